@@ -119,6 +119,9 @@ void release_derived(Ctx &c) {
         b->release();
     for (DBuf<int> *b : {&c.sp_slot, &c.sp_ndx, &c.sp_edge, &c.sp_av, &c.sp_nbr, &c.sp_lab, &c.sp_pos, &c.sp_ndf})
         b->release();
+    for (DBuf<uint64_t> *b : {&c.join_box, &c.join_leaf, &c.join_tile}) b->release();
+    c.join_ctl.release();
+    c.joined = false;
     for (DBuf<YRangeF> *b : {&c.eyr, &c.lend_yr, &c.cov_yr}) b->release();
     c.lend_bl.release();
     c.ep_lohi.release();
@@ -179,17 +182,15 @@ int need_space(int64_t n, int64_t cap, int64_t *need) {
     return n > cap ? SEGCLIP_ESPACE : SEGCLIP_OK;
 }
 
+// a clip's candidate pairs need no tree: build it for calls that show it
+int need_tree(segclip_ctx *h) {
+    if (!h->c.joined) return SEGCLIP_OK;
+    return guarded(h, [](sc::Ctx &x) { sc::tree_after_join(x); });
+}
+
 template <class T> void d2h(sc::Ctx &c, T *dst, const T *src, int64_t n) {
     if (n <= 0) return;
     SC_HIP(hipMemcpyAsync(dst, src, sizeof(T) * size_t(n), hipMemcpyDeviceToHost, c.stream));
-}
-
-void tree_all(sc::Ctx &c) {
-    sc::build_edges(c);
-    sc::build_elementary(c);
-    sc::build_node_intervals(c);
-    sc::build_leaf_end_entries(c);
-    sc::build_cover_lists(c);
 }
 
 } // namespace
@@ -251,25 +252,44 @@ int segclip_set_pairs_device(segclip_ctx *h, const double *b, const int *bsz, co
 }
 int segclip_build_elementary(segclip_ctx *h) {
     return guarded(h, [&](sc::Ctx &x) {
-        sc::build_edges(x);
-        sc::build_elementary(x);
+        if (x.joined && x.T == 0) {
+            sc::build_tree(x); // the later stages' results show with it, as after any clip
+        } else {
+            sc::build_edges(x);
+            sc::build_elementary(x);
+        }
     });
 }
 int segclip_build_node_intervals(segclip_ctx *h) {
-    return guarded(h, [&](sc::Ctx &x) { sc::build_node_intervals(x); });
+    return guarded(h, [&](sc::Ctx &x) {
+        sc::tree_after_join(x);
+        sc::build_node_intervals(x);
+    });
 }
 int segclip_build_end_lists(segclip_ctx *h) {
-    return guarded(h, [&](sc::Ctx &x) { sc::build_leaf_end_entries(x); });
+    return guarded(h, [&](sc::Ctx &x) {
+        sc::tree_after_join(x);
+        sc::build_leaf_end_entries(x);
+    });
 }
 int segclip_build_cover_lists(segclip_ctx *h) {
-    return guarded(h, [&](sc::Ctx &x) { sc::build_cover_lists(x); });
+    return guarded(h, [&](sc::Ctx &x) {
+        sc::tree_after_join(x);
+        sc::build_cover_lists(x);
+    });
 }
 int segclip_materialize_end_lists(segclip_ctx *h) {
-    return guarded(h, [&](sc::Ctx &x) { sc::materialize_end_lists(x); });
+    return guarded(h, [&](sc::Ctx &x) {
+        sc::tree_after_join(x);
+        sc::materialize_end_lists(x);
+    });
 }
-int segclip_build_tree(segclip_ctx *h) { return guarded(h, [&](sc::Ctx &x) { tree_all(x); }); }
+int segclip_build_tree(segclip_ctx *h) { return guarded(h, [&](sc::Ctx &x) { sc::build_tree(x); }); }
 int segclip_find_candidates(segclip_ctx *h) {
-    return guarded(h, [&](sc::Ctx &x) { sc::find_candidates(x); });
+    return guarded(h, [&](sc::Ctx &x) {
+        sc::tree_after_join(x);
+        sc::find_candidates(x);
+    });
 }
 int segclip_intersections(segclip_ctx *h, int k) {
     int rc = guarded(h, [&](sc::Ctx &x) { sc::post_overlay(x, k); });
@@ -385,6 +405,7 @@ int segclip_reset(segclip_ctx *h) {
         x.n_lend = x.n_cov = x.n_cand = x.n_pairs = x.n_mend = x.n_near = 0;
         x.cur_k = 0;
         x.pair_off.clear();
+        x.joined = false;
         x.jobs.J = 0;
         x.jobs.AB.clear();
         x.jobs.ring_off.clear();
@@ -424,7 +445,10 @@ int segclip_copy_batch_status(segclip_ctx *h, int32_t *status, int64_t cap, int6
 
 int segclip_get_counts(segclip_ctx *h, segclip_counts *o) {
     if (!h || !o) return SEGCLIP_EINVAL;
-    int frc = guarded(h, [&](sc::Ctx &x) { sc::fetch_flags(x); });
+    int frc = guarded(h, [&](sc::Ctx &x) {
+        sc::fetch_flags(x);
+        sc::stab_after_join(x); // the tree's and the stab's sizes are part of the answer
+    });
     if (frc != SEGCLIP_OK) return frc;
     const sc::Ctx &c = h->c;
     std::memset(o, 0, sizeof(*o));
@@ -451,6 +475,7 @@ int segclip_get_counts(segclip_ctx *h, segclip_counts *o) {
 
 int segclip_copy_elementary(segclip_ctx *h, double *out, int64_t cap, int64_t *need) {
     if (!h) return SEGCLIP_EINVAL;
+    if (int trc = need_tree(h)) return trc;
     int rc = need_space(h->c.epc, cap, need);
     if (rc || !out) return rc;
     return guarded(h, [&](sc::Ctx &c) {
@@ -461,6 +486,7 @@ int segclip_copy_elementary(segclip_ctx *h, double *out, int64_t cap, int64_t *n
 
 int segclip_copy_node_intervals(segclip_ctx *h, double *out, int64_t cap, int64_t *need) {
     if (!h) return SEGCLIP_EINVAL;
+    if (int trc = need_tree(h)) return trc;
     int rc = need_space(2 * int64_t(h->c.T), cap, need);
     if (rc || !out) return rc;
     return guarded(h, [&](sc::Ctx &c) {
@@ -471,6 +497,7 @@ int segclip_copy_node_intervals(segclip_ctx *h, double *out, int64_t cap, int64_
 
 int segclip_copy_cover_lists(segclip_ctx *h, uint32_t *off, uint32_t *edges, int64_t cap, int64_t *need) {
     if (!h) return SEGCLIP_EINVAL;
+    if (int trc = need_tree(h)) return trc;
     int rc = need_space(h->c.n_cov, cap, need);
     if (rc || !off || !edges) return rc;
     return guarded(h, [&](sc::Ctx &c) {
@@ -493,6 +520,7 @@ int segclip_copy_end_lists(segclip_ctx *h, uint32_t *off, uint32_t *edges, int64
 
 int segclip_copy_leaf_targets(segclip_ctx *h, int32_t *after, int32_t *before, int64_t cap, int64_t *need) {
     if (!h) return SEGCLIP_EINVAL;
+    if (int trc = need_tree(h)) return trc;
     int rc = need_space(h->c.ne, cap, need);
     if (rc || !after || !before) return rc;
     return guarded(h, [&](sc::Ctx &c) {

@@ -47,6 +47,8 @@ struct Ctx {
     std::vector<int> eoff;          // overlay edge offsets in the edge index space (K+1), eoff[0] = nb
     DBuf<double> bpoly, cpoly;      // (nb+nbr)*2, (nct+K)*2
     DBuf<int> d_coff, d_eoff, d_bvoff, d_beoff;
+    std::vector<int> loff;          // first leaf (64 consecutive edges) of every base ring, then of every overlay
+    DBuf<int> d_loff;
     DBuf<double> d_shift;           // per base/overlay ring x shift of the tree keys (paired mode)
     // per-edge SoA (edge index e in [0,ne): base edges, then overlay 1, 2, ...)
     DBuf<double> ex0, ey0, ex1, ey1; // endpoints in ring order
@@ -86,6 +88,12 @@ struct Ctx {
     DBuf<YRangeF> cov_yr;                // the edge's single-precision y-extent, beside each cover entry
     DBuf<uint64_t> cov_key, cov_key_alt; // (node, class) << 32 | edge sort keys, and their sort partner
     int64_t n_cov = 0;
+    // ---- box join (sc_join.hip): the pairs of a clip without the tree ----
+    bool joined = false;                 // pairs come from the join: no tree, no stab counts
+    DBuf<uint64_t> join_box, join_leaf;  // boxes of leaves and base groups; first vertex, size, edge, ring of leaves
+    DBuf<uint64_t> join_tile;            // (base leaf, overlay leaf) tiles in segments of join_seg_cap entries
+    DBuf<uint32_t> join_ctl;             // totals, flag, segment counters
+    int64_t join_seg_cap = 0;
     // ---- A8/A10 candidates and unique pairs ----
     DBuf<uint64_t> unit_desc;            // stab work units: 32-byte records
     DBuf<uint64_t> cand;                 // packed (k, b, c) keys
@@ -181,7 +189,7 @@ struct Ctx {
 
     bool timing = false;
     StageTimes times;
-    hipEvent_t ev[10] = {};
+    hipEvent_t ev[11] = {};
     bool ev_ready = false;
     void ensure_events();
     bool flags_pending = false; // jobs.flags / undefined still on the device
@@ -211,6 +219,15 @@ void build_leaf_end_entries(Ctx &c);
 void materialize_end_lists(Ctx &c);
 void build_cover_lists(Ctx &c);
 void find_candidates(Ctx &c);          // all overlays at once, then unique pairs
+// the same pairs from bounding boxes alone (no tree); false: rings that the
+// tree must pair (vertical edges, coordinates without an order), nothing done
+bool join_candidates(Ctx &c);
+void pair_offsets(Ctx &c);             // pair_off of c.n_pairs sorted pairs
+// after a clip whose pairs came from the join: the tree (tree_after_join), and
+// the stab's counts as well (stab_after_join), for calls that show them
+void build_tree(Ctx &c);
+void tree_after_join(Ctx &c);
+void stab_after_join(Ctx &c);
 void post_jobs(Ctx &c, int k0, int k1); // A11-A15 for overlays k0..k1 in one batch
 // the batch's per-job flags (jobs.flags, undefined) from the device, when the
 // post stage left them there (labelling fetches them with its first read-back)

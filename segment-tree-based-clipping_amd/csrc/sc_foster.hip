@@ -2862,7 +2862,12 @@ void clip_jobs(Ctx &c, int k0, int k1) {
             return;
         }
     }
-    const bool tree = c.T == 0, cand = tree || int(c.pair_off.size()) != c.K + 1;
+    // candidate pairs: from the box join, or from the tree where the join
+    // refuses the rings or the tree is already there with its own pairs
+    const bool cand = int(c.pair_off.size()) != c.K + 1;
+    c.mark(10);
+    const bool joined = cand && join_candidates(c);
+    const bool tree = cand && !joined && c.T == 0;
     c.mark(0);
     if (tree) {
         build_edges(c);
@@ -2875,7 +2880,7 @@ void clip_jobs(Ctx &c, int k0, int k1) {
     c.mark(3);
     if (tree) build_cover_lists(c);
     c.mark(4);
-    if (cand) find_candidates(c);
+    if (cand && !joined) find_candidates(c);
     c.mark(5);
     post_jobs(c, k0, k1);
     c.mark(6);
@@ -2887,7 +2892,7 @@ void clip_jobs(Ctx &c, int k0, int k1) {
         t.tree = c.elapsed(1, 2);
         t.endlist = c.elapsed(2, 3);
         t.cover = c.elapsed(3, 4);
-        t.candidates = c.elapsed(4, 5);
+        t.candidates = c.elapsed(joined ? 10 : 4, 5);
         t.stab_kernel = cand ? c.elapsed(8, 9) : 0.0f;
         t.post = c.elapsed(5, 6);
         t.label = c.elapsed(6, 7);

@@ -28,6 +28,7 @@
 // in the same pass: a pair key carries the overlay.
 #include "sc_ctx.hpp"
 #include "sc_fp64.hpp"
+#include "sc_wave.hpp"
 
 namespace sc {
 
@@ -223,46 +224,6 @@ struct StabArgs {
     uint64_t cap;
     unsigned long long *counter;              // NEAR_SEGS counters, NEAR_PAD apart
 };
-
-// value of lane 'src' broadcast to the wave (src is uniform)
-__device__ inline double bcast(double v, int src) {
-    long long b = __double_as_longlong(v);
-    int lo = __builtin_amdgcn_readlane(int(b), src);
-    int hi = __builtin_amdgcn_readlane(int(b >> 32), src);
-    return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
-}
-__device__ inline uint32_t uni(uint32_t v) { return uint32_t(__builtin_amdgcn_readfirstlane(int(v))); }
-
-// Wave-wide reductions (every lane active): four DPP steps combine the 16
-// lanes of each row (quad swaps, half-row and row mirrors), four reads of
-// lanes 0/16/32/48 combine the rows.
-template <class Op> __device__ inline uint32_t wave_reduce(uint32_t v, Op op) {
-    v = op(v, uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0xB1, 0xF, 0xF, false))); // quad_perm 1,0,3,2
-    v = op(v, uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x4E, 0xF, 0xF, false))); // quad_perm 2,3,0,1
-    v = op(v, uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x141, 0xF, 0xF, false))); // row_half_mirror
-    v = op(v, uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x140, 0xF, 0xF, false))); // row_mirror
-    const uint32_t a = uint32_t(__builtin_amdgcn_readlane(int(v), 0)), b = uint32_t(__builtin_amdgcn_readlane(int(v), 16));
-    const uint32_t c = uint32_t(__builtin_amdgcn_readlane(int(v), 32)), d = uint32_t(__builtin_amdgcn_readlane(int(v), 48));
-    return op(op(a, b), op(c, d));
-}
-__device__ inline uint32_t wave_or32(uint32_t v) {
-    return wave_reduce(v, [](uint32_t x, uint32_t y) { return x | y; });
-}
-// min / max of floats through an order-preserving integer key (NaN excluded:
-// callers handle NaN extents before)
-__device__ inline int fkey(float f) {
-    const int b = __float_as_int(f);
-    return b ^ ((b >> 31) & 0x7fffffff);
-}
-__device__ inline float funkey(int k) { return __int_as_float(k ^ ((k >> 31) & 0x7fffffff)); }
-__device__ inline float wave_min(float v) {
-    auto f = [](uint32_t x, uint32_t y) { return uint32_t(min(int(x), int(y))); };
-    return funkey(int(wave_reduce(uint32_t(fkey(v)), f)));
-}
-__device__ inline float wave_max(float v) {
-    auto f = [](uint32_t x, uint32_t y) { return uint32_t(max(int(x), int(y))); };
-    return funkey(int(wave_reduce(uint32_t(fkey(v)), f)));
-}
 
 // y-bins of a unit: the span [ulo, uhi] of its rows' y-extents cut into 32
 // bins.  bin_of is monotone in y (a subtraction and a multiplication by a
@@ -709,12 +670,12 @@ __global__ void k_compact_unique(const uint64_t *__restrict__ k, const uint32_t 
 }
 
 // first unique pair of every overlay k (pairs are sorted by overlay first)
-// koff[k] = first pair of overlay k; the pair count is read on the device
-__global__ void k_overlay_offsets(const uint64_t *__restrict__ pairs, const uint32_t *__restrict__ npairs, int K,
-                                  int sh, uint32_t *off) {
+// koff[k] = first pair of overlay k; the pair count is read on the device when npairs is given
+__global__ void k_overlay_offsets(const uint64_t *__restrict__ pairs, const uint32_t *__restrict__ npairs, int64_t n,
+                                  int K, int sh, uint32_t *off) {
     int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k > K + 1) return;
-    int64_t lo = 0, hi = int64_t(*npairs);
+    int64_t lo = 0, hi = npairs ? int64_t(*npairs) : n;
     while (lo < hi) {
         int64_t mid = (lo + hi) >> 1;
         if (int64_t(pairs[mid] >> sh) < k) lo = mid + 1;
@@ -896,7 +857,7 @@ void find_candidates(Ctx &c) {
         k_compact_unique<<<grid_for(n), BLK, 0, s>>>(c.cand, flag, n, c.pairs);
         SC_HIP(hipGetLastError());
     }
-    k_overlay_offsets<<<grid_for(int64_t(c.K) + 2), BLK, 0, s>>>(c.pairs, tot, c.K, c.bits_b + c.bits_c, koff);
+    k_overlay_offsets<<<grid_for(int64_t(c.K) + 2), BLK, 0, s>>>(c.pairs, tot, 0, c.K, c.bits_b + c.bits_c, koff);
     SC_HIP(hipGetLastError());
     // koff[k] = first pair of overlay k (k = 1..K+1): pairs of overlay k are [koff[k], koff[k+1])
     std::vector<uint32_t> h(size_t(c.K) + 2);
@@ -909,6 +870,22 @@ void find_candidates(Ctx &c) {
     }
     c.n_pairs = np;
     c.pair_off.assign(size_t(c.K) + 1, 0);
+    for (int k = 1; k <= c.K; ++k) c.pair_off[k] = h[k + 1];
+    c.joined = false;
+}
+
+void pair_offsets(Ctx &c) {
+    c.pair_off.assign(size_t(c.K) + 1, 0);
+    c.pair_off[c.K] = c.n_pairs;
+    if (c.K == 1) return;
+    uint32_t *koff = c.d_pair_off.ensure(size_t(c.K) + 2);
+    k_overlay_offsets<<<grid_for(int64_t(c.K) + 2), BLK, 0, c.stream>>>(c.pairs, nullptr, c.n_pairs, c.K,
+                                                                       c.bits_b + c.bits_c, koff);
+    SC_HIP(hipGetLastError());
+    std::vector<uint32_t> h(size_t(c.K) + 2);
+    ReadBack rb(c);
+    rb.add(h.data(), static_cast<const uint32_t *>(koff), h.size());
+    rb.run();
     for (int k = 1; k <= c.K; ++k) c.pair_off[k] = h[k + 1];
 }
 

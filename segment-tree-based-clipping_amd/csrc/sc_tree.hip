@@ -506,6 +506,7 @@ void reset_derived(Ctx &c) {
     c.n_lend = c.n_cov = c.n_cand = c.n_pairs = c.n_mend = c.n_near = 0;
     c.cur_k = 0;
     c.pair_off.clear();
+    c.joined = false;
 }
 
 void load(Ctx &c, const double *bxy, const int *bsz, int nbr, const double *cxy, const int *csz, int K,
@@ -548,6 +549,11 @@ void load(Ctx &c, const double *bxy, const int *bsz, int nbr, const double *cxy,
         c.eoff[i + 1] = c.eoff[i] + csz[i];
         c.maxcsz = std::max(c.maxcsz, csz[i]);
     }
+    c.loff.assign(size_t(nbr) + K + 1, 0);
+    for (int i = 0; i < nbr + K; ++i)
+        c.loff[i + 1] = c.loff[i] + int(ceil_div(i < nbr ? bsz[i] : csz[i - nbr], WAVE));
+    SC_HIP(hipMemcpyAsync(c.d_loff.ensure(c.loff.size()), c.loff.data(), sizeof(int) * c.loff.size(),
+                          hipMemcpyHostToDevice, c.stream));
     layout_rings(c, bxy, nb, c.bsz, c.bvoff, c.d_bvoff, c.beoff, 0, c.d_beoff, c.bpoly, device_ptrs);
     layout_rings(c, cxy, nct, c.csz, c.coff, c.d_coff, c.eoff, c.nb, c.d_eoff, c.cpoly, device_ptrs);
     if (paired) {
@@ -779,6 +785,24 @@ void build_cover_lists(Ctx &c) {
     scan_inclusive_max_u32(off + 1, off + 1, T, s);
     k_cover_split<<<grid_for(T), BLK, 0, s>>>(T, off, bend, split);
     SC_HIP(hipGetLastError());
+}
+
+void build_tree(Ctx &c) {
+    build_edges(c);
+    build_elementary(c);
+    build_node_intervals(c);
+    build_leaf_end_entries(c);
+    build_cover_lists(c);
+}
+
+void tree_after_join(Ctx &c) {
+    if (c.joined && c.T == 0) build_tree(c);
+}
+
+void stab_after_join(Ctx &c) {
+    if (!c.joined) return;
+    tree_after_join(c);
+    find_candidates(c); // the same pairs again, with the stab's counts
 }
 
 void materialize_end_lists(Ctx &c) {
