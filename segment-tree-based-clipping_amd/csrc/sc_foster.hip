@@ -40,6 +40,7 @@
 // as g, a Q slot g as ~g, none as SRC_NONE) for the area gradient.
 #include "sc_ctx.hpp"
 #include "sc_fp64.hpp"
+#include "sc_seqroute.hpp"
 
 #include <algorithm>
 #include <climits>
@@ -55,20 +56,10 @@ inline unsigned grid_for(int64_t n, int per = BLK) {
     return unsigned(g);
 }
 
-enum : int {
-    L_NONE = 0, L_CROSSING = 1, L_BOUNCING = 2, L_LEFT_ON = 3, L_RIGHT_ON = 4, L_ON_ON = 5,
-    L_ON_LEFT = 6, L_ON_RIGHT = 7, L_DCROSS = 8, L_DBOUNCE = 9
-};
-enum : int { EXIT = 0, ENTRY = 1, NEITHER = 2 };
-enum : int { UB_TRAVERSAL = 4 };
-constexpr int SRC_NONE = INT_MIN;
-
 // reasons for taking the sequential route
 enum : int { SLOW_LABEL = 1, SLOW_NOPLAIN = 2, SLOW_ODD = 4, SLOW_SPLIT = 8, SLOW_LINK = 16, SLOW_UNION = 32 };
 // routes
 enum : int { K_CROSS = 0, K_NOCROSS = 1, K_SEQ = 2 };
-
-constexpr uint32_t NIL = 0xffffffffu;
 
 // one side (all P rings or all Q rings) of a batch
 struct Side {
@@ -1058,8 +1049,6 @@ __device__ inline int seq_src(const SeqArgs &a, int V) {
     return V < a.nP ? a.P0 + a.vslot[V] : ~(a.Q0 + a.vslot[V]);
 }
 
-__device__ int seq_toggle(int s) { return s == ENTRY ? EXIT : (s == EXIT ? ENTRY : s); }
-
 // node records -> the job's linked rings (all threads of the block)
 // createResult2's walks, one per lane (see seq_run).  Returns PT_DONE with
 // rings/outn advanced and the rings written, PT_FAIL when the single walk
@@ -1412,17 +1401,6 @@ __device__ __attribute__((always_inline)) int seq_par_traverse(SeqArgs &a, SeqSh
     return PT_DONE;
 }
 
-// the entry/exit walk's state (status, first of a delayed pair) as 2 bits
-// x = st | first << 1 (EXIT = 0, ENTRY = 1); a node's effect on it is a
-// 4-entry table of 2-bit states, and tables compose along the ring
-__device__ inline int seq_tapply(uint32_t t, int x) { return int((t >> (2 * x)) & 3u); }
-__device__ inline uint32_t seq_tcompose(uint32_t f, uint32_t g) { // f first, then g
-    uint32_t h = 0;
-#pragma unroll
-    for (int x = 0; x < 4; ++x) h |= ((g >> (2 * ((f >> (2 * x)) & 3u))) & 3u) << (2 * x);
-    return h;
-}
-
 // The entry/exit walks of the rings marked in sh.scan, on every thread of the
 // block: ring s from the node after sh.sV[s] around to sh.sV[s], WAVE x
 // waves nodes per round.  Each wave scans its nodes' tables, the waves'
@@ -1455,13 +1433,7 @@ __device__ __attribute__((always_inline)) void seq_enex_block(SeqArgs &a, SeqSha
                 lab = a.lab[I];
                 it = a.inter[I] != 0;
             }
-            uint32_t tab = 0xE4u; // identity
-            if (it) {
-                if (lab == L_CROSSING) tab = 0xB1u;     // status toggles
-                else if (lab == L_DCROSS) tab = 0x4Bu;  // first: clear it; else set it, toggle
-                else if (lab == L_DBOUNCE) tab = 0x1Bu; // first flips, status toggles
-            }
-            uint32_t P = tab;
+            uint32_t P = it ? seq_table(lab) : SEQ_TAB_ID;
             for (int d = 1; d < WAVE; d <<= 1) {
                 const uint32_t o = uint32_t(__shfl_up(int(P), d, WAVE));
                 if (lane >= d) P = seq_tcompose(o, P);
@@ -2003,36 +1975,10 @@ done:
 }
 
 
-// sequential route for several jobs: one block per job, its first wave runs seq_run
-struct SeqJob {
-    int j;                     // job
-    int nP, nQ, P0, Q0;        // ring sizes (slots) and first slots in the dense ring arrays
-    int node0, nPn, nQn;       // first node, node counts of P and Q
-    int cap, out_cap, ring_cap;
-    int64_t vbase, obase, rbase; // scratch bases: vertices, output vertices, ring offsets
-};
-
-struct SeqBatch {
-    const SeqJob *jobs;
-    const double *px, *py, *qx, *qy;
-    const double *nx0, *ny0, *nx1, *ny1;
-    const int *nlen, *nslot, *ninter, *nlab, *nnb;
-    const int *windP, *windQ;
-    double *vx, *vy, *vx1, *vy1;
-    int *vlen, *vslot, *nx, *pv, *nb, *lab, *enex, *vsrc, *cand, *seen;
-    uint8_t *inter;
-    int4 *rec;
-    int *pstep;
-    int2 *emit;
-    double *ox, *oy;
-    int *osrc, *ring_off, *result;
-    int uni;
-    int par;
-};
-
 // one block per sequential job: its threads lay out the rings, its first wave
 // runs the algorithm (no barrier after that point)
 __global__ __launch_bounds__(SEQ_BLK) void k_sequential(SeqBatch b) {
+    if (b.done && b.done[blockIdx.x]) return;
     const SeqJob jb = b.jobs[blockIdx.x];
     SeqArgs a;
     a.nP = jb.nPn;
@@ -2090,6 +2036,7 @@ __global__ __launch_bounds__(SEQ_BLK) void k_sequential(SeqBatch b) {
 // Every sequential job's working rings before any insertion: its P and Q
 // rings in node order (node v of the job at slot vbase + v), nothing
 // inserted, no walk state.  Job q owns nodes [nodeoff[2q], nodeoff[2q+2]).
+// Again before k_sequential for the jobs that the device-wide steps left.
 __global__ void k_seq_init(SeqBatch b, const int64_t *__restrict__ nodeoff, int nseq, int64_t N) {
     const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (t >= N) return;
@@ -2099,9 +2046,12 @@ __global__ void k_seq_init(SeqBatch b, const int64_t *__restrict__ nodeoff, int 
         if (nodeoff[2 * mid] <= t) lo = mid;
         else hi = mid - 1;
     }
+    if (b.done && b.done[lo]) return;
     const SeqJob &jb = b.jobs[lo];
     const int v = int(t - jb.node0);
     const int64_t w = jb.vbase + v;
+    b.seen[2 * w] = 0;
+    b.seen[2 * w + 1] = 0;
     b.vx[w] = b.nx0[t];
     b.vy[w] = b.ny0[t];
     b.vx1[w] = b.nx1[t];
@@ -2216,9 +2166,10 @@ __global__ void k_node_finish(NodeArgs a, int64_t N, const int64_t *nodeoff, con
 }
 
 // rings of the sequential jobs into the batch output (one block per job)
-__global__ void k_jseq_copy(const SeqJob *jobs, const int *result, const uint32_t *JV, const uint32_t *JR,
+__global__ void k_jseq_copy(const SeqJob *jobs, const int *done, const int *result, const uint32_t *JV, const uint32_t *JR,
                             const double *sx, const double *sy, const int *ssrc, const int *sroff, double *ox,
                             double *oy, int *osrc, int *off) {
+    if (done && done[blockIdx.x]) return; // written by walk_emit
     const SeqJob jb = jobs[blockIdx.x];
     const int rings = result[3 * blockIdx.x], verts = result[3 * blockIdx.x + 1];
     const int64_t o = JV[jb.j];
@@ -2259,6 +2210,7 @@ struct FosterScratch {
     DBuf<uint32_t> jmoved; // per doubling round: some cycle minimum moved
     DBuf<int> spstep;
     DBuf<int2> semit;
+    DBuf<int> sdone;
 };
 
 FosterScratch &fscratch() {
@@ -2398,6 +2350,8 @@ void release_foster_scratch() {
     f.srec.release();
     f.spstep.release();
     f.semit.release();
+    f.sdone.release();
+    release_walk_scratch();
     f.jrec.release();
     f.kstatus.release();
     f.jrec2.release();
@@ -2578,6 +2532,9 @@ void label_and_traverse(Ctx &c) {
     // sequential route
     const int nseq = int(seq_jobs.size());
     std::vector<SeqJob> sj(static_cast<size_t>(nseq));
+    WalkIn wi;
+    int *done = nullptr; // per sequential job: run by walk_jobs
+    bool walked = false;
     if (nseq > 0) {
         std::vector<int> hsidx(static_cast<size_t>(J), -1);
         int64_t mb = 0;
@@ -2602,6 +2559,7 @@ void label_and_traverse(Ctx &c) {
         SC_HIP(hipMemcpyAsync(sidx, hsidx.data(), sizeof(int) * J, hipMemcpyHostToDevice, s));
         SeqBatch b;
         b.jobs = djobs;
+        b.done = nullptr;
         b.uni = c.uni;
         b.par = c.seq_par;
         b.px = c.aug_bx; b.py = c.aug_by; b.qx = c.aug_cx; b.qy = c.aug_cy;
@@ -2701,6 +2659,28 @@ void label_and_traverse(Ctx &c) {
         c.ensure_side_stream();
         SC_HIP(hipEventRecord(c.ev_fork, s));
         SC_HIP(hipStreamWaitEvent(c.stream2, c.ev_fork, 0));
+        if (c.seq_par) {
+            wi.b = b;
+            wi.jobs = &sj;
+            wi.nodeoff = dnodeoff;
+            wi.segoff = dseg;
+            wi.nidx = nidx;
+            wi.N = N;
+            wi.firstP = st.firstP;
+            wi.firstQ = st.firstQ;
+            done = f.sdone.ensure(nseq);
+            {
+                FillBatch fb(c.stream2);
+                fb.add(done, nseq, 0u);
+                fb.flush();
+            }
+            walked = walk_jobs(wi, done, c.stream2);
+            if (walked) { // the others from their initial state
+                b.done = done;
+                k_seq_init<<<grid_for(N), BLK, 0, c.stream2>>>(b, dnodeoff, nseq, N);
+                SC_HIP(hipGetLastError());
+            }
+        }
         k_sequential<<<nseq, SEQ_BLK, 0, c.stream2>>>(b);
         SC_HIP(hipGetLastError());
         SC_HIP(hipEventRecord(c.ev_join, c.stream2));
@@ -2821,7 +2801,8 @@ void label_and_traverse(Ctx &c) {
     }
     std::vector<int> hres(3 * size_t(nseq));
     if (nseq > 0) {
-        k_jseq_copy<<<nseq, BLK, 0, s>>>(f.sjobs, f.sres, jv, jr, f.sox, f.soy, f.sosrc, f.sroff, f.ox, f.oy,
+        if (walked) walk_emit(wi, done, jv, jr, f.ox, f.oy, f.osrc, off, s);
+        k_jseq_copy<<<nseq, BLK, 0, s>>>(f.sjobs, walked ? done : nullptr, f.sres, jv, jr, f.sox, f.soy, f.sosrc, f.sroff, f.ox, f.oy,
                                           f.osrc, off);
         SC_HIP(hipGetLastError());
     }
