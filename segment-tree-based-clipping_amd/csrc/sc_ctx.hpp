@@ -146,6 +146,7 @@ struct Ctx {
     DBuf<double> d_ring_x, d_ring_y;
     DBuf<int> d_ring_src;                // provenance of each output vertex (P slot g, Q slot ~g)
     int64_t n_out = 0;
+    DBuf<uint64_t> out_xy;               // a piece of the output on its way to the host
     int undefined = 0;                   // bitmask like the oracle's status
 
     // scratch
@@ -268,6 +269,7 @@ void arr_init_labels(Ctx &c, int nba, int nca, const double *inter_b, const doub
 void init_labels_one(Ctx &c, int nba, int nca, const double *bx, const double *by, const int *avb, const int *nbrb,
                      const double *cx, const double *cy, int *labb, int *labc, int *flags);
 void release_foster_scratch();
+void rings_to_host(Ctx &c, int32_t *ring_off, double *xy); // ring offsets and x,y pairs of the last result
 
 // Device-to-host read-backs through the context's pinned staging, one wait
 // for all of them: add() up to RB_MAX pieces, then run().

@@ -77,7 +77,9 @@ struct WalkIn {
     int64_t N;                       // nodes of all jobs
     const int *firstP, *firstQ;      // per batch job: first plain slot of each ring
 };
-constexpr int WALK_MIN_NODES = 2048;
+// below, one block per job is as fast: on unions of 300 nodes 0.99 ms a clip against
+// 0.98 device-wide, of 1,000 nodes 1.22 against 0.98 (the launches cost 0.15 ms)
+constexpr int WALK_MIN_NODES = 512;
 bool walk_jobs(const WalkIn &in, int *done, hipStream_t s); // false: no job is large enough
 void walk_emit(const WalkIn &in, const int *done, const uint32_t *JV, const uint32_t *JR, double *ox, double *oy,
                int *osrc, int *off, hipStream_t s);
