@@ -694,245 +694,210 @@ __global__ void k_root_loop(int nr, const int *off, const double *x, const doubl
     rstart[r] = root;
 }
 
-// keep0 keeps the decisions (bytes) for the clean-up rounds: a vertex whose
-// last kept predecessor is the vertex before it is decided exactly so again
-__global__ void k_keep0(int64_t n, const int *ringid, const int *off, const int *rstart, const double *x,
-                        const double *y, uint32_t *keep, uint8_t *keep0) {
-    int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    int r = ringid[i];
-    int rs = rstart[r], last = off[r + 1] - 1;
-    uint32_t k;
-    if (i < rs) k = 0;
-    else if (i == rs) k = 1;
-    else {
-        int nx = i == last ? rs : int(i) + 1;
-        k = collinear(x, y, int(i) - 1, int(i), nx) ? 0u : 1u;
-    }
-    keep[i] = k;
-    keep0[i] = uint8_t(k);
-}
+// Which vertices stay.  In a ring, the vertices before its root go, the root
+// stays, and a later vertex stays unless it is collinear with the last vertex
+// kept before it and its successor (the root, for the ring's last vertex).
+// One wave decides a span from left to right, 64 vertices a window: while the
+// vertex before is kept a vertex's decision needs only its two neighbours (k0,
+// all lanes at once), so a step goes to the next vertex dropped that way;
+// after a drop the last kept vertex L is fixed until the next kept one, so one
+// step tests all later lanes against L.  A step is one test per lane and a
+// ballot, however long the run of dropped vertices is.  Rounds that each let
+// one more vertex of every run see its last kept vertex took 6 launches of 15
+// us on 1.4 M vertices, and 48 of 54 us and then 6.4 ms of one lane per ring on
+// 27 M (short edges drop in long runs); now 39 us and 0.26 ms.
+constexpr int KEEP_WIN = 4;                  // windows per tile, their loads issued together
+constexpr int KEEP_TILE = KEEP_WIN * WAVE;
+constexpr int KEEP_ROUNDS = 50;              // rounds before one wave per ring
+constexpr uint32_t KEEP_ANY = 0xffffffffu;   // the tile's first vertex needs no vertex before it
 
-// One clean-up round in one launch.  A vertex after its ring's root stays
-// unless it is collinear with the last vertex kept before it (under the
-// previous round's flags) and its successor (the root, for the ring's last
-// vertex); the rounds repeat until no flag changes.
-// Tile t is block t.  A block waits only for tiles of lower index, and every
-// XCD dispatches its blocks in index order, so the lowest block not yet
-// dispatched waits for nothing that does not finish: every wait ends (and a
-// wait is also bounded, reported as an error).  A ticket counter instead of
-// the block index costs one contended atomic per tile.  A tile publishes the
-// largest mark (kept index + 1) among its vertices under the previous round's
-// flags; wave 0 then walks back over earlier tiles' words, 64 per round trip,
-// until one carries an inclusive prefix.  Each vertex so learns the last
-// vertex kept before it and its new flag is written in place: a tile reads
-// only its own flags, other tiles' only through the published words.
-constexpr int KEEP_ITEMS = 8;
-constexpr int KEEP_TILE = BLK * KEEP_ITEMS;
-constexpr int KEEP_ROUNDS = 48;                // rounds before the exact sequential pass
-constexpr int KEEP_BATCH = 3;                  // rounds launched per convergence check
-constexpr int KEEP_SPIN_LIMIT = 1 << 20;       // polls of a predecessor window before giving up
-constexpr int KS_EPOCH_SHIFT = 56;             // status word: epoch | flag | value
-constexpr unsigned long long KS_PRE = 1ull << 54, KS_VAL = 0xffffffffull;
-
-struct KeepRound {
+struct KeepArgs {
     int64_t n;
     const int *ringid, *off, *rstart;
     const double *x, *y;
     uint32_t *keep;
-    const uint8_t *keep0;       // k_keep0's decisions (predecessor = the vertex before)
-    unsigned long long *status; // per tile; no word carries this round's epoch before the launch
-    unsigned long long epoch;   // 1..KEEP_ROUNDS, shifted into place
-    uint32_t *changed;          // set when a flag changes
-    uint32_t *err;              // set when a wait gives up (the result is then invalid)
-    uint32_t *tstate;           // per tile: flags changed in its last round, the prefix that round saw, its largest mark
-    int first;                  // the first round: every tile decides
+    uint32_t *used;      // per tile: the mark (last kept index + 1) before it that it was decided with
+    const uint32_t *last; // per tile, previous round: its last kept index + 1, 0 for none
+    uint32_t *last_out;
+    uint32_t *changed;   // per round: some tile's last kept vertex moved
+    int64_t ntiles;
 };
 
-__global__ __launch_bounds__(BLK) void k_keep_round(KeepRound a) {
-    __shared__ uint32_t s_prefix, s_skip, s_ch, s_fast, s_agg;
-    __shared__ uint32_t s_wmax[BLK / WAVE];
-    const int tid = threadIdx.x, lane = tid & (WAVE - 1), w = tid / WAVE;
-    const uint32_t tile = blockIdx.x;
-    const int64_t i0 = int64_t(tile) * KEEP_TILE + int64_t(tid) * KEEP_ITEMS;
-    // a tile whose flags did not change in its last round still has the
-    // largest mark it computed then: it publishes that without reading its
-    // flags, and reads them only if its incoming prefix changed
-    if (tid == 0) {
-        const bool f = !a.first && a.tstate[3 * tile] == 0u;
-        s_fast = f ? 1u : 0u;
-        s_agg = f ? a.tstate[3 * tile + 2] : 0u;
+__device__ inline double lane_value(double v, int l) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_readlane(int(b), l), hi = __builtin_amdgcn_readlane(int(b >> 32), l);
+    return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
+}
+
+// vertices [base, min(base + NW * 64, end)), flags written from 'out' (a window's
+// start) on; mark: last kept index + 1 before base.  Returns the span's last
+// kept index + 1, or mark; used: the mark before 'out', KEEP_ANY when the vertex
+// there needs none.  Run by a whole wave, uniform arguments.
+template <int NW>
+__device__ inline uint32_t keep_span(const KeepArgs &a, int64_t base, int64_t out, int64_t end, uint32_t mark,
+                                     uint32_t &used) {
+    const int lane = threadIdx.x & (WAVE - 1);
+    int rs[NW], rl[NW];
+    double X[NW], Y[NW], XN[NW], YN[NW];
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+        const int64_t i = base + w * WAVE + lane;
+        rs[w] = rl[w] = -1;
+        X[w] = Y[w] = XN[w] = YN[w] = 0.0;
+        if (i < end) {
+            rl[w] = a.ringid[i];
+            X[w] = a.x[i];
+            Y[w] = a.y[i];
+        }
     }
-    __syncthreads();
-    const bool fast = s_fast != 0u;
-    uint32_t kp[KEEP_ITEMS];
-    uint32_t ex = 0, agg = 0;
-    // the tile's flags, the largest mark before each thread's vertices and
-    // the tile's largest (every thread of the block calls it)
-    auto load_scan = [&]() {
-        uint32_t mine = 0; // marks grow with the index: the thread's largest is its last kept vertex
 #pragma unroll
-        for (int it = 0; it < KEEP_ITEMS; ++it) {
-            const int64_t i = i0 + it;
-            kp[it] = i < a.n ? a.keep[i] : 0u;
-            if (kp[it]) mine = uint32_t(i) + 1u;
+    for (int w = 0; w < NW; ++w) {
+        const int64_t i = base + w * WAVE + lane;
+        if (i < end) {
+            rs[w] = a.rstart[rl[w]];
+            rl[w] = a.off[rl[w] + 1] - 1; // the ring's last vertex
         }
-        uint32_t inc = mine;
+    }
 #pragma unroll
-        for (int d = 1; d < WAVE; d <<= 1) {
-            const uint32_t y = __shfl_up(inc, d, WAVE);
-            if (lane >= d) inc = inc > y ? inc : y;
-        }
-        ex = __shfl_up(inc, 1, WAVE);
-        if (lane == 0) ex = 0;
-        if (lane == WAVE - 1) s_wmax[w] = inc;
-        __syncthreads();
-        agg = 0;
-#pragma unroll
-        for (int q = 0; q < BLK / WAVE; ++q) {
-            const uint32_t m = s_wmax[q];
-            if (q < w) ex = ex > m ? ex : m;
-            agg = agg > m ? agg : m;
-        }
-    };
-    if (fast) agg = s_agg;
-    else load_scan();
-    // marks grow with the index, so a tile holding a kept vertex knows its
-    // inclusive prefix already (its own largest mark) and publishes it as one;
-    // a look-back then normally stops at the nearest predecessor
-    unsigned long long *my = a.status + tile;
-    if (tid == 0)
-        __hip_atomic_store(my, a.epoch | (tile == 0 || agg != 0 ? KS_PRE : 0ull) | agg, __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
-    if (w == 0) {
-        uint32_t prefix = 0;
-        if (tile > 0) {
-            const unsigned long long EM = 0xffull << KS_EPOCH_SHIFT;
-            int64_t t = int64_t(tile) - 1; // nearest predecessor not yet accounted for
-            int spins = 0;
-            while (true) {
-                const int64_t q = t - lane;
-                const unsigned long long word =
-                    q >= 0 ? __hip_atomic_load(a.status + q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                           : (a.epoch | KS_PRE); // before tile 0: an empty prefix
-                const bool ready = (word & EM) == a.epoch;
-                const uint64_t notready = __ballot(!ready);
-                const uint64_t pre = __ballot(ready && (word & KS_PRE));
-                int upto = -1; // lanes 0..upto are summed
-                bool finished = false;
-                if (pre) {
-                    const int p = __builtin_ctzll(pre);
-                    const uint64_t need = p == WAVE - 1 ? ~0ull : ((2ull << p) - 1ull);
-                    if ((notready & need) == 0) {
-                        upto = p;
-                        finished = true;
-                    }
-                } else if (notready == 0) {
-                    upto = WAVE - 1;
-                }
-                if (upto >= 0) {
-                    uint32_t v = lane <= upto ? uint32_t(word & KS_VAL) : 0u;
-#pragma unroll
-                    for (int d = 1; d < WAVE; d <<= 1) {
-                        const uint32_t y = __shfl_xor(v, d, WAVE);
-                        v = v > y ? v : y;
-                    }
-                    prefix = prefix > v ? prefix : v;
-                    if (finished) break;
-                    t -= WAVE;
-                    spins = 0;
-                } else {
-                    if (++spins > KEEP_SPIN_LIMIT) {
-                        if (lane == 0) atomicOr(a.err, 1u);
-                        break;
-                    }
-                    __builtin_amdgcn_s_sleep(1);
-                }
+    for (int w = 0; w < NW; ++w) {
+        const int64_t i = base + w * WAVE + lane;
+        if (i < end) {
+            const int64_t nx = i == rl[w] ? rs[w] : i + 1;
+            if (rs[w] <= rl[w]) { // else no vertex of the ring stays and none is tested
+                XN[w] = a.x[nx];
+                YN[w] = a.y[nx];
             }
-            if (lane == 0 && agg == 0)
-                __hip_atomic_store(my, a.epoch | KS_PRE | prefix, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
+    }
+    double px = 0.0, py = 0.0; // the vertex before the window
+    if (base > 0) {
+        px = a.x[base - 1];
+        py = a.y[base - 1];
+    }
+    used = KEEP_ANY;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+        const int64_t b = base + w * WAVE, i = b + lane;
+        if (b >= end) break; // uniform
+        const bool valid = i < end, fixed = valid && i <= rs[w];
+        double XP = __shfl_up(X[w], 1, WAVE), YP = __shfl_up(Y[w], 1, WAVE); // every lane active
         if (lane == 0) {
-            s_prefix = prefix;
-            // a tile whose flags did not change in its last round and whose
-            // incoming prefix is the same sees the same last-kept vertices:
-            // its decisions, and so its flags, stay as they are
-            s_skip = fast && a.tstate[3 * tile + 1] == prefix ? 1u : 0u;
-            s_ch = 0u;
+            XP = px;
+            YP = py;
         }
-    }
-    __syncthreads();
-    if (s_skip) {
-        if (tid == 0) a.tstate[3 * tile] = 0u;
-        return;
-    }
-    if (fast) load_scan(); // its maximum is the one published
-    uint32_t cur = s_prefix > ex ? s_prefix : ex; // mark of the last vertex kept before i
-    // the thread's initial decisions, one byte per vertex (i0 is a multiple of 8)
-    uint64_t k0w = 0;
-    if (i0 + KEEP_ITEMS <= a.n) {
-        k0w = *reinterpret_cast<const uint64_t *>(a.keep0 + i0);
-    } else {
-        for (int it = 0; it < KEEP_ITEMS; ++it)
-            if (i0 + it < a.n) k0w |= uint64_t(a.keep0[i0 + it]) << (8 * it);
-    }
-    bool ch = false;
-#pragma unroll
-    for (int it = 0; it < KEEP_ITEMS; ++it) {
-        const int64_t i = i0 + it;
-        if (i < a.n) {
-            uint32_t k = kp[it];
-            if (cur == uint32_t(i)) {
-                // the last vertex kept before i is i - 1: the initial decision's
-                // inputs (for a vertex up to its ring's root that decision is
-                // its flag, which no round changes)
-                k = uint32_t(k0w >> (8 * it)) & 0xffu;
+        const bool k0 = fixed ? i == rs[w] : valid && !(fabs(areaA(XP, YP, X[w], Y[w], XN[w], YN[w])) < EPS);
+        const uint64_t K0 = __ballot(k0), FIX = __ballot(fixed);
+        const int nv = int(end - b < WAVE ? end - b : WAVE);
+        const uint64_t V = nv == WAVE ? ~0ull : ((1ull << nv) - 1ull);
+        uint64_t K = 0;
+        int p = 0;
+        double Lx = 0.0, Ly = 0.0;
+        bool yes = (FIX & 1ull) || mark == uint32_t(b); // the vertex before lane p is kept, or lane p needs none
+        if (b == out) used = (FIX & 1ull) ? KEEP_ANY : mark;
+        if (!yes) {
+            Lx = a.x[mark - 1u];
+            Ly = a.y[mark - 1u];
+        }
+        while (p < nv) {
+            const uint64_t from = ~0ull << p;
+            if (yes) {
+                const uint64_t D = V & ~K0 & ~FIX & from;
+                const int z = D ? int(__builtin_ctzll(D)) : nv;
+                K |= K0 & from & (z == WAVE ? ~0ull : ((1ull << z) - 1ull));
+                if (z < nv) {
+                    Lx = z ? lane_value(X[w], z - 1) : px;
+                    Ly = z ? lane_value(Y[w], z - 1) : py;
+                    yes = false;
+                }
+                p = z + 1;
             } else {
-                const int r = a.ringid[i];
-                const int rs = a.rstart[r], last = a.off[r + 1] - 1;
-                if (i > rs) {
-                    const int pv = int(cur) - 1; // >= rs: the ring's root is always kept
-                    const int nx = i == last ? rs : int(i) + 1;
-                    k = collinear(a.x, a.y, pv, int(i), nx) ? 0u : 1u;
+                const bool stop = valid && lane >= p &&
+                                  (fixed || !(fabs(areaA(Lx, Ly, X[w], Y[w], XN[w], YN[w])) < EPS));
+                const uint64_t F = __ballot(stop);
+                if (!F) break;
+                const int f = int(__builtin_ctzll(F));
+                yes = true;
+                if ((FIX >> f) & 1ull) {
+                    p = f;
+                } else {
+                    K |= 1ull << f;
+                    p = f + 1;
                 }
             }
-            if (k != kp[it]) {
-                a.keep[i] = k;
-                ch = true;
-            }
         }
-        if (kp[it]) cur = uint32_t(i) + 1u;
+        if (valid && i >= out) a.keep[i] = uint32_t((K >> lane) & 1ull);
+        if (K) mark = uint32_t(b) + uint32_t(WAVE - __builtin_clzll(K));
+        px = lane_value(X[w], WAVE - 1);
+        py = lane_value(Y[w], WAVE - 1);
     }
-    if (__ballot(ch) != 0ull && lane == 0) {
-        atomicOr(a.changed, 1u);
-        s_ch = 1u;
-    }
-    __syncthreads();
-    if (tid == 0) {
-        a.tstate[3 * tile] = s_ch;
-        a.tstate[3 * tile + 1] = s_prefix;
-        a.tstate[3 * tile + 2] = agg;
+    return mark;
+}
+
+// Round 0: every tile, one wave each, from one window before it, as if the
+// vertex before that window were kept: only a run of dropped vertices as long
+// as the window leaves the tile with another start than its true one.
+__global__ __launch_bounds__(BLK) void k_keep_first(KeepArgs a) {
+    const int64_t t = int64_t(__builtin_amdgcn_readfirstlane(int(blockIdx.x * (BLK / WAVE) + threadIdx.x / WAVE)));
+    if (t >= a.ntiles) return;
+    const int64_t out = t * KEEP_TILE, end = min(out + KEEP_TILE, a.n);
+    uint32_t used, m;
+    if (t == 0) m = keep_span<KEEP_WIN>(a, 0, 0, end, 0u, used);
+    else m = keep_span<KEEP_WIN + 1>(a, out - WAVE, out, end, uint32_t(out - WAVE), used);
+    if ((threadIdx.x & (WAVE - 1)) == 0) {
+        a.used[t] = used;
+        a.last_out[t] = m > uint32_t(out) ? m : 0u;
     }
 }
 
-// exact sequential pass per ring (used when the fixed point needs too many rounds)
-__global__ void k_cleanup_seq(int nr, const int *off, const int *rstart, const double *x, const double *y,
-                              uint32_t *keep) {
-    int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= nr) return;
-    int s = off[r], last = off[r + 1] - 1, rs = rstart[r];
-    for (int i = s; i < rs && i <= last; ++i) keep[i] = 0;
-    if (rs > last) return;
-    keep[rs] = 1;
-    int lk = rs;
-    for (int i = rs + 1; i <= last; ++i) {
-        int nx = i == last ? rs : i + 1;
-        if (collinear(x, y, lk, i, nx)) keep[i] = 0;
-        else {
-            keep[i] = 1;
-            lk = i;
+// Later rounds: a tile whose last kept vertex before it is another one than it
+// was decided with is decided again.  A round that moves no tile's last kept
+// vertex leaves every tile right, and later rounds return at once.  One wave
+// looks at 64 tiles; hardly any is decided again (a run of dropped vertices has
+// to cross a tile's edge).
+__global__ __launch_bounds__(BLK) void k_keep_fix(KeepArgs a, int round) {
+    if (round > 1 && a.changed[round - 1] == 0u) return;
+    const int lane = threadIdx.x & (WAVE - 1);
+    const int64_t t0 = int64_t(__builtin_amdgcn_readfirstlane(int(blockIdx.x * (BLK / WAVE) + threadIdx.x / WAVE))) * WAVE;
+    if (t0 >= a.ntiles) return;
+    const int64_t t = t0 + lane;
+    uint32_t in = 0u;
+    bool again = false;
+    if (t < a.ntiles) {
+        const uint32_t u = a.used[t];
+        if (u != KEEP_ANY) { // its ring's root, which is kept, lies before the tile
+            int64_t q = t - 1;
+            while (q > 0 && a.last[q] == 0u) --q;
+            in = a.last[q];
+            again = in != u;
+        }
+        if (!again) a.last_out[t] = a.last[t];
+    }
+    uint64_t m = __ballot(again);
+    while (m) {
+        const int l = int(__builtin_ctzll(m));
+        m &= m - 1ull;
+        const int64_t tt = t0 + l, base = tt * KEEP_TILE;
+        const uint32_t mk = uint32_t(__builtin_amdgcn_readlane(int(in), l));
+        uint32_t used;
+        const uint32_t r = keep_span<KEEP_WIN>(a, base, base, min(base + KEEP_TILE, a.n), mk, used);
+        if (lane == 0) {
+            const uint32_t lk = r > uint32_t(base) ? r : 0u;
+            a.used[tt] = mk;
+            a.last_out[tt] = lk;
+            if (lk != a.last[tt]) a.changed[round] = 1u;
         }
     }
+}
+
+// one wave per ring from its first vertex to its last (runs that need too many rounds)
+__global__ __launch_bounds__(BLK) void k_keep_rings(KeepArgs a, int nr) {
+    const int r = __builtin_amdgcn_readfirstlane(int(blockIdx.x * (BLK / WAVE) + threadIdx.x / WAVE));
+    if (r >= nr) return;
+    const int64_t end = a.off[r + 1];
+    uint32_t mark = 0u;
+    uint32_t used;
+    for (int64_t b = a.off[r]; b < end; b += KEEP_TILE)
+        mark = keep_span<KEEP_WIN>(a, b, b, min(b + KEEP_TILE, end), mark, used);
 }
 
 // ring heads carry their ring index; an inclusive max-scan spreads it
@@ -942,11 +907,13 @@ __global__ void k_ring_heads(int nr, const int *off, uint32_t *head) {
     if (off[r + 1] > off[r]) head[off[r]] = uint32_t(r);
 }
 
-__global__ void k_ring_counts(int nr, const int *off, const uint32_t *kscan, uint32_t *cnt) {
-    int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= nr) return;
-    uint32_t c = kscan[off[r + 1]] - kscan[off[r]];
-    cnt[r] = c;
+// vertices left of every ring, and whether there are any (nr + 1 threads: the closing entry)
+__global__ void k_ring_counts(int nr, const int *off, const uint32_t *kscan, uint32_t *cnt, uint32_t *nonempty) {
+    const int r = blockIdx.x * blockDim.x + threadIdx.x;
+    if (r > nr) return;
+    const uint32_t c = r < nr ? kscan[off[r + 1]] - kscan[off[r]] : 0u;
+    if (r < nr) cnt[r] = c;
+    nonempty[r] = c > 0u ? 1u : 0u;
 }
 
 __global__ void k_compact_out(int64_t n, const uint32_t *keep, const uint32_t *kscan, const double *x,
@@ -965,12 +932,6 @@ __global__ void k_ring_off_final(int nr, const uint32_t *cnt, const uint32_t *rs
     if (cnt[r]) off2[nonempty[r]] = int(kscan[off[r]]);
 }
 
-__global__ void k_nonempty(int nr, const uint32_t *cnt, uint32_t *flag) {
-    int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r < nr) flag[r] = cnt[r] ? 1u : 0u;
-}
-
-// per job: its first ring after clean-up (jr = first ring before it)
 __global__ void k_job_rings(int J, const uint32_t *jr, const uint32_t *nonempty, uint32_t *out) {
     int j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j <= J) out[j] = nonempty[jr[j]];
@@ -2198,8 +2159,6 @@ struct FosterScratch {
     DBuf<uint32_t> nflag, nidx;
     DBuf<int> off, rstart, ringid;
     DBuf<uint32_t> keep, kscan, rcnt, nonempty, kctl, ktstate;
-    DBuf<uint8_t> keep0;
-    DBuf<unsigned long long> kstatus; // clean-up rounds: per tile status words
     // sequential route
     DBuf<SeqJob> sjobs;
     DBuf<int> sres, sroff, sosrc;
@@ -2250,73 +2209,66 @@ void cleanup_rings(Ctx &c, FosterScratch &f, int nr, int64_t n, int J, const uin
     k_ring_heads<<<grid_for(nr), BLK, 0, s>>>(nr, f.off, reinterpret_cast<uint32_t *>(ringid));
     scan_inclusive_max_u32(reinterpret_cast<uint32_t *>(ringid), reinterpret_cast<uint32_t *>(ringid), n, s);
     uint32_t *keep = f.keep.ensure(size_t(n) + 1);
-    uint8_t *keep0 = f.keep0.ensure(size_t(n) + KEEP_ITEMS);
-    k_keep0<<<grid_for(n), BLK, 0, s>>>(n, ringid, f.off, rstart, f.ox, f.oy, keep, keep0);
-    SC_HIP(hipGetLastError());
-    // clean-up rounds, KEEP_BATCH per look at the per-round change flags; a
-    // round after one without change changes nothing either
     const int64_t ntiles = (n + KEEP_TILE - 1) / KEEP_TILE;
-    uint32_t *ctl = f.kctl.ensure(KEEP_ROUNDS + 1); // changed flags, error word
-    unsigned long long *kst = f.kstatus.ensure(size_t(ntiles));
-    uint32_t *nonempty = f.nonempty.ensure(nr + 1);
+    uint32_t *changed = f.kctl.ensure(KEEP_ROUNDS);
+    uint32_t *state = f.ktstate.ensure(3 * size_t(ntiles));
+    uint32_t *nonempty = f.nonempty.ensure(size_t(nr) + 1);
     {
         FillBatch fb(s);
-        fb.add(ctl, KEEP_ROUNDS + 1, 0u);
-        fb.add(kst, 2 * ntiles, 0u);
-        fb.add(keep + n, 1, 0u);         // closing entries of the two scans below
-        fb.add(nonempty + nr, 1, 0u);
+        fb.add(changed, KEEP_ROUNDS, 0u);
+        fb.add(keep + n, 1, 0u); // closing entry of the scan below
         fb.flush();
     }
-    KeepRound kr;
-    kr.n = n;
-    kr.ringid = ringid;
-    kr.off = f.off;
-    kr.rstart = rstart;
-    kr.x = f.ox;
-    kr.y = f.oy;
-    kr.keep = keep;
-    kr.keep0 = keep0;
-    kr.status = kst;
-    kr.err = ctl + KEEP_ROUNDS;
-    kr.tstate = f.ktstate.ensure(3 * size_t(ntiles)); // written by every tile in the first round
-    bool converged = false;
-    for (int it = 0; it < KEEP_ROUNDS && !converged;) {
-        const int end = std::min(it + KEEP_BATCH, KEEP_ROUNDS);
-        for (; it < end; ++it) {
-            kr.epoch = (unsigned long long)(it + 1) << KS_EPOCH_SHIFT;
-            kr.changed = ctl + it;
-            kr.first = it == 0 ? 1 : 0;
-            k_keep_round<<<unsigned(ntiles), BLK, 0, s>>>(kr);
-            SC_HIP(hipGetLastError());
-        }
-        // one copy from the batch's last change flag up to the error word
-        uint32_t h[KEEP_ROUNDS + 1];
-        d2h_sync(c, h, ctl + it - 1, int64_t(KEEP_ROUNDS - it + 2));
-        SC_REQUIRE(h[KEEP_ROUNDS - it + 1] == 0, SC_EHIP, "clean-up scan gave up waiting for an earlier tile");
-        converged = h[0] == 0;
-    }
-    if (!converged) {
-        k_cleanup_seq<<<grid_for(nr), BLK, 0, s>>>(nr, f.off, rstart, f.ox, f.oy, keep);
-        SC_HIP(hipGetLastError());
-    }
-    // compaction
+    KeepArgs ka;
+    ka.n = n;
+    ka.ringid = ringid;
+    ka.off = f.off;
+    ka.rstart = rstart;
+    ka.x = f.ox;
+    ka.y = f.oy;
+    ka.keep = keep;
+    ka.used = state;
+    ka.last = nullptr;
+    ka.last_out = state + ntiles;
+    ka.changed = changed;
+    ka.ntiles = ntiles;
+    k_keep_first<<<grid_for(ntiles, BLK / WAVE), BLK, 0, s>>>(ka);
+    SC_HIP(hipGetLastError());
+    ka.last = state + 2 * ntiles;
     uint32_t *kscan = f.kscan.ensure(size_t(n) + 1);
-    uint32_t *tot = c.d_u32_total.ensure(2);
-    scan_exclusive_u32(keep, kscan, n + 1, tot, s);
-    uint32_t *rcnt = f.rcnt.ensure(nr + 1);
-    k_ring_counts<<<grid_for(nr), BLK, 0, s>>>(nr, f.off, kscan, rcnt);
-    SC_HIP(hipGetLastError());
-    // surviving rings: exclusive scan of the non-empty flags; both totals and
-    // the jobs' first rings come back in one copy
-    k_nonempty<<<grid_for(nr), BLK, 0, s>>>(nr, rcnt, nonempty);
-    SC_HIP(hipGetLastError());
-    scan_exclusive_u32(nonempty, nonempty, int64_t(nr) + 1, tot + 1, s);
+    uint32_t *rcnt = f.rcnt.ensure(size_t(nr) + 1);
     uint32_t *jring = f.jring.ensure(size_t(J) + 3);
-    k_job_rings<<<grid_for(int64_t(J) + 1), BLK, 0, s>>>(J, jr, nonempty, jring);
-    SC_HIP(hipGetLastError());
-    SC_HIP(hipMemcpyAsync(jring + J + 1, tot, sizeof(uint32_t) * 2, hipMemcpyDeviceToDevice, s));
     job_ring.resize(size_t(J) + 3);
-    d2h_sync(c, job_ring.data(), jring, int64_t(J) + 3);
+    // rounds until one moves nothing; the counts that follow are taken before
+    // that is known (one wait instead of two), and again if it was not the last
+    for (int it = 1;;) {
+        const int end = std::min(it + (it == 1 ? 2 : 8), KEEP_ROUNDS);
+        const bool rings = it >= end;
+        if (rings) {
+            k_keep_rings<<<grid_for(nr, BLK / WAVE), BLK, 0, s>>>(ka, nr);
+        } else {
+            for (; it < end; ++it) {
+                const uint32_t *prev = ka.last_out;
+                ka.last_out = const_cast<uint32_t *>(ka.last);
+                ka.last = prev;
+                k_keep_fix<<<grid_for(ntiles, BLK), BLK, 0, s>>>(ka, it);
+            }
+        }
+        SC_HIP(hipGetLastError());
+        // compaction counts: vertices, surviving rings, the jobs' first rings
+        scan_exclusive_u32(keep, kscan, n + 1, jring + J + 1, s);
+        k_ring_counts<<<grid_for(int64_t(nr) + 1), BLK, 0, s>>>(nr, f.off, kscan, rcnt, nonempty);
+        SC_HIP(hipGetLastError());
+        scan_exclusive_u32(nonempty, nonempty, int64_t(nr) + 1, jring + J + 2, s);
+        k_job_rings<<<grid_for(int64_t(J) + 1), BLK, 0, s>>>(J, jr, nonempty, jring);
+        SC_HIP(hipGetLastError());
+        uint32_t moved = 0;
+        ReadBack rb(c);
+        rb.add(job_ring.data(), static_cast<const uint32_t *>(jring), size_t(J) + 3);
+        if (!rings) rb.add(&moved, static_cast<const uint32_t *>(changed + it - 1), 1);
+        rb.run();
+        if (!moved) break;
+    }
     const uint32_t nout = job_ring[size_t(J) + 1];
     c.nrings = int(job_ring[size_t(J) + 2]);
     job_ring.resize(size_t(J) + 1);
@@ -2346,14 +2298,12 @@ void release_foster_scratch() {
                               &f.jv, &f.jr, &f.keep, &f.kscan, &f.rcnt, &f.nonempty, &f.kctl, &f.ktstate,
                               &f.jmoved})
         b->release();
-    f.keep0.release();
     f.srec.release();
     f.spstep.release();
     f.semit.release();
     f.sdone.release();
     release_walk_scratch();
     f.jrec.release();
-    f.kstatus.release();
     f.jrec2.release();
     for (DBuf<int> *b : {&f.enexP, &f.enexQ, &f.cposP, &f.cposQ, &f.ppos, &f.plen, &f.pdir, &f.pj, &f.jst,
                          &f.osrc, &f.off, &f.rstart, &f.ringid, &f.sres, &f.sroff, &f.sosrc, &f.nx, &f.pv, &f.nb,
