@@ -336,8 +336,7 @@ void job_rings_to_device(Ctx &c) {
     JobSet &js = c.jobs;
     SC_REQUIRE(js.J >= 1 && int(js.ring_off.size()) == js.J + 1, SC_ESTATE, "no clipped batch");
     js.d_ring.ensure(js.J + 1);
-    SC_HIP(hipMemcpyAsync(js.d_ring.p, js.ring_off.data(), sizeof(int) * (js.J + 1), hipMemcpyHostToDevice,
-                          c.stream));
+    c.upload(js.d_ring.p, js.ring_off.data(), sizeof(int) * (js.J + 1));
 }
 
 } // namespace
@@ -396,7 +395,7 @@ void batch_area_backward(Ctx &c, const double *g_area, const double *g_iou, doub
     std::vector<int> cinall(size_t(c.K) + 1);
     for (int k = 0; k <= c.K; ++k) cinall[k] = c.eoff[k] - c.nb;
     int *dci = a.bin_off.ensure(c.K + 1);
-    SC_HIP(hipMemcpyAsync(dci, cinall.data(), sizeof(int) * (c.K + 1), hipMemcpyHostToDevice, s));
+    c.upload(dci, cinall.data(), sizeof(int) * (c.K + 1));
     k_input_ring_grad<<<grid_for(c.nct), BLK, 0, s>>>(c.nct, dci, c.K, c.cpoly, cQ, grad_c);
     SC_HIP(hipGetLastError());
     // output vertices of the batch

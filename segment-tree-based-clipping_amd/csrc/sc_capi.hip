@@ -39,6 +39,22 @@ __global__ void k_readback(GatherArgs a) {
     for (int q = 0; q < a.n; ++q)
         for (uint32_t i = threadIdx.x; i < a.words[q]; i += blockDim.x) a.dst[q][i] = a.src[q][i];
 }
+// Two pinned upload buffers per host thread, used in turn: a table is written
+// there and a kernel copies it, which costs a launch instead of a copy command
+// from pageable memory (10 us of host time each).  The event tells when a
+// buffer's last kernel is done.
+struct UploadStage {
+    char *p = nullptr, *dev = nullptr;
+    size_t cap = 0;
+    hipEvent_t ev = nullptr;
+    int device = -1;
+};
+thread_local UploadStage tl_up[2];
+thread_local int tl_up_next = 0;
+constexpr size_t UPLOAD_MAX = size_t(4) << 20; // larger tables are copied
+__global__ void k_upload(const uint32_t *src, uint32_t *dst, uint32_t words) {
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < words; i += gridDim.x * blockDim.x) dst[i] = src[i];
+}
 constexpr size_t RB_GATHER_MAX = 65536; // larger items go through the copy engine path
 } // namespace
 void *Ctx::pinned(size_t bytes) {
@@ -55,6 +71,44 @@ void *Ctx::pinned(size_t bytes) {
         ps.cap = want;
     }
     return ps.p;
+}
+void Ctx::upload(void *dst, const void *src, size_t bytes) {
+    if (bytes == 0) return;
+    if (bytes > UPLOAD_MAX || bytes % 4 != 0) {
+        SC_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, stream));
+        SC_HIP(hipStreamSynchronize(stream)); // the source may be pinned: it is free on return either way
+        return;
+    }
+    UploadStage &u = tl_up[tl_up_next];
+    tl_up_next ^= 1;
+    if (u.ev && u.device != device) { // events belong to a device
+        SC_HIP(hipEventSynchronize(u.ev));
+        SC_HIP(hipEventDestroy(u.ev));
+        u.ev = nullptr;
+    }
+    if (u.ev) SC_HIP(hipEventSynchronize(u.ev));
+    if (bytes > u.cap) {
+        if (u.p) SC_HIP(hipHostFree(u.p));
+        u.p = u.dev = nullptr;
+        u.cap = 0;
+        const size_t want = std::max(size_t(65536), bytes + bytes / 4);
+        void *hp = nullptr, *dp = nullptr;
+        SC_HIP(hipHostMalloc(&hp, want, hipHostMallocDefault));
+        u.p = static_cast<char *>(hp);
+        SC_HIP(hipHostGetDevicePointer(&dp, hp, 0));
+        u.dev = static_cast<char *>(dp);
+        u.cap = want;
+    }
+    if (!u.ev) {
+        SC_HIP(hipEventCreateWithFlags(&u.ev, hipEventDisableTiming));
+        u.device = device;
+    }
+    std::memcpy(u.p, src, bytes);
+    const uint32_t words = uint32_t(bytes / 4);
+    k_upload<<<std::min(1024u, (words + 255u) / 256u), 256, 0, stream>>>(reinterpret_cast<const uint32_t *>(u.dev),
+                                                                       static_cast<uint32_t *>(dst), words);
+    SC_HIP(hipGetLastError());
+    SC_HIP(hipEventRecord(u.ev, stream));
 }
 void Ctx::wait() {
     for (;;) {

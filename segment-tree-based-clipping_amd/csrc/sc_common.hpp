@@ -153,6 +153,25 @@ __device__ inline int seg_of(const int *off, int n, int64_t i) {
     return lo;
 }
 
+// The same for the lanes of a wave that hold consecutive i (lane l: i of the
+// first active lane + l): one search for the wave where it lies in one segment
+// (scalar loads, no divergence), else a search between the first and the last
+// lane's segments.
+__device__ inline int seg_of_wave(const int *off, int n, int64_t i) {
+    const uint64_t u = uint64_t(i);
+    const int64_t first = int64_t((uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(int(u >> 32)))) << 32) |
+                                  uint32_t(__builtin_amdgcn_readfirstlane(int(u))));
+    int lo = seg_of(off, n, first);
+    if (lo + 1 >= n || int64_t(off[lo + 1]) > first + (WAVE - 1)) return lo;
+    int hi = seg_of(off, n, first + (WAVE - 1));
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (off[mid] <= i) lo = mid;
+        else hi = mid - 1;
+    }
+    return lo;
+}
+
 // ---------------------------------------------------------------------------
 // primitives (sc_prims.hip)
 // ---------------------------------------------------------------------------

@@ -46,10 +46,12 @@ struct Ctx {
     std::vector<int> csz, coff;     // overlay sizes; vertex offsets with closing vertices
     std::vector<int> eoff;          // overlay edge offsets in the edge index space (K+1), eoff[0] = nb
     DBuf<double> bpoly, cpoly;      // (nb+nbr)*2, (nct+K)*2
-    DBuf<int> d_coff, d_eoff, d_bvoff, d_beoff;
     std::vector<int> loff;          // first leaf (64 consecutive edges) of every base ring, then of every overlay
-    DBuf<int> d_loff;
+    DBuf<int> d_tab;                // the offsets below, back to back
+    std::vector<int> h_tab;
+    int *d_coff = nullptr, *d_eoff = nullptr, *d_bvoff = nullptr, *d_beoff = nullptr, *d_loff = nullptr;
     DBuf<double> d_shift;           // per base/overlay ring x shift of the tree keys (paired mode)
+    bool shift_ready = false;
     // per-edge SoA (edge index e in [0,ne): base edges, then overlay 1, 2, ...)
     DBuf<double> ex0, ey0, ex1, ey1; // endpoints in ring order
     DBuf<double> estart, eend;       // x-extent (tree keys; shifted per pair in paired mode)
@@ -200,6 +202,8 @@ struct Ctx {
     // and the next launch)
     static void *pinned(size_t bytes);
     void wait();
+    // host words to device memory, in stream order; the host array is free on return
+    void upload(void *dst, const void *src, size_t bytes);
     void mark(int i) {
         if (timing) SC_HIP(hipEventRecord(ev[i], stream));
     }
@@ -213,6 +217,7 @@ void ctx_set_polygons(Ctx &c, const double *bxy, int nb, const double *cxy, cons
 void ctx_set_pairs(Ctx &c, const double *bxy, const int *bsz, const double *cxy, const int *csz, int P,
                    bool device_ptrs);
 inline int job_base(const Ctx &c, int k) { return c.paired ? k - 1 : 0; } // base ring of overlay k (1-based)
+void key_shifts(Ctx &c); // d_shift of a paired context, on first use
 void build_edges(Ctx &c);
 void build_elementary(Ctx &c);
 void build_node_intervals(Ctx &c);

@@ -2505,8 +2505,8 @@ void label_and_traverse(Ctx &c) {
             hsidx[j] = q;
         }
         SeqJob *djobs = f.sjobs.ensure(nseq);
-        SC_HIP(hipMemcpyAsync(djobs, sj.data(), sizeof(SeqJob) * nseq, hipMemcpyHostToDevice, s));
-        SC_HIP(hipMemcpyAsync(sidx, hsidx.data(), sizeof(int) * J, hipMemcpyHostToDevice, s));
+        c.upload(djobs, sj.data(), sizeof(SeqJob) * nseq);
+        c.upload(sidx, hsidx.data(), sizeof(int) * J);
         SeqBatch b;
         b.jobs = djobs;
         b.done = nullptr;
@@ -2519,8 +2519,8 @@ void label_and_traverse(Ctx &c) {
             int *mav = f.mav.ensure(mb), *mnbr = f.mnbr.ensure(mb), *mlab = f.mlab.ensure(mb);
             int *djob = f.mjob.ensure(nseq);
             int64_t *dmoff = f.moff.ensure(nseq);
-            SC_HIP(hipMemcpyAsync(djob, seq_jobs.data(), sizeof(int) * nseq, hipMemcpyHostToDevice, s));
-            SC_HIP(hipMemcpyAsync(dmoff, moff.data(), sizeof(int64_t) * nseq, hipMemcpyHostToDevice, s));
+            c.upload(djob, seq_jobs.data(), sizeof(int) * nseq);
+            c.upload(dmoff, moff.data(), sizeof(int64_t) * nseq);
             for (int q0 = 0; q0 < nseq; q0 += 65535) {
                 dim3 g(64, unsigned(std::min(65535, nseq - q0)));
                 k_sp_materialize<<<g, BLK, 0, s>>>(q0, nseq, djob, dmoff, sp, c.sp_av, c.sp_nbr, c.sp_lab, mx, my,
@@ -2534,7 +2534,7 @@ void label_and_traverse(Ctx &c) {
         const int nseg = 2 * nseq;
         const int64_t S = segoff[nseg];
         int64_t *dseg = f.segoff.ensure(nseg + 1);
-        SC_HIP(hipMemcpyAsync(dseg, segoff.data(), sizeof(int64_t) * (nseg + 1), hipMemcpyHostToDevice, s));
+        c.upload(dseg, segoff.data(), sizeof(int64_t) * (nseg + 1));
         NodeArgs na;
         na.nseg = nseg;
         na.segoff = dseg;
@@ -2580,7 +2580,7 @@ void label_and_traverse(Ctx &c) {
             ob += j.out_cap;
             rb += j.ring_cap + 1;
         }
-        SC_HIP(hipMemcpyAsync(djobs, sj.data(), sizeof(SeqJob) * nseq, hipMemcpyHostToDevice, s));
+        c.upload(djobs, sj.data(), sizeof(SeqJob) * nseq);
         b.nx0 = nx0; b.ny0 = ny0; b.nx1 = nx1; b.ny1 = ny1;
         b.nlen = nlen; b.nslot = nslot; b.ninter = ninter; b.nlab = nlab; b.nnb = nnb;
         b.windP = st.windP;

@@ -104,7 +104,7 @@ __global__ __launch_bounds__(BLK) void k_join_leaves(RingTab t, BoxF *box, Leaf 
     const int lane = threadIdx.x & (WAVE - 1);
     const uint32_t w = uni(blockIdx.x * WPB + threadIdx.x / WAVE);
     if (w >= t.nleaf) return;
-    const int r = int(uni(uint32_t(seg_of(t.loff, t.nbr + t.K, w))));
+    const int r = seg_of(t.loff, t.nbr + t.K, w);
     const bool base = r < t.nbr;
     const int k = r - t.nbr;
     const double2 *P = base ? t.bpoly : t.cpoly;
@@ -409,6 +409,7 @@ bool join_candidates(Ctx &c) {
     c.bits_c = bits_for(c.maxcsz);
     c.bits_k = bits_for(int64_t(c.K) + 1);
     SC_REQUIRE(c.bits_b + c.bits_c + c.bits_k <= 64, SC_ERANGE, "pair key does not fit in 64 bits");
+    key_shifts(c);
     const int R = c.nbr + c.K;
     const uint32_t nleaf = uint32_t(c.loff[R]), lb = uint32_t(c.loff[c.nbr]), lc = nleaf - lb;
     RingTab t;

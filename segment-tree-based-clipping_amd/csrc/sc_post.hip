@@ -424,7 +424,7 @@ void post_jobs(Ctx &c, int k0, int k1) {
             *views[q] = dp + at;
             at += parts[q]->size();
         }
-        SC_HIP(hipMemcpyAsync(dp, js.h_pack.data(), sizeof(int) * tot, hipMemcpyHostToDevice, s));
+        c.upload(dp, js.h_pack.data(), sizeof(int) * tot);
     }
     JobArgs ja;
     ja.J = J;

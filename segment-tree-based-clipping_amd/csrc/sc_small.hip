@@ -711,7 +711,7 @@ bool clip_small_batch(Ctx &c, int k0, int k1) {
         h[3 * J + j] = c.csz[k - 1];
     }
     int *dj = S.jobs.ensure(4 * size_t(J));
-    SC_HIP(hipMemcpyAsync(dj, h.data(), sizeof(int) * h.size(), hipMemcpyHostToDevice, s));
+    c.upload(dj, h.data(), sizeof(int) * h.size());
     SmallArgs a;
     a.J = J;
     a.bvoff = dj;
@@ -871,6 +871,7 @@ void pairs_area_graph(Ctx &c, const double *bxy, const double *cxy, double *out4
         g.out4 = out4;
     }
     SC_HIP(hipGraphLaunch(g.exec, s));
+    c.shift_ready = false; // the rings hold other coordinates now
     uint32_t anyfail = 0;
     {
         ReadBack rb(c);

@@ -43,24 +43,30 @@ __device__ inline int find_overlay(const int *eoff, int K, int e) {
     return lo;
 }
 
-// overlay input vertex g (concatenated, no closing vertices) -> reference cPoly slot
-__global__ void k_layout_overlays(const double *__restrict__ cxy, int nct, const int *__restrict__ eoff,
-                                  const int *__restrict__ coff, int K, int nb, double *__restrict__ cpoly) {
-    int64_t g = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (g >= nct) return;
-    int j = find_overlay(eoff, K, int(g) + nb);
-    int local = int(g) + nb - eoff[j];
-    int dst = coff[j] + local;
-    double x = cxy[2 * g], y = cxy[2 * g + 1];
-    cpoly[2 * int64_t(dst)] = x;
-    cpoly[2 * int64_t(dst) + 1] = y;
-    if (local == 0) {
-        int cl = coff[j] + (eoff[j + 1] - eoff[j]);
-        cpoly[2 * int64_t(cl)] = x;
-        cpoly[2 * int64_t(cl) + 1] = y;
+// The reference's ring layout: input vertex g (base rings' vertices, then the
+// overlays', no closing vertices; g is also its edge's index) to its slot, every
+// ring's first vertex again as its closing one.  Both sides in one launch,
+// straight from the caller's arrays; bound by 16 bytes read and written per vertex.
+__global__ void k_layout(const double2 *__restrict__ bxy, const double2 *__restrict__ cxy, int nb, int ne,
+                         const int *__restrict__ beoff, const int *__restrict__ bvoff, int nbr,
+                         const int *__restrict__ eoff, const int *__restrict__ coff, int K,
+                         double2 *__restrict__ bpoly, double2 *__restrict__ cpoly) {
+    const int64_t g = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (g >= ne) return;
+    if (g < nb) {
+        const int j = seg_of_wave(beoff, nbr, g);
+        const double2 v = bxy[g];
+        const int at = bvoff[j] + int(g) - beoff[j];
+        bpoly[at] = v;
+        if (int(g) == beoff[j]) bpoly[bvoff[j + 1] - 1] = v;
+    } else {
+        const int j = seg_of_wave(eoff, K, g);
+        const double2 v = cxy[g - nb];
+        const int at = coff[j] + int(g) - eoff[j];
+        cpoly[at] = v;
+        if (int(g) == eoff[j]) cpoly[coff[j + 1] - 1] = v;
     }
 }
-
 
 // smallest and largest x of a laid-out ring array (nv vertices), per block;
 // min / max are exact, so the result does not depend on the reduction order
@@ -88,15 +94,29 @@ __global__ void k_xrange_blocks(const double *__restrict__ poly, int64_t nv, dou
         bmax[blockIdx.x] = smax[0];
     }
 }
-__global__ void k_xrange_final(const double *__restrict__ bmin, const double *__restrict__ bmax, int n, double *out) {
-    if (blockIdx.x != 0 || threadIdx.x != 0) return;
-    double lo = bmin[0], hi = bmax[0];
-    for (int i = 1; i < n; ++i) {
+// Per-pair key shifts: pairs are laid side by side along x, each in a window
+// wider than the span [lo, hi] of all rings, which every block takes from the
+// XR_BLOCKS * 2 partial ranges itself.
+__global__ __launch_bounds__(BLK) void k_key_shifts(const double *__restrict__ bmin, const double *__restrict__ bmax,
+                                                    int n, int K, double *__restrict__ shift) {
+    __shared__ double slo[BLK], shi[BLK];
+    double lo = INFINITY, hi = -INFINITY;
+    for (int i = threadIdx.x; i < n; i += BLK) {
         lo = fmin(lo, bmin[i]);
         hi = fmax(hi, bmax[i]);
     }
-    out[0] = lo;
-    out[1] = hi;
+    slo[threadIdx.x] = lo;
+    shi[threadIdx.x] = hi;
+    __syncthreads();
+    for (int d = BLK / 2; d > 0; d >>= 1) {
+        if (int(threadIdx.x) < d) {
+            slo[threadIdx.x] = fmin(slo[threadIdx.x], slo[threadIdx.x + d]);
+            shi[threadIdx.x] = fmax(shi[threadIdx.x], shi[threadIdx.x + d]);
+        }
+        __syncthreads();
+    }
+    const double span = (shi[0] - slo[0]) + 1.0;
+    for (int k = blockIdx.x * BLK + threadIdx.x; k < K; k += gridDim.x * BLK) shift[k] = double(k) * span - slo[0];
 }
 
 // Edge records.  In paired mode the x-extents used as tree keys are moved by a
@@ -482,25 +502,6 @@ uint64_t read_u64(Ctx &c, const uint64_t *d) {
 }
 
 namespace {
-// lay out a set of rings (concatenated, no closing vertices) with closing vertices
-void layout_rings(Ctx &c, const double *src, int64_t nverts, const std::vector<int> &sizes,
-                  const std::vector<int> &voff, DBuf<int> &d_voff, std::vector<int> &edge_off, int edge_base,
-                  DBuf<int> &d_eoff, DBuf<double> &dst, bool device_ptrs) {
-    hipStream_t s = c.stream;
-    const int R = int(sizes.size());
-    d_voff.ensure(R + 1);
-    d_eoff.ensure(R + 1);
-    SC_HIP(hipMemcpyAsync(d_voff.p, voff.data(), sizeof(int) * (R + 1), hipMemcpyHostToDevice, s));
-    SC_HIP(hipMemcpyAsync(d_eoff.p, edge_off.data(), sizeof(int) * (R + 1), hipMemcpyHostToDevice, s));
-    dst.ensure(2 * size_t(nverts + R));
-    double *stage = reinterpret_cast<double *>(c.u64a.ensure(2 * size_t(nverts)));
-    SC_HIP(hipMemcpyAsync(stage, src, sizeof(double) * 2 * size_t(nverts),
-                          device_ptrs ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, s));
-    k_layout_overlays<<<grid_for(nverts), BLK, 0, s>>>(stage, int(nverts), d_eoff.p, d_voff.p, R, edge_base, dst.p);
-    SC_HIP(hipGetLastError());
-    SC_HIP(hipStreamSynchronize(s)); // staging buffer is reused by the next call
-}
-
 void reset_derived(Ctx &c) {
     c.epc = c.nleaves = c.T = c.ea_count = 0;
     c.n_lend = c.n_cov = c.n_cand = c.n_pairs = c.n_mend = c.n_near = 0;
@@ -552,37 +553,39 @@ void load(Ctx &c, const double *bxy, const int *bsz, int nbr, const double *cxy,
     c.loff.assign(size_t(nbr) + K + 1, 0);
     for (int i = 0; i < nbr + K; ++i)
         c.loff[i + 1] = c.loff[i] + int(ceil_div(i < nbr ? bsz[i] : csz[i - nbr], WAVE));
-    SC_HIP(hipMemcpyAsync(c.d_loff.ensure(c.loff.size()), c.loff.data(), sizeof(int) * c.loff.size(),
-                          hipMemcpyHostToDevice, c.stream));
-    layout_rings(c, bxy, nb, c.bsz, c.bvoff, c.d_bvoff, c.beoff, 0, c.d_beoff, c.bpoly, device_ptrs);
-    layout_rings(c, cxy, nct, c.csz, c.coff, c.d_coff, c.eoff, c.nb, c.d_eoff, c.cpoly, device_ptrs);
-    if (paired) {
-        // per-pair key shift: pairs are laid side by side along x, each in a
-        // window wider than the span of all rings
-        // x-range of all rings, reduced on the device from the laid-out rings
-        // (their closing vertices repeat first vertices: the same range)
-        double lo = 0, hi = 0;
-        {
-            double *part = reinterpret_cast<double *>(c.u64b.ensure(4 * XR_BLOCKS + 2));
-            k_xrange_blocks<<<XR_BLOCKS, BLK, 0, c.stream>>>(c.bpoly, nb + nbr, part, part + 2 * XR_BLOCKS);
-            k_xrange_blocks<<<XR_BLOCKS, BLK, 0, c.stream>>>(c.cpoly, nct + K, part + XR_BLOCKS,
-                                                             part + 3 * XR_BLOCKS);
-            k_xrange_final<<<1, 1, 0, c.stream>>>(part, part + 2 * XR_BLOCKS, 2 * XR_BLOCKS, part + 4 * XR_BLOCKS);
-            SC_HIP(hipGetLastError());
-            double h[2];
-            ReadBack rb(c);
-            rb.add(h, static_cast<const double *>(part + 4 * XR_BLOCKS), 2);
-            rb.run();
-            lo = h[0];
-            hi = h[1];
-        }
-        double span = (hi - lo) + 1.0;
-        std::vector<double> sh(static_cast<size_t>(K));
-        for (int k = 0; k < K; ++k) sh[k] = double(k) * span - lo;
-        c.d_shift.ensure(K);
-        SC_HIP(hipMemcpyAsync(c.d_shift.p, sh.data(), sizeof(double) * K, hipMemcpyHostToDevice, c.stream));
-        SC_HIP(hipStreamSynchronize(c.stream));
+    // the offset tables in one upload
+    const std::vector<int> *parts[] = {&c.bvoff, &c.beoff, &c.coff, &c.eoff, &c.loff};
+    int **views[] = {&c.d_bvoff, &c.d_beoff, &c.d_coff, &c.d_eoff, &c.d_loff};
+    size_t tot = 0, at = 0;
+    for (const std::vector<int> *v : parts) tot += v->size();
+    c.h_tab.resize(tot);
+    int *dp = c.d_tab.ensure(tot);
+    for (int q = 0; q < 5; ++q) {
+        std::copy(parts[q]->begin(), parts[q]->end(), c.h_tab.begin() + at);
+        *views[q] = dp + at;
+        at += parts[q]->size();
     }
+    hipStream_t s = c.stream;
+    c.upload(dp, c.h_tab.data(), tot * sizeof(int));
+    c.bpoly.ensure(2 * size_t(nb + nbr));
+    c.cpoly.ensure(2 * size_t(nct + K));
+    // device rings are read in place (by double2 where they are aligned for it), others staged
+    const double *bsrc = bxy, *csrc = cxy;
+    if (!device_ptrs || ((reinterpret_cast<uintptr_t>(bxy) | reinterpret_cast<uintptr_t>(cxy)) & 15) != 0) {
+        double *stage = reinterpret_cast<double *>(c.u64a.ensure(2 * size_t(nb + nct)));
+        const hipMemcpyKind kind = device_ptrs ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
+        SC_HIP(hipMemcpyAsync(stage, bxy, sizeof(double) * 2 * size_t(nb), kind, s));
+        SC_HIP(hipMemcpyAsync(stage + 2 * nb, cxy, sizeof(double) * 2 * size_t(nct), kind, s));
+        bsrc = stage;
+        csrc = stage + 2 * nb;
+    }
+    k_layout<<<grid_for(c.ne), BLK, 0, s>>>(reinterpret_cast<const double2 *>(bsrc),
+                                            reinterpret_cast<const double2 *>(csrc), c.nb, c.ne, c.d_beoff, c.d_bvoff,
+                                            nbr, c.d_eoff, c.d_coff, K, reinterpret_cast<double2 *>(c.bpoly.p),
+                                            reinterpret_cast<double2 *>(c.cpoly.p));
+    SC_HIP(hipGetLastError());
+    c.wait(); // the caller's arrays are free on return
+    c.shift_ready = false;
     reset_derived(c);
 }
 } // namespace
@@ -598,8 +601,24 @@ void ctx_set_pairs(Ctx &c, const double *bxy, const int *bsz, const double *cxy,
     load(c, bxy, bsz, P, cxy, csz, P, true, device_ptrs);
 }
 
+// x-range of all rings, reduced on the device from the laid-out rings (their
+// closing vertices repeat first vertices: the same range), to the shifts
+void key_shifts(Ctx &c) {
+    if (!c.paired || c.shift_ready) return;
+    double *part = reinterpret_cast<double *>(c.u64b.ensure(4 * XR_BLOCKS));
+    double *shift = c.d_shift.ensure(c.K);
+    k_xrange_blocks<<<XR_BLOCKS, BLK, 0, c.stream>>>(c.bpoly, int64_t(c.nb) + c.nbr, part, part + 2 * XR_BLOCKS);
+    k_xrange_blocks<<<XR_BLOCKS, BLK, 0, c.stream>>>(c.cpoly, int64_t(c.nct) + c.K, part + XR_BLOCKS,
+                                                     part + 3 * XR_BLOCKS);
+    k_key_shifts<<<unsigned(std::min<int64_t>(64, ceil_div(c.K, BLK))), BLK, 0, c.stream>>>(
+        part, part + 2 * XR_BLOCKS, 2 * XR_BLOCKS, c.K, shift);
+    SC_HIP(hipGetLastError());
+    c.shift_ready = true;
+}
+
 void build_edges(Ctx &c) {
     SC_REQUIRE(c.ne > 0, SC_ESTATE, "polygons not set");
+    key_shifts(c);
     int ne = c.ne;
     c.ex0.ensure(ne); c.ey0.ensure(ne); c.ex1.ensure(ne); c.ey1.ensure(ne);
     c.estart.ensure(ne); c.eend.ensure(ne); c.etype.ensure(ne); c.eid.ensure(ne);

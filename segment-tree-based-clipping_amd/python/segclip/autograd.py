@@ -120,4 +120,6 @@ class AreaIoU(torch.autograd.Function):
 
 def clip_area_iou(base_xy, base_sizes, ov_xy, ov_sizes, paired=True, recompute=False, tuning=None):
     """Per pair (or overlay): intersection area and IoU, differentiable w.r.t. the vertices."""
-    return AreaIoU.apply(base_xy, ov_xy, list(base_sizes), list(ov_sizes), paired, recompute, tuning)
+    # arrays as they are: a list of 16,384 numbers costs half a millisecond each way
+    base_sizes, ov_sizes = (s if isinstance(s, np.ndarray) else list(s) for s in (base_sizes, ov_sizes))
+    return AreaIoU.apply(base_xy, ov_xy, base_sizes, ov_sizes, paired, recompute, tuning)
