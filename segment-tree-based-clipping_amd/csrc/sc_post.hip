@@ -125,15 +125,21 @@ __global__ void k_pair_decode(JobArgs ja, const uint64_t *__restrict__ pairs, in
 // pairs are then ranked by (quantised alpha, pair index), keys that are all
 // distinct.  The result equals a stable sort of the pairs (in pair order) by
 // (edge slot, quantised alpha): ties keep pair order.
-__global__ void k_seg_scatter(int I, const int *__restrict__ edge_of, const int *__restrict__ pj,
-                              const int *__restrict__ JX, const int *__restrict__ scan, const int *__restrict__ arr,
-                              const int *__restrict__ q, uint64_t *K) {
+struct ScatterSide {
+    const int *edge_of, *JX, *scan, *arr, *q;
+    uint64_t *K;
+};
+struct ScatterSides {
+    ScatterSide s[2];
+};
+__global__ void k_seg_scatter(int I, const int *__restrict__ pj, ScatterSides sides) {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= I) return;
-    const int a = arr[p];
+    const ScatterSide &z = sides.s[blockIdx.y];
+    const int a = z.arr[p];
     if (a < 0) return; // not counted (flagged job)
-    const int pos = scan[JX[pj[p]] + edge_of[p]] + a;
-    K[pos] = (uint64_t(uint32_t(q[p] % 1000000000)) << 32) | uint32_t(p);
+    const int pos = z.scan[z.JX[pj[p]] + z.edge_of[p]] + a;
+    z.K[pos] = (uint64_t(uint32_t(z.q[p] % 1000000000)) << 32) | uint32_t(p);
 }
 
 // keys for the per-edge alpha order: the edge's slot over the batch above
@@ -154,82 +160,143 @@ __global__ void k_copy_order(const uint32_t *__restrict__ vals, int I, int *ord)
     if (i < I) ord[i] = int(vals[i]);
 }
 
-// per job: augmented sizes nb + (non-degenerate intersections on the base), likewise overlay
-__global__ void k_job_sizes(JobArgs ja, const int *__restrict__ nd_b, const int *__restrict__ nd_c, int *nba,
-                            int *nca) {
-    int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= ja.J) return;
-    if (nd_b) nba[j] = ja.nb[j] + (nd_b[ja.JB[j + 1]] - nd_b[ja.JB[j]]);
-    nca[j] = ja.nc[j] + (nd_c[ja.JC[j + 1]] - nd_c[ja.JC[j]]);
+// Augmented ring offsets per job: sizes nb + (non-degenerate intersections on
+// the base; ndg: their counts by pair position in the sparse layout), likewise
+// overlay, scanned by one block (J + 1 entries each), JOB_PER jobs per thread
+// and chunk: one launch where sizes, closing entries and their scans took five.
+constexpr int JOB_BLK = 1024, JOB_PER = 4;
+__global__ __launch_bounds__(JOB_BLK) void k_job_offsets(JobArgs ja, const int *__restrict__ nd_b,
+                                                       const uint32_t *__restrict__ ndg,
+                                                       const int *__restrict__ nd_c, int *nba, int *nca) {
+    __shared__ int sb[JOB_BLK / WAVE], sc[JOB_BLK / WAVE];
+    const int lane = threadIdx.x & (WAVE - 1), wid = threadIdx.x / WAVE;
+    int cb = 0, cc = 0;
+    for (int64_t c0 = 0; c0 <= ja.J; c0 += JOB_BLK * JOB_PER) {
+        const int64_t j0 = c0 + int64_t(threadIdx.x) * JOB_PER;
+        int vb[JOB_PER], vc[JOB_PER], tb = 0, tc = 0;
+#pragma unroll
+        for (int q = 0; q < JOB_PER; ++q) {
+            const int64_t j = j0 + q;
+            vb[q] = vc[q] = 0;
+            if (j < ja.J) {
+                vb[q] = ja.nb[j] + (nd_b ? nd_b[ja.JB[j + 1]] - nd_b[ja.JB[j]] : int(ndg[ja.p0[j + 1]] - ndg[ja.p0[j]]));
+                vc[q] = ja.nc[j] + (nd_c[ja.JC[j + 1]] - nd_c[ja.JC[j]]);
+            }
+            tb += vb[q];
+            tc += vc[q];
+        }
+        int ib = tb, ic = tc;
+        for (int d = 1; d < WAVE; d <<= 1) {
+            const int ob = __shfl_up(ib, d, WAVE), oc = __shfl_up(ic, d, WAVE);
+            if (lane >= d) {
+                ib += ob;
+                ic += oc;
+            }
+        }
+        if (lane == WAVE - 1) {
+            sb[wid] = ib;
+            sc[wid] = ic;
+        }
+        __syncthreads();
+        int bb = cb + ib - tb, bc = cc + ic - tc; // before this thread's jobs
+        for (int w = 0; w < JOB_BLK / WAVE; ++w) {
+            if (w < wid) {
+                bb += sb[w];
+                bc += sc[w];
+            }
+            cb += sb[w];
+            cc += sc[w];
+        }
+        __syncthreads(); // sb and sc are rewritten in the next chunk
+#pragma unroll
+        for (int q = 0; q < JOB_PER; ++q) {
+            if (j0 + q <= ja.J) {
+                nba[j0 + q] = bb;
+                nca[j0 + q] = bc;
+            }
+            bb += vb[q];
+            bc += vc[q];
+        }
+    }
 }
 
-__global__ void k_init_aug(int64_t n, double *ax, double *ay, int *av, int *nbr, int *lab, int *sv, int *sp) {
-    int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    ax[i] = 0.0;
-    ay[i] = 0.0;
-    av[i] = -100;
-    nbr[i] = -100;
-    lab[i] = 0;
-    if (sv) {
-        sv[i] = -1;
-        sp[i] = -1;
+// the two sides of the augmented rings, one per blockIdx.y (a null ax: not in this batch)
+struct AugSide {
+    int64_t n;             // slots
+    const int *JX, *nverts, *voff, *AX;
+    const double *poly;
+    const int *all_scan, *nd_scan, *edge_of, *ord, *q;
+    double *ax, *ay;
+    int *av, *nbr, *lab, *sv, *sp, *slot;
+};
+struct AugSides {
+    AugSide s[2];
+};
+
+__global__ void k_init_aug(AugSides sides) {
+    const AugSide &z = sides.s[blockIdx.y];
+    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (!z.ax || i >= z.n) return;
+    z.ax[i] = 0.0;
+    z.ay[i] = 0.0;
+    z.av[i] = -100;
+    z.nbr[i] = -100;
+    z.lab[i] = 0;
+    if (z.sv) {
+        z.sv[i] = -1;
+        z.sp[i] = -1;
     }
 }
 
 // source vertices: count slot i of job j is vertex i - JX[j] (the last slot of a job is padding)
-__global__ void k_aug_sources(int J, const int *__restrict__ JX, const int *__restrict__ nverts,
-                              const int *__restrict__ voff, const int *__restrict__ AX,
-                              const double *__restrict__ poly, const int *__restrict__ nd_scan, double *ax,
-                              double *ay, int *sv) {
-    int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= JX[J]) return;
-    int j = seg_of(JX, J, i);
-    int v = int(i - JX[j]);
-    if (v >= nverts[j]) return;
-    int64_t pos = AX[j] + v + (nd_scan[i] - nd_scan[JX[j]]);
-    int64_t g = 2 * int64_t(voff[j] + v);
-    ax[pos] = poly[g];
-    ay[pos] = poly[g + 1];
-    if (sv) sv[pos] = v;
+__global__ void k_aug_sources(int J, AugSides sides) {
+    const AugSide &z = sides.s[blockIdx.y];
+    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (!z.ax || i >= z.JX[J]) return;
+    const int j = seg_of_wave(z.JX, J, i);
+    const int j0 = z.JX[j], v = int(i - j0);
+    if (v >= z.nverts[j]) return;
+    const int64_t pos = z.AX[j] + v + (z.nd_scan[i] - z.nd_scan[j0]);
+    const double2 V = reinterpret_cast<const double2 *>(z.poly)[int64_t(z.voff[j]) + v];
+    z.ax[pos] = V.x;
+    z.ay[pos] = V.y;
+    if (z.sv) z.sv[pos] = v;
 }
 
 // one thread per position of the per-edge alpha order: a leading degenerate
 // intersection marks its edge's source vertex, the non-degenerate ones fill
 // the slots after it in order
-template <bool SIDE_B>
-__global__ void k_aug_segments(const int *__restrict__ edge_of, const int *__restrict__ pj, int I,
-                               const int *__restrict__ ord, const int *__restrict__ JX, const int *__restrict__ AX,
-                               const int *__restrict__ all_scan, const int *__restrict__ nd_scan,
-                               const int *__restrict__ pt, const double *__restrict__ px,
-                               const double *__restrict__ py, const int *__restrict__ q, double *ax, double *ay,
-                               int *av, int *slot, int *flags, int *sp) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= I) return;
-    const int p = ord[i];
+__global__ void k_aug_segments(const int *__restrict__ pj, int I, const int *__restrict__ pt,
+                               const double *__restrict__ px, const double *__restrict__ py, int *flags,
+                               AugSides sides) {
+    const bool side_b = blockIdx.y == 0;
+    const AugSide &z = sides.s[blockIdx.y];
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (!z.ax || i >= I) return;
+    const int p = z.ord[i];
     const int j = pj[p];
-    const int e = edge_of[p];
-    const int gi = JX[j] + e;
-    const int s = all_scan[gi], t = all_scan[gi + 1];
-    const int nd = nd_scan[gi + 1] - nd_scan[gi];
-    const int src = AX[j] + e + (nd_scan[gi] - nd_scan[JX[j]]);
-    const int first = i == s ? p : ord[s];
-    const int k0 = (SIDE_B ? degen_b_first(pt[first]) : degen_c_first(pt[first])) ? 1 : 0;
+    const int e = z.edge_of[p];
+    const int gi = z.JX[j] + e;
+    const int s = z.all_scan[gi], t = z.all_scan[gi + 1];
+    const int nd = z.nd_scan[gi + 1] - z.nd_scan[gi];
+    const int src = z.AX[j] + e + (z.nd_scan[gi] - z.nd_scan[z.JX[j]]);
+    const int first = i == s ? p : z.ord[s];
+    const int k0 = (side_b ? degen_b_first(pt[first]) : degen_c_first(pt[first])) ? 1 : 0;
     if (i == s && k0 + nd != t - s) atomicOr(&flags[j], UB_UNASSIGNED);
     if (i == s && k0) {
-        av[src] = q[p];
-        slot[p] = src;
+        z.av[src] = z.q[p];
+        z.slot[p] = src;
         return;
     }
     const int k = i - s - k0;
     if (k >= nd) return; // more positions than non-degenerate slots: flagged above
-    if (!(SIDE_B ? nondeg_b(pt[p]) : nondeg_c(pt[p]))) atomicOr(&flags[j], UB_UNASSIGNED);
+    if (!(side_b ? nondeg_b(pt[p]) : nondeg_c(pt[p]))) atomicOr(&flags[j], UB_UNASSIGNED);
     const int sl = src + 1 + k;
-    ax[sl] = px[p];
-    ay[sl] = py[p];
-    av[sl] = q[p];
-    slot[p] = sl;
-    if (sp) sp[sl] = p;
+    z.ax[sl] = px[p];
+    z.ay[sl] = py[p];
+    z.av[sl] = z.q[p];
+    z.slot[p] = sl;
+    if (z.sp) z.sp[sl] = p;
 }
 
 // neighbour links, 1-based and local to the job's rings (as the reference's arrays)
@@ -315,13 +382,6 @@ __global__ void k_sp_fill(int I, const int *__restrict__ ord, const int *__restr
         y[i] = V[1];
     }
     pos[p] = i;
-}
-
-__global__ void k_sp_sizes(int J, const int *__restrict__ p0, const uint32_t *__restrict__ ndg,
-                           const int *__restrict__ nb, int *nba) {
-    int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= J) return;
-    nba[j] = nb[j] + int(ndg[p0[j + 1]] - ndg[p0[j]]);
 }
 
 __global__ void k_sp_link(int I, const int *__restrict__ pos, const int *__restrict__ pj,
@@ -459,6 +519,9 @@ void post_jobs(Ctx &c, int k0, int k1) {
     fb.add(nd_c, nJC + 1, 0u);
     fb.add(c.slot_b.p, Ia, ~0u);
     fb.add(c.slot_c.p, Ia, ~0u);
+    uint32_t *segctl = c.seg_ctl.ensure(2 * SEG_CTL); // per side: list counts, too-large flag
+    fb.add(segctl, 2 * SEG_CTL, 0u);
+    if (sparse) fb.add(c.sp_ndf.ensure(size_t(I) + 1) + I, 1, 0u); // closing entry of its scan
     fb.flush();
     if (I > 0) {
         k_pair_decode<<<grid_for(I), BLK, 0, s>>>(ja, c.pairs.p + P0, I, c.bits_b, c.bits_c, c.bpoly, c.cpoly, c.p_j,
@@ -467,15 +530,12 @@ void post_jobs(Ctx &c, int k0, int k1) {
                                                   c.arr_c.ensure(Ia));
         SC_HIP(hipGetLastError());
     }
-    auto scan = [&](int *a, int64_t n) {
-        scan_exclusive_u32(reinterpret_cast<uint32_t *>(a), reinterpret_cast<uint32_t *>(a), n, nullptr, s);
-    };
-    if (!sparse) {
-        scan(all_b, nJB + 1);
-        scan(nd_b, nJB + 1);
+    {
+        uint32_t *arr[4] = {reinterpret_cast<uint32_t *>(all_c), reinterpret_cast<uint32_t *>(nd_c),
+                            reinterpret_cast<uint32_t *>(all_b), reinterpret_cast<uint32_t *>(nd_b)};
+        const int64_t n[4] = {int64_t(nJC) + 1, int64_t(nJC) + 1, int64_t(nJB) + 1, int64_t(nJB) + 1};
+        scan_exclusive_u32_4(sparse ? 2 : 4, arr, n, s);
     }
-    scan(all_c, nJC + 1);
-    scan(nd_c, nJC + 1);
 
     // Per edge alpha order on each side (positions = the edge groups' count
     // offsets): by ranking inside the groups, or (a group beyond SEG_LDS_MAX,
@@ -496,33 +556,32 @@ void post_jobs(Ctx &c, int k0, int k1) {
         k_copy_order<<<grid_for(I), BLK, 0, s>>>(c.ord_val, I, side_b ? c.ordB : c.ordC);
         SC_HIP(hipGetLastError());
     };
-    uint32_t *segctl = c.seg_ctl.ensure(2 * SEG_CTL); // per side: list counts, too-large flag
     if (I > 0) {
-        {
-            FillBatch fb(s);
-            fb.add(segctl, 2 * SEG_CTL, 0u);
-            fb.flush();
-        }
-        auto seg_order = [&](const int *edge_of, const int *JX, const int *scan, const int *arr, const int *q,
-                             int nseg, DBuf<uint64_t> &K, DBuf<uint32_t> &wl, DBuf<uint32_t> &bl, uint32_t *ctl,
-                             int *ord) {
-            k_seg_scatter<<<grid_for(I), BLK, 0, s>>>(I, edge_of, c.p_j, JX, scan, arr, q, K.ensure(Ia));
+        // the sides sorted inside their groups: the overlays, then the base rings (not sparse)
+        ScatterSides sc{};
+        SegSets ss{};
+        auto side = [&](const int *edge_of, const int *JX, const int *scan, const int *arr, const int *q, int nseg,
+                        DBuf<uint64_t> &K, DBuf<uint32_t> &wl, DBuf<uint32_t> &bl, uint32_t *ctl, int *ord) {
             // listed groups hold more than SEG_THREAD (wave list) or SEG_WAVE_MAX (block list) pairs each
             const int64_t nw = std::min<int64_t>(nseg, int64_t(I) / (SEG_THREAD + 1)) + 1;
             const int64_t nb = std::min<int64_t>(nseg, int64_t(I) / (SEG_WAVE_MAX + 1)) + 1;
-            seg_sort<false>(nseg, scan, K, ord, wl.ensure(size_t(nw)), bl.ensure(size_t(nb)), ctl, s);
+            sc.s[ss.count] = ScatterSide{edge_of, JX, scan, arr, q, K.ensure(Ia)};
+            ss.s[ss.count] = SegSet{nseg, scan, K.p, ord, wl.ensure(size_t(nw)), bl.ensure(size_t(nb)), ctl};
+            ++ss.count;
         };
+        side(c.p_c, ja.JC, all_c, c.arr_c, c.p_qb, nJC, c.seg_kc, c.seg_wc, c.seg_bc, segctl + SEG_CTL, c.ordC);
         if (sparse) radix_order(true);
-        else seg_order(c.p_b, ja.JB, all_b, c.arr_b, c.p_qa, nJB, c.seg_kb, c.seg_wb, c.seg_bb, segctl, c.ordB);
-        seg_order(c.p_c, ja.JC, all_c, c.arr_c, c.p_qb, nJC, c.seg_kc, c.seg_wc, c.seg_bc, segctl + SEG_CTL, c.ordC);
+        else side(c.p_b, ja.JB, all_b, c.arr_b, c.p_qa, nJB, c.seg_kb, c.seg_wb, c.seg_bb, segctl, c.ordB);
+        k_seg_scatter<<<dim3(grid_for(I), unsigned(ss.count)), BLK, 0, s>>>(I, c.p_j, sc);
+        SC_HIP(hipGetLastError());
+        seg_sort<false>(ss, s);
     }
     // augmented ring sizes and offsets per job
     int *nba = js.d_AB.ensure(J + 1), *nca = js.d_AC.ensure(J + 1);
     if (sparse) {
         // virtual slot of every base-side intersection
         int *kind = reinterpret_cast<int *>(c.u32c.ensure(Ia));
-        uint32_t *ndf = reinterpret_cast<uint32_t *>(c.sp_ndf.ensure(size_t(I) + 1));
-        SC_HIP(hipMemsetAsync(ndf + I, 0, sizeof(uint32_t), s));
+        uint32_t *ndf = reinterpret_cast<uint32_t *>(c.sp_ndf.p);
         if (I > 0) {
             k_sp_mark<<<grid_for(I), BLK, 0, s>>>(I, c.ordB, c.p_j, c.p_b, c.p_type, ja.p0, kind, ndf, flags);
             SC_HIP(hipGetLastError());
@@ -538,20 +597,11 @@ void post_jobs(Ctx &c, int k0, int k1) {
                                                   kind);
             SC_HIP(hipGetLastError());
         }
-        k_sp_sizes<<<grid_for(J), BLK, 0, s>>>(J, ja.p0, ndf, ja.nb, nba);
-        SC_HIP(hipGetLastError());
     }
-    k_job_sizes<<<grid_for(J), BLK, 0, s>>>(ja, nd_b, nd_c, nba, nca);
+    k_job_offsets<<<1, JOB_BLK, 0, s>>>(ja, sparse ? nullptr : nd_b,
+                                        sparse ? reinterpret_cast<const uint32_t *>(c.sp_ndf.p) : nullptr, nd_c, nba,
+                                        nca);
     SC_HIP(hipGetLastError());
-    {
-        FillBatch fb(s);
-        fb.add(nba + J, 1, 0u);
-        fb.add(nca + J, 1, 0u);
-        fb.flush();
-    }
-    uint32_t *tot = c.d_u32_total.ensure(2);
-    scan_exclusive_u32_2(reinterpret_cast<uint32_t *>(nba), reinterpret_cast<uint32_t *>(nba), J + 1, tot,
-                         reinterpret_cast<uint32_t *>(nca), reinterpret_cast<uint32_t *>(nca), J + 1, tot + 1, s);
     js.AB.resize(J + 1);
     js.AC.resize(J + 1);
     uint32_t hseg[2 * SEG_CTL] = {};
@@ -578,24 +628,20 @@ void post_jobs(Ctx &c, int k0, int k1) {
         svc = c.sv_c.ensure(ncaA);
         spc = c.sp_c.ensure(ncaA);
     }
+    AugSides as{};
     if (!sparse) {
         c.aug_bx.ensure(nbaA); c.aug_by.ensure(nbaA); c.av_b.ensure(nbaA); c.nbr_b.ensure(nbaA); c.lab_b.ensure(nbaA);
-        k_init_aug<<<grid_for(nba_tot), BLK, 0, s>>>(nba_tot, c.aug_bx, c.aug_by, c.av_b, c.nbr_b, c.lab_b, svb, spb);
-        k_aug_sources<<<grid_for(nJB), BLK, 0, s>>>(J, ja.JB, ja.nb, ja.bvoff, nba, c.bpoly, nd_b, c.aug_bx,
-                                                    c.aug_by, svb);
+        as.s[0] = AugSide{nba_tot, ja.JB, ja.nb, ja.bvoff, nba, c.bpoly, all_b, nd_b, c.p_b, c.ordB, c.p_qa, c.aug_bx,
+                          c.aug_by, c.av_b, c.nbr_b, c.lab_b, svb, spb, c.slot_b};
     }
-    k_init_aug<<<grid_for(nca_tot), BLK, 0, s>>>(nca_tot, c.aug_cx, c.aug_cy, c.av_c, c.nbr_c, c.lab_c, svc, spc);
-    k_aug_sources<<<grid_for(nJC), BLK, 0, s>>>(J, ja.JC, ja.nc, ja.cvoff, nca, c.cpoly, nd_c, c.aug_cx, c.aug_cy,
-                                                svc);
+    as.s[1] = AugSide{nca_tot, ja.JC, ja.nc, ja.cvoff, nca, c.cpoly, all_c, nd_c, c.p_c, c.ordC, c.p_qb, c.aug_cx,
+                      c.aug_cy, c.av_c, c.nbr_c, c.lab_c, svc, spc, c.slot_c};
+    // (the sparse base side has slots by the hundred million and none of these arrays)
+    k_init_aug<<<dim3(grid_for(sparse ? nca_tot : std::max(nba_tot, nca_tot)), 2), BLK, 0, s>>>(as);
+    k_aug_sources<<<dim3(grid_for(sparse ? nJC : std::max(nJB, nJC)), 2), BLK, 0, s>>>(J, as);
     SC_HIP(hipGetLastError());
     if (I > 0) {
-        if (!sparse)
-            k_aug_segments<true><<<grid_for(I), BLK, 0, s>>>(c.p_b, c.p_j, I, c.ordB, ja.JB, nba, all_b, nd_b,
-                                                             c.p_type, c.p_x, c.p_y, c.p_qa, c.aug_bx, c.aug_by,
-                                                             c.av_b, c.slot_b, flags, spb);
-        k_aug_segments<false><<<grid_for(I), BLK, 0, s>>>(c.p_c, c.p_j, I, c.ordC, ja.JC, nca, all_c, nd_c,
-                                                          c.p_type, c.p_x, c.p_y, c.p_qb, c.aug_cx, c.aug_cy, c.av_c,
-                                                          c.slot_c, flags, spc);
+        k_aug_segments<<<dim3(grid_for(I), 2), BLK, 0, s>>>(c.p_j, I, c.p_type, c.p_x, c.p_y, flags, as);
         SC_HIP(hipGetLastError());
         if (sparse) {
             k_sp_link<<<grid_for(I), BLK, 0, s>>>(I, c.sp_pos, c.p_j, c.sp_slot, c.slot_c, nca, int(nca_tot),

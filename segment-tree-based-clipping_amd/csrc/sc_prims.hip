@@ -702,6 +702,12 @@ void scan_exclusive_u32_2(const uint32_t *in0, uint32_t *out0, int64_t n0, uint3
     const int64_t n[2] = {n0, n1};
     scan_u32_set<OpSum, false>(2, in, out, n, tot, s);
 }
+void scan_exclusive_u32_4(int count, uint32_t *const *inout, const int64_t *n, hipStream_t s) {
+    const uint32_t *in[SCAN_SET];
+    uint32_t *tot[SCAN_SET] = {};
+    for (int k = 0; k < count && k < SCAN_SET; ++k) in[k] = inout[k];
+    scan_u32_set<OpSum, false>(count, in, inout, n, tot, s);
+}
 void scan_inclusive_max_u32_2(const uint32_t *in0, uint32_t *out0, int64_t n0, const uint32_t *in1,
                               uint32_t *out1, int64_t n1, hipStream_t s) {
     const uint32_t *in[2] = {in0, in1};

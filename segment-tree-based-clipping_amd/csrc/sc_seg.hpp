@@ -42,13 +42,31 @@ template <int N> __device__ inline void reg_bitonic(uint64_t (&v)[N]) {
             }
 }
 
+// One set of groups: group offsets, keys, output, the lists of groups for a wave
+// and for a block, and their control words.  Up to two sets share each launch
+// (blockIdx.y picks one): at small sizes a launch costs more than its work.
+struct SegSet {
+    int nseg;
+    const int *scan;
+    const uint64_t *K;
+    void *out;
+    uint32_t *wlist, *blist, *ctl;
+};
+struct SegSets {
+    SegSet s[2];
+    int count;
+};
+
 // one thread per edge group: groups of up to SEG_THREAD sorted in registers,
 // larger ones listed for a wave or a block, groups beyond SEG_LDS_MAX reported
-template <bool FULL>
-__global__ void k_seg_small(int nseg, const int *__restrict__ scan, const uint64_t *__restrict__ K, void *out,
-                            uint32_t *wlist, uint32_t *blist, uint32_t *ctl) {
+template <bool FULL> __global__ void k_seg_small(SegSets a) {
+    const SegSet &q = a.s[blockIdx.y];
+    const int *__restrict__ scan = q.scan;
+    const uint64_t *__restrict__ K = q.K;
+    void *out = q.out;
+    uint32_t *wlist = q.wlist, *blist = q.blist, *ctl = q.ctl;
     const int g = blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= nseg) return;
+    if (g >= q.nseg) return;
     const int s = scan[g], n = scan[g + 1] - s;
     if (n <= 0) return;
     if (n == 1) {
@@ -118,10 +136,12 @@ __device__ inline void wave_sort(const uint64_t *__restrict__ K, int s, int n, v
 
 // one wave per listed group of SEG_THREAD+1..SEG_WAVE_MAX keys, with the
 // fewest keys per lane that hold the group
-template <bool FULL>
-__global__ __launch_bounds__(SEG_BLK) void k_seg_wave(const int *__restrict__ scan, const uint64_t *__restrict__ K,
-                                                  void *out, const uint32_t *__restrict__ wlist,
-                                                  const uint32_t *__restrict__ ctl) {
+template <bool FULL> __global__ __launch_bounds__(SEG_BLK) void k_seg_wave(SegSets a) {
+    const SegSet &q = a.s[blockIdx.y];
+    const int *__restrict__ scan = q.scan;
+    const uint64_t *__restrict__ K = q.K;
+    void *out = q.out;
+    const uint32_t *__restrict__ wlist = q.wlist, *__restrict__ ctl = q.ctl;
     const int lane = threadIdx.x & (WAVE - 1);
     const uint32_t nw = ctl[0];
     const uint32_t stride = gridDim.x * (SEG_BLK / WAVE);
@@ -136,10 +156,12 @@ __global__ __launch_bounds__(SEG_BLK) void k_seg_wave(const int *__restrict__ sc
 }
 
 // one block per listed group of SEG_WAVE_MAX+1..SEG_LDS_MAX keys: bitonic sort in LDS
-template <bool FULL>
-__global__ __launch_bounds__(SEG_BLK) void k_seg_block(const int *__restrict__ scan, const uint64_t *__restrict__ K,
-                                                   void *out, const uint32_t *__restrict__ blist,
-                                                   const uint32_t *__restrict__ ctl) {
+template <bool FULL> __global__ __launch_bounds__(SEG_BLK) void k_seg_block(SegSets a) {
+    const SegSet &q = a.s[blockIdx.y];
+    const int *__restrict__ scan = q.scan;
+    const uint64_t *__restrict__ K = q.K;
+    void *out = q.out;
+    const uint32_t *__restrict__ blist = q.blist, *__restrict__ ctl = q.ctl;
     __shared__ uint64_t sk[SEG_LDS_MAX];
     const uint32_t nb = ctl[1];
     for (uint32_t b = blockIdx.x; b < nb; b += gridDim.x) {
@@ -169,16 +191,17 @@ __global__ __launch_bounds__(SEG_BLK) void k_seg_block(const int *__restrict__ s
 }
 
 
-// the three launches for groups 0..nseg-1; wl and bl hold the listed groups
-// (capacity: more than SEG_THREAD, resp. SEG_WAVE_MAX keys per listed group),
-// ctl[0..SEG_CTL) is zero before the call
-template <bool FULL>
-inline void seg_sort(int nseg, const int *scan, const uint64_t *K, void *out, uint32_t *wl, uint32_t *bl,
-                     uint32_t *ctl, hipStream_t s) {
-    if (nseg <= 0) return;
-    k_seg_small<FULL><<<unsigned((nseg + SEG_BLK - 1) / SEG_BLK), SEG_BLK, 0, s>>>(nseg, scan, K, out, wl, bl, ctl);
-    k_seg_wave<FULL><<<1024, SEG_BLK, 0, s>>>(scan, K, out, wl, ctl);
-    k_seg_block<FULL><<<1280, SEG_BLK, 0, s>>>(scan, K, out, bl, ctl); // five 32 KB blocks per CU
+// the three launches for the groups of every set; wlist and blist hold the
+// listed groups (capacity: more than SEG_THREAD, resp. SEG_WAVE_MAX keys per
+// listed group), ctl[0..SEG_CTL) is zero before the call
+template <bool FULL> inline void seg_sort(const SegSets &a, hipStream_t s) {
+    int most = 0;
+    for (int k = 0; k < a.count; ++k) most = a.s[k].nseg > most ? a.s[k].nseg : most;
+    if (most <= 0) return;
+    const unsigned y = unsigned(a.count);
+    k_seg_small<FULL><<<dim3(unsigned((most + SEG_BLK - 1) / SEG_BLK), y), SEG_BLK, 0, s>>>(a);
+    k_seg_wave<FULL><<<dim3(1024, y), SEG_BLK, 0, s>>>(a);
+    k_seg_block<FULL><<<dim3(1280, y), SEG_BLK, 0, s>>>(a); // five 32 KB blocks per CU
     SC_HIP(hipGetLastError());
 }
 
