@@ -71,63 +71,87 @@ struct Side {
 
 __device__ inline bool inter_at(const Side &s, int64_t i) { return s.av ? s.av[i] != -100 : s.nbr[i] != -100; }
 
-// crossing flags; label and link checks
-__global__ void k_jclassify(Side s, int J, int64_t n, uint32_t *cross, int *slow) {
-    int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    int j = seg_of(s.off, J, i);
-    uint32_t c = 0;
-    if (inter_at(s, i)) {
-        int lab = s.lab[i];
-        if (lab != L_CROSSING && lab != L_BOUNCING) atomicOr(&slow[j], SLOW_LABEL);
-        int nb = s.nbr[i];
-        if (nb < 1 || nb > s.ooff[j + 1] - s.ooff[j]) atomicOr(&slow[j], SLOW_LINK);
-        c = lab == L_CROSSING ? 1u : 0u;
+// Crossing flags with their closing entry, label and link checks of both sides
+// (blockIdx.y 0: P, 1: Q), and the first plain vertex of each job's rings
+// (blockIdx.y 2: P, skipped for the sparse base; 3: Q).  At ordinary sizes the
+// stage is bound by its launches, not by their work, so steps of both sides share
+// one: two stars of 1,000 and 1,100 vertices are labelled in 0.24 ms instead of
+// 0.39, 20,000 against 51,000 in 0.30 instead of 0.39.
+struct ClassifyArgs {
+    Side s[2];
+    int J;
+    int64_t n[2];
+    uint32_t *cross[2];
+    int *slow, *first[2];
+};
+__global__ __launch_bounds__(BLK) void k_jclassify(ClassifyArgs a) {
+    const int y = blockIdx.y & 1;
+    const Side &s = a.s[y];
+    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (blockIdx.y < 2) {
+        if (i > a.n[y]) return;
+        uint32_t c = 0;
+        if (i < a.n[y] && inter_at(s, i)) {
+            const int j = seg_of(s.off, a.J, i); // only intersections look their job up
+            const int lab = s.lab[i];
+            if (lab != L_CROSSING && lab != L_BOUNCING) atomicOr(&a.slow[j], SLOW_LABEL);
+            const int nb = s.nbr[i];
+            if (nb < 1 || nb > s.ooff[j + 1] - s.ooff[j]) atomicOr(&a.slow[j], SLOW_LINK);
+            c = lab == L_CROSSING ? 1u : 0u;
+        }
+        a.cross[y][i] = c;
+        return;
     }
-    cross[i] = c;
-}
-
-// first plain vertex of each job's ring (local index, -1 if none): one wave per job
-__global__ __launch_bounds__(BLK) void k_first_plain(Side s, int J, int *first) {
-    const int j = int((int64_t(blockIdx.x) * blockDim.x + threadIdx.x) / WAVE);
-    const int lane = threadIdx.x & (WAVE - 1);
-    if (j >= J) return; // whole wave
-    const int64_t a = s.off[j], b = s.off[j + 1];
+    // first plain vertex (local index, -1 if none): one wave per job
+    const int j = int(i / WAVE), lane = threadIdx.x & (WAVE - 1);
+    if (!a.first[y] || j >= a.J) return; // whole wave
+    const int64_t b = s.off[j], e = s.off[j + 1];
     int res = -1;
-    for (int64_t base = a; base < b; base += WAVE) {
-        int64_t i = base + lane;
-        bool plain = i < b && !inter_at(s, i);
-        uint64_t m = __ballot(plain);
+    for (int64_t base = b; base < e; base += WAVE) {
+        const int64_t v = base + lane;
+        const uint64_t m = __ballot(v < e && !inter_at(s, v));
         if (m) {
-            res = int(base - a) + __ffsll((unsigned long long)m) - 1;
+            res = int(base - b) + __ffsll((unsigned long long)m) - 1;
             break;
         }
     }
-    if (lane == 0) first[j] = res;
+    if (lane == 0) a.first[y][j] = res;
 }
 
 // winding test of polygon::pointInPoly (polygon.h:435-457) of each job's
 // query point (the other ring's first plain vertex) against this side's
-// rings, summed per job
-__global__ __launch_bounds__(BLK) void k_jwinding(Side r, int J, int64_t n, const double *qx, const double *qy,
-                                                  const int *qok, int *wind) {
-    // qx[2j], qy[2j]: the query point of job j (interleaved x,y)
-    int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+// rings, summed per job; blockIdx.y picks the side (a null wind: not this way)
+struct WindSide {
+    Side r;
+    int64_t n;
+    const double *q; // query points, x,y per job
+    const int *ok;
+    int *wind;
+};
+struct WindSides {
+    WindSide s[2];
+    int J;
+};
+__global__ __launch_bounds__(BLK) void k_jwinding(WindSides a) {
+    const WindSide &z = a.s[blockIdx.y];
+    if (!z.wind) return;
+    const Side &r = z.r;
+    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     int w = 0, j = -1;
-    if (i < n) {
-        j = seg_of(r.off, J, i);
-        if (qok[j]) {
-            int64_t nx = i + 1 == r.off[j + 1] ? r.off[j] : i + 1;
-            w = wind_edge(r.x[i], r.y[i], r.x[nx], r.y[nx], qx[2 * j], qy[2 * j]);
+    if (i < z.n) {
+        j = seg_of_wave(r.off, a.J, i);
+        if (z.ok[j]) {
+            const int64_t nx = i + 1 == r.off[j + 1] ? r.off[j] : i + 1;
+            w = wind_edge(r.x[i], r.y[i], r.x[nx], r.y[nx], z.q[2 * j], z.q[2 * j + 1]);
         }
     }
     // a wave inside one job adds once; a wave across jobs adds per lane
     const int j0 = __shfl(j, 0, WAVE), j1 = __shfl(j, WAVE - 1, WAVE);
     if (j0 == j1 && j0 >= 0) {
         for (int d = WAVE / 2; d > 0; d >>= 1) w += __shfl_down(w, d, WAVE);
-        if ((threadIdx.x & (WAVE - 1)) == 0 && w) atomicAdd(&wind[j0], w);
+        if ((threadIdx.x & (WAVE - 1)) == 0 && w) atomicAdd(&z.wind[j0], w);
     } else if (w && j >= 0) {
-        atomicAdd(&wind[j], w);
+        atomicAdd(&z.wind[j], w);
     }
 }
 
@@ -241,10 +265,11 @@ __global__ void k_sp_wind_fix(int I, int J, SparseP sp, const double *__restrict
 
 // entry/exit status on the sparse base ring (positions = its intersections)
 __global__ void k_sp_enex(int I, int J, SparseP sp, const int *lab, const uint32_t *cross, const uint32_t *cc,
-                          const int *first, const int *wind, const int *kind, int *enex, uint8_t *split) {
+                          const int *first, const int *wind, const int *kind, int *enex, uint8_t *split, int *cpos) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= I) return;
-    const int j = seg_of(sp.P0, J, i);
+    if (cross[i]) cpos[cc[i]] = i;
+    const int j = seg_of_wave(sp.P0, J, i);
     if (kind[j] != K_CROSS) {
         enex[i] = NEITHER;
         split[i] = 0;
@@ -288,23 +313,39 @@ __global__ void k_jdecide(JobState s, const uint32_t *ccP, const uint32_t *ccQ) 
 // entry/exit status of every crossing vertex from the parity of crossings
 // since the first plain vertex V; bouncing vertices met with status EXIT are
 // split candidates (labelIntersections2 step 4, polyclip.h:551-635)
-__global__ void k_jenex(Side s, int J, int64_t n, const uint32_t *cross, const uint32_t *cc, const int *first,
-                        const int *wind, const int *kind, int *enex, uint8_t *split) {
-    int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    int j = seg_of(s.off, J, i);
-    if (kind[j] != K_CROSS) {
-        enex[i] = NEITHER;
-        split[i] = 0;
+struct EnexSide {
+    Side r;
+    int64_t n;
+    const uint32_t *cross, *cc;
+    const int *first, *wind;
+    int *enex;
+    uint8_t *split;
+    int *cpos; // crossing -> slot (null enex: not this side)
+};
+struct EnexSides {
+    EnexSide s[2];
+    int J;
+    const int *kind;
+};
+__global__ void k_jenex(EnexSides a) {
+    const EnexSide &z = a.s[blockIdx.y];
+    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (!z.enex || i >= z.n) return;
+    const uint32_t cr = z.cross[i], ci = z.cc[i];
+    if (cr) z.cpos[ci] = int(i);
+    const int j = seg_of_wave(z.r.off, a.J, i);
+    if (a.kind[j] != K_CROSS) {
+        z.enex[i] = NEITHER;
+        z.split[i] = 0;
         return;
     }
-    int64_t V = s.off[j] + first[j];
-    uint32_t m = cc[s.off[j + 1]] - cc[s.off[j]];
-    uint32_t c = cc[i] - cc[V] + (i < V ? m : 0u);
-    int st0 = (wind[j] % 2) != 0 ? EXIT : ENTRY;
-    int st = st0 ^ int(c & 1u);
-    enex[i] = cross[i] ? st : NEITHER;
-    split[i] = (inter_at(s, i) && s.lab[i] == L_BOUNCING && st == EXIT) ? 1 : 0;
+    const int64_t r0 = z.r.off[j], V = r0 + z.first[j];
+    const uint32_t m = z.cc[z.r.off[j + 1]] - z.cc[r0];
+    const uint32_t c = ci - z.cc[V] + (i < V ? m : 0u);
+    const int st0 = (z.wind[j] % 2) != 0 ? EXIT : ENTRY;
+    const int st = st0 ^ int(c & 1u);
+    z.enex[i] = cr ? st : NEITHER;
+    z.split[i] = (st == EXIT && inter_at(z.r, i) && z.r.lab[i] == L_BOUNCING) ? 1 : 0;
 }
 
 __global__ void k_jsplit_pairs(Side P, int J, int64_t nP, const uint8_t *splitP, const uint8_t *splitQ, int *slow) {
@@ -313,11 +354,6 @@ __global__ void k_jsplit_pairs(Side P, int J, int64_t nP, const uint8_t *splitP,
     int j = seg_of(P.off, J, i);
     int64_t q = P.ooff[j] + P.nbr[i] - 1;
     if (splitQ[q]) atomicOr(&slow[j], SLOW_SPLIT);
-}
-
-__global__ void k_compact_cross(int64_t n, const uint32_t *cross, const uint32_t *ccount, int *cpos) {
-    int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i < n && cross[i]) cpos[ccount[i]] = int(i);
 }
 
 struct PieceArgs {
@@ -407,15 +443,14 @@ __global__ void k_jpieces(PieceArgs a) {
     a.val[x] = onP ? min(2u * uint32_t(sl), 2u * uint32_t(slW) + 1u) : NIL;
 }
 
-// jobs found inconsistent while building pieces take the sequential route
-__global__ void k_jredecide(int J, const int *slow, int *kind) {
-    int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j < J && kind[j] == K_CROSS && slow[j]) kind[j] = K_SEQ;
-}
-
-__global__ void k_jmask(int M, const int *pj, const int *kind, uint32_t *succ, uint32_t *val) {
-    int x = blockIdx.x * blockDim.x + threadIdx.x;
-    if (x >= M || kind[pj[x]] == K_CROSS) return;
+// jobs found inconsistent while building pieces take the sequential route;
+// their crossings leave the graph (the other jobs' are in it only for K_CROSS)
+__global__ void k_jmask(int J, int M, const int *pj, const int *slow, int *kind, uint32_t *succ, uint32_t *val) {
+    const int x = blockIdx.x * blockDim.x + threadIdx.x;
+    if (x < J && kind[x] == K_CROSS && slow[x]) kind[x] = K_SEQ;
+    if (x >= M) return;
+    const int j = pj[x];
+    if (kind[j] == K_CROSS && !slow[j]) return;
     succ[x] = uint32_t(x);
     val[x] = NIL;
 }
@@ -430,14 +465,24 @@ __global__ void k_jmask(int M, const int *pj, const int *kind, uint32_t *succ, u
 // the P crossing after the window.  A window sum is read only when the window
 // holds no occurrence of the cycle's minimum, so does not wrap and stays below
 // the cycle's total; the 32-bit wrap-around of longer windows is never read.
-__global__ void k_jump_init(int mP, int M, const uint32_t *val, const uint32_t *succ, const int *plen, uint4 *rec) {
-    int x = blockIdx.x * blockDim.x + threadIdx.x;
-    if (x >= mP) return;
+__device__ inline uint4 jump_first(int x, int mP, int M, const uint32_t *val, const uint32_t *succ, const int *plen) {
     const uint32_t q = succ[x];
     uint32_t n2 = q < uint32_t(M) ? succ[q] : uint32_t(x);
     if (n2 >= uint32_t(mP)) n2 = uint32_t(x); // not a P-Q-P step: a crossing outside the traversed jobs
     const uint32_t w = uint32_t(plen[x]) + (q < uint32_t(M) && q != uint32_t(x) ? uint32_t(plen[q]) : 0u);
-    rec[x] = make_uint4(val[x], 0u, w, n2);
+    return make_uint4(val[x], 0u, w, n2);
+}
+__device__ inline uint4 jump_join(const uint4 &a, const uint4 &b) { // the window of a, then that of b
+    uint4 o;
+    o.x = a.x <= b.x ? a.x : b.x;
+    o.y = a.x <= b.x ? a.y : a.z + b.y;
+    o.z = a.z + b.z;
+    o.w = b.w;
+    return o;
+}
+__global__ void k_jump_init(int mP, int M, const uint32_t *val, const uint32_t *succ, const int *plen, uint4 *rec) {
+    const int x = blockIdx.x * blockDim.x + threadIdx.x;
+    if (x < mP) rec[x] = jump_first(x, mP, M, val, succ, plen);
 }
 
 // Round r doubles every window (2^r crossings to 2^(r+1)) and sets moved[r]
@@ -451,14 +496,45 @@ __global__ void k_jump_rank(int mP, const uint4 *__restrict__ rec, uint4 *__rest
     int x = blockIdx.x * blockDim.x + threadIdx.x;
     if (x >= mP) return;
     const uint4 a = rec[x];
-    const uint4 b = rec[a.w];
-    uint4 o;
-    o.x = a.x <= b.x ? a.x : b.x;
-    o.y = a.x <= b.x ? a.y : a.z + b.y;
-    o.z = a.z + b.z;
-    o.w = b.w;
+    const uint4 o = jump_join(a, rec[a.w]);
     rec2[x] = o;
     if (o.x != a.x) moved[r] = 1u;
+}
+
+// Every round of k_jump_rank for at most JUMP_SMALL P crossings, by one block
+// with the records in LDS (64 KB): a round is a barrier instead of a launch
+// (12 launches of 2.5 us and their gaps at 1,400 crossings).
+constexpr int JUMP_SMALL = 4096, JUMP_BLK = 1024, JUMP_PER = JUMP_SMALL / JUMP_BLK;
+__global__ __launch_bounds__(JUMP_BLK) void k_jump_small(int mP, int M, const uint32_t *val, const uint32_t *succ,
+                                                       const int *plen, int rounds, uint4 *rec) {
+    __shared__ uint4 r[JUMP_SMALL];
+    uint4 a[JUMP_PER];
+    for (int q = 0; q < JUMP_PER; ++q) {
+        const int x = q * JUMP_BLK + int(threadIdx.x);
+        if (x < mP) r[x] = a[q] = jump_first(x, mP, M, val, succ, plen);
+    }
+    __syncthreads();
+    for (int k = 0; k < rounds; ++k) {
+        int moved = 0;
+        for (int q = 0; q < JUMP_PER; ++q) {
+            const int x = q * JUMP_BLK + int(threadIdx.x);
+            if (x >= mP) continue;
+            const uint4 o = jump_join(a[q], r[a[q].w]);
+            moved |= o.x != a[q].x ? 1 : 0;
+            a[q] = o;
+        }
+        moved = __syncthreads_or(moved); // every record is read before the next round's are written
+        if (!moved) break;
+        for (int q = 0; q < JUMP_PER; ++q) {
+            const int x = q * JUMP_BLK + int(threadIdx.x);
+            if (x < mP) r[x] = a[q];
+        }
+        __syncthreads();
+    }
+    for (int q = 0; q < JUMP_PER; ++q) {
+        const int x = q * JUMP_BLK + int(threadIdx.x);
+        if (x < mP) rec[x] = a[q];
+    }
 }
 
 // Per crossing (P and Q): its cycle's minimum, the list start of a traversed
@@ -466,10 +542,13 @@ __global__ void k_jump_rank(int mP, const uint4 *__restrict__ rec, uint4 *__rest
 // value on the cycle is larger) and the summed piece lengths from the
 // crossing up to that start, the whole cycle's total at the start itself.
 // Equivalent to the list ranking of the cycle broken before its start.
+// For the P crossings also the ring starts and their totals in base-ring
+// order, each with a closing entry.
 __global__ void k_rank_final(int M, int mP, const uint4 *__restrict__ rec, const uint32_t *succ, const int *pj,
                              const int *AB, int sparse, SparseP sp, const uint32_t *ccountP, const int *plen,
-                             uint32_t *cmin, uint32_t *inode, uint32_t *dist) {
-    int x = blockIdx.x * blockDim.x + threadIdx.x;
+                             const int *ppos, uint32_t *inode, uint32_t *dist, uint32_t *tot, uint32_t *isstart) {
+    const int x = blockIdx.x * blockDim.x + threadIdx.x;
+    if (x == 0) tot[mP] = isstart[mP] = 0u;
     if (x >= M) return;
     // the P crossing whose record describes x's cycle: x itself, or a Q crossing's successor
     const uint32_t p = x < mP ? uint32_t(x) : succ[x];
@@ -486,7 +565,6 @@ __global__ void k_rank_final(int M, int mP, const uint4 *__restrict__ rec, const
         I = k >= 0 ? ccountP[k] : NIL;
         trav = k >= 0;
     }
-    cmin[x] = m;
     inode[x] = I;
     uint32_t d = 0u;
     if (trav) {
@@ -500,18 +578,11 @@ __global__ void k_rank_final(int M, int mP, const uint4 *__restrict__ rec, const
         }
     }
     dist[x] = d;
-}
-
-// component totals at their starts (base-ring order)
-__global__ void k_start_totals(int mP, const int *cposP, const int *pj, const int *AB, const int *pslot,
-                               const uint32_t *cmin, const uint32_t *dist, uint32_t *tot, uint32_t *isstart) {
-    int x = blockIdx.x * blockDim.x + threadIdx.x;
-    if (x >= mP) return;
-    uint32_t m = cmin[x];
-    const int sl = pslot ? pslot[cposP[x]] : cposP[x] - AB[pj[x]];
-    bool s = m != NIL && (m & 1u) == 0u && (m >> 1) == uint32_t(sl);
-    tot[x] = s ? dist[x] : 0u;
-    isstart[x] = s ? 1u : 0u;
+    if (x < mP) { // ppos: the crossing's slot on its ring
+        const bool st = m != NIL && (m & 1u) == 0u && (m >> 1) == uint32_t(ppos[x]);
+        tot[x] = st ? d : 0u;
+        isstart[x] = st ? 1u : 0u;
+    }
 }
 
 struct CountArgs {
@@ -524,7 +595,11 @@ struct CountArgs {
 // output vertices and rings of every job before clean-up
 __global__ void k_jcounts(CountArgs a) {
     int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= a.J) return;
+    if (j > a.J) return;
+    if (j == a.J) { // closing entries of their scans
+        a.jv[j] = a.jr[j] = 0u;
+        return;
+    }
     uint32_t v = 0, r = 0;
     const int k = a.kind[j];
     if (k == K_CROSS) {
@@ -543,22 +618,18 @@ __global__ void k_jcounts(CountArgs a) {
     a.jr[j] = r;
 }
 
-__global__ void k_jring_offsets(int mP, const uint32_t *isstart, const uint32_t *ridx, const uint32_t *base,
-                                const int *pj, const int *cP0, const uint32_t *JV, const uint32_t *JR, int *off) {
-    int x = blockIdx.x * blockDim.x + threadIdx.x;
-    if (x >= mP || !isstart[x]) return;
-    int j = pj[x];
-    off[JR[j] + ridx[x] - ridx[cP0[j]]] = int(JV[j] + base[x] - base[cP0[j]]);
-}
-
-__global__ void k_jheads(int M, const uint32_t *inode, const uint32_t *dist, const uint32_t *base, const int *pj,
-                         const int *cP0, const uint32_t *JV, uint32_t *head, uint32_t *piece_at) {
-    int x = blockIdx.x * blockDim.x + threadIdx.x;
+// every piece's first output vertex carries the piece; ring offsets at the starts
+__global__ void k_jheads(int M, int mP, const uint32_t *inode, const uint32_t *dist, const uint32_t *base,
+                         const uint32_t *ridx, const int *pj, const int *cP0, const uint32_t *JV, const uint32_t *JR,
+                         uint32_t *head, uint32_t *piece_at, int *off) {
+    const int x = blockIdx.x * blockDim.x + threadIdx.x;
     if (x >= M) return;
-    uint32_t I = inode[x];
+    const int j = pj[x];
+    const int c0 = cP0[j];
+    if (x < mP && ridx[x + 1] != ridx[x]) off[JR[j] + ridx[x] - ridx[c0]] = int(JV[j] + base[x] - base[c0]);
+    const uint32_t I = inode[x];
     if (I == NIL) return;
-    int j = pj[x];
-    uint32_t o = JV[j] + (base[I] - base[cP0[j]]) + (dist[I] - dist[x]);
+    const uint32_t o = JV[j] + (base[I] - base[c0]) + (dist[I] - dist[x]);
     head[o] = o;
     piece_at[o] = uint32_t(x);
 }
@@ -579,7 +650,7 @@ struct EmitArgs {
 __global__ void k_jemit(EmitArgs a, int64_t n_out) {
     int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i >= n_out) return;
-    const int j = seg_of(reinterpret_cast<const int *>(a.JV), a.J, i);
+    const int j = seg_of_wave(reinterpret_cast<const int *>(a.JV), a.J, i);
     if (a.kind[j] != K_CROSS) return;
     uint32_t s = a.head[i];
     uint32_t x = a.piece_at[s];
@@ -916,20 +987,17 @@ __global__ void k_ring_counts(int nr, const int *off, const uint32_t *kscan, uin
     nonempty[r] = c > 0u ? 1u : 0u;
 }
 
+// the vertices kept, and the offsets of the rings that have any (with the closing one)
 __global__ void k_compact_out(int64_t n, const uint32_t *keep, const uint32_t *kscan, const double *x,
-                              const double *y, const int *src, double *x2, double *y2, int *src2) {
-    int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+                              const double *y, const int *src, double *x2, double *y2, int *src2, int nr,
+                              const uint32_t *cnt, const uint32_t *nonempty, const int *off, int *off2) {
+    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i <= nr && (i == nr || cnt[i])) off2[nonempty[i]] = int(kscan[off[i]]);
     if (i >= n || !keep[i]) return;
-    x2[kscan[i]] = x[i];
-    y2[kscan[i]] = y[i];
-    src2[kscan[i]] = src[i];
-}
-
-__global__ void k_ring_off_final(int nr, const uint32_t *cnt, const uint32_t *rscan, const uint32_t *nonempty,
-                                 const int *off, const uint32_t *kscan, int *off2) {
-    int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= nr) return;
-    if (cnt[r]) off2[nonempty[r]] = int(kscan[off[r]]);
+    const uint32_t o = kscan[i];
+    x2[o] = x[i];
+    y2[o] = y[i];
+    src2[o] = src[i];
 }
 
 __global__ void k_job_rings(int J, const uint32_t *jr, const uint32_t *nonempty, uint32_t *out) {
@@ -2150,14 +2218,14 @@ struct FosterScratch {
     DBuf<uint8_t> splitP, splitQ;
     DBuf<int> ppos, plen, pdir, pj;
     DBuf<uint4> jrec, jrec2; // doubling records of the crossing cycles
-    DBuf<uint32_t> succ, val, val2, inode, dist, tot, isstart, ringidx, head, piece_at;
+    DBuf<uint32_t> succ, val, ringid, inode, dist, tot, isstart, ringidx, head, piece_at;
     DBuf<int> jst;
     DBuf<uint32_t> jv, jr;
     DBuf<double> ox, oy, qpts, mx, my, nx0, ny0, nx1, ny1, vx1, vy1;
     DBuf<int> osrc, qoks, mav, mnbr, mlab, mjob, nslot, ninter, nlab, nnb, nlen, vlen, vslot, seen;
     DBuf<int64_t> moff, segoff, nodeoff;
     DBuf<uint32_t> nflag, nidx;
-    DBuf<int> off, rstart, ringid;
+    DBuf<int> off, rstart;
     DBuf<uint32_t> keep, kscan, rcnt, nonempty, kctl, ktstate;
     // sequential route
     DBuf<SeqJob> sjobs;
@@ -2183,9 +2251,9 @@ template <class T> void d2h_sync(Ctx &c, T *h, const T *d, int64_t n) {
     rb.run();
 }
 
-// clean-up of nr rings laid out at off[0..nr] in (ox, oy, osrc); result into
-// Ctx; ring_idx[r] = index of ring r among the non-empty rings (nr+1 entries)
-// clean-up of the rings; job_ring gets, per job, its first ring after it (J+1
+// clean-up of nr rings laid out at off[0..nr] in (ox, oy, osrc), the vertices'
+// rings in ringid and keep's closing entry and the round flags cleared by the
+// caller; result into Ctx.  job_ring gets, per job, its first ring after it (J+1
 // entries, from the jobs' first rings before it, jr on the device)
 void cleanup_rings(Ctx &c, FosterScratch &f, int nr, int64_t n, int J, const uint32_t *jr,
                    std::vector<uint32_t> &job_ring) {
@@ -2199,29 +2267,15 @@ void cleanup_rings(Ctx &c, FosterScratch &f, int nr, int64_t n, int J, const uin
         return;
     }
     int *rstart = f.rstart.ensure(nr);
-    int *ringid = f.ringid.ensure(size_t(n));
     k_root_loop<<<grid_for(nr), BLK, 0, s>>>(nr, f.off, f.ox, f.oy, rstart);
-    {
-        FillBatch fb(s);
-        fb.add(ringid, n, 0u);
-        fb.flush();
-    }
-    k_ring_heads<<<grid_for(nr), BLK, 0, s>>>(nr, f.off, reinterpret_cast<uint32_t *>(ringid));
-    scan_inclusive_max_u32(reinterpret_cast<uint32_t *>(ringid), reinterpret_cast<uint32_t *>(ringid), n, s);
-    uint32_t *keep = f.keep.ensure(size_t(n) + 1);
+    uint32_t *keep = f.keep;
     const int64_t ntiles = (n + KEEP_TILE - 1) / KEEP_TILE;
-    uint32_t *changed = f.kctl.ensure(KEEP_ROUNDS);
+    uint32_t *changed = f.kctl;
     uint32_t *state = f.ktstate.ensure(3 * size_t(ntiles));
     uint32_t *nonempty = f.nonempty.ensure(size_t(nr) + 1);
-    {
-        FillBatch fb(s);
-        fb.add(changed, KEEP_ROUNDS, 0u);
-        fb.add(keep + n, 1, 0u); // closing entry of the scan below
-        fb.flush();
-    }
     KeepArgs ka;
     ka.n = n;
-    ka.ringid = ringid;
+    ka.ringid = reinterpret_cast<const int *>(f.ringid.p);
     ka.off = f.off;
     ka.rstart = rstart;
     ka.x = f.ox;
@@ -2277,15 +2331,10 @@ void cleanup_rings(Ctx &c, FosterScratch &f, int nr, int64_t n, int J, const uin
     c.d_ring_y.ensure(nout);
     c.d_ring_src.ensure(nout);
     int *off2 = c.d_ring_off.ensure(size_t(c.nrings) + 1);
-    k_compact_out<<<grid_for(n), BLK, 0, s>>>(n, keep, kscan, f.ox, f.oy, f.osrc, c.d_ring_x, c.d_ring_y,
-                                              c.d_ring_src);
-    k_ring_off_final<<<grid_for(nr), BLK, 0, s>>>(nr, rcnt, nullptr, nonempty, f.off, kscan, off2);
+    k_compact_out<<<grid_for(std::max(n, int64_t(nr) + 1)), BLK, 0, s>>>(n, keep, kscan, f.ox, f.oy, f.osrc,
+                                                                        c.d_ring_x, c.d_ring_y, c.d_ring_src, nr,
+                                                                        rcnt, nonempty, f.off, off2);
     SC_HIP(hipGetLastError());
-    {
-        FillBatch fb(s);
-        fb.add(off2 + c.nrings, 1, uint32_t(int(nout)));
-        fb.flush();
-    }
     c.wait();
 }
 
@@ -2293,7 +2342,7 @@ void cleanup_rings(Ctx &c, FosterScratch &f, int nr, int64_t n, int J, const uin
 
 void release_foster_scratch() {
     FosterScratch &f = fscratch();
-    for (DBuf<uint32_t> *b : {&f.jring, &f.crossP, &f.crossQ, &f.ccP, &f.ccQ, &f.succ, &f.val, &f.val2,
+    for (DBuf<uint32_t> *b : {&f.jring, &f.crossP, &f.crossQ, &f.ccP, &f.ccQ, &f.succ, &f.val, &f.ringid,
                               &f.inode, &f.dist, &f.tot, &f.isstart, &f.ringidx, &f.head, &f.piece_at,
                               &f.jv, &f.jr, &f.keep, &f.kscan, &f.rcnt, &f.nonempty, &f.kctl, &f.ktstate,
                               &f.jmoved})
@@ -2306,7 +2355,7 @@ void release_foster_scratch() {
     f.jrec.release();
     f.jrec2.release();
     for (DBuf<int> *b : {&f.enexP, &f.enexQ, &f.cposP, &f.cposQ, &f.ppos, &f.plen, &f.pdir, &f.pj, &f.jst,
-                         &f.osrc, &f.off, &f.rstart, &f.ringid, &f.sres, &f.sroff, &f.sosrc, &f.nx, &f.pv, &f.nb,
+                         &f.osrc, &f.off, &f.rstart, &f.sres, &f.sroff, &f.sosrc, &f.nx, &f.pv, &f.nb,
                          &f.lab, &f.enex, &f.vsrc, &f.cand})
         b->release();
     for (DBuf<double> *b : {&f.ox, &f.oy, &f.vx, &f.vy, &f.sox, &f.soy, &f.qpts, &f.mx, &f.my, &f.nx0, &f.ny0,
@@ -2366,18 +2415,21 @@ void label_and_traverse(Ctx &c) {
     st.cQ0 = jw + 9 * J + 1;      // J+1
     int *sidx = jw + 10 * J + 2;  // J
     uint32_t *crossP = f.crossP.ensure(nP + 1), *crossQ = f.crossQ.ensure(nQ + 1);
-    if (nP > 0) k_jclassify<<<grid_for(nP), BLK, 0, s>>>(P, J, nP, crossP, st.slow);
-    k_jclassify<<<grid_for(nQ), BLK, 0, s>>>(Q, J, nQ, crossQ, st.slow);
+    ClassifyArgs cl;
+    cl.s[0] = P;
+    cl.s[1] = Q;
+    cl.J = J;
+    cl.n[0] = nP;
+    cl.n[1] = nQ;
+    cl.cross[0] = crossP;
+    cl.cross[1] = crossQ;
+    cl.slow = st.slow;
+    cl.first[0] = sparse ? nullptr : st.firstP;
+    cl.first[1] = st.firstQ;
+    const int64_t most = std::max(nP, nQ); // slots of the larger side
+    k_jclassify<<<dim3(grid_for(std::max(most + 1, int64_t(J) * WAVE)), 4), BLK, 0, s>>>(cl);
     if (sparse) k_sp_first_plain<<<grid_for(int64_t(J) * WAVE), BLK, 0, s>>>(sp, J, st.firstP);
-    else k_first_plain<<<grid_for(int64_t(J) * WAVE), BLK, 0, s>>>(P, J, st.firstP);
-    k_first_plain<<<grid_for(int64_t(J) * WAVE), BLK, 0, s>>>(Q, J, st.firstQ);
     SC_HIP(hipGetLastError());
-    {
-        FillBatch fb(s);
-        fb.add(crossP + nP, 1, 0u);
-        fb.add(crossQ + nQ, 1, 0u);
-        fb.flush();
-    }
     uint32_t *ccP = f.ccP.ensure(nP + 1), *ccQ = f.ccQ.ensure(nQ + 1);
     uint32_t *tot = c.d_u32_total.ensure(2);
     scan_exclusive_u32_2(crossP, ccP, nP + 1, tot, crossQ, ccQ, nQ + 1, tot + 1, s);
@@ -2388,13 +2440,15 @@ void label_and_traverse(Ctx &c) {
     int *pok = qoks, *qok = qoks + J;
     k_query_pts<<<grid_for(J), BLK, 0, s>>>(J, P, Q, sparse ? 1 : 0, sp, st.firstP, st.firstQ, pq, pok, qq, qok);
     SC_HIP(hipGetLastError());
-    k_jwinding<<<grid_for(nQ), BLK, 0, s>>>(Q, J, nQ, pq, pq + 1, pok, st.windP);
+    WindSides wd;
+    wd.s[0] = WindSide{Q, nQ, pq, pok, st.windP};
+    wd.s[1] = WindSide{P, nP, qq, qok, sparse ? nullptr : st.windQ};
+    wd.J = J;
+    k_jwinding<<<dim3(grid_for(sparse ? nQ : most), sparse ? 1 : 2), BLK, 0, s>>>(wd);
     if (sparse) {
         const int chunks = (c.nb + WCH - 1) / WCH;
         k_sp_wind_base<<<unsigned(int64_t(J) * chunks), BLK, 0, s>>>(J, c.nb, c.bpoly, qq, qok, st.windQ);
         if (nP > 0) k_sp_wind_fix<<<grid_for(nP), BLK, 0, s>>>(int(nP), J, sp, qq, qok, st.windQ);
-    } else {
-        k_jwinding<<<grid_for(nP), BLK, 0, s>>>(P, J, nP, qq, qq + 1, qok, st.windQ);
     }
     k_jdecide<<<grid_for(J + 1), BLK, 0, s>>>(st, ccP, ccQ);
     SC_HIP(hipGetLastError());
@@ -2419,17 +2473,17 @@ void label_and_traverse(Ctx &c) {
     uint8_t *splitP = f.splitP.ensure(nP), *splitQ = f.splitQ.ensure(nQ);
     PieceArgs pa;
     if (M > 0) {
+        int *cposP = f.cposP.ensure(mP + 1), *cposQ = f.cposQ.ensure(mQ + 1);
         if (sparse)
             k_sp_enex<<<grid_for(nP), BLK, 0, s>>>(int(nP), J, sp, c.sp_lab, crossP, ccP, st.firstP, st.windP,
-                                                   st.kind, enexP, splitP);
-        else
-            k_jenex<<<grid_for(nP), BLK, 0, s>>>(P, J, nP, crossP, ccP, st.firstP, st.windP, st.kind, enexP,
-                                                 splitP);
-        k_jenex<<<grid_for(nQ), BLK, 0, s>>>(Q, J, nQ, crossQ, ccQ, st.firstQ, st.windQ, st.kind, enexQ, splitQ);
+                                                   st.kind, enexP, splitP, cposP);
+        EnexSides en;
+        en.s[0] = EnexSide{Q, nQ, crossQ, ccQ, st.firstQ, st.windQ, enexQ, splitQ, cposQ};
+        en.s[1] = EnexSide{P, nP, crossP, ccP, st.firstP, st.windP, sparse ? nullptr : enexP, splitP, cposP};
+        en.J = J;
+        en.kind = st.kind;
+        k_jenex<<<dim3(grid_for(sparse ? nQ : most), sparse ? 1 : 2), BLK, 0, s>>>(en);
         k_jsplit_pairs<<<grid_for(nP), BLK, 0, s>>>(P, J, nP, splitP, splitQ, st.slow);
-        int *cposP = f.cposP.ensure(mP + 1), *cposQ = f.cposQ.ensure(mQ + 1);
-        k_compact_cross<<<grid_for(nP), BLK, 0, s>>>(nP, crossP, ccP, cposP);
-        k_compact_cross<<<grid_for(nQ), BLK, 0, s>>>(nQ, crossQ, ccQ, cposQ);
         pa.J = J;
         pa.P = P;
         pa.Q = Q;
@@ -2457,17 +2511,20 @@ void label_and_traverse(Ctx &c) {
         pa.val = f.val.ensure(M);
         pa.slow = st.slow;
         k_jpieces<<<grid_for(M), BLK, 0, s>>>(pa);
-        k_jredecide<<<grid_for(J), BLK, 0, s>>>(J, st.slow, st.kind);
-        k_jmask<<<grid_for(M), BLK, 0, s>>>(M, pa.pj, st.kind, pa.succ, pa.val);
+        k_jmask<<<grid_for(std::max(M, J)), BLK, 0, s>>>(J, M, pa.pj, st.slow, st.kind, pa.succ, pa.val);
         SC_HIP(hipGetLastError());
     }
     // routes and crossing counts on the host
     std::vector<int> hk(3 * size_t(J));
-    d2h_sync(c, hk.data(), st.kind, 3 * int64_t(J));
+    js.reason.resize(size_t(J));
+    {
+        ReadBack rb(c);
+        rb.add(hk.data(), static_cast<const int *>(st.kind), 3 * size_t(J));
+        rb.add(js.reason.data(), static_cast<const int *>(st.slow), size_t(J));
+        rb.run();
+    }
     const int *hkind = hk.data(), *hmP = hk.data() + J, *hmQ = hk.data() + 2 * J;
     js.route.assign(hkind, hkind + J);
-    js.reason.resize(size_t(J));
-    SC_HIP(hipMemcpyAsync(js.reason.data(), st.slow, sizeof(int) * size_t(J), hipMemcpyDeviceToHost, s));
     int maxm = 0, maxmP = 0; // crossings of the largest traversed job, and its P crossings
     std::vector<int> seq_jobs;
     bool any_nocross = false;
@@ -2636,14 +2693,17 @@ void label_and_traverse(Ctx &c) {
         SC_HIP(hipEventRecord(c.ev_join, c.stream2));
     }
     // cycles of the crossing jobs: minimum and distance to it by doubling
-    uint32_t *cmin = nullptr, *dist = nullptr, *inode = nullptr;
+    uint32_t *dist = nullptr, *inode = nullptr;
     uint32_t *base = f.tot.ensure(int64_t(mP) + 1), *ridx = f.ringidx.ensure(int64_t(mP) + 1);
     if (maxm > 0) {
-        uint4 *rec = f.jrec.ensure(mP > 0 ? mP : 1), *rec2 = f.jrec2.ensure(mP > 0 ? mP : 1);
-        if (mP > 0) {
+        uint4 *rec = f.jrec.ensure(mP > 0 ? mP : 1);
+        // a cycle of a traversed job holds at most maxmP P crossings
+        const int rounds = ilog2_exact(maxmP);
+        if (mP > 0 && mP <= JUMP_SMALL) {
+            k_jump_small<<<1, JUMP_BLK, 0, s>>>(mP, M, pa.val, pa.succ, pa.plen, rounds, rec);
+        } else if (mP > 0) {
+            uint4 *rec2 = f.jrec2.ensure(mP);
             k_jump_init<<<grid_for(mP), BLK, 0, s>>>(mP, M, pa.val, pa.succ, pa.plen, rec);
-            // a cycle of a traversed job holds at most maxmP P crossings
-            const int rounds = ilog2_exact(maxmP);
             uint32_t *moved = f.jmoved.ensure(size_t(rounds > 0 ? rounds : 1));
             {
                 FillBatch fb(s);
@@ -2655,21 +2715,11 @@ void label_and_traverse(Ctx &c) {
                 std::swap(rec, rec2);
             }
         }
-        cmin = f.val2.ensure(M);
         inode = f.inode.ensure(M);
         dist = f.dist.ensure(M);
-        k_rank_final<<<grid_for(M), BLK, 0, s>>>(M, mP, rec, pa.succ, pa.pj, AB, sparse ? 1 : 0, sp, ccP, pa.plen, cmin,
-                                                 inode, dist);
-        SC_HIP(hipGetLastError());
         uint32_t *isstart = f.isstart.ensure(int64_t(mP) + 1);
-        k_start_totals<<<grid_for(mP), BLK, 0, s>>>(mP, pa.cposP, pa.pj, AB, sparse ? c.sp_slot.p : nullptr, cmin,
-                                                    dist, base, isstart);
-        {
-            FillBatch fb(s);
-            fb.add(base + mP, 1, 0u);
-            fb.add(isstart + mP, 1, 0u);
-            fb.flush();
-        }
+        k_rank_final<<<grid_for(M), BLK, 0, s>>>(M, mP, rec, pa.succ, pa.pj, AB, sparse ? 1 : 0, sp, ccP, pa.plen,
+                                                 pa.ppos, inode, dist, base, isstart);
         SC_HIP(hipGetLastError());
         scan_exclusive_u32_2(base, base, int64_t(mP) + 1, nullptr, isstart, ridx, int64_t(mP) + 1, nullptr, s);
     }
@@ -2690,14 +2740,8 @@ void label_and_traverse(Ctx &c) {
     ca.jv = jv;
     ca.jr = jr;
     if (nseq > 0) SC_HIP(hipStreamWaitEvent(s, c.ev_join, 0));
-    k_jcounts<<<grid_for(J), BLK, 0, s>>>(ca);
+    k_jcounts<<<grid_for(int64_t(J) + 1), BLK, 0, s>>>(ca);
     SC_HIP(hipGetLastError());
-    {
-        FillBatch fb(s);
-        fb.add(jv + J, 1, 0u);
-        fb.add(jr + J, 1, 0u);
-        fb.flush();
-    }
     scan_exclusive_u32_2(jv, jv, int64_t(J) + 1, tot, jr, jr, int64_t(J) + 1, tot + 1, s);
     d2h_sync(c, htot, tot, 2);
     const int64_t NV = htot[0];
@@ -2706,17 +2750,48 @@ void label_and_traverse(Ctx &c) {
     f.oy.ensure(NV + 1);
     f.osrc.ensure(NV + 1);
     int *off = f.off.ensure(int64_t(NR) + 1);
-    if (maxm > 0 && NV > 0) {
-        k_jring_offsets<<<grid_for(mP), BLK, 0, s>>>(mP, f.isstart, ridx, base, pa.pj, st.cP0, jv, jr, off);
-        uint32_t *head = f.head.ensure(NV + 1), *piece_at = f.piece_at.ensure(NV + 1);
-        {
-            FillBatch fb(s);
-            fb.add(head, NV + 1, 0u);
-            fb.flush();
-        }
-        k_jheads<<<grid_for(M), BLK, 0, s>>>(M, inode, dist, base, pa.pj, st.cP0, jv, head, piece_at);
+    // the rings' first vertices and the pieces' by position, each the maximum up
+    // to it after one scan of both; ring offsets come from every route first
+    uint32_t *head = f.head.ensure(NV + 1), *piece_at = f.piece_at.ensure(NV + 1);
+    uint32_t *ringid = f.ringid.ensure(size_t(NV) + 1);
+    const bool cross = maxm > 0 && NV > 0;
+    {
+        FillBatch fb(s);
+        fb.add(off + NR, 1, uint32_t(int(NV)));
+        fb.add(head, cross ? NV : 0, 0u);
+        fb.add(ringid, NV, 0u);
+        fb.add(f.keep.ensure(size_t(NV) + 1) + NV, 1, 0u); // closing entry of the clean-up's scan
+        fb.add(f.kctl.ensure(KEEP_ROUNDS), KEEP_ROUNDS, 0u);
+        fb.flush();
+    }
+    if (cross)
+        k_jheads<<<grid_for(M), BLK, 0, s>>>(M, mP, inode, dist, base, ridx, pa.pj, st.cP0, jv, jr, head, piece_at,
+                                             off);
+    SC_HIP(hipGetLastError());
+    if (any_nocross) {
+        if (sparse)
+            k_sp_nocross_p<<<grid_for(NV), BLK, 0, s>>>(NV, J, jv, st.kind, st.windP, sp, f.ox, f.oy, f.osrc);
+        else
+            k_jcopy_nocross<<<grid_for(nP), BLK, 0, s>>>(P, true, J, nP, st.kind, st.windP, st.windQ, AB, jv, f.ox,
+                                                         f.oy, f.osrc);
+        k_jcopy_nocross<<<grid_for(nQ), BLK, 0, s>>>(Q, false, J, nQ, st.kind, st.windP, st.windQ, AB, jv, f.ox,
+                                                     f.oy, f.osrc);
+        k_jnocross_off<<<grid_for(J), BLK, 0, s>>>(J, st.kind, st.windP, st.windQ, AB, jv, jr, off);
         SC_HIP(hipGetLastError());
-        scan_inclusive_max_u32(head, head, NV, s);
+    }
+    std::vector<int> hres(3 * size_t(nseq));
+    if (nseq > 0) {
+        if (walked) walk_emit(wi, done, jv, jr, f.ox, f.oy, f.osrc, off, s);
+        k_jseq_copy<<<nseq, BLK, 0, s>>>(f.sjobs, walked ? done : nullptr, f.sres, jv, jr, f.sox, f.soy, f.sosrc, f.sroff, f.ox, f.oy,
+                                          f.osrc, off);
+        SC_HIP(hipGetLastError());
+    }
+    if (NR > 0 && NV > 0) {
+        k_ring_heads<<<grid_for(NR), BLK, 0, s>>>(NR, off, ringid);
+        SC_HIP(hipGetLastError());
+        scan_inclusive_max_u32_2(ringid, ringid, NV, head, head, cross ? NV : 0, s);
+    }
+    if (cross) {
         EmitArgs ea;
         ea.J = J;
         ea.mP = mP;
@@ -2737,29 +2812,6 @@ void label_and_traverse(Ctx &c) {
         ea.osrc = f.osrc;
         k_jemit<<<grid_for(NV), BLK, 0, s>>>(ea, NV);
         SC_HIP(hipGetLastError());
-    }
-    if (any_nocross) {
-        if (sparse)
-            k_sp_nocross_p<<<grid_for(NV), BLK, 0, s>>>(NV, J, jv, st.kind, st.windP, sp, f.ox, f.oy, f.osrc);
-        else
-            k_jcopy_nocross<<<grid_for(nP), BLK, 0, s>>>(P, true, J, nP, st.kind, st.windP, st.windQ, AB, jv, f.ox,
-                                                         f.oy, f.osrc);
-        k_jcopy_nocross<<<grid_for(nQ), BLK, 0, s>>>(Q, false, J, nQ, st.kind, st.windP, st.windQ, AB, jv, f.ox,
-                                                     f.oy, f.osrc);
-        k_jnocross_off<<<grid_for(J), BLK, 0, s>>>(J, st.kind, st.windP, st.windQ, AB, jv, jr, off);
-        SC_HIP(hipGetLastError());
-    }
-    std::vector<int> hres(3 * size_t(nseq));
-    if (nseq > 0) {
-        if (walked) walk_emit(wi, done, jv, jr, f.ox, f.oy, f.osrc, off, s);
-        k_jseq_copy<<<nseq, BLK, 0, s>>>(f.sjobs, walked ? done : nullptr, f.sres, jv, jr, f.sox, f.soy, f.sosrc, f.sroff, f.ox, f.oy,
-                                          f.osrc, off);
-        SC_HIP(hipGetLastError());
-    }
-    {
-        FillBatch fb(s);
-        fb.add(off + NR, 1, uint32_t(int(NV)));
-        fb.flush();
     }
     if (nseq > 0) {
         ReadBack rb(c);
