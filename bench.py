@@ -16,7 +16,7 @@ GPU loop on a sample of the same pairs):
                 (log-uniform 8..20,000 vertices): one tree, every overlay
                 clipped in one batch
   small_pairs   16,384 pairs of 4..64-vertex rings: clip + area/IoU forward
-                (the persistent small-pair kernel; also replayed as a
+                (the small-pair kernel; also replayed as a
                 captured hipGraph, and on the staged path for comparison),
                 and forward + backward of the area / IoU
   large_pairs   256 pairs of 10k..200k-vertex harmonic stars: forward +

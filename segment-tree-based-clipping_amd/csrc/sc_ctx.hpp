@@ -168,7 +168,7 @@ struct Ctx {
     int stab_tiles = 2;
     // tuning: consecutive stab work units per wave (1..32); results do not depend on it
     int stab_upw = 2;
-    // independent pairs of up to 64 + 64 vertices clipped by the persistent
+    // independent pairs of up to 64 + 64 vertices clipped by the one-launch
     // small-pair kernel (1) or the staged path (0); results do not depend on it
     int uni = 0; // operation: 0 intersection, 1 union (UNION of foster/polyclip.h:39)
     int small_fused = 1;
@@ -185,9 +185,8 @@ struct Ctx {
         const double *bxy = nullptr, *cxy = nullptr;
         double *out4 = nullptr;
         DBuf<int> tables;      // job table and the rings' input / output offsets
-        DBuf<uint32_t> words;  // queue counter, fallback word
-        DBuf<int> fail, route, nv, nr, olen;
-        DBuf<double> ox, oy;
+        DBuf<uint32_t> words;  // fallback word
+        DBuf<int> fail, route, nv, nr;
     } pg;
 
     bool timing = false;
@@ -243,7 +242,7 @@ void post_overlay(Ctx &c, int k);      // A11-A15 for overlay k
 void label_and_traverse(Ctx &c);       // A16-A17 for the jobs of the last post_jobs
 void clip_all(Ctx &c, int k);          // full pipeline for one overlay
 void clip_jobs(Ctx &c, int k0, int k1); // full pipeline for overlays k0..k1 as one batch
-// paired batches of small rings in one persistent launch: whether batch k0..k1
+// paired batches of small rings in one launch: whether batch k0..k1
 // qualifies, and the clip (false: some pair needs the staged path; nothing
 // of the batch's results was written)
 bool small_batch_eligible(const Ctx &c, int k0, int k1);

@@ -2831,7 +2831,7 @@ void label_and_traverse(Ctx &c) {
 void clip_jobs(Ctx &c, int k0, int k1) {
     SC_REQUIRE(k0 >= 1 && k1 <= c.K && k0 <= k1, SC_EINVAL, "overlay index out of range");
     StageTimes t;
-    // independent small pairs: one persistent launch (sc_small.hip); a batch
+    // independent small pairs: one launch (sc_small.hip); a batch
     // it does not cover runs on the staged path below
     if (small_batch_eligible(c, k0, k1)) {
         for (int i = 0; i <= 6; ++i) c.mark(i);
