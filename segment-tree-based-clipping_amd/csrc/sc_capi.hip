@@ -240,7 +240,7 @@ void release_derived(Ctx &c) {
     for (DBuf<double> *b : {&c.ex0, &c.ey0, &c.ex1, &c.ey1, &c.estart, &c.eend, &c.uxs, &c.uxe, &c.eymin, &c.eymax,
                             &c.ea, &c.niv, &c.p_x, &c.p_y, &c.aug_bx, &c.aug_by, &c.aug_cx, &c.aug_cy})
         b->release();
-    for (DBuf<int> *b : {&c.sp_slot, &c.sp_ndx, &c.sp_edge, &c.sp_av, &c.sp_nbr, &c.sp_lab, &c.sp_pos, &c.sp_ndf})
+    for (DBuf<int> *b : {&c.sp_slot, &c.sp_ndx, &c.sp_edge, &c.sp_av, &c.sp_nbr, &c.sp_lab, &c.sp_pos, &c.sp_ndf, &c.run_start})
         b->release();
     for (DBuf<uint64_t> *b : {&c.join_box, &c.join_leaf, &c.join_tile}) b->release();
     c.join_ctl.release();
@@ -262,7 +262,7 @@ void release_derived(Ctx &c) {
                          &c.sv_c, &c.sp_c, &c.arr_b, &c.arr_c})
         b->release();
     for (DBuf<uint32_t> *b : {&c.lend_off, &c.lend_e, &c.mend_off, &c.mend_e, &c.cov_off, &c.cov_e, &c.cov_split,
-                              &c.d_pair_off, &c.u32a, &c.u32b, &c.u32c, &c.u32d, &c.lend_e_alt,
+                              &c.d_pair_off, &c.run_head, &c.u32a, &c.u32b, &c.u32c, &c.u32d, &c.lend_e_alt,
                               &c.ord_val, &c.ord_val_alt, &c.seg_wb, &c.seg_wc, &c.seg_bb,
                               &c.seg_bc, &c.seg_ctl})
         b->release();

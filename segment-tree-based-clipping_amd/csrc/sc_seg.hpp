@@ -1,9 +1,9 @@
 // Sorting of many small key groups (segments) at once, each group held at
 // [scan[g], scan[g+1]) of a u64 key array.  Keys inside a group must be
 // distinct or, where equal, interchangeable.  A group of up to SEG_THREAD
-// keys is sorted by a register bitonic network in one thread, up to
-// SEG_WAVE_MAX by a bitonic sort in one wave's registers (1, 2, 4 or 8 keys
-// per lane, no barriers), up to SEG_LDS_MAX in one block's LDS; a larger
+// keys is sorted by a register bitonic network in one thread, up to SEG_WAVE
+// placed by a wave, up to SEG_WAVE_MAX by a bitonic sort in one wave's
+// registers (2, 4 or 8 keys per lane, no barriers), up to SEG_LDS_MAX in one block's LDS; a larger
 // group is only reported (the caller then sorts another way).  The output is
 // the key's low word as an int (FULL = false) or the whole key.
 #pragma once
@@ -134,8 +134,23 @@ __device__ inline void wave_sort(const uint64_t *__restrict__ K, int s, int n, v
         if (base + r < n) seg_put<FULL>(out, s + base + r, v[r]);
 }
 
-// one wave per listed group of SEG_THREAD+1..SEG_WAVE_MAX keys, with the
-// fewest keys per lane that hold the group
+// Up to SEG_WAVE keys, one per lane: a key's place is the number of smaller keys
+// (equal ones by position), read lane by lane: as many steps as keys, where the
+// bitonic network takes 21 exchanges through LDS whatever their number.
+template <bool FULL>
+__device__ inline void wave_rank(const uint64_t *__restrict__ K, int s, int n, void *out, int lane) {
+    const uint64_t v = lane < n ? K[s + lane] : ~0ull;
+    const int lo = int(uint32_t(v)), hi = int(uint32_t(v >> 32));
+    int r = 0;
+    for (int i = 0; i < n; ++i) {
+        const uint64_t o = (uint64_t(uint32_t(__builtin_amdgcn_readlane(hi, i))) << 32) |
+                           uint32_t(__builtin_amdgcn_readlane(lo, i));
+        r += (o < v || (o == v && i < lane)) ? 1 : 0;
+    }
+    if (lane < n) seg_put<FULL>(out, s + r, v);
+}
+
+// one wave per listed group of SEG_THREAD+1..SEG_WAVE_MAX keys
 template <bool FULL> __global__ __launch_bounds__(SEG_BLK) void k_seg_wave(SegSets a) {
     const SegSet &q = a.s[blockIdx.y];
     const int *__restrict__ scan = q.scan;
@@ -146,9 +161,9 @@ template <bool FULL> __global__ __launch_bounds__(SEG_BLK) void k_seg_wave(SegSe
     const uint32_t nw = ctl[0];
     const uint32_t stride = gridDim.x * (SEG_BLK / WAVE);
     for (uint32_t w = blockIdx.x * (SEG_BLK / WAVE) + threadIdx.x / WAVE; w < nw; w += stride) {
-        const int g = int(wlist[w]);
-        const int s = scan[g], n = scan[g + 1] - s;
-        if (n <= SEG_WAVE) wave_sort<1, FULL>(K, s, n, out, lane);
+        const int g = __builtin_amdgcn_readfirstlane(int(wlist[w]));
+        const int s = __builtin_amdgcn_readfirstlane(scan[g]), n = __builtin_amdgcn_readfirstlane(scan[g + 1]) - s;
+        if (n <= SEG_WAVE) wave_rank<FULL>(K, s, n, out, lane);
         else if (n <= 2 * SEG_WAVE) wave_sort<2, FULL>(K, s, n, out, lane);
         else if (n <= 4 * SEG_WAVE) wave_sort<4, FULL>(K, s, n, out, lane);
         else wave_sort<8, FULL>(K, s, n, out, lane);
