@@ -420,18 +420,30 @@ __global__ void k_sp_link(int I, const int *__restrict__ pos, const int *__restr
     nbr_c[b] = a + 1;
 }
 
-__global__ void k_sp_init_labels(int I, int J, SparseP sp, const int *__restrict__ av, const int *__restrict__ nbr,
+__global__ void k_sp_init_labels(int I, const int *__restrict__ pj, SparseP sp, const int *__restrict__ nbr,
                                  const int *__restrict__ AC, const double *__restrict__ cx,
                                  const double *__restrict__ cy, int *lab, int *labc, int *flags) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= I) return;
     const int q = sp.slot[i];
     if (q < 0) return;
-    const int j = seg_of(sp.P0, J, i);
+    const int j = pj[i];
     const int nbaug = sp.AB[j + 1] - sp.AB[j], C0 = AC[j], ncaug = AC[j + 1] - C0;
     const int tm = q - 1 < 0 ? nbaug - 1 : q - 1;
     const int tp = q + 1 == nbaug ? 0 : q + 1;
-    const SlotInfo pm = sp_slot(sp, j, tm), pp = sp_slot(sp, j, tp);
+    // The slots beside q are held by the positions beside i or plain (slots ascend
+    // with the positions unless the job was flagged); at the ring's ends by the
+    // last position, or one past it, and by the first.
+    SlotInfo pm, pp;
+    if (flags[j] & UB_UNASSIGNED) {
+        pm = sp_slot(sp, j, tm);
+        pp = sp_slot(sp, j, tp);
+    } else {
+        const int a = sp.P0[j], b = sp.P0[j + 1];
+        const int last = sp.slot[b - 1] == nbaug - 1 ? b - 1 : b;
+        pm = sp_slot_at(sp, j, tm, q == 0 ? last : (i > a && sp.slot[i - 1] == tm ? i - 1 : i));
+        pp = sp_slot_at(sp, j, tp, q + 1 == nbaug ? a : i + 1);
+    }
     const int pMN = pm.pos >= 0 ? nbr[pm.pos] - 1 : -100;
     const int pPN = pp.pos >= 0 ? nbr[pp.pos] - 1 : -100;
     const int nId = nbr[i] - 1;
@@ -687,7 +699,7 @@ void post_jobs(Ctx &c, int k0, int k1) {
             k_sp_link<<<grid_for(I), BLK, 0, s>>>(I, c.sp_pos, c.p_j, c.sp_slot, c.slot_c, nca, int(nca_tot),
                                                   c.sp_nbr, c.nbr_c, flags);
             SC_HIP(hipGetLastError());
-            k_sp_init_labels<<<grid_for(I), BLK, 0, s>>>(I, J, sparse_view(c), c.sp_av, c.sp_nbr, nca, c.aug_cx,
+            k_sp_init_labels<<<grid_for(I), BLK, 0, s>>>(I, c.p_j, sparse_view(c), c.sp_nbr, nca, c.aug_cx,
                                                          c.aug_cy, c.sp_lab, c.lab_c, flags);
             SC_HIP(hipGetLastError());
         } else {

@@ -140,7 +140,7 @@ template <class T> void scan_impl(const T *in, T *out, int64_t n, T *d_total, hi
 }
 
 // ---------------------------------------------------------------------------
-// two-launch scan of u32 (exclusive sum, inclusive max)
+// two-launch scan of u32 (exclusive sum, inclusive max and last)
 // ---------------------------------------------------------------------------
 // The first launch reduces each 2048-item tile to one value; in the second,
 // each block combines the values of the tiles before its own (at most
@@ -153,6 +153,10 @@ constexpr int64_t PREF_TILES = 2048;
 struct OpSum {
     static __device__ uint32_t id() { return 0u; }
     static __device__ uint32_t f(uint32_t a, uint32_t b) { return a + b; }
+};
+struct OpLast { // the last value that is not zero
+    static __device__ uint32_t id() { return 0u; }
+    static __device__ uint32_t f(uint32_t a, uint32_t b) { return b ? b : a; }
 };
 struct OpMax {
     static __device__ uint32_t id() { return 0u; }
@@ -195,12 +199,20 @@ template <class Op> __device__ inline uint32_t block_excl_op(uint32_t x, uint32_
 template <class Op>
 __device__ inline void tile_reduce_body(const uint32_t *in, int64_t n, uint32_t *sums, uint32_t tile,
                                         uint32_t *s_wave) {
-    const int64_t base = int64_t(tile) * SCAN_TILE;
+    // a thread's items are consecutive, so an Op need not commute
+    const int64_t i0 = int64_t(tile) * SCAN_TILE + int64_t(threadIdx.x) * SCAN_ITEMS;
     uint32_t acc = Op::id();
+    if (i0 + SCAN_ITEMS <= n && (reinterpret_cast<uintptr_t>(in) & 15) == 0) {
+        const uint4 *v = reinterpret_cast<const uint4 *>(in + i0);
 #pragma unroll
-    for (int it = 0; it < SCAN_ITEMS; ++it) {
-        const int64_t i = base + int64_t(it) * SCAN_BLOCK + threadIdx.x;
-        if (i < n) acc = Op::f(acc, in[i]);
+        for (int it = 0; it < SCAN_ITEMS / 4; ++it) {
+            const uint4 u = v[it];
+            acc = Op::f(Op::f(acc, u.x), u.y);
+            acc = Op::f(Op::f(acc, u.z), u.w);
+        }
+    } else {
+        for (int it = 0; it < SCAN_ITEMS; ++it)
+            if (i0 + it < n) acc = Op::f(acc, in[i0 + it]);
     }
     uint32_t total;
     (void)block_excl_op<Op>(acc, s_wave, total);
@@ -217,8 +229,10 @@ __device__ inline void tile_scan_body(const uint32_t *in, uint32_t *out, int64_t
                                       uint32_t *s_wave) {
     const int64_t base = int64_t(tile) * SCAN_TILE;
     uint32_t pacc = Op::id();
-    if (!pre)
-        for (uint32_t i = threadIdx.x; i < tile; i += SCAN_BLOCK) pacc = Op::f(pacc, sums[i]);
+    if (!pre) {
+        const uint32_t c = (tile + SCAN_BLOCK - 1) / SCAN_BLOCK, i0 = threadIdx.x * c;
+        for (uint32_t i = i0; i < i0 + c && i < tile; ++i) pacc = Op::f(pacc, sums[i]);
+    }
 #pragma unroll
     for (int it = 0; it < SCAN_ITEMS; ++it) {
         const int64_t i = base + int64_t(it) * SCAN_BLOCK + threadIdx.x;
@@ -729,6 +743,15 @@ void scan_inclusive_max_u32_2(const uint32_t *in0, uint32_t *out0, int64_t n0, c
     const int64_t n[2] = {n0, n1};
     if (n0 <= 0 && n1 <= 0) return;
     scan_u32_set<OpMax, true>(2, in, out, n, tot, s);
+}
+
+void scan_inclusive_last_u32_2(const uint32_t *in0, uint32_t *out0, int64_t n0, const uint32_t *in1,
+                               uint32_t *out1, int64_t n1, hipStream_t s) {
+    const uint32_t *in[2] = {in0, in1};
+    uint32_t *out[2] = {out0, out1}, *tot[2] = {nullptr, nullptr};
+    const int64_t n[2] = {n0, n1};
+    if (n0 <= 0 && n1 <= 0) return;
+    scan_u32_set<OpLast, true>(2, in, out, n, tot, s);
 }
 
 namespace {

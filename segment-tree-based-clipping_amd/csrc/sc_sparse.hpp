@@ -32,9 +32,8 @@ struct SlotInfo {
     double x, y;
 };
 
-// first position of job j whose slot is >= q
-__device__ inline int sp_lower(const SparseP &s, int j, int q) {
-    int lo = s.P0[j], hi = s.P0[j + 1];
+// first position in [lo, hi) whose slot is >= q, else hi
+__device__ inline int sp_lower_in(const SparseP &s, int q, int lo, int hi) {
     while (lo < hi) {
         int mid = (lo + hi) >> 1;
         if (s.slot[mid] < q) lo = mid + 1;
@@ -42,6 +41,7 @@ __device__ inline int sp_lower(const SparseP &s, int j, int q) {
     }
     return lo;
 }
+__device__ inline int sp_lower(const SparseP &s, int j, int q) { return sp_lower_in(s, q, s.P0[j], s.P0[j + 1]); }
 
 // position holding local slot q of job j, or -1
 __device__ inline int sp_find(const SparseP &s, int j, int q) {
@@ -49,10 +49,9 @@ __device__ inline int sp_find(const SparseP &s, int j, int q) {
     return (k < s.P0[j + 1] && s.slot[k] == q) ? k : -1;
 }
 
-// content of local slot q of job j
-__device__ inline SlotInfo sp_slot(const SparseP &s, int j, int q) {
+// content of local slot q of job j, whose first position with a slot >= q is k
+__device__ inline SlotInfo sp_slot_at(const SparseP &s, int j, int q, int k) {
     SlotInfo r;
-    const int k = sp_lower(s, j, q);
     if (k < s.P0[j + 1] && s.slot[k] == q) {
         r.pos = k;
         r.x = s.x[k];
@@ -68,6 +67,11 @@ __device__ inline SlotInfo sp_slot(const SparseP &s, int j, int q) {
     r.x = P[0];
     r.y = P[1];
     return r;
+}
+__device__ inline SlotInfo sp_slot(const SparseP &s, int j, int q) { return sp_slot_at(s, j, q, sp_lower(s, j, q)); }
+// the same where that position is known to lie in [lo, hi]
+__device__ inline SlotInfo sp_slot_in(const SparseP &s, int j, int q, int lo, int hi) {
+    return sp_slot_at(s, j, q, sp_lower_in(s, q, lo, hi));
 }
 
 // the winding test of polygon::pointInPoly (foster/polygon.h:435-457) for
