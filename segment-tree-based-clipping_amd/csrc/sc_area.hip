@@ -229,7 +229,7 @@ struct ProvArgs {
     const double *ox, *oy;
     const double *cI;
     const double *ring2; // signed 2A of every output ring
-    const int *sv_b, *sp_b, *sv_c, *sp_c;
+    const int *from_b, *from_c;
     const int *p_b, *p_c, *p_type;
     const int *bvoff, *beoff, *nb, *cvoff, *cin, *nc; // per job
     const double *bpoly, *cpoly;
@@ -308,16 +308,13 @@ __global__ void k_output_grad(ProvArgs a, int64_t v0, int64_t v1) {
         return;
     }
     if (s >= 0) {
-        const int v = a.sv_b[s];
+        const int v = a.from_b[s];
         if (v >= 0) add_b(a, j, v, gx, gy);
-        else if (a.sp_b[s] >= 0) pair_grad(a, j, a.sp_b[s], true, gx, gy);
-        else atomicOr(a.bad, 1);
+        else pair_grad(a, j, ~v, true, gx, gy);
     } else {
-        const int g = ~s;
-        const int v = a.sv_c[g];
+        const int v = a.from_c[~s];
         if (v >= 0) add_c(a, j, v, gx, gy);
-        else if (a.sp_c[g] >= 0) pair_grad(a, j, a.sp_c[g], false, gx, gy);
-        else atomicOr(a.bad, 1);
+        else pair_grad(a, j, ~v, false, gx, gy);
     }
 }
 
@@ -409,10 +406,8 @@ void batch_area_backward(Ctx &c, const double *g_area, const double *g_iou, doub
     p.oy = c.d_ring_y;
     p.cI = cI;
     p.ring2 = a.ring2;
-    p.sv_b = c.sv_b;
-    p.sp_b = c.sp_b;
-    p.sv_c = c.sv_c;
-    p.sp_c = c.sp_c;
+    p.from_b = c.from_b;
+    p.from_c = c.from_c;
     p.p_b = c.p_b;
     p.p_c = c.p_c;
     p.p_type = c.p_type;

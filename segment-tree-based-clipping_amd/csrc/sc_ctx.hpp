@@ -141,7 +141,7 @@ struct Ctx {
     bool sparseP = false;
     DBuf<int> sp_slot, sp_ndx, sp_edge, sp_av, sp_nbr, sp_lab, sp_pos, sp_ndf;
     DBuf<double> sp_x, sp_y;
-    DBuf<int> sv_b, sp_b, sv_c, sp_c;    // per slot: source vertex (local) or pair index, else -1
+    DBuf<int> from_b, from_c;            // per slot: source vertex (local), or ~ the pair inserted there
     DBuf<int> flags;                     // device status words
     int nrings = 0;
     std::vector<int> ring_off;           // host copy of the result

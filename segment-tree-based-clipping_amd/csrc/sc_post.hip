@@ -238,33 +238,21 @@ __global__ __launch_bounds__(JOB_BLK) void k_job_offsets(JobArgs ja, const int *
 
 // the two sides of the augmented rings, one per blockIdx.y (a null ax: not in this batch)
 struct AugSide {
-    int64_t n;             // slots
     const int *JX, *nverts, *voff, *AX;
     const double *poly;
     const int *all_scan, *nd_scan, *edge_of, *ord, *q;
     double *ax, *ay;
-    int *av, *nbr, *lab, *sv, *sp, *slot;
+    int *av, *nbr, *lab, *from, *slot;
 };
 struct AugSides {
     AugSide s[2];
 };
 
-__global__ void k_init_aug(AugSides sides) {
-    const AugSide &z = sides.s[blockIdx.y];
-    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (!z.ax || i >= z.n) return;
-    z.ax[i] = 0.0;
-    z.ay[i] = 0.0;
-    z.av[i] = -100;
-    z.nbr[i] = -100;
-    z.lab[i] = 0;
-    if (z.sv) {
-        z.sv[i] = -1;
-        z.sp[i] = -1;
-    }
-}
-
-// source vertices: count slot i of job j is vertex i - JX[j] (the last slot of a job is padding)
+// Source vertices: count slot i of job j is vertex i - JX[j] (the last slot of
+// a job is padding).  Every slot of the augmented rings is written once, in
+// full: a source's here, an inserted intersection's in k_aug_segments (an edge
+// has a slot per non-degenerate intersection, and no fewer positions to fill
+// them from), so nothing is cleared first.  Bound by the stores, 32 bytes a slot.
 __global__ void k_aug_sources(int J, AugSides sides) {
     const AugSide &z = sides.s[blockIdx.y];
     const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -276,7 +264,10 @@ __global__ void k_aug_sources(int J, AugSides sides) {
     const double2 V = reinterpret_cast<const double2 *>(z.poly)[int64_t(z.voff[j]) + v];
     z.ax[pos] = V.x;
     z.ay[pos] = V.y;
-    if (z.sv) z.sv[pos] = v;
+    z.av[pos] = -100;
+    z.nbr[pos] = -100;
+    z.lab[pos] = 0;
+    if (z.from) z.from[pos] = v;
 }
 
 // one thread per position of the per-edge alpha order: a leading degenerate
@@ -311,8 +302,10 @@ __global__ void k_aug_segments(const int *__restrict__ pj, int I, const int *__r
     z.ax[sl] = px[p];
     z.ay[sl] = py[p];
     z.av[sl] = z.q[p];
+    z.nbr[sl] = -100;
+    z.lab[sl] = 0;
     z.slot[p] = sl;
-    if (z.sp) z.sp[sl] = p;
+    if (z.from) z.from[sl] = ~p;
 }
 
 // neighbour links, 1-based and local to the job's rings (as the reference's arrays)
@@ -673,23 +666,16 @@ void post_jobs(Ctx &c, int k0, int k1) {
 
     const int64_t nbaA = nba_tot > 0 ? nba_tot : 1, ncaA = nca_tot > 0 ? nca_tot : 1;
     c.aug_cx.ensure(ncaA); c.aug_cy.ensure(ncaA); c.av_c.ensure(ncaA); c.nbr_c.ensure(ncaA); c.lab_c.ensure(ncaA);
-    int *svb = nullptr, *spb = nullptr, *svc = nullptr, *spc = nullptr;
-    if (c.prov) {
-        svb = c.sv_b.ensure(nbaA);
-        spb = c.sp_b.ensure(nbaA);
-        svc = c.sv_c.ensure(ncaA);
-        spc = c.sp_c.ensure(ncaA);
-    }
+    int *from_b = c.prov ? c.from_b.ensure(nbaA) : nullptr, *from_c = c.prov ? c.from_c.ensure(ncaA) : nullptr;
     AugSides as{};
     if (!sparse) {
         c.aug_bx.ensure(nbaA); c.aug_by.ensure(nbaA); c.av_b.ensure(nbaA); c.nbr_b.ensure(nbaA); c.lab_b.ensure(nbaA);
-        as.s[0] = AugSide{nba_tot, ja.JB, ja.nb, ja.bvoff, nba, c.bpoly, all_b, nd_b, c.p_b, c.ordB, c.p_qa, c.aug_bx,
-                          c.aug_by, c.av_b, c.nbr_b, c.lab_b, svb, spb, c.slot_b};
+        as.s[0] = AugSide{ja.JB, ja.nb, ja.bvoff, nba, c.bpoly, all_b, nd_b, c.p_b, c.ordB, c.p_qa, c.aug_bx,
+                          c.aug_by, c.av_b, c.nbr_b, c.lab_b, from_b, c.slot_b};
     }
-    as.s[1] = AugSide{nca_tot, ja.JC, ja.nc, ja.cvoff, nca, c.cpoly, all_c, nd_c, c.p_c, c.ordC, c.p_qb, c.aug_cx,
-                      c.aug_cy, c.av_c, c.nbr_c, c.lab_c, svc, spc, c.slot_c};
+    as.s[1] = AugSide{ja.JC, ja.nc, ja.cvoff, nca, c.cpoly, all_c, nd_c, c.p_c, c.ordC, c.p_qb, c.aug_cx,
+                      c.aug_cy, c.av_c, c.nbr_c, c.lab_c, from_c, c.slot_c};
     // (the sparse base side has slots by the hundred million and none of these arrays)
-    k_init_aug<<<dim3(grid_for(sparse ? nca_tot : std::max(nba_tot, nca_tot)), 2), BLK, 0, s>>>(as);
     k_aug_sources<<<dim3(grid_for(sparse ? nJC : std::max(nJB, nJC)), 2), BLK, 0, s>>>(J, as);
     SC_HIP(hipGetLastError());
     if (I > 0) {
