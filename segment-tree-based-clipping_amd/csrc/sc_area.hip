@@ -51,43 +51,76 @@ __device__ inline double block_sum(double v, double *sh) {
     return sh[0];
 }
 
-// twice the signed area of input ring r (vertices voff[r] .. voff[r+1]-1, the
-// last one the repeated closing vertex); one block per ring
-__global__ __launch_bounds__(BLK) void k_ring_area2(const double *__restrict__ poly, const int *__restrict__ voff,
-                                                    int r0, double *out) {
+// Twice the signed area of the input rings of both sides (blockIdx.z; vertices
+// voff[r] .. voff[r+1]-1, the last one the repeated closing vertex), a block per
+// RING_CHUNK vertices: one block per ring left 256 rings of 10,000 to 200,000
+// vertices to as many blocks (0.25 ms for 32 million vertices, now 0.09).
+// Chunk q of ring r is part[voff[r] / RING_CHUNK + r + q]: no two rings meet.
+constexpr int64_t RING_CHUNK = 4096;
+struct RingSide {
+    int rings, r0;
+    const double *poly;
+    const int *voff;
+    double *part, *out;
+};
+struct RingSides {
+    RingSide s[2];
+};
+__global__ __launch_bounds__(BLK) void k_ring_area2(RingSides sides) {
     __shared__ double sh[BLK];
-    const int r = r0 + blockIdx.x;
-    const int64_t a = voff[r], n = voff[r + 1] - a - 1;
-    // thread t adds the terms of vertices t, t + BLK, ... in that order; four
-    // terms are loaded before they are added (the same order and bits)
-    double s = 0.0;
-    int64_t i = threadIdx.x;
-    for (; i + 3 * BLK < n; i += 4 * BLK) {
-        const double *p0 = poly + 2 * (a + i), *p1 = p0 + 2 * BLK, *p2 = p1 + 2 * BLK, *p3 = p2 + 2 * BLK;
-        const double t0 = p0[0] * p0[3] - p0[2] * p0[1], t1 = p1[0] * p1[3] - p1[2] * p1[1];
-        const double t2 = p2[0] * p2[3] - p2[2] * p2[1], t3 = p3[0] * p3[3] - p3[2] * p3[1];
-        s += t0;
-        s += t1;
-        s += t2;
-        s += t3;
+    const RingSide &z = sides.s[blockIdx.z];
+    if (int(blockIdx.y) >= z.rings) return;
+    const int r = z.r0 + blockIdx.y;
+    const int64_t a = z.voff[r], n = z.voff[r + 1] - a - 1;
+    for (int64_t q = blockIdx.x; q == 0 || q * RING_CHUNK < n; q += gridDim.x) {
+        const int64_t end = n < (q + 1) * RING_CHUNK ? n : (q + 1) * RING_CHUNK;
+        // thread t adds the terms of vertices t, t + BLK, ... in that order; four
+        // terms are loaded before they are added (the same order and bits)
+        double s = 0.0;
+        int64_t i = q * RING_CHUNK + threadIdx.x;
+        for (; i + 3 * BLK < end; i += 4 * BLK) {
+            const double *p0 = z.poly + 2 * (a + i), *p1 = p0 + 2 * BLK, *p2 = p1 + 2 * BLK, *p3 = p2 + 2 * BLK;
+            const double t0 = p0[0] * p0[3] - p0[2] * p0[1], t1 = p1[0] * p1[3] - p1[2] * p1[1];
+            const double t2 = p2[0] * p2[3] - p2[2] * p2[1], t3 = p3[0] * p3[3] - p3[2] * p3[1];
+            s += t0;
+            s += t1;
+            s += t2;
+            s += t3;
+        }
+        for (; i < end; i += BLK) {
+            const double *p = z.poly + 2 * (a + i);
+            s += p[0] * p[3] - p[2] * p[1];
+        }
+        const double t = block_sum(s, sh);
+        if (threadIdx.x == 0) (n <= RING_CHUNK ? z.out[blockIdx.y] : z.part[a / RING_CHUNK + r + q]) = t;
+        __syncthreads(); // sh is written again
     }
-    for (; i < n; i += BLK) {
-        const double *p = poly + 2 * (a + i);
-        s += p[0] * p[3] - p[2] * p[1];
-    }
-    double t = block_sum(s, sh);
-    if (threadIdx.x == 0) out[blockIdx.x] = t;
+}
+// rings of more than one chunk: its chunks in order
+__global__ void k_ring_parts(RingSides sides) {
+    const RingSide &z = sides.s[blockIdx.y];
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= z.rings) return;
+    const int r = z.r0 + k;
+    const int64_t a = z.voff[r], n = z.voff[r + 1] - a - 1;
+    if (n <= RING_CHUNK) return;
+    const double *p = z.part + (a / RING_CHUNK + r);
+    double s = p[0];
+    for (int64_t q = 1; q * RING_CHUNK < n; ++q) s += p[q];
+    z.out[k] = s;
 }
 
 // Twice the signed area of every output ring.  A ring of at most AREA_CHUNK
 // vertices is summed by one wave: lanes stride the ring and a fixed shuffle
-// tree adds their sums (the order of the small-pair kernel); the waves of a
-// fixed grid take rings in turn, so a batch of many small rings costs no
-// launch of a wave per ring.  A longer ring is summed in chunks of
-// AREA_CHUNK vertices the same way, one wave per chunk, and its chunk sums
-// are added in chunk order.
+// tree adds their sums (the order of the small-pair kernel).  Four rings of at
+// most 16 vertices share the wave: the tree's steps over 32 and 16 lanes would
+// add zeros to such a ring, and most are this short (the output rings of 256
+// large pairs: 0.19 -> 0.06 ms).
+// A longer ring is summed in chunks of AREA_CHUNK vertices, one wave per
+// chunk, and its chunk sums are added in chunk order.
 constexpr int AREA_CHUNK = 64 * WAVE;
 constexpr int AREA_WAVES = 8192; // waves of the short-ring grid (32 per CU)
+constexpr int RING_LANES = 16, RING_SET = WAVE / RING_LANES; // lanes of a short ring, rings a wave takes at once
 
 __device__ inline double wave_ring_sum(const double *__restrict__ x, const double *__restrict__ y, int64_t a,
                                        int64_t b, int64_t c0, int64_t c1, int lane) {
@@ -103,13 +136,24 @@ __device__ inline double wave_ring_sum(const double *__restrict__ x, const doubl
 __global__ __launch_bounds__(BLK) void k_out_ring_area2(int nrings, const int *__restrict__ roff,
                                                         const double *__restrict__ x, const double *__restrict__ y,
                                                         double *out) {
-    const int lane = int(threadIdx.x) & (WAVE - 1);
-    const int stride = int(gridDim.x) * (BLK / WAVE);
-    for (int r = int(blockIdx.x) * (BLK / WAVE) + int(threadIdx.x) / WAVE; r < nrings; r += stride) {
-        const int64_t a = roff[r], b = roff[r + 1];
-        if (b - a > AREA_CHUNK) continue; // chunked below
-        const double s = wave_ring_sum(x, y, a, b, a, b, lane);
-        if (lane == 0) out[r] = s;
+    const int lane = int(threadIdx.x) & (WAVE - 1), l = lane & (RING_LANES - 1), q = lane / RING_LANES;
+    const int stride = int(gridDim.x) * (BLK / WAVE) * RING_SET;
+    for (int r0 = (int(blockIdx.x) * (BLK / WAVE) + int(threadIdx.x) / WAVE) * RING_SET; r0 < nrings; r0 += stride) {
+        const int r = r0 + q;
+        const int64_t a = r < nrings ? roff[r] : 0, b = r < nrings ? roff[r + 1] : 0;
+        double s = 0.0;
+        if (b - a <= RING_LANES && a + l < b) {
+            const int64_t i = a + l, nx = i + 1 == b ? a : i + 1;
+            s += x[i] * y[nx] - x[nx] * y[i];
+        }
+        for (int d = RING_LANES / 2; d > 0; d >>= 1) s += __shfl_down(s, d, RING_LANES);
+        if (l == 0 && r < nrings && b - a <= RING_LANES) out[r] = s;
+        for (uint64_t m = __ballot(l == 0 && b - a > RING_LANES && b - a <= AREA_CHUNK); m; m &= m - 1) {
+            const int from = __ffsll((unsigned long long)m) - 1;
+            const int64_t ra = __shfl(int(a), from, WAVE), rb = __shfl(int(b), from, WAVE);
+            const double t = wave_ring_sum(x, y, ra, rb, ra, rb, lane);
+            if (lane == 0) out[r0 + from / RING_LANES] = t;
+        }
     }
 }
 
@@ -348,7 +392,8 @@ struct GatherGrad {
     int *inv_p, *inv_q;  // per pair: the output vertex of its base / overlay visit
     double4 *rec;        // per pair: shares of c1 and c2
     const int *ord_c, *pj;
-    uint32_t *found;     // output vertices found from the other side
+    uint32_t *found;     // output vertices found from the other side, per block of the kernels that look
+    int nfound;
 };
 
 // first output vertex of each job (J + 1 threads)
@@ -381,9 +426,18 @@ __global__ __launch_bounds__(BLK) void k_output_terms(GatherGrad g, int per) {
     }
 }
 
-__device__ inline void add_count(uint32_t *ctl, uint32_t n) { // all lanes: one atomic per wave
+// a block's count at its place in the list (an atomic per wave on one word took
+// longer than the kernels' own work)
+__device__ inline void put_count(uint32_t *at, uint32_t n) { // all threads
+    __shared__ uint32_t part[BLK / WAVE];
     for (int d = WAVE / 2; d > 0; d >>= 1) n += uint32_t(__shfl_xor(int(n), d, WAVE));
-    if ((threadIdx.x & (WAVE - 1)) == 0 && n) atomicAdd(ctl, n);
+    if ((threadIdx.x & (WAVE - 1)) == 0) part[threadIdx.x / WAVE] = n;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint32_t t = 0;
+        for (int q = 0; q < BLK / WAVE; ++q) t += part[q];
+        *at = t;
+    }
 }
 
 // Sums g over each run of lanes with the same key (n lanes hold one) and gives
@@ -438,7 +492,7 @@ __global__ __launch_bounds__(BLK) void k_pair_terms(GatherGrad g) {
             if (gb[2] != 0.0 || gb[3] != 0.0) add_b(a, j, b + 1 == a.nb[j] ? 0 : b + 1, gb[2], gb[3]);
         }
     }
-    add_count(g.found, found);
+    put_count(g.found + blockIdx.x, found);
 }
 
 // pairs in (job, overlay edge) order: the overlay side's
@@ -502,14 +556,22 @@ __global__ __launch_bounds__(BLK) void k_vertex_grad(VertexSides a) {
         z.grad[2 * i] = gx;
         z.grad[2 * i + 1] = gy;
     }
-    add_count(a.found, found);
+    put_count(a.found + blockIdx.y * gridDim.x + blockIdx.x, found);
 }
 
 // Output vertices that share their input vertex or visit with another one, of
 // which only the last was found; returns at once where there is none.
 __global__ __launch_bounds__(BLK) void k_grad_rest(GatherGrad g) {
     const ProvArgs &a = g.a;
-    if (int64_t(*g.found) == g.n_out) return;
+    __shared__ uint32_t total;
+    if (threadIdx.x == 0) total = 0;
+    __syncthreads();
+    uint32_t n = 0;
+    for (int k = threadIdx.x; k < g.nfound; k += BLK) n += g.found[k];
+    for (int d = WAVE / 2; d > 0; d >>= 1) n += uint32_t(__shfl_xor(int(n), d, WAVE));
+    if ((threadIdx.x & (WAVE - 1)) == 0) atomicAdd(&total, n);
+    __syncthreads();
+    if (int64_t(total) == g.n_out) return;
     const int64_t step = int64_t(gridDim.x) * blockDim.x;
     for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < g.n_out; i += step) {
         const int s = a.src[i];
@@ -528,9 +590,9 @@ __global__ __launch_bounds__(BLK) void k_grad_rest(GatherGrad g) {
 }
 
 struct AreaScratch {
-    DBuf<double> out2, ring2, barea2, carea2, out4, cI, cQ, cPr, part;
+    DBuf<double> out2, ring2, barea2, carea2, out4, cI, cQ, cPr, part, rpart;
     DBuf<int> bad, bin_off;
-    DBuf<uint32_t> chunks, choff, tot, rid, gctl;
+    DBuf<uint32_t> chunks, choff, tot, rid, gfound;
     // gathered gradients
     DBuf<int> jv0, inv;
     DBuf<double2> og;
@@ -562,7 +624,8 @@ void batch_area(Ctx &c, double *out4) {
     double *ring2 = a.ring2.ensure(size_t(c.nrings > 0 ? c.nrings : 1));
     if (c.nrings > 0) {
         const int nr = c.nrings;
-        const int64_t wgrid = std::min<int64_t>(ceil_div(int64_t(nr), BLK / WAVE), AREA_WAVES / (BLK / WAVE));
+        const int64_t wgrid =
+            std::min<int64_t>(ceil_div(int64_t(nr), RING_SET * (BLK / WAVE)), AREA_WAVES / (BLK / WAVE));
         k_out_ring_area2<<<unsigned(wgrid), BLK, 0, s>>>(nr, c.d_ring_off, c.d_ring_x, c.d_ring_y, ring2);
         uint32_t *cnt = a.chunks.ensure(size_t(nr) + 1), *choff = a.choff.ensure(size_t(nr) + 1);
         uint32_t *tot = a.tot.ensure(1);
@@ -577,9 +640,24 @@ void batch_area(Ctx &c, double *out4) {
         k_ring_chunk_sum<<<grid_for(nr), BLK, 0, s>>>(nr, choff, cap, part, ring2);
     }
     k_job_out_area2<<<J, BLK, 0, s>>>(js.d_ring, ring2, out2);
-    if (c.paired) k_ring_area2<<<J, BLK, 0, s>>>(c.bpoly, c.d_bvoff, js.k0 - 1, barea2);
-    else k_ring_area2<<<1, BLK, 0, s>>>(c.bpoly, c.d_bvoff, 0, barea2);
-    k_ring_area2<<<J, BLK, 0, s>>>(c.cpoly, c.d_coff, js.k0 - 1, carea2);
+    RingSides rs;
+    const int64_t pb = (c.nb + c.nbr) / RING_CHUNK + c.nbr + 1, pc = (c.nct + c.K) / RING_CHUNK + c.K + 1;
+    double *part = a.rpart.ensure(size_t(pb + pc));
+    rs.s[0] = RingSide{c.paired ? J : 1, c.paired ? js.k0 - 1 : 0, c.bpoly, c.d_bvoff, part, barea2};
+    rs.s[1] = RingSide{J, js.k0 - 1, c.cpoly, c.d_coff, part + pb, carea2};
+    // blocks for a ring's chunks, where there are not many rings anyway
+    const int64_t longest = ceil_div(int64_t(std::max(c.maxbsz, c.maxcsz)), RING_CHUNK);
+    const int64_t bx = std::max<int64_t>(1, std::min<int64_t>(longest, 32768 / J));
+    for (int r = 0; r < J; r += 65535) { // grid dimension limit
+        RingSides part_of = rs;
+        for (RingSide &z : part_of.s) {
+            z.rings = std::max(0, std::min(65535, z.rings - r));
+            z.r0 += r;
+            z.out += r;
+        }
+        k_ring_area2<<<dim3(unsigned(bx), unsigned(std::min(65535, J - r)), 2), BLK, 0, s>>>(part_of);
+    }
+    if (longest > 1) k_ring_parts<<<dim3(grid_for(J), 2), BLK, 0, s>>>(rs);
     k_job_final<<<grid_for(J), BLK, 0, s>>>(J, c.paired ? 1 : 0, out2, barea2, carea2, out4);
     SC_HIP(hipGetLastError());
 }
@@ -650,9 +728,7 @@ void batch_area_backward(Ctx &c, const double *g_area, const double *g_iou, doub
             g.inv_c = inv + c.nb;
             g.inv_p = inv + nv;
             g.inv_q = inv + nv + I;
-            g.found = a.gctl.ensure(1);
             fb.add(inv, nv + 2 * int64_t(I), ~0u);
-            fb.add(g.found, 1, 0u);
         }
         fb.flush();
     }
@@ -678,19 +754,23 @@ void batch_area_backward(Ctx &c, const double *g_area, const double *g_iou, doub
             const int per = span_per(g.n_out);
             k_output_terms<<<grid_for(g.n_out, BLK * per), BLK, 0, s>>>(g, per);
         }
-        const int blocks = 2048; // eight waves per SIMD; a count per wave
+        const int blocks = 2048; // eight waves per SIMD
         VertexSides vs{};
         vs.s[0] = VertexSide{c.nb, boff, c.nbr, c.bpoly, cPr, g.inv_b, grad_b};
         vs.s[1] = VertexSide{c.nct, dci, c.K, c.cpoly, cQ, g.inv_c, grad_c};
         vs.og = g.og;
-        vs.found = g.found;
         const int64_t most = std::max<int64_t>(c.nb, c.nct);
         vs.per = int(std::max<int64_t>(1, ceil_div(most, int64_t(blocks) * BLK)));
-        k_vertex_grad<<<dim3(grid_for(most, BLK * vs.per), 2), BLK, 0, s>>>(vs);
+        const int vblocks = int(grid_for(most, BLK * vs.per)), pblocks = I > 0 ? std::min(blocks, int(grid_for(I))) : 0;
+        g.nfound = 2 * vblocks + pblocks;
+        vs.found = a.gfound.ensure(size_t(g.nfound));
+        k_vertex_grad<<<dim3(unsigned(vblocks), 2), BLK, 0, s>>>(vs);
+        g.found = vs.found + 2 * vblocks;
         if (I > 0) {
-            k_pair_terms<<<std::min(blocks, int(grid_for(I))), BLK, 0, s>>>(g);
+            k_pair_terms<<<pblocks, BLK, 0, s>>>(g);
             k_pair_terms_c<<<grid_for(I), BLK, 0, s>>>(g);
         }
+        g.found = vs.found;
         if (g.n_out > 0) k_grad_rest<<<std::min(blocks, int(grid_for(g.n_out))), BLK, 0, s>>>(g);
     }
     SC_HIP(hipGetLastError());
