@@ -251,6 +251,9 @@ struct RadixScratch {
     DBuf<uint64_t> keys_alt;
     DBuf<uint32_t> vals_alt;
 };
+// ascending, n <= SMALL_SORT_MAX whole keys; tmp: as many
+constexpr int SMALL_SORT_MAX = 16384;
+void sort_small_u64(uint64_t *keys, uint64_t *tmp, int n, hipStream_t s);
 void radix_sort_u64(uint64_t *keys, uint32_t *vals, int64_t n, int bit_lo, int bit_hi, RadixScratch &rs,
                     hipStream_t s);
 // The same sort on keys/vals held in buffers, with alternate buffers of the

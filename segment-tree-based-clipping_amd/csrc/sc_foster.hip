@@ -134,15 +134,58 @@ __global__ __launch_bounds__(BLK) void k_jclassify(ClassifyArgs a) {
 struct WindSide {
     Side r;
     int64_t n;
-    const double *q; // query points, x,y per job
-    const int *ok;
+    Side from;        // the other side, whose first plain vertices are the query points
+    const int *first;
+    const double *q;  // or the points, x,y per job (sparse base side)
     int *wind;
+};
+struct JobState {
+    int J;
+    int uni; // the union: every job takes the sequential route
+    const int *AB, *AC;
+    int *slow, *firstP, *firstQ, *windP, *windQ, *kind, *mP, *mQ, *cP0, *cQ0;
+    int *vP, *vQ; // crossings of the batch before each ring's first plain vertex
 };
 struct WindSides {
     WindSide s[2];
     int J, per;
+    JobState st;
+    const uint32_t *ccP, *ccQ;
+    int sparse;
+    SparseP sp;
+    const int *flags;
 };
+// route of each job; first crossing index of each job on both sides (J+1 threads)
+__device__ inline void decide(const WindSides &a, int j) {
+    const JobState &s = a.st;
+    const uint32_t *ccP = a.ccP, *ccQ = a.ccQ;
+    if (j > s.J) return;
+    s.cP0[j] = int(ccP[s.AB[j]]);
+    s.cQ0[j] = int(ccQ[s.AC[j]]);
+    if (j == s.J) return;
+    int mp = int(ccP[s.AB[j + 1]] - ccP[s.AB[j]]), mq = int(ccQ[s.AC[j + 1]] - ccQ[s.AC[j]]);
+    s.mP[j] = mp;
+    s.mQ[j] = mq;
+    int sl = s.slow[j];
+    const int fp = s.firstP[j], fq = s.firstQ[j];
+    if (fp < 0 || fq < 0) {
+        sl |= SLOW_NOPLAIN;
+    } else {
+        // sparse: the slots before the first plain one are the job's first positions
+        // (a flagged job's slots may not ascend: as the searches find it)
+        s.vP[j] = int(ccP[!a.sparse ? s.AB[j] + fp : (a.flags[j] ? sp_lower(a.sp, j, fp) : a.sp.P0[j] + fp)]);
+        s.vQ[j] = int(ccQ[s.AC[j] + fq]);
+    }
+    if (mp != mq || (mp & 1)) sl |= SLOW_ODD;
+    if (s.uni) sl |= SLOW_UNION;
+    s.slow[j] = sl;
+    s.kind[j] = sl ? K_SEQ : (mp == 0 ? K_NOCROSS : K_CROSS);
+}
 __global__ __launch_bounds__(BLK) void k_jwinding(WindSides a) {
+    if (blockIdx.y == 2) { // the routes need no winding and share the launch
+        decide(a, blockIdx.x * blockDim.x + threadIdx.x);
+        return;
+    }
     const WindSide &z = a.s[blockIdx.y];
     if (!z.wind) return;
     const Side &r = z.r;
@@ -158,9 +201,12 @@ __global__ __launch_bounds__(BLK) void k_jwinding(WindSides a) {
         const int64_t i = s.at + lane;
         const int j = s.of(r.off, a.J, lane);
         int w = 0;
-        if (i < z.n && z.ok[j]) {
+        const int fp = i < z.n ? z.first[j] : -1;
+        if (fp >= 0) {
             const int64_t nx = i + 1 == r.off[j + 1] ? r.off[j] : i + 1;
-            w = wind_edge(r.x[i], r.y[i], r.x[nx], r.y[nx], z.q[2 * j], z.q[2 * j + 1]);
+            const int64_t v = z.q ? 0 : int64_t(z.from.off[j]) + fp;
+            const double qx = z.q ? z.q[2 * j] : z.from.x[v], qy = z.q ? z.q[2 * j + 1] : z.from.y[v];
+            w = wind_edge(r.x[i], r.y[i], r.x[nx], r.y[nx], qx, qy);
         }
         const int j0 = __builtin_amdgcn_readfirstlane(j);
         if (j0 != of) {
@@ -177,24 +223,18 @@ __global__ __launch_bounds__(BLK) void k_jwinding(WindSides a) {
     add();
 }
 
-// query points: each ring's first plain vertex (dense rings, or the sparse base ring)
-__global__ void k_query_pts(int J, Side P, Side Q, int sparse, SparseP sp, const int *firstP, const int *firstQ,
-                            double *pq, int *pok, double *qq, int *qok) {
+// query points of a batch with a sparse base ring: each ring's first plain vertex
+__global__ void k_query_pts(int J, Side Q, SparseP sp, const int *firstP, const int *firstQ, double *pq, double *qq,
+                            int *qok) {
     int j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= J) return;
     const int fp = firstP[j], fq = firstQ[j];
-    pok[j] = fp >= 0;
     qok[j] = fq >= 0;
     double x = 0, y = 0;
     if (fp >= 0) {
-        if (sparse) {
-            SlotInfo si = sp_slot(sp, j, fp);
-            x = si.x;
-            y = si.y;
-        } else {
-            x = P.x[P.off[j] + fp];
-            y = P.y[P.off[j] + fp];
-        }
+        const SlotInfo si = sp_slot(sp, j, fp);
+        x = si.x;
+        y = si.y;
     }
     pq[2 * j] = x;
     pq[2 * j + 1] = y;
@@ -283,41 +323,6 @@ __global__ void k_sp_wind_fix(int I, const int *__restrict__ pj, SparseP sp, con
     if (first) w -= wind_edge(ax, ay, bx, by, rx, ry);
     if (last) w += wind_edge(x, y, bx, by, rx, ry);
     if (w) atomicAdd(&wind[j], w);
-}
-
-struct JobState {
-    int J;
-    int uni; // the union: every job takes the sequential route
-    const int *AB, *AC;
-    int *slow, *firstP, *firstQ, *windP, *windQ, *kind, *mP, *mQ, *cP0, *cQ0;
-    int *vP, *vQ; // crossings of the batch before each ring's first plain vertex
-};
-
-// route of each job; first crossing index of each job on both sides (J+1 threads)
-__global__ void k_jdecide(JobState s, const uint32_t *ccP, const uint32_t *ccQ, int sparse, SparseP sp,
-                          const int *flags) {
-    int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j > s.J) return;
-    s.cP0[j] = int(ccP[s.AB[j]]);
-    s.cQ0[j] = int(ccQ[s.AC[j]]);
-    if (j == s.J) return;
-    int mp = int(ccP[s.AB[j + 1]] - ccP[s.AB[j]]), mq = int(ccQ[s.AC[j + 1]] - ccQ[s.AC[j]]);
-    s.mP[j] = mp;
-    s.mQ[j] = mq;
-    int sl = s.slow[j];
-    const int fp = s.firstP[j], fq = s.firstQ[j];
-    if (fp < 0 || fq < 0) {
-        sl |= SLOW_NOPLAIN;
-    } else {
-        // sparse: the slots before the first plain one are the job's first positions
-        // (a flagged job's slots may not ascend: as the searches find it)
-        s.vP[j] = int(ccP[!sparse ? s.AB[j] + fp : (flags[j] ? sp_lower(sp, j, fp) : sp.P0[j] + fp)]);
-        s.vQ[j] = int(ccQ[s.AC[j] + fq]);
-    }
-    if (mp != mq || (mp & 1)) sl |= SLOW_ODD;
-    if (s.uni) sl |= SLOW_UNION;
-    s.slow[j] = sl;
-    s.kind[j] = sl ? K_SEQ : (mp == 0 ? K_NOCROSS : K_CROSS);
 }
 
 // Entry/exit status of every crossing vertex from the parity of crossings
@@ -494,18 +499,6 @@ __global__ __launch_bounds__(BLK) void k_jpieces(PieceArgs a) {
     a.val[x] = onP ? min(2u * uint32_t(x), 2u * uint32_t(xw) + 1u) : NIL;
 }
 
-// jobs found inconsistent while building pieces take the sequential route;
-// their crossings leave the graph (the other jobs' are in it only for K_CROSS)
-__global__ void k_jmask(int J, int M, const int *pj, const int *slow, int *kind, uint32_t *succ, uint32_t *val) {
-    const int x = blockIdx.x * blockDim.x + threadIdx.x;
-    if (x < J && kind[x] == K_CROSS && slow[x]) kind[x] = K_SEQ;
-    if (x >= M) return;
-    const int j = pj[x];
-    if (kind[j] == K_CROSS && !slow[j]) return;
-    succ[x] = uint32_t(x);
-    val[x] = NIL;
-}
-
 // Cycles of the crossing graph by doubling.  On a crossing job successors
 // alternate between P and Q crossings and only P crossings carry values, so
 // the doubling runs over the P crossings alone, stepping two pieces at a time
@@ -516,12 +509,21 @@ __global__ void k_jmask(int J, int M, const int *pj, const int *slow, int *kind,
 // the P crossing after the window.  A window sum is read only when the window
 // holds no occurrence of the cycle's minimum, so does not wrap and stays below
 // the cycle's total; the 32-bit wrap-around of longer windows is never read.
-__device__ inline uint4 jump_first(int x, int mP, int M, const uint32_t *val, const uint32_t *succ, const int *plen) {
-    const uint32_t q = succ[x];
-    uint32_t n2 = q < uint32_t(M) ? succ[q] : uint32_t(x);
-    if (n2 >= uint32_t(mP)) n2 = uint32_t(x); // not a P-Q-P step: a crossing outside the traversed jobs
-    const uint32_t w = uint32_t(plen[x]) + (q < uint32_t(M) && q != uint32_t(x) ? uint32_t(plen[q]) : 0u);
-    return make_uint4(val[x], 0u, w, n2);
+struct JumpArgs {
+    int mP, M;
+    const uint32_t *val, *succ;
+    const int *plen, *pj, *kind, *slow;
+};
+// A job found inconsistent while its pieces were built takes the sequential
+// route: its crossings stand alone.
+__device__ inline uint4 jump_first(const JumpArgs &a, int x) {
+    const int j = a.pj[x];
+    if (a.kind[j] != K_CROSS || a.slow[j]) return make_uint4(NIL, 0u, 0u, uint32_t(x));
+    const uint32_t q = a.succ[x];
+    uint32_t n2 = q < uint32_t(a.M) ? a.succ[q] : uint32_t(x);
+    if (n2 >= uint32_t(a.mP)) n2 = uint32_t(x); // not a P-Q-P step: a crossing outside the traversed jobs
+    const uint32_t w = uint32_t(a.plen[x]) + (q < uint32_t(a.M) && q != uint32_t(x) ? uint32_t(a.plen[q]) : 0u);
+    return make_uint4(a.val[x], 0u, w, n2);
 }
 __device__ inline uint4 jump_join(const uint4 &a, const uint4 &b) { // the window of a, then that of b
     uint4 o;
@@ -531,11 +533,10 @@ __device__ inline uint4 jump_join(const uint4 &a, const uint4 &b) { // the windo
     o.w = b.w;
     return o;
 }
-__global__ void k_jump_init(int mP, int M, const uint32_t *val, const uint32_t *succ, const int *plen, uint4 *rec,
-                            uint2 *cov) {
+__global__ void k_jump_init(JumpArgs a, uint4 *rec, uint2 *cov) {
     const int x = blockIdx.x * blockDim.x + threadIdx.x;
-    if (x >= mP) return;
-    rec[x] = jump_first(x, mP, M, val, succ, plen);
+    if (x >= a.mP) return;
+    rec[x] = jump_first(a, x);
     cov[x] = make_uint2(NIL, 0u);
 }
 
@@ -632,24 +633,22 @@ __global__ void k_jump_rank(int mP, const uint4 *__restrict__ rec, uint4 *__rest
     if (o.x != a.x) moved[r] = 1u;
 }
 
-// Every round of k_jump_rank for at most JUMP_SMALL P crossings, by one block
-// with the records in LDS (64 KB): a round is a barrier instead of a launch
-// (12 launches of 2.5 us and their gaps at 1,400 crossings).
+// Every round of k_jump_rank for at most JUMP_SMALL records, by one block with
+// the records in LDS (64 KB): a round is a barrier instead of a launch (12
+// launches of 2.5 us and their gaps at 1,400 crossings).
 constexpr int JUMP_SMALL = 4096, JUMP_BLK = 1024, JUMP_PER = JUMP_SMALL / JUMP_BLK;
-__global__ __launch_bounds__(JUMP_BLK) void k_jump_small(int mP, int M, const uint32_t *val, const uint32_t *succ,
-                                                       const int *plen, int rounds, uint2 *out) {
+__device__ inline void jump_all(uint4 (&a)[JUMP_PER], int n, int rounds) { // thread t: records t, t + JUMP_BLK, ...
     __shared__ uint4 r[JUMP_SMALL];
-    uint4 a[JUMP_PER];
     for (int q = 0; q < JUMP_PER; ++q) {
         const int x = q * JUMP_BLK + int(threadIdx.x);
-        if (x < mP) r[x] = a[q] = jump_first(x, mP, M, val, succ, plen);
+        if (x < n) r[x] = a[q];
     }
     __syncthreads();
     for (int k = 0; k < rounds; ++k) {
         int moved = 0;
         for (int q = 0; q < JUMP_PER; ++q) {
             const int x = q * JUMP_BLK + int(threadIdx.x);
-            if (x >= mP) continue;
+            if (x >= n) continue;
             const uint4 o = jump_join(a[q], r[a[q].w]);
             moved |= o.x != a[q].x ? 1 : 0;
             a[q] = o;
@@ -658,13 +657,35 @@ __global__ __launch_bounds__(JUMP_BLK) void k_jump_small(int mP, int M, const ui
         if (!moved) break;
         for (int q = 0; q < JUMP_PER; ++q) {
             const int x = q * JUMP_BLK + int(threadIdx.x);
-            if (x < mP) r[x] = a[q];
+            if (x < n) r[x] = a[q];
         }
         __syncthreads();
     }
+}
+// the crossings' own records
+__global__ __launch_bounds__(JUMP_BLK) void k_jump_small(JumpArgs ja, int rounds, uint2 *out) {
+    uint4 a[JUMP_PER];
     for (int q = 0; q < JUMP_PER; ++q) {
         const int x = q * JUMP_BLK + int(threadIdx.x);
-        if (x < mP) out[x] = make_uint2(a[q].x, a[q].y);
+        if (x < ja.mP) a[q] = jump_first(ja, x);
+    }
+    jump_all(a, ja.mP, rounds);
+    for (int q = 0; q < JUMP_PER; ++q) {
+        const int x = q * JUMP_BLK + int(threadIdx.x);
+        if (x < ja.mP) out[x] = make_uint2(a[q].x, a[q].y);
+    }
+}
+// the rulers'
+__global__ __launch_bounds__(JUMP_BLK) void k_rule_small(uint4 *rec, int n, int rounds) {
+    uint4 a[JUMP_PER];
+    for (int q = 0; q < JUMP_PER; ++q) {
+        const int x = q * JUMP_BLK + int(threadIdx.x);
+        if (x < n) a[q] = rec[x];
+    }
+    jump_all(a, n, rounds);
+    for (int q = 0; q < JUMP_PER; ++q) {
+        const int x = q * JUMP_BLK + int(threadIdx.x);
+        if (x < n) rec[x] = a[q];
     }
 }
 
@@ -712,7 +733,7 @@ __global__ void k_rank_final(int M, int mP, const uint2 *__restrict__ rec, const
 
 struct CountArgs {
     int J;
-    const int *AB, *AC, *kind, *windP, *windQ, *cP0, *sidx, *seq_res;
+    const int *AB, *AC, *kind, *slow, *windP, *windQ, *cP0, *sidx, *seq_res; // seq_res null: not run (yet)
     const uint32_t *base, *ridx;
     uint32_t *jv, *jr;
 };
@@ -727,14 +748,14 @@ __global__ void k_jcounts(CountArgs a) {
     }
     uint32_t v = 0, r = 0;
     const int k = a.kind[j];
-    if (k == K_CROSS) {
+    if (k == K_CROSS && !a.slow[j]) {
         v = a.base[a.cP0[j + 1]] - a.base[a.cP0[j]];
         r = a.ridx[a.cP0[j + 1]] - a.ridx[a.cP0[j]];
     } else if (k == K_NOCROSS) {
         bool ip = (a.windP[j] % 2) != 0, iq = (a.windQ[j] % 2) != 0;
         v = (ip ? uint32_t(a.AB[j + 1] - a.AB[j]) : 0u) + (iq ? uint32_t(a.AC[j + 1] - a.AC[j]) : 0u);
         r = uint32_t(ip) + uint32_t(iq);
-    } else {
+    } else if (a.seq_res) {
         int s = a.sidx[j];
         r = uint32_t(a.seq_res[3 * s]);
         v = uint32_t(a.seq_res[3 * s + 1]);
@@ -935,6 +956,7 @@ __global__ void k_root_loop(int nr, const int *off, const double *x, const doubl
 // 27 M (short edges drop in long runs); now 39 us and 0.26 ms.
 constexpr int KEEP_WIN = 4;                  // windows per tile, their loads issued together
 constexpr int KEEP_TILE = KEEP_WIN * WAVE;
+constexpr int64_t KEEP_FIRST_TWO = 1 << 18; // vertices beyond which two rounds are run before the first check
 constexpr int KEEP_ROUNDS = 50;              // rounds before one wave per ring
 constexpr uint32_t KEEP_ANY = 0xffffffffu;   // the tile's first vertex needs no vertex before it
 
@@ -2450,10 +2472,11 @@ void cleanup_rings(Ctx &c, FosterScratch &f, int nr, int64_t n, int J, const uin
     uint32_t *rcnt = f.rcnt.ensure(size_t(nr) + 1);
     uint32_t *jring = f.jring.ensure(size_t(J) + 3);
     job_ring.resize(size_t(J) + 3);
-    // rounds until one moves nothing; the counts that follow are taken before
+    // rounds until one moves nothing (of many vertices some tile nearly always
+    // moves in the first); the counts that follow are taken before
     // that is known (one wait instead of two), and again if it was not the last
     for (int it = 1;;) {
-        const int end = std::min(it + (it == 1 ? 2 : 8), KEEP_ROUNDS);
+        const int end = std::min(it + (it > 1 ? 8 : (n > KEEP_FIRST_TWO ? 2 : 1)), KEEP_ROUNDS);
         const bool rings = it >= end;
         if (rings) {
             k_keep_rings<<<grid_for(nr, BLK / WAVE), BLK, 0, s>>>(ka, nr);
@@ -2599,24 +2622,32 @@ void label_and_traverse(Ctx &c) {
     uint32_t *tot = c.d_u32_total.ensure(2);
     scan_exclusive_u32_2(crossP, ccP, nP + 1, tot, crossQ, ccQ, nQ + 1, tot + 1, s);
     // point-in-polygon of each ring's first plain vertex w.r.t. the other ring
-    double *qpts = f.qpts.ensure(4 * size_t(J));
-    int *qoks = f.qoks.ensure(2 * size_t(J));
-    double *pq = qpts, *qq = qpts + 2 * size_t(J);
-    int *pok = qoks, *qok = qoks + J;
-    k_query_pts<<<grid_for(J), BLK, 0, s>>>(J, P, Q, sparse ? 1 : 0, sp, st.firstP, st.firstQ, pq, pok, qq, qok);
-    SC_HIP(hipGetLastError());
+    double *pq = nullptr, *qq = nullptr;
+    int *qok = nullptr;
+    if (sparse) {
+        pq = f.qpts.ensure(4 * size_t(J));
+        qq = pq + 2 * size_t(J);
+        qok = f.qoks.ensure(size_t(J));
+        k_query_pts<<<grid_for(J), BLK, 0, s>>>(J, Q, sp, st.firstP, st.firstQ, pq, qq, qok);
+        SC_HIP(hipGetLastError());
+    }
     WindSides wd;
-    wd.s[0] = WindSide{Q, nQ, pq, pok, st.windP};
-    wd.s[1] = WindSide{P, nP, qq, qok, sparse ? nullptr : st.windQ};
+    wd.s[0] = WindSide{Q, nQ, P, st.firstP, pq, st.windP};
+    wd.s[1] = WindSide{P, nP, Q, st.firstQ, nullptr, sparse ? nullptr : st.windQ};
     wd.J = J;
     wd.per = per;
-    k_jwinding<<<dim3(grid_for(sparse ? nQ : most, BLK * per), sparse ? 1 : 2), BLK, 0, s>>>(wd);
+    wd.st = st;
+    wd.ccP = ccP;
+    wd.ccQ = ccQ;
+    wd.sparse = sparse ? 1 : 0;
+    wd.sp = sp;
+    wd.flags = c.flags;
+    k_jwinding<<<dim3(std::max(grid_for(sparse ? nQ : most, BLK * per), grid_for(int64_t(J) + 1)), 3), BLK, 0, s>>>(wd);
     if (sparse) {
         const int chunks = (c.nb + WCH - 1) / WCH;
         k_sp_wind_base<<<unsigned(int64_t(J) * chunks), BLK, 0, s>>>(J, c.nb, c.bpoly, qq, qok, st.windQ);
         if (nP > 0) k_sp_wind_fix<<<grid_for(nP), BLK, 0, s>>>(int(nP), c.p_j, sp, qq, qok, st.windQ);
     }
-    k_jdecide<<<grid_for(J + 1), BLK, 0, s>>>(st, ccP, ccQ, sparse ? 1 : 0, sp, c.flags);
     SC_HIP(hipGetLastError());
     uint32_t htot[2];
     {
@@ -2679,30 +2710,129 @@ void label_and_traverse(Ctx &c) {
         pa.slow = st.slow;
         pa.flags = c.flags;
         k_jpieces<<<dim3(grid_for(std::max(mP, mQ)), 2), BLK, 0, s>>>(pa);
-        k_jmask<<<grid_for(std::max(M, J)), BLK, 0, s>>>(J, M, pa.pj, st.slow, st.kind, pa.succ, pa.val);
         SC_HIP(hipGetLastError());
     }
     // routes and crossing counts on the host
     std::vector<int> hk(3 * size_t(J));
-    js.reason.resize(size_t(J));
-    {
-        ReadBack rb(c);
-        rb.add(hk.data(), static_cast<const int *>(st.kind), 3 * size_t(J));
-        rb.add(js.reason.data(), static_cast<const int *>(st.slow), size_t(J));
-        rb.run();
-    }
     const int *hkind = hk.data(), *hmP = hk.data() + J, *hmQ = hk.data() + 2 * J;
-    js.route.assign(hkind, hkind + J);
+    js.reason.resize(size_t(J));
     int maxm = 0, maxmP = 0; // crossings of the largest traversed job, and its P crossings
     std::vector<int> seq_jobs;
     bool any_nocross = false;
-    for (int j = 0; j < J; ++j) {
-        if (hkind[j] == K_CROSS) {
-            maxm = std::max(maxm, hmP[j] + hmQ[j]);
-            maxmP = std::max(maxmP, hmP[j]);
+    auto add_routes = [&](ReadBack &rb) {
+        rb.add(hk.data(), static_cast<const int *>(st.kind), 3 * size_t(J));
+        rb.add(js.reason.data(), static_cast<const int *>(st.slow), size_t(J));
+    };
+    auto take_routes = [&] {
+        js.route.assign(hkind, hkind + J);
+        for (int j = 0; j < J; ++j) {
+            if (hkind[j] == K_CROSS && js.reason[j]) js.route[j] = K_SEQ; // found inconsistent later
+            if (js.route[j] == K_CROSS) {
+                maxm = std::max(maxm, hmP[j] + hmQ[j]);
+                maxmP = std::max(maxmP, hmP[j]);
+            }
+            else if (js.route[j] == K_SEQ) seq_jobs.push_back(j);
+            else any_nocross = true;
         }
-        else if (hkind[j] == K_SEQ) seq_jobs.push_back(j);
-        else any_nocross = true;
+    };
+    // cycles of the crossing jobs: minimum and distance to it by doubling
+    uint32_t *dist = nullptr, *inode = nullptr;
+    uint32_t *base = f.tot.ensure(int64_t(mP) + 1), *ridx = f.ringidx.ensure(int64_t(mP) + 1);
+    const uint32_t *gave_up = nullptr; // set where the crossings' links are no permutation
+    // longest: as many P crossings as a cycle may hold
+    auto rank_cycles = [&](int longest, bool every) {
+        const int rounds = ilog2_exact(longest);
+        const JumpArgs ja{mP, M, pa.val, pa.succ, pa.plen, pa.pj, st.kind, st.slow};
+        uint2 *ends = f.jend.ensure(mP > 0 ? mP : 1);
+        uint32_t *moved = f.jmoved.ensure(size_t(rounds) + 1); // per round, and whether a walk gave up
+        // the windows of the n records a, doubled until they hold whole cycles
+        auto doubled = [&](int n, uint4 *a, uint4 *b) {
+            for (int r = 0; r < rounds; ++r) {
+                k_jump_rank<<<grid_for(n), BLK, 0, s>>>(n, a, b, moved, r);
+                std::swap(a, b);
+            }
+            return a;
+        };
+        if (mP > 0 && mP <= JUMP_SMALL) {
+            k_jump_small<<<1, JUMP_BLK, 0, s>>>(ja, rounds, ends);
+        } else if (mP > 0) {
+            const int G = int(ceil_div(int64_t(mP), int64_t(RULE)));
+            uint4 *rec = f.jrec.ensure(mP), *rule = f.jrule.ensure(3 * size_t(G));
+            uint2 *cov = f.jcov.ensure(mP);
+            {
+                FillBatch fb(s);
+                fb.add(moved, rounds + 1, 0u);
+                fb.flush();
+            }
+            k_jump_init<<<grid_for(mP), BLK, 0, s>>>(ja, rec, cov);
+            if (every) {
+                const uint4 *whole = doubled(mP, rec, f.jrec2.ensure(mP));
+                k_jump_out<<<grid_for(mP), BLK, 0, s>>>(mP, whole, ends);
+            } else {
+                k_ruler_walk<<<grid_for(G), BLK, 0, s>>>(mP, G, rec, cov, rule, moved + rounds);
+                const uint4 *whole = rule + G;
+                if (G <= JUMP_SMALL) k_rule_small<<<1, JUMP_BLK, 0, s>>>(rule + G, G, rounds);
+                else whole = doubled(G, rule + G, rule + 2 * size_t(G));
+                k_ruler_final<<<grid_for(mP), BLK, 0, s>>>(mP, rec, cov, rule, whole, ends, moved + rounds);
+                gave_up = moved + rounds;
+            }
+        }
+        inode = f.inode.ensure(M);
+        dist = f.dist.ensure(M);
+        uint32_t *isstart = f.isstart.ensure(int64_t(mP) + 1);
+        k_rank_final<<<grid_for(M), BLK, 0, s>>>(M, mP, ends, pa.succ, pa.plen, inode, dist, base, isstart);
+        SC_HIP(hipGetLastError());
+        scan_exclusive_u32_2(base, base, int64_t(mP) + 1, nullptr, isstart, ridx, int64_t(mP) + 1, nullptr, s);
+    };
+    // per-job output sizes before clean-up, and their offsets
+    uint32_t *jv = f.jv.ensure(J + 1), *jr = f.jr.ensure(J + 1);
+    CountArgs ca;
+    ca.J = J;
+    ca.AB = AB;
+    ca.AC = AC;
+    ca.kind = st.kind;
+    ca.slow = st.slow;
+    ca.windP = st.windP;
+    ca.windQ = st.windQ;
+    ca.cP0 = st.cP0;
+    ca.sidx = sidx;
+    ca.seq_res = nullptr;
+    ca.base = base;
+    ca.ridx = ridx;
+    ca.jv = jv;
+    ca.jr = jr;
+    auto totals = [&](bool routes) {
+        k_jcounts<<<grid_for(int64_t(J) + 1), BLK, 0, s>>>(ca);
+        SC_HIP(hipGetLastError());
+        scan_exclusive_u32_2(jv, jv, int64_t(J) + 1, tot, jr, jr, int64_t(J) + 1, tot + 1, s);
+        uint32_t over = 0;
+        ReadBack rb(c);
+        rb.add(htot, static_cast<const uint32_t *>(tot), 2);
+        if (gave_up) rb.add(&over, gave_up, 1);
+        if (routes) add_routes(rb);
+        rb.run();
+        return over == 0u;
+    };
+    // Few crossings: their cycles are ranked before the routes are known, and
+    // one read-back brings the routes and the totals (which stand where no job
+    // is sequential).  Many: the routes come first, so that the sequential jobs
+    // run beside the ranking.
+    const bool few = mP <= RULE * JUMP_SMALL; // no launch per round
+    bool counted = false;
+    if (few) {
+        if (mP > 0) rank_cycles(mP, false);
+        if (!totals(true)) {
+            gave_up = nullptr;
+            rank_cycles(mP, true);
+            totals(true);
+        }
+        take_routes();
+        counted = seq_jobs.empty();
+    } else {
+        ReadBack rb(c);
+        add_routes(rb);
+        rb.run();
+        take_routes();
     }
     // sequential route
     const int nseq = int(seq_jobs.size());
@@ -2860,85 +2990,17 @@ void label_and_traverse(Ctx &c) {
         SC_HIP(hipGetLastError());
         SC_HIP(hipEventRecord(c.ev_join, c.stream2));
     }
-    // cycles of the crossing jobs: minimum and distance to it by doubling
-    uint32_t *dist = nullptr, *inode = nullptr;
-    uint32_t *base = f.tot.ensure(int64_t(mP) + 1), *ridx = f.ringidx.ensure(int64_t(mP) + 1);
-    const uint32_t *gave_up = nullptr; // set where the crossings' links are no permutation
-    auto rank_cycles = [&](bool every) {
-        // a cycle of a traversed job holds at most maxmP P crossings
-        const int rounds = ilog2_exact(maxmP);
-        uint2 *ends = f.jend.ensure(mP > 0 ? mP : 1);
-        uint32_t *moved = f.jmoved.ensure(size_t(rounds) + 1); // per round, and whether a walk gave up
-        // the windows of the n records a, doubled until they hold whole cycles
-        auto doubled = [&](int n, uint4 *a, uint4 *b) {
-            for (int r = 0; r < rounds; ++r) {
-                k_jump_rank<<<grid_for(n), BLK, 0, s>>>(n, a, b, moved, r);
-                std::swap(a, b);
-            }
-            return a;
-        };
-        if (mP > 0 && mP <= JUMP_SMALL) {
-            k_jump_small<<<1, JUMP_BLK, 0, s>>>(mP, M, pa.val, pa.succ, pa.plen, rounds, ends);
-        } else if (mP > 0) {
-            const int G = int(ceil_div(int64_t(mP), int64_t(RULE)));
-            uint4 *rec = f.jrec.ensure(mP), *rule = f.jrule.ensure(3 * size_t(G));
-            uint2 *cov = f.jcov.ensure(mP);
-            {
-                FillBatch fb(s);
-                fb.add(moved, rounds + 1, 0u);
-                fb.flush();
-            }
-            k_jump_init<<<grid_for(mP), BLK, 0, s>>>(mP, M, pa.val, pa.succ, pa.plen, rec, cov);
-            if (every) {
-                const uint4 *whole = doubled(mP, rec, f.jrec2.ensure(mP));
-                k_jump_out<<<grid_for(mP), BLK, 0, s>>>(mP, whole, ends);
-            } else {
-                k_ruler_walk<<<grid_for(G), BLK, 0, s>>>(mP, G, rec, cov, rule, moved + rounds);
-                const uint4 *whole = doubled(G, rule + G, rule + 2 * size_t(G));
-                k_ruler_final<<<grid_for(mP), BLK, 0, s>>>(mP, rec, cov, rule, whole, ends, moved + rounds);
-                gave_up = moved + rounds;
-            }
+    if (!few && maxm > 0) rank_cycles(maxmP, false);
+    if (!counted) {
+        if (nseq > 0) {
+            ca.seq_res = f.sres;
+            SC_HIP(hipStreamWaitEvent(s, c.ev_join, 0));
         }
-        inode = f.inode.ensure(M);
-        dist = f.dist.ensure(M);
-        uint32_t *isstart = f.isstart.ensure(int64_t(mP) + 1);
-        k_rank_final<<<grid_for(M), BLK, 0, s>>>(M, mP, ends, pa.succ, pa.plen, inode, dist, base, isstart);
-        SC_HIP(hipGetLastError());
-        scan_exclusive_u32_2(base, base, int64_t(mP) + 1, nullptr, isstart, ridx, int64_t(mP) + 1, nullptr, s);
-    };
-    if (maxm > 0) rank_cycles(false);
-    // per-job output sizes before clean-up, and their offsets
-    uint32_t *jv = f.jv.ensure(J + 1), *jr = f.jr.ensure(J + 1);
-    CountArgs ca;
-    ca.J = J;
-    ca.AB = AB;
-    ca.AC = AC;
-    ca.kind = st.kind;
-    ca.windP = st.windP;
-    ca.windQ = st.windQ;
-    ca.cP0 = st.cP0;
-    ca.sidx = sidx;
-    ca.seq_res = nseq > 0 ? f.sres.p : nullptr;
-    ca.base = base;
-    ca.ridx = ridx;
-    ca.jv = jv;
-    ca.jr = jr;
-    if (nseq > 0) SC_HIP(hipStreamWaitEvent(s, c.ev_join, 0));
-    auto totals = [&] {
-        k_jcounts<<<grid_for(int64_t(J) + 1), BLK, 0, s>>>(ca);
-        SC_HIP(hipGetLastError());
-        scan_exclusive_u32_2(jv, jv, int64_t(J) + 1, tot, jr, jr, int64_t(J) + 1, tot + 1, s);
-        uint32_t over = 0;
-        ReadBack rb(c);
-        rb.add(htot, static_cast<const uint32_t *>(tot), 2);
-        if (gave_up) rb.add(&over, gave_up, 1);
-        rb.run();
-        return over == 0u;
-    };
-    if (!totals()) {
-        gave_up = nullptr;
-        rank_cycles(true);
-        totals();
+        if (!totals(false)) {
+            gave_up = nullptr;
+            rank_cycles(maxmP, true);
+            totals(false);
+        }
     }
     const int64_t NV = htot[0];
     const int NR = int(htot[1]);

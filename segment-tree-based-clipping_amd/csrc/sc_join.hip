@@ -295,7 +295,14 @@ __global__ __launch_bounds__(BLK) void k_join_pairs(PairArgs a) {
         }
     }
     __syncthreads();
-    const uint32_t ntile = toff[TILE_SEGS];
+    // Fewer tiles than waves: 2 to 16 waves share a tile, each walking every
+    // 2nd to 16th of its rows or columns (two stars of 1,000 and 1,100 vertices
+    // have 272 tiles, which took 36 us a wave each, 13 shared).
+    const uint32_t nw = gridDim.x * WPB;
+    uint32_t parts = 1;
+    while (parts < 16u && toff[TILE_SEGS] * parts * 2u <= nw) parts *= 2u;
+    const uint32_t ntile = toff[TILE_SEGS] * parts; // shares of tiles
+    const uint64_t share = ~0ull / ((1ull << parts) - 1ull); // every parts-th row
     uint32_t *vb = qb[wv], *vc = qc[wv], *vk = qk[wv];
     uint64_t *hits = hits_all[wv];
     const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (WAVE - lane));
@@ -346,7 +353,6 @@ __global__ __launch_bounds__(BLK) void k_join_pairs(PairArgs a) {
             nh += add;
         }
     };
-    const uint32_t nw = gridDim.x * WPB;
     const uint32_t per = min(8u, max(1u, ntile / (4u * nw))); // tiles per turn
     int sg = 0;
     for (uint32_t t0 = (blockIdx.x * WPB + wv) * per; t0 < ntile; t0 += nw * per) {
@@ -354,12 +360,13 @@ __global__ __launch_bounds__(BLK) void k_join_pairs(PairArgs a) {
         int hi = TILE_SEGS; // toff[sg] <= t0 < toff[hi]: later turns search on from the last segment
         while (hi - sg > 1) {
             const int mid = (sg + hi) >> 1;
-            if (toff[mid] <= t0) sg = mid;
+            if (toff[mid] * parts <= t0) sg = mid;
             else hi = mid;
         }
         for (uint32_t t = t0; t < t1; ++t) {
-            while (toff[sg + 1] <= t) ++sg; // t < ntile = toff[TILE_SEGS]: ends at the last non-empty segment
-            const uint2 tl = a.tiles[size_t(sg) * a.cap + (t - toff[sg])];
+            const uint32_t tile = t / parts;
+            while (toff[sg + 1] <= tile) ++sg; // tile < toff[TILE_SEGS]: ends at the last non-empty segment
+            const uint2 tl = a.tiles[size_t(sg) * a.cap + (tile - toff[sg])];
             const uint32_t lb = uni(tl.x), lc = uni(tl.y);
             const Leaf db = a.desc[lb], dc = a.desc[lc];
             const BoxF bb = a.box[lb], cb = a.box[lc];
@@ -369,7 +376,7 @@ __global__ __launch_bounds__(BLK) void k_join_pairs(PairArgs a) {
             const uint64_t R = meets(rb, cb), C = meets(cl, bb);
             // walk the side with fewer survivors, the other side in lanes
             const bool rows = __popcll(R) <= __popcll(C);
-            uint64_t set = rows ? R : C;
+            uint64_t set = (rows ? R : C) & (share << (t % parts));
             const uint64_t other = rows ? C : R;
             const BoxF mine = rows ? cl : rb, walk = rows ? rb : cl;
             while (set) {
@@ -513,7 +520,8 @@ bool join_candidates(Ctx &c) {
     // the pair order, so both leave that field out of the sort.
     const int64_t n = int64_t(h[0]);
     const int kb = c.bits_b + c.bits_c + (c.paired || c.K == 1 ? 0 : c.bits_k);
-    radix_sort_u64_buf(c.pairs, c.cand, nullptr, nullptr, n, 0, kb, c.rs, s);
+    if (n <= SMALL_SORT_MAX) sort_small_u64(c.pairs, c.cand.ensure(size_t(n) + 1), int(n), s); // whole keys: the same order
+    else radix_sort_u64_buf(c.pairs, c.cand, nullptr, nullptr, n, 0, kb, c.rs, s);
     c.n_pairs = n;
     pair_offsets(c);
     c.n_cand = c.n_near = c.n_tests = c.n_units = 0;

@@ -256,12 +256,11 @@ struct AugSides {
 
 // Source vertices: count slot i of job j is vertex i - JX[j] (the last slot of
 // a job is padding).  Every slot of the augmented rings is written once, in
-// full: a source's here, an inserted intersection's in k_aug_segments (an edge
+// full: a source's here, an inserted intersection's by aug_segment (an edge
 // has a slot per non-degenerate intersection, and no fewer positions to fill
 // them from), so nothing is cleared first.  Bound by the stores, 32 bytes a slot.
-__global__ void k_aug_sources(int J, AugSides sides) {
-    const AugSide &z = sides.s[blockIdx.y];
-    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+template <bool ONE>
+__device__ inline void aug_source(int J, const AugSide &z, bool side_b, const int *__restrict__ pt, int64_t i) {
     if (!z.ax || i >= z.JX[J]) return;
     const int j = seg_of_wave(z.JX, J, i);
     const int j0 = z.JX[j], v = int(i - j0);
@@ -270,21 +269,27 @@ __global__ void k_aug_sources(int J, AugSides sides) {
     const double2 V = reinterpret_cast<const double2 *>(z.poly)[int64_t(z.voff[j]) + v];
     z.ax[pos] = V.x;
     z.ay[pos] = V.y;
-    z.av[pos] = -100;
+    int av = -100; // or the parameter of the degenerate intersection that leads its edge's order
+    if (ONE) {
+        const int s = z.all_scan[i];
+        if (z.all_scan[i + 1] > s) {
+            const int p = z.ord[s];
+            if (side_b ? degen_b_first(pt[p]) : degen_c_first(pt[p])) av = z.q[p];
+        }
+    }
+    z.av[pos] = av;
     z.nbr[pos] = -100;
     z.lab[pos] = 0;
     if (z.from) z.from[pos] = v;
 }
 
 // one thread per position of the per-edge alpha order: a leading degenerate
-// intersection marks its edge's source vertex, the non-degenerate ones fill
+// intersection takes its edge's source slot, the non-degenerate ones fill
 // the slots after it in order
-__global__ void k_aug_segments(const int *__restrict__ pj, int I, const int *__restrict__ pt,
-                               const double *__restrict__ px, const double *__restrict__ py, int *flags,
-                               AugSides sides) {
-    const bool side_b = blockIdx.y == 0;
-    const AugSide &z = sides.s[blockIdx.y];
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+template <bool ONE>
+__device__ inline void aug_segment(const int *__restrict__ pj, int I, const int *__restrict__ pt,
+                                   const double *__restrict__ px, const double *__restrict__ py, int *flags,
+                                   const AugSide &z, bool side_b, int i) {
     if (!z.ax || i >= I) return;
     const int p = z.ord[i];
     const int j = pj[p];
@@ -297,7 +302,7 @@ __global__ void k_aug_segments(const int *__restrict__ pj, int I, const int *__r
     const int k0 = (side_b ? degen_b_first(pt[first]) : degen_c_first(pt[first])) ? 1 : 0;
     if (i == s && k0 + nd != t - s) atomicOr(&flags[j], UB_UNASSIGNED);
     if (i == s && k0) {
-        z.av[src] = z.q[p];
+        if (!ONE) z.av[src] = z.q[p];
         z.slot[p] = src;
         return;
     }
@@ -312,6 +317,21 @@ __global__ void k_aug_segments(const int *__restrict__ pj, int I, const int *__r
     z.lab[sl] = 0;
     z.slot[p] = sl;
     if (z.from) z.from[sl] = ~p;
+}
+// blockIdx.y: the sources of either side, then the intersections.  In one
+// launch (ONE) a source looks up whether an intersection leads its edge's
+// order; many slots take two, and the intersection tells its source slot (256
+// pairs with 40 million slots: 0.1 ms less than the look-ups).
+template <bool ONE>
+__global__ __launch_bounds__(BLK) void k_augment(int J, const int *__restrict__ pj, int I, const int *__restrict__ pt,
+                                               const double *__restrict__ px, const double *__restrict__ py,
+                                               int *flags, AugSides sides, int y0) {
+    const int y = int(blockIdx.y) + y0;
+    const AugSide &z = sides.s[y & 1];
+    const bool side_b = (y & 1) == 0;
+    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (y < 2) aug_source<ONE>(J, z, side_b, pt, i);
+    else if (i < I) aug_segment<ONE>(pj, I, pt, px, py, flags, z, side_b, int(i));
 }
 
 // neighbour links, 1-based and local to the job's rings (as the reference's arrays)
@@ -619,7 +639,7 @@ void post_jobs(Ctx &c, int k0, int k1) {
         }
         k_seg_scatter<<<dim3(grid_for(I), sparse ? 1 : 2), BLK, 0, s>>>(I, c.p_j, sc);
         SC_HIP(hipGetLastError());
-        seg_sort<false>(ss, s);
+        seg_sort<false>(ss, I, s);
     }
     // augmented ring sizes and offsets per job
     int *nba = js.d_AB.ensure(J + 1), *nca = js.d_AC.ensure(J + 1);
@@ -687,11 +707,17 @@ void post_jobs(Ctx &c, int k0, int k1) {
     as.s[1] = AugSide{ja.JC, ja.nc, ja.cvoff, nca, c.cpoly, all_c, nd_c, c.p_c, c.ordC, c.p_qb, c.aug_cx,
                       c.aug_cy, c.av_c, c.nbr_c, c.lab_c, from_c, c.slot_c};
     // (the sparse base side has slots by the hundred million and none of these arrays)
-    k_aug_sources<<<dim3(grid_for(sparse ? nJC : std::max(nJB, nJC)), 2), BLK, 0, s>>>(J, as);
+    const int64_t nsrc = sparse ? nJC : std::max(nJB, nJC);
+    if (std::max<int64_t>(I, nsrc) < SPAN_MIN) {
+        k_augment<true><<<dim3(grid_for(std::max<int64_t>(I, nsrc)), I > 0 ? 4 : 2), BLK, 0, s>>>(
+            J, c.p_j, I, c.p_type, c.p_x, c.p_y, flags, as, 0);
+    } else {
+        k_augment<false><<<dim3(grid_for(nsrc), 2), BLK, 0, s>>>(J, c.p_j, I, c.p_type, c.p_x, c.p_y, flags, as, 0);
+        if (I > 0)
+            k_augment<false><<<dim3(grid_for(I), 2), BLK, 0, s>>>(J, c.p_j, I, c.p_type, c.p_x, c.p_y, flags, as, 2);
+    }
     SC_HIP(hipGetLastError());
     if (I > 0) {
-        k_aug_segments<<<dim3(grid_for(I), 2), BLK, 0, s>>>(c.p_j, I, c.p_type, c.p_x, c.p_y, flags, as);
-        SC_HIP(hipGetLastError());
         if (sparse) {
             k_sp_link<<<grid_for(I), BLK, 0, s>>>(I, c.sp_pos, c.p_j, c.sp_slot, c.slot_c, nca, int(nca_tot),
                                                   c.sp_nbr, c.nbr_c, flags);

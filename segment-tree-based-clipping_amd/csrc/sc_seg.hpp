@@ -206,17 +206,18 @@ template <bool FULL> __global__ __launch_bounds__(SEG_BLK) void k_seg_block(SegS
 }
 
 
-// the three launches for the groups of every set; wlist and blist hold the
-// listed groups (capacity: more than SEG_THREAD, resp. SEG_WAVE_MAX keys per
-// listed group), ctl[0..SEG_CTL) is zero before the call
-template <bool FULL> inline void seg_sort(const SegSets &a, hipStream_t s) {
+// the launches for the groups of every set, which hold at most 'keys' keys in
+// all; wlist and blist hold the listed groups (capacity: more than SEG_THREAD,
+// resp. SEG_WAVE_MAX keys per listed group), ctl[0..SEG_CTL) is zero before the
+// call
+template <bool FULL> inline void seg_sort(const SegSets &a, int64_t keys, hipStream_t s) {
     int most = 0;
     for (int k = 0; k < a.count; ++k) most = a.s[k].nseg > most ? a.s[k].nseg : most;
     if (most <= 0) return;
     const unsigned y = unsigned(a.count);
     k_seg_small<FULL><<<dim3(unsigned((most + SEG_BLK - 1) / SEG_BLK), y), SEG_BLK, 0, s>>>(a);
-    k_seg_wave<FULL><<<dim3(1024, y), SEG_BLK, 0, s>>>(a);
-    k_seg_block<FULL><<<dim3(1280, y), SEG_BLK, 0, s>>>(a); // five 32 KB blocks per CU
+    if (keys > SEG_THREAD) k_seg_wave<FULL><<<dim3(1024, y), SEG_BLK, 0, s>>>(a);
+    if (keys > SEG_WAVE_MAX) k_seg_block<FULL><<<dim3(1280, y), SEG_BLK, 0, s>>>(a); // five 32 KB blocks per CU
     SC_HIP(hipGetLastError());
 }
 
