@@ -124,8 +124,21 @@ constexpr int RING_LANES = 16, RING_SET = WAVE / RING_LANES; // lanes of a short
 
 __device__ inline double wave_ring_sum(const double *__restrict__ x, const double *__restrict__ y, int64_t a,
                                        int64_t b, int64_t c0, int64_t c1, int lane) {
+    // four terms are loaded before they are added (the same order and bits): a
+    // wave alone on a long ring does little but wait for its loads
     double s = 0.0;
-    for (int64_t i = c0 + lane; i < c1; i += WAVE) {
+    int64_t i = c0 + lane;
+    for (; i + 3 * WAVE < c1 && i + 3 * WAVE + 1 < b; i += 4 * WAVE) {
+        double t[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int64_t k = i + q * WAVE;
+            t[q] = x[k] * y[k + 1] - x[k + 1] * y[k];
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) s += t[q];
+    }
+    for (; i < c1; i += WAVE) {
         const int64_t nx = i + 1 == b ? a : i + 1;
         s += x[i] * y[nx] - x[nx] * y[i];
     }
@@ -204,24 +217,21 @@ __global__ void k_ring_chunk_sum(int nrings, const uint32_t *__restrict__ choff,
 }
 
 // twice the unsigned area of each job's output: one block per job, thread t
-// adds |S| of rings t, t + 256, ... of the job, then a fixed tree
-__global__ __launch_bounds__(BLK) void k_job_out_area2(const int *__restrict__ jring,
-                                                       const double *__restrict__ ring2, double *out) {
+// adds |S| of rings t, t + 256, ... of the job, then a fixed tree; with the
+// input rings' sums, the job's areas and IoU
+__global__ __launch_bounds__(BLK) void k_job_areas(int J, int paired, const int *__restrict__ jring,
+                                                   const double *__restrict__ ring2,
+                                                   const double *__restrict__ barea2,
+                                                   const double *__restrict__ carea2, double *out4) {
     __shared__ double sh[BLK];
     const int j = blockIdx.x;
     const int r0 = jring[j], r1 = jring[j + 1];
     double s = 0.0;
     for (int r = r0 + int(threadIdx.x); r < r1; r += BLK) s += fabs(ring2[r]);
     const double t = block_sum(s, sh);
-    if (threadIdx.x == 0) out[j] = t;
-}
-
-__global__ void k_job_final(int J, int paired, const double *out2, const double *barea2, const double *carea2,
-                            double *out4) {
-    int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= J) return;
-    double I = 0.5 * out2[j], P = 0.5 * fabs(barea2[paired ? j : 0]), Q = 0.5 * fabs(carea2[j]);
-    double U = P + Q - I;
+    if (threadIdx.x != 0) return;
+    const double I = 0.5 * t, P = 0.5 * fabs(barea2[paired ? j : 0]), Q = 0.5 * fabs(carea2[j]);
+    const double U = P + Q - I;
     out4[j] = I;
     out4[J + j] = P;
     out4[2 * J + j] = Q;
@@ -590,7 +600,7 @@ __global__ __launch_bounds__(BLK) void k_grad_rest(GatherGrad g) {
 }
 
 struct AreaScratch {
-    DBuf<double> out2, ring2, barea2, carea2, out4, cI, cQ, cPr, part, rpart;
+    DBuf<double> ring2, barea2, carea2, out4, cI, cQ, cPr, part, rpart;
     DBuf<int> bad, bin_off;
     DBuf<uint32_t> chunks, choff, tot, rid, gfound;
     // gathered gradients
@@ -604,23 +614,16 @@ AreaScratch &ascratch(Ctx &) {
     return *p;
 }
 
-void job_rings_to_device(Ctx &c) {
-    JobSet &js = c.jobs;
-    SC_REQUIRE(js.J >= 1 && int(js.ring_off.size()) == js.J + 1, SC_ESTATE, "no clipped batch");
-    js.d_ring.ensure(js.J + 1);
-    c.upload(js.d_ring.p, js.ring_off.data(), sizeof(int) * (js.J + 1));
-}
-
 } // namespace
 
 void batch_area(Ctx &c, double *out4) {
     SC_REQUIRE(!c.uni, SC_ESTATE, "area / IoU are defined for the intersection (a union output may hold holes)");
     JobSet &js = c.jobs;
-    job_rings_to_device(c);
+    SC_REQUIRE(js.J >= 1 && int(js.ring_off.size()) == js.J + 1, SC_ESTATE, "no clipped batch");
     hipStream_t s = c.stream;
     AreaScratch &a = ascratch(c);
     const int J = js.J;
-    double *out2 = a.out2.ensure(J), *barea2 = a.barea2.ensure(c.nbr), *carea2 = a.carea2.ensure(J);
+    double *barea2 = a.barea2.ensure(c.nbr), *carea2 = a.carea2.ensure(J);
     double *ring2 = a.ring2.ensure(size_t(c.nrings > 0 ? c.nrings : 1));
     if (c.nrings > 0) {
         const int nr = c.nrings;
@@ -639,7 +642,6 @@ void batch_area(Ctx &c, double *out4) {
                                                                     c.d_ring_y, part);
         k_ring_chunk_sum<<<grid_for(nr), BLK, 0, s>>>(nr, choff, cap, part, ring2);
     }
-    k_job_out_area2<<<J, BLK, 0, s>>>(js.d_ring, ring2, out2);
     RingSides rs;
     const int64_t pb = (c.nb + c.nbr) / RING_CHUNK + c.nbr + 1, pc = (c.nct + c.K) / RING_CHUNK + c.K + 1;
     double *part = a.rpart.ensure(size_t(pb + pc));
@@ -658,7 +660,7 @@ void batch_area(Ctx &c, double *out4) {
         k_ring_area2<<<dim3(unsigned(bx), unsigned(std::min(65535, J - r)), 2), BLK, 0, s>>>(part_of);
     }
     if (longest > 1) k_ring_parts<<<dim3(grid_for(J), 2), BLK, 0, s>>>(rs);
-    k_job_final<<<grid_for(J), BLK, 0, s>>>(J, c.paired ? 1 : 0, out2, barea2, carea2, out4);
+    k_job_areas<<<J, BLK, 0, s>>>(J, c.paired ? 1 : 0, js.d_ring, ring2, barea2, carea2, out4);
     SC_HIP(hipGetLastError());
 }
 

@@ -56,7 +56,7 @@ constexpr size_t UPLOAD_MAX = size_t(4) << 20; // larger tables are copied
 __global__ void k_upload(const uint32_t *src, uint32_t *dst, uint32_t words) {
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < words; i += gridDim.x * blockDim.x) dst[i] = src[i];
 }
-constexpr size_t RB_GATHER_MAX = 65536; // larger items go through the copy engine path
+constexpr size_t RB_GATHER_MAX = size_t(1) << 20; // larger items go through the copy engine path
 } // namespace
 void *Ctx::pinned(size_t bytes) {
     PinnedStage &ps = tl_pin;

@@ -1178,9 +1178,12 @@ __global__ void k_compact_out(int64_t n, const uint32_t *keep, const uint32_t *k
     src2[o] = src[i];
 }
 
-__global__ void k_job_rings(int J, const uint32_t *jr, const uint32_t *nonempty, uint32_t *out) {
+__global__ void k_job_rings(int J, const uint32_t *jr, const uint32_t *nonempty, uint32_t *out, int *ring) {
     int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j <= J) out[j] = nonempty[jr[j]];
+    if (j > J) return;
+    const uint32_t r = nonempty[jr[j]];
+    out[j] = r;
+    ring[j] = int(r);
 }
 
 // ---------------------------------------------------------------------------
@@ -2437,12 +2440,15 @@ template <class T> void d2h_sync(Ctx &c, T *h, const T *d, int64_t n) {
 void cleanup_rings(Ctx &c, FosterScratch &f, int nr, int64_t n, int J, const uint32_t *jr,
                    std::vector<uint32_t> &job_ring) {
     hipStream_t s = c.stream;
+    int *dring = c.jobs.d_ring.ensure(size_t(J) + 1); // job_ring on the device, for the areas
     if (nr == 0 || n == 0) {
         job_ring.assign(size_t(J) + 1, 0u);
         c.nrings = 0;
         c.n_out = 0;
-        c.d_ring_off.ensure(1);
-        SC_HIP(hipMemsetAsync(c.d_ring_off.p, 0, sizeof(int), s));
+        FillBatch fb(s);
+        fb.add(c.d_ring_off.ensure(1), 1, 0u);
+        fb.add(dring, int64_t(J) + 1, 0u);
+        fb.flush();
         return;
     }
     int *rstart = f.rstart.ensure(nr);
@@ -2494,7 +2500,7 @@ void cleanup_rings(Ctx &c, FosterScratch &f, int nr, int64_t n, int J, const uin
         k_ring_counts<<<grid_for(int64_t(nr) + 1), BLK, 0, s>>>(nr, f.off, kscan, rcnt, nonempty);
         SC_HIP(hipGetLastError());
         scan_exclusive_u32(nonempty, nonempty, int64_t(nr) + 1, jring + J + 2, s);
-        k_job_rings<<<grid_for(int64_t(J) + 1), BLK, 0, s>>>(J, jr, nonempty, jring);
+        k_job_rings<<<grid_for(int64_t(J) + 1), BLK, 0, s>>>(J, jr, nonempty, jring, dring);
         SC_HIP(hipGetLastError());
         uint32_t moved = 0;
         ReadBack rb(c);

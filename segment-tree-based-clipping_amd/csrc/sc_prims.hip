@@ -382,35 +382,45 @@ constexpr int RS_TILE = RS_BLOCK * RS_ITEMS;
 constexpr int RS_WAVES = RS_BLOCK / WAVE;
 constexpr int RS_MAXPASS = 8;
 
-// Digit counts of every pass in one read of the keys.  Bound by LDS atomics to
-// the same address: keys that come nearly ordered share their high digits, so a
-// wave with one digit adds once, and the lanes spread over HIST_COPIES counters
-// (24 million keys of six passes: 290 -> 108 us).
-constexpr int HIST_COPIES = 4;
-__global__ __launch_bounds__(RS_BLOCK) void k_global_hist(const uint64_t *keys, int64_t n, int bit_lo, int bit_hi,
+// Digit counts of every pass in one read of the keys.  Bound by atomics: in
+// LDS to the same address, as keys that come nearly ordered share their high
+// digits, so a wave with one digit adds once and the lanes spread over
+// HIST_COPIES counters; in memory by a block's 256 counters per pass, so large
+// blocks and no more of them than CUs (24 million keys of six passes: 290 ->
+// 108 us, 260,000 of eight: 16 -> 11).
+constexpr int HIST_COPIES = 4, HIST_BLK = 1024, HIST_PER = 4;
+inline int hist_blocks(int64_t n) { return int(std::max<int64_t>(1, std::min<int64_t>(256, n / (HIST_BLK * 2 * HIST_PER)))); }
+__global__ __launch_bounds__(HIST_BLK) void k_global_hist(const uint64_t *keys, int64_t n, int bit_lo, int bit_hi,
                                                           int npass, uint32_t *ghist) {
     __shared__ uint32_t h[HIST_COPIES][RS_MAXPASS][256];
-    for (int i = threadIdx.x; i < HIST_COPIES * RS_MAXPASS * 256; i += RS_BLOCK) (&h[0][0][0])[i] = 0;
+    for (int i = threadIdx.x; i < HIST_COPIES * RS_MAXPASS * 256; i += HIST_BLK) (&h[0][0][0])[i] = 0;
     __syncthreads();
-    const int copy = threadIdx.x & (HIST_COPIES - 1);
-    for (int64_t i = int64_t(blockIdx.x) * RS_BLOCK + threadIdx.x; i < n; i += int64_t(gridDim.x) * RS_BLOCK) {
-        const uint64_t k = keys[i];
-        for (int p = 0; p < npass; ++p) {
-            const int sh = bit_lo + 8 * p;
-            const int bits = bit_hi - sh < 8 ? bit_hi - sh : 8;
-            const uint32_t d = uint32_t(k >> sh) & ((1u << bits) - 1u);
-            const uint32_t d0 = uint32_t(__builtin_amdgcn_readfirstlane(int(d)));
-            const uint64_t here = __ballot(1);
-            if (__ballot(d != d0) == 0) {
-                if (int(threadIdx.x & (WAVE - 1)) == __ffsll((unsigned long long)here) - 1)
-                    atomicAdd(&h[0][p][d0], uint32_t(__popcll(here)));
-            } else {
-                atomicAdd(&h[copy][p][d], 1u);
+    const int copy = threadIdx.x & (HIST_COPIES - 1), lane = threadIdx.x & (WAVE - 1);
+    const int64_t step = int64_t(gridDim.x) * HIST_BLK;
+    for (int64_t i0 = int64_t(blockIdx.x) * HIST_BLK + threadIdx.x; i0 - lane < n; i0 += HIST_PER * step) {
+        uint64_t k[HIST_PER];
+#pragma unroll
+        for (int q = 0; q < HIST_PER; ++q) k[q] = i0 + q * step < n ? keys[i0 + q * step] : 0ull;
+#pragma unroll
+        for (int q = 0; q < HIST_PER; ++q) {
+            const bool have = i0 + q * step < n;
+            const uint64_t here = __ballot(have);
+            if (!here) break;
+            for (int p = 0; p < npass; ++p) {
+                const int sh = bit_lo + 8 * p;
+                const int bits = bit_hi - sh < 8 ? bit_hi - sh : 8;
+                const uint32_t d = uint32_t(k[q] >> sh) & ((1u << bits) - 1u);
+                const uint32_t d0 = uint32_t(__builtin_amdgcn_readfirstlane(int(d))); // lane 0 has a key if any has
+                if (__ballot(have && d != d0) == 0) {
+                    if (lane == 0) atomicAdd(&h[0][p][d0], uint32_t(__popcll(here)));
+                } else if (have) {
+                    atomicAdd(&h[copy][p][d], 1u);
+                }
             }
         }
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < npass * 256; i += RS_BLOCK) {
+    for (int i = threadIdx.x; i < npass * 256; i += HIST_BLK) {
         uint32_t v = 0;
         for (int q = 0; q < HIST_COPIES; ++q) v += (&h[q][0][0])[i];
         if (v) atomicAdd(&ghist[i], v);
@@ -810,9 +820,7 @@ bool radix_passes(uint64_t *keys, uint32_t *vals, uint64_t *kalt, uint32_t *valt
     const size_t GH = size_t(RS_MAXPASS) * 256;
     uint32_t *gh = rs.global_hist.ensure(GH);
     SC_HIP(hipMemsetAsync(gh, 0, sizeof(uint32_t) * GH, s));
-    int ghb = int(ceil_div(n, RS_BLOCK * 16));
-    if (ghb > 1024) ghb = 1024;
-    k_global_hist<<<ghb, RS_BLOCK, 0, s>>>(keys, n, bit_lo, bit_hi, npass, gh);
+    k_global_hist<<<hist_blocks(n), HIST_BLK, 0, s>>>(keys, n, bit_lo, bit_hi, npass, gh);
     SC_HIP(hipGetLastError());
 
     const int64_t ntiles = ceil_div(n, RS_TILE);
@@ -879,9 +887,7 @@ bool radix_sort_u64_fixed(uint64_t *keys, uint32_t *vals, uint64_t *kalt, uint32
         fb.add(st, 2 * ntiles * 256, 0u);
         fb.flush();
     }
-    int ghb = int(ceil_div(n, RS_BLOCK * 16));
-    if (ghb > 1024) ghb = 1024;
-    k_global_hist<<<ghb, RS_BLOCK, 0, s>>>(keys, n, bit_lo, bit_hi, npass, gh);
+    k_global_hist<<<hist_blocks(n), HIST_BLK, 0, s>>>(keys, n, bit_lo, bit_hi, npass, gh);
     SC_HIP(hipGetLastError());
     uint64_t *kc = keys, *ko = kalt;
     uint32_t *vc = vals, *vo = valt;

@@ -689,12 +689,8 @@ __global__ void k_small_emit(int J, const int *__restrict__ voff, const int *__r
             ring_off[r0 + r] = at;
             at += olen[int64_t(j) * SP_OUTR + r];
         }
+        if (j == J - 1) ring_off[roff[J]] = voff[J]; // the closing entry
     }
-}
-
-// the totals after the exclusive scans of the per-job counts: ring_off[NR] = NV
-__global__ void k_small_tail(int J, const int *__restrict__ voff, const int *__restrict__ roff, int *ring_off) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) ring_off[roff[J]] = voff[J];
 }
 
 // rings given back to back without closing vertices (the set_pairs layout)
@@ -717,7 +713,7 @@ __global__ void k_pairs_layout(const double *__restrict__ xy, int64_t n, const i
 }
 
 struct SmallScratch {
-    DBuf<int> jobs, fail, route, nv, nr, voff, roff, olen;
+    DBuf<int> jobs, fail, route, nv, nr, voff, olen;
     DBuf<double> ox, oy;
 };
 
@@ -774,7 +770,7 @@ bool clip_small_batch(Ctx &c, int k0, int k1) {
     a.anyfail = nullptr;
     k_small_pairs<<<J, WAVE, 0, s>>>(a);
     SC_HIP(hipGetLastError());
-    int *voff = S.voff.ensure(size_t(J) + 1), *roff = S.roff.ensure(size_t(J) + 1);
+    int *voff = S.voff.ensure(size_t(J) + 1), *roff = c.jobs.d_ring.ensure(size_t(J) + 1); // rings: for the areas too
     scan_exclusive_u32_2(reinterpret_cast<const uint32_t *>(a.job_nv), reinterpret_cast<uint32_t *>(voff), J + 1,
                          nullptr, reinterpret_cast<const uint32_t *>(a.job_nr), reinterpret_cast<uint32_t *>(roff),
                          J + 1, nullptr, s);
@@ -801,7 +797,6 @@ bool clip_small_batch(Ctx &c, int k0, int k1) {
     c.d_ring_y.ensure(size_t(NV > 0 ? NV : 1));
     k_small_emit<<<J, 256, 0, s>>>(J, voff, roff, a.job_nr, a.out_x, a.out_y, a.out_len, c.d_ring_x, c.d_ring_y,
                                    c.d_ring_off);
-    k_small_tail<<<1, 1, 0, s>>>(J, voff, roff, c.d_ring_off);
     SC_HIP(hipGetLastError());
     c.nrings = NR;
     c.n_out = NV;
