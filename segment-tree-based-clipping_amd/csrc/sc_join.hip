@@ -254,7 +254,11 @@ struct PairArgs {
 
 constexpr int QNEAR = 2 * WAVE;      // near pairs classified per step, two per lane
 constexpr int QCAP = QNEAR + WAVE;   // queue: a row adds at most 64
-constexpr int HSTG = 4 * WAVE;       // found pairs staged per wave
+// Found pairs staged per wave.  A flush takes its place in the output with an
+// atomic on one word, and those queue up: 20 million pairs with 256 staged took
+// 1.35 ms, with 640 (five blocks of LDS still fit a CU) 0.87; eight counters
+// with parts of the output to pack afterwards gain nothing more.
+constexpr int HSTG = 10 * WAVE;
 
 // One wave per run of tiles; the grid covers the chip and strides over the
 // tiles.  Bound by VALU issue: about 14 instructions per surviving row and
