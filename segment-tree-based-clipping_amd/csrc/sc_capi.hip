@@ -242,7 +242,7 @@ void release_derived(Ctx &c) {
     for (DBuf<double> *b : {&c.ex0, &c.ey0, &c.ex1, &c.ey1, &c.estart, &c.eend, &c.uxs, &c.uxe, &c.eymin, &c.eymax,
                             &c.ea, &c.niv, &c.p_x, &c.p_y, &c.aug_bx, &c.aug_by, &c.aug_cx, &c.aug_cy})
         b->release();
-    for (DBuf<int> *b : {&c.sp_slot, &c.sp_ndx, &c.sp_edge, &c.sp_av, &c.sp_nbr, &c.sp_lab, &c.sp_pos, &c.sp_ndf, &c.run_start})
+    for (DBuf<int> *b : {&c.sp_slot, &c.sp_ndx, &c.sp_edge, &c.sp_av, &c.sp_nbr, &c.sp_lab, &c.sp_ndf, &c.run_start})
         b->release();
     for (DBuf<uint64_t> *b : {&c.join_box, &c.join_leaf, &c.join_tile}) b->release();
     c.join_ctl.release();

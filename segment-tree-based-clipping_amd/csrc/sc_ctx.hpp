@@ -22,6 +22,8 @@ struct JobSet {
     std::vector<int> cin;      // first input vertex (no closing vertices) of each job's overlay
     std::vector<int> route, reason; // labelling route per job (0 crossing, 1 no crossing, 2 sequential), why sequential
     DBuf<int> d_AB, d_AC, d_ring;
+    bool late = false;         // AB and AC are still on the device (below: the most they end with)
+    int64_t cap_b = 0, cap_c = 0;
     // device copies of p0, bvoff, beoff, nb, nc, cvoff, JB, JC, cin: views into
     // one buffer filled by one host-to-device copy
     DBuf<int> d_pack;
@@ -95,6 +97,7 @@ struct Ctx {
     DBuf<uint64_t> join_box, join_leaf;  // boxes of leaves and base groups; first vertex, size, edge, ring of leaves
     DBuf<uint64_t> join_tile;            // (base leaf, overlay leaf) tiles in segments of join_seg_cap entries
     DBuf<uint32_t> join_ctl;             // totals, flag, segment counters
+    uint32_t join_call = 0; // number of the last join
     int64_t join_seg_cap = 0;
     // ---- A8/A10 candidates and unique pairs ----
     DBuf<uint64_t> unit_desc;            // stab work units: 32-byte records
@@ -139,7 +142,7 @@ struct Ctx {
     // sparse base ring (one-to-many batches without provenance): per position
     // (pair in (job, base edge, alpha) order) its virtual slot and slot data
     bool sparseP = false;
-    DBuf<int> sp_slot, sp_ndx, sp_edge, sp_av, sp_nbr, sp_lab, sp_pos, sp_ndf;
+    DBuf<int> sp_slot, sp_ndx, sp_edge, sp_av, sp_nbr, sp_lab, sp_ndf;
     DBuf<double> sp_x, sp_y;
     DBuf<int> from_b, from_c;            // per slot: source vertex (local), or ~ the pair inserted there
     DBuf<int> flags;                     // device status words
@@ -235,7 +238,7 @@ void pair_offsets(Ctx &c);             // pair_off of c.n_pairs sorted pairs
 void build_tree(Ctx &c);
 void tree_after_join(Ctx &c);
 void stab_after_join(Ctx &c);
-void post_jobs(Ctx &c, int k0, int k1); // A11-A15 for overlays k0..k1 in one batch
+void post_jobs(Ctx &c, int k0, int k1, bool late = false); // A11-A15 for overlays k0..k1 in one batch
 // the batch's per-job flags (jobs.flags, undefined) from the device, when the
 // post stage left them there (labelling fetches them with its first read-back)
 void fetch_flags(Ctx &c);
@@ -279,7 +282,7 @@ void rings_to_host(Ctx &c, int32_t *ring_off, double *xy); // ring offsets and x
 
 // Device-to-host read-backs through the context's pinned staging, one wait
 // for all of them: add() up to RB_MAX pieces, then run().
-constexpr int RB_MAX = 4;
+constexpr int RB_MAX = 6;
 struct ReadBack {
     Ctx &c;
     int n = 0;

@@ -40,6 +40,7 @@
 // as g, a Q slot g as ~g, none as SRC_NONE) for the area gradient.
 #include "sc_ctx.hpp"
 #include "sc_fp64.hpp"
+#include "sc_seg.hpp"
 #include "sc_seqroute.hpp"
 
 #include <algorithm>
@@ -80,7 +81,7 @@ __device__ inline bool inter_at(const Side &s, int64_t i) { return s.av ? s.av[i
 struct ClassifyArgs {
     Side s[2];
     int J, per;
-    int64_t n[2];
+    int64_t n[2];  // flags of the sides: their slots or more
     const int *pj; // jobs of a sparse base side's slots (its pairs' jobs), else null
     uint32_t *cross[2];
     int *slow, *first[2];
@@ -92,12 +93,12 @@ __global__ __launch_bounds__(BLK) void k_jclassify(ClassifyArgs a) {
     const int lane = threadIdx.x & (WAVE - 1);
     if (blockIdx.y < 2) {
         const int *pj = y ? nullptr : a.pj;
-        const int64_t n = a.n[y];
+        const int64_t n = s.off[a.J];
         WaveSpan w(s.off, a.J, pj ? 0 : n, a.per);
-        for (int q = 0; q < a.per && w.at <= n; ++q, w.at += WAVE) {
+        for (int q = 0; q < a.per && w.at <= a.n[y]; ++q, w.at += WAVE) {
             const int64_t i = w.at + lane;
             const int js = pj ? 0 : w.of(s.off, a.J, lane);
-            if (i > n) continue;
+            if (i > a.n[y]) continue;
             uint32_t c = 0;
             if (i < n && inter_at(s, i)) {
                 const int j = pj ? pj[i] : js;
@@ -133,7 +134,6 @@ __global__ __launch_bounds__(BLK) void k_jclassify(ClassifyArgs a) {
 // rings, summed per job; blockIdx.y picks the side (a null wind: not this way)
 struct WindSide {
     Side r;
-    int64_t n;
     Side from;        // the other side, whose first plain vertices are the query points
     const int *first;
     const double *q;  // or the points, x,y per job (sparse base side)
@@ -189,19 +189,20 @@ __global__ __launch_bounds__(BLK) void k_jwinding(WindSides a) {
     const WindSide &z = a.s[blockIdx.y];
     if (!z.wind) return;
     const Side &r = z.r;
+    const int64_t n = r.off[a.J];
     const int lane = threadIdx.x & (WAVE - 1);
-    WaveSpan s(r.off, a.J, z.n, a.per);
+    WaveSpan s(r.off, a.J, n, a.per);
     int sum = 0, of = s.seg; // terms of job 'of', not added yet
     auto add = [&]() {
         for (int d = WAVE / 2; d > 0; d >>= 1) sum += __shfl_down(sum, d, WAVE);
         if (lane == 0 && sum) atomicAdd(&z.wind[of], sum);
         sum = 0;
     };
-    for (int q = 0; q < a.per && s.at < z.n; ++q, s.at += WAVE) {
+    for (int q = 0; q < a.per && s.at < n; ++q, s.at += WAVE) {
         const int64_t i = s.at + lane;
         const int j = s.of(r.off, a.J, lane);
         int w = 0;
-        const int fp = i < z.n ? z.first[j] : -1;
+        const int fp = i < n ? z.first[j] : -1;
         if (fp >= 0) {
             const int64_t nx = i + 1 == r.off[j + 1] ? r.off[j] : i + 1;
             const int64_t v = z.q ? 0 : int64_t(z.from.off[j]) + fp;
@@ -2565,7 +2566,8 @@ void release_foster_scratch() {
 
 void label_and_traverse(Ctx &c) {
     JobSet &js = c.jobs;
-    SC_REQUIRE(js.J >= 1 && int(js.AB.size()) == js.J + 1, SC_ESTATE, "segclip_intersections must run first");
+    SC_REQUIRE(js.J >= 1 && (js.late || int(js.AB.size()) == js.J + 1), SC_ESTATE,
+               "segclip_intersections must run first");
     hipStream_t s = c.stream;
     FosterScratch &f = fscratch();
     const int J = js.J;
@@ -2575,7 +2577,9 @@ void label_and_traverse(Ctx &c) {
     // its intersections (positions); the overlay side is always dense
     const SparseP sp = sparse ? sparse_view(c) : SparseP{};
     const int *PO = sparse ? js.d_p0 : AB; // offsets of the base-side arrays
-    const int64_t nP = sparse ? js.p0[J] : js.AB[J], nQ = js.AC[J];
+    // slots of either side, or the most they can be until the offsets are read back
+    const bool late = js.late;
+    int64_t nP = sparse ? js.p0[J] : (late ? js.cap_b : js.AB[J]), nQ = late ? js.cap_c : js.AC[J];
     const Side P = sparse ? Side{PO, AC, c.sp_x, c.sp_y, c.sp_lab, c.sp_nbr, c.sp_av}
                           : Side{AB, AC, c.aug_bx, c.aug_by, c.lab_b, c.nbr_b, c.av_b};
     const Side Q{AC, AB, c.aug_cx, c.aug_cy, c.lab_c, c.nbr_c, nullptr};
@@ -2619,8 +2623,8 @@ void label_and_traverse(Ctx &c) {
     cl.bounce = bounce;
     cl.first[0] = sparse ? nullptr : st.firstP;
     cl.first[1] = st.firstQ;
-    const int64_t most = std::max(nP, nQ); // slots of the larger side
-    const int per = cl.per = span_per(most);
+    int64_t most = std::max(nP, nQ); // slots of the larger side
+    int per = cl.per = span_per(most);
     k_jclassify<<<dim3(std::max(grid_for(most + 1, BLK * per), grid_for(int64_t(J) * WAVE)), 4), BLK, 0, s>>>(cl);
     if (sparse) k_sp_first_plain<<<grid_for(int64_t(J) * WAVE), BLK, 0, s>>>(sp, J, st.firstP);
     SC_HIP(hipGetLastError());
@@ -2638,8 +2642,8 @@ void label_and_traverse(Ctx &c) {
         SC_HIP(hipGetLastError());
     }
     WindSides wd;
-    wd.s[0] = WindSide{Q, nQ, P, st.firstP, pq, st.windP};
-    wd.s[1] = WindSide{P, nP, Q, st.firstQ, nullptr, sparse ? nullptr : st.windQ};
+    wd.s[0] = WindSide{Q, P, st.firstP, pq, st.windP};
+    wd.s[1] = WindSide{P, Q, st.firstQ, nullptr, sparse ? nullptr : st.windQ};
     wd.J = J;
     wd.per = per;
     wd.st = st;
@@ -2655,12 +2659,19 @@ void label_and_traverse(Ctx &c) {
         if (nP > 0) k_sp_wind_fix<<<grid_for(nP), BLK, 0, s>>>(int(nP), c.p_j, sp, qq, qok, st.windQ);
     }
     SC_HIP(hipGetLastError());
-    uint32_t htot[2];
+    uint32_t htot[2], hseg[2 * SEG_CTL] = {};
     {
-        ReadBack rb(c); // with the post stage's job flags, when still on the device
+        ReadBack rb(c); // with the post stage's job flags and offsets, when still on the device
         rb.add(htot, static_cast<const uint32_t *>(tot), 2);
         const bool fl = c.flags_pending;
         if (fl) rb.add(js.flags.data(), static_cast<const int *>(c.flags.p), size_t(J));
+        if (late) {
+            js.AB.resize(size_t(J) + 1);
+            js.AC.resize(size_t(J) + 1);
+            rb.add(js.AB.data(), AB, size_t(J) + 1);
+            rb.add(js.AC.data(), AC, size_t(J) + 1);
+            if (c.I > 0) rb.add(hseg, static_cast<const uint32_t *>(c.seg_ctl.p), 2 * SEG_CTL);
+        }
         rb.run();
         if (fl) {
             c.flags_pending = false;
@@ -2668,6 +2679,20 @@ void label_and_traverse(Ctx &c) {
             for (int v : js.flags) any |= v;
             c.undefined = any;
         }
+    }
+    if (late) {
+        js.late = false;
+        if (hseg[2] | hseg[SEG_CTL + 2]) { // a group too large for the ordering: again, with the radix sort
+            post_jobs(c, js.k0, js.k0 + J - 1);
+            label_and_traverse(c);
+            return;
+        }
+        c.nbaug = js.AB[J];
+        c.ncaug = js.AC[J];
+        if (!sparse) nP = js.AB[J];
+        nQ = js.AC[J];
+        most = std::max(nP, nQ);
+        per = span_per(most);
     }
     const int mP = int(htot[0]), mQ = int(htot[1]);
     const int M = mP + mQ;
@@ -3145,7 +3170,7 @@ void clip_jobs(Ctx &c, int k0, int k1) {
     c.mark(4);
     if (cand && !joined) find_candidates(c);
     c.mark(5);
-    post_jobs(c, k0, k1);
+    post_jobs(c, k0, k1, true);
     c.mark(6);
     label_and_traverse(c);
     c.mark(7);

@@ -68,6 +68,7 @@ struct RingTab {
     const double *shift; // per ring of a pair, or null
     int nbr, K;
     uint32_t lb, nleaf; // base leaves, all leaves
+    uint32_t call;      // this join's number: what "bad" holds where its rings are not for the join
 };
 // first vertex, edges, first edge (base: global, overlay: 0) and ring (overlay: 1-based) of a leaf
 struct __align__(16) Leaf {
@@ -99,10 +100,25 @@ __device__ inline BoxF edge_boxf(const double2 &a, const double2 &b) {
     return boxf_of(box_of(a.x, a.y, b.x, b.y));
 }
 
+// Tiles (base leaf, overlay leaf) go to TILE_SEGS segments, each with its own
+// counter on its own 128-byte line, staged per wave (one same-address counter
+// costs about 5 ns an atomic).
+constexpr int TILE_SEGS = 512;
+constexpr int TILE_PAD = 32; // u32 per counter line
+constexpr int TSTG = 256;
+
 // One wave per leaf.  Bound by the read of the vertices (16 bytes each).
-__global__ __launch_bounds__(BLK) void k_join_leaves(RingTab t, BoxF *box, Leaf *desc, uint32_t *bad) {
+// Clears the words that the tiles and pairs are counted in as well.
+__global__ __launch_bounds__(BLK) void k_join_leaves(RingTab t, BoxF *__restrict__ box, Leaf *__restrict__ desc,
+                                                     uint32_t *__restrict__ bad,
+                                                     unsigned long long *__restrict__ sum,
+                                                     uint32_t *__restrict__ counter) {
     const int lane = threadIdx.x & (WAVE - 1);
     const uint32_t w = uni(blockIdx.x * WPB + threadIdx.x / WAVE);
+    for (uint32_t i = blockIdx.x * BLK + threadIdx.x; i < TILE_SEGS; i += gridDim.x * BLK) {
+        counter[size_t(i) * TILE_PAD] = 0u;
+        if (i < 3) sum[i] = 0ull;
+    }
     if (w >= t.nleaf) return;
     const int r = seg_of(t.loff, t.nbr + t.K, w);
     const bool base = r < t.nbr;
@@ -124,7 +140,7 @@ __global__ __launch_bounds__(BLK) void k_join_leaves(RingTab t, BoxF *box, Leaf 
              !(fabs(q.y) < INFINITY);
     }
     if (__ballot(no)) {
-        if (lane == 0) atomicOr(bad, 1u);
+        if (lane == 0) *bad = t.call;
         return; // the join's results are not used
     }
     b = boxf_wave(b);
@@ -148,7 +164,7 @@ __global__ __launch_bounds__(BLK) void k_join_groups(RingTab t, const BoxF *__re
                                                      BoxF *__restrict__ gbox, const uint32_t *__restrict__ bad) {
     const int lane = threadIdx.x & (WAVE - 1);
     const uint32_t w = uni(blockIdx.x * WPB + threadIdx.x / WAVE);
-    if (w >= nslot || *bad) return;
+    if (w >= nslot || *bad == t.call) return;
     int lo = 0, hi = t.nbr - 1; // last ring whose first slot is <= w
     while (lo < hi) {
         const int mid = (lo + hi + 1) >> 1;
@@ -161,13 +177,6 @@ __global__ __launch_bounds__(BLK) void k_join_groups(RingTab t, const BoxF *__re
     b = boxf_wave(b);
     if (lane == 0) gbox[w] = b;
 }
-
-// Tiles (base leaf, overlay leaf) go to TILE_SEGS segments, each with its own
-// counter on its own 128-byte line, staged per wave (one same-address counter
-// costs about 5 ns an atomic).
-constexpr int TILE_SEGS = 512;
-constexpr int TILE_PAD = 32; // u32 per counter line
-constexpr int TSTG = 256;
 
 struct TileArgs {
     RingTab t;
@@ -188,7 +197,7 @@ __global__ __launch_bounds__(BLK) void k_join_tiles(TileArgs a) {
     const uint32_t wv = uni(threadIdx.x / WAVE);
     const uint32_t w = blockIdx.x * WPB + wv;
     const uint32_t L = a.t.lb + w;
-    if (L >= a.t.nleaf || *a.bad) return;
+    if (L >= a.t.nleaf || *a.bad == a.t.call) return;
     const BoxF cb = a.box[L];
     const int r = a.paired ? int(a.desc[L].ring) - 1 : 0;
     const uint32_t l0 = uint32_t(a.t.loff[r]), nl = uint32_t(a.t.loff[r + 1]) - l0;
@@ -243,6 +252,7 @@ struct PairArgs {
     const int *coff;
     bool paired;
     const uint32_t *bad;
+    uint32_t call;
     const uint2 *tiles;
     uint32_t cap;
     const uint32_t *counter;
@@ -267,7 +277,7 @@ __global__ __launch_bounds__(BLK) void k_join_pairs(PairArgs a) {
     __shared__ uint32_t toff[TILE_SEGS + 1]; // first tile of each segment
     __shared__ uint32_t qb[WPB][QCAP], qc[WPB][QCAP], qk[WPB][QCAP];
     __shared__ uint64_t hits_all[WPB][HSTG];
-    if (*a.bad) return; // every block reads the same word
+    if (*a.bad == a.call) return; // every block reads the same word
     const int lane = threadIdx.x & (WAVE - 1);
     const uint32_t wv = uni(threadIdx.x / WAVE);
     if (wv == 0) { // segment counts to offsets, eight segments per lane
@@ -442,6 +452,9 @@ bool join_candidates(Ctx &c) {
     BoxF *gbox = box + nleaf;
     Leaf *desc = reinterpret_cast<Leaf *>(c.join_leaf.ensure(2 * size_t(nleaf)));
     // control words: pairs, tiles, largest segment (64 bits each), the "bad" flag, then the segment counters
+    const bool fresh = c.join_ctl.cap == 0; // holds nothing yet
+    if (++c.join_call == 0) c.join_call = 1;
+    t.call = c.join_call;
     uint32_t *ctl = c.join_ctl.ensure(size_t(TILE_PAD) * (TILE_SEGS + 1));
     unsigned long long *sum = reinterpret_cast<unsigned long long *>(ctl);
     uint32_t *bad = ctl + 6, *counter = ctl + TILE_PAD;
@@ -456,14 +469,14 @@ bool join_candidates(Ctx &c) {
     for (int attempt = 0; attempt < 3; ++attempt) {
         c.join_tile.ensure(size_t(c.join_seg_cap) * TILE_SEGS);
         c.pairs.ensure(size_t(c.cand_cap));
-        {
+        if (attempt > 0 || fresh) {
             FillBatch fb(s);
             fb.add(ctl, int64_t(TILE_PAD) * (TILE_SEGS + 1), 0u);
             fb.flush();
         }
         c.mark(8);
         if (attempt == 0) {
-            k_join_leaves<<<grid_for(nleaf, WPB), BLK, 0, s>>>(t, box, desc, bad);
+            k_join_leaves<<<grid_for(nleaf, WPB), BLK, 0, s>>>(t, box, desc, bad, sum, counter);
             SC_HIP(hipGetLastError());
             if (maxng > 1) {
                 k_join_groups<<<grid_for(nslot, WPB), BLK, 0, s>>>(t, box, nslot, gbox, bad);
@@ -491,6 +504,7 @@ bool join_candidates(Ctx &c) {
         p.coff = t.coff;
         p.paired = c.paired;
         p.bad = bad;
+        p.call = t.call;
         p.tiles = a.out;
         p.cap = a.cap;
         p.counter = counter;
@@ -507,7 +521,7 @@ bool join_candidates(Ctx &c) {
         ReadBack rb(c);
         rb.add(h, reinterpret_cast<const uint64_t *>(ctl), 4);
         rb.run();
-        if (uint32_t(h[3])) return false;
+        if (uint32_t(h[3]) == t.call) return false;
         const int64_t seg_max = int64_t(h[2]), np = int64_t(h[0]);
         if (seg_max > int64_t(UINT32_MAX / TILE_SEGS)) return false; // tiles are counted in 32 bits
         if (seg_max > c.join_seg_cap) {

@@ -182,6 +182,7 @@ __global__ void k_copy_order(const uint32_t *__restrict__ vals, int I, int *ord)
 // one launch where sizes, closing entries and their scans took five.  More jobs
 // than one chunk are gathered by as many blocks and scanned in two launches
 // (16,384 jobs: 81 us in four chunks of one block, 14 so).
+constexpr int LATE_MAX = 1 << 16; // pairs up to which launches and read-backs are saved at the price of more loads
 constexpr int JOB_BLK = 1024, JOB_PER = 4;
 __global__ void k_job_sizes(JobArgs ja, const int *__restrict__ nd_b, const uint32_t *__restrict__ ndg,
                             const int *__restrict__ nd_c, int *nba, int *nca) {
@@ -318,23 +319,81 @@ __device__ inline void aug_segment(const int *__restrict__ pj, int I, const int 
     z.slot[p] = sl;
     if (z.from) z.from[sl] = ~p;
 }
-// blockIdx.y: the sources of either side, then the intersections.  In one
-// launch (ONE) a source looks up whether an intersection leads its edge's
-// order; many slots take two, and the intersection tells its source slot (256
-// pairs with 40 million slots: 0.1 ms less than the look-ups).
-template <bool ONE>
+// words of the ordering that say that a group was too large for it
+__device__ inline bool unordered_words(const uint32_t *over) { return over && (over[2] | over[SEG_CTL + 2]) != 0u; }
+// blockIdx.y: the sources of either side, then the intersections, in one
+// launch: a source looks up whether an intersection leads its edge's order
 __global__ __launch_bounds__(BLK) void k_augment(int J, const int *__restrict__ pj, int I, const int *__restrict__ pt,
                                                const double *__restrict__ px, const double *__restrict__ py,
-                                               int *flags, AugSides sides, int y0) {
-    const int y = int(blockIdx.y) + y0;
-    const AugSide &z = sides.s[y & 1];
-    const bool side_b = (y & 1) == 0;
+                                               int *flags, AugSides sides, const uint32_t *over) {
+    if (unordered_words(over)) return;
+    const AugSide &z = sides.s[blockIdx.y & 1];
+    const bool side_b = (blockIdx.y & 1) == 0;
     const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (y < 2) aug_source<ONE>(J, z, side_b, pt, i);
-    else if (i < I) aug_segment<ONE>(pj, I, pt, px, py, flags, z, side_b, int(i));
+    if (blockIdx.y < 2) aug_source<true>(J, z, side_b, pt, i);
+    else if (i < I) aug_segment<true>(pj, I, pt, px, py, flags, z, side_b, int(i));
+}
+// Many slots take two launches, and the intersection tells its source slot (256
+// pairs with 32 million sources: 0.7 ms, with the look-ups 0.8; one kernel with
+// both parts takes 0.15 longer than two).
+__global__ void k_aug_sources(int J, AugSides sides) {
+    aug_source<false>(J, sides.s[blockIdx.y], blockIdx.y == 0, nullptr,
+                      int64_t(blockIdx.x) * blockDim.x + threadIdx.x);
+}
+__global__ void k_aug_segments(const int *__restrict__ pj, int I, const int *__restrict__ pt,
+                               const double *__restrict__ px, const double *__restrict__ py, int *flags,
+                               AugSides sides) {
+    aug_segment<false>(pj, I, pt, px, py, flags, sides.s[blockIdx.y], blockIdx.y == 0,
+                       int(blockIdx.x * blockDim.x + threadIdx.x));
 }
 
-// neighbour links, 1-based and local to the job's rings (as the reference's arrays)
+// Neighbour links, 1-based and local to the job's rings (as the reference's
+// arrays), and initial labels, by position on the base rings: the slots beside
+// an intersection's are those of the positions beside it, or plain (a position
+// without a slot, in a flagged job, is passed over).  over: words that say that
+// an order is still to come.
+struct LabelArgs {
+    int J, I;
+    const int *pj, *ord, *JB, *scan, *slot_b, *slot_c, *AB, *AC;
+    const double *bx, *by, *cx, *cy;
+    int *nbr_b, *nbr_c, *lab_b, *lab_c, *flags;
+    const uint32_t *over;
+};
+__global__ __launch_bounds__(BLK) void k_link_labels(LabelArgs a) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (unordered_words(a.over) || i >= a.scan[a.JB[a.J]]) return;
+    const int p = a.ord[i], j = a.pj[p];
+    const int g = a.slot_b[p], h = a.slot_c[p];
+    if (g < 0 || h < 0) {
+        atomicOr(&a.flags[j], UB_UNASSIGNED);
+        return;
+    }
+    const int B0 = a.AB[j], C0 = a.AC[j], nbaug = a.AB[j + 1] - B0, ncaug = a.AC[j + 1] - C0;
+    a.nbr_b[g] = h - C0 + 1;
+    a.nbr_c[h] = g - B0 + 1;
+    const int first = a.scan[a.JB[j]], end = a.scan[a.JB[j + 1]]; // the job's positions
+    // the partner of slot s (-100: a plain vertex, -101: an intersection without one), from position k on in steps d
+    auto partner = [&](int s, int k, int d) {
+        while (k >= first && k < end && a.slot_b[a.ord[k]] < 0) k += d;
+        if (k < first || k >= end) return -100;
+        const int q = a.ord[k];
+        if (a.slot_b[q] != s) return -100;
+        return a.slot_c[q] < 0 ? -101 : a.slot_c[q] - C0;
+    };
+    const int t = g - B0, tm = t == 0 ? nbaug - 1 : t - 1, tp = t + 1 == nbaug ? 0 : t + 1;
+    const int pMN = partner(B0 + tm, t == 0 ? end - 1 : i - 1, -1);
+    const int pPN = partner(B0 + tp, t + 1 == nbaug ? first : i + 1, 1);
+    const int n = h - C0, qm = n == 0 ? ncaug - 1 : n - 1, qp = n + 1 == ncaug ? 0 : n + 1;
+    const int lab = label_of(pMN, pPN, qm, qp, a.cx[C0 + qm], a.cy[C0 + qm], a.cx[C0 + qp], a.cy[C0 + qp],
+                             a.bx[B0 + tm], a.by[B0 + tm], a.bx[g], a.by[g], a.bx[B0 + tp], a.by[B0 + tp]);
+    a.lab_b[g] = lab;
+    a.lab_c[h] = lab;
+}
+
+// The same in two launches, by pair and by slot: for many pairs, whose
+// neighbours' pairs are worth more loads than a look at every slot (256 pairs
+// with 40 million slots: 0.15 ms less).  The labels also of rings whose links
+// are given.
 __global__ void k_link(const int *__restrict__ sb, const int *__restrict__ scn, const int *__restrict__ pj, int I,
                        const int *__restrict__ AB, const int *__restrict__ AC, int *nbr_b, int *nbr_c, int *flags) {
     int p = blockIdx.x * blockDim.x + threadIdx.x;
@@ -347,7 +406,6 @@ __global__ void k_link(const int *__restrict__ sb, const int *__restrict__ scn, 
     nbr_b[a] = b - AC[j] + 1;
     nbr_c[b] = a - AB[j] + 1;
 }
-
 __global__ void k_init_labels(int J, const int *__restrict__ AB, const int *__restrict__ AC,
                               const double *__restrict__ bx, const double *__restrict__ by,
                               const int *__restrict__ avb, const int *__restrict__ nbrb,
@@ -400,7 +458,7 @@ __global__ void k_sp_fill(int I, const int *__restrict__ ord, const int *__restr
                           const int *__restrict__ p0, const uint32_t *__restrict__ ndg, const int *__restrict__ bvoff,
                           const double *__restrict__ bpoly, const double *__restrict__ px,
                           const double *__restrict__ py, const int *__restrict__ qa, int *slot, int *ndx, int *edge,
-                          int *av, int *nbr, int *lab, double *x, double *y, int *pos, const int *kind,
+                          int *av, int *nbr, int *lab, double *x, double *y, const int *kind,
                           const uint32_t *__restrict__ unordered) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= I || (unordered && *unordered)) return;
@@ -421,61 +479,58 @@ __global__ void k_sp_fill(int I, const int *__restrict__ ord, const int *__restr
         x[i] = V[0];
         y[i] = V[1];
     }
-    pos[p] = i;
 }
 
-__global__ void k_sp_link(int I, const int *__restrict__ pos, const int *__restrict__ pj,
-                          const int *__restrict__ slot, const int *__restrict__ scn, const int *__restrict__ AC,
-                          int nca, int *nbr_p, int *nbr_c, int *flags) {
-    int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= I) return;
-    int i = pos[p], j = pj[p];
-    int a = slot[i], b = scn[p];
-    if (a < 0 || b < 0 || b >= nca) {
-        atomicOr(&flags[j], UB_UNASSIGNED);
+// links and labels on the sparse base ring
+struct SpLabelArgs {
+    int I, J;
+    const int *pj, *ord, *slot_c, *AC;
+    SparseP sp;
+    const double *cx, *cy;
+    int *nbr_p, *nbr_c, *lab_p, *lab_c, *flags;
+    const uint32_t *over;
+};
+__global__ __launch_bounds__(BLK) void k_sp_link_labels(SpLabelArgs a) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= a.I || unordered_words(a.over)) return;
+    const SparseP &sp = a.sp;
+    const int j = a.pj[i], q = sp.slot[i], h = a.slot_c[a.ord[i]];
+    if (q < 0 || h < 0 || h >= a.AC[a.J]) {
+        atomicOr(&a.flags[j], UB_UNASSIGNED);
         return;
     }
-    nbr_p[i] = b - AC[j] + 1;
-    nbr_c[b] = a + 1;
-}
-
-__global__ void k_sp_init_labels(int I, const int *__restrict__ pj, SparseP sp, const int *__restrict__ nbr,
-                                 const int *__restrict__ AC, const double *__restrict__ cx,
-                                 const double *__restrict__ cy, int *lab, int *labc, int *flags) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= I) return;
-    const int q = sp.slot[i];
-    if (q < 0) return;
-    const int j = pj[i];
-    const int nbaug = sp.AB[j + 1] - sp.AB[j], C0 = AC[j], ncaug = AC[j + 1] - C0;
-    const int tm = q - 1 < 0 ? nbaug - 1 : q - 1;
-    const int tp = q + 1 == nbaug ? 0 : q + 1;
+    const int C0 = a.AC[j], ncaug = a.AC[j + 1] - C0, nbaug = sp.AB[j + 1] - sp.AB[j];
+    a.nbr_p[i] = h - C0 + 1;
+    a.nbr_c[h] = q + 1;
+    const int tm = q == 0 ? nbaug - 1 : q - 1, tp = q + 1 == nbaug ? 0 : q + 1;
     // The slots beside q are held by the positions beside i or plain (slots ascend
     // with the positions unless the job was flagged); at the ring's ends by the
     // last position, or one past it, and by the first.
     SlotInfo pm, pp;
-    if (flags[j] & UB_UNASSIGNED) {
+    if (a.flags[j] & UB_UNASSIGNED) {
         pm = sp_slot(sp, j, tm);
         pp = sp_slot(sp, j, tp);
     } else {
-        const int a = sp.P0[j], b = sp.P0[j + 1];
-        const int last = sp.slot[b - 1] == nbaug - 1 ? b - 1 : b;
-        pm = sp_slot_at(sp, j, tm, q == 0 ? last : (i > a && sp.slot[i - 1] == tm ? i - 1 : i));
-        pp = sp_slot_at(sp, j, tp, q + 1 == nbaug ? a : i + 1);
+        const int first = sp.P0[j], end = sp.P0[j + 1];
+        const int last = sp.slot[end - 1] == nbaug - 1 ? end - 1 : end;
+        pm = sp_slot_at(sp, j, tm, q == 0 ? last : (i > first && sp.slot[i - 1] == tm ? i - 1 : i));
+        pp = sp_slot_at(sp, j, tp, q + 1 == nbaug ? first : i + 1);
     }
-    const int pMN = pm.pos >= 0 ? nbr[pm.pos] - 1 : -100;
-    const int pPN = pp.pos >= 0 ? nbr[pp.pos] - 1 : -100;
-    const int nId = nbr[i] - 1;
-    if (nId < 0 || nId >= ncaug) {
-        atomicOr(&flags[j], UB_UNASSIGNED);
+    auto partner = [&](const SlotInfo &s) {
+        if (s.pos < 0) return -100;
+        const int o = a.slot_c[a.ord[s.pos]];
+        return o < 0 || o >= a.AC[a.J] ? -101 : o - C0;
+    };
+    const int n = h - C0;
+    if (n < 0 || n >= ncaug) {
+        atomicOr(&a.flags[j], UB_UNASSIGNED);
         return;
     }
-    const int qm = nId - 1 < 0 ? ncaug - 1 : nId - 1;
-    const int qp = nId + 1 == ncaug ? 0 : nId + 1;
-    const int l = label_of(pMN, pPN, qm, qp, cx[C0 + qm], cy[C0 + qm], cx[C0 + qp], cy[C0 + qp], pm.x, pm.y,
-                           sp.x[i], sp.y[i], pp.x, pp.y);
-    lab[i] = l;
-    labc[C0 + nId] = l;
+    const int qm = n == 0 ? ncaug - 1 : n - 1, qp = n + 1 == ncaug ? 0 : n + 1;
+    const int lab = label_of(partner(pm), partner(pp), qm, qp, a.cx[C0 + qm], a.cy[C0 + qm], a.cx[C0 + qp],
+                             a.cy[C0 + qp], pm.x, pm.y, sp.x[i], sp.y[i], pp.x, pp.y);
+    a.lab_p[i] = lab;
+    a.lab_c[h] = lab;
 }
 
 int bits_for(int64_t n) {
@@ -486,7 +541,11 @@ int bits_for(int64_t n) {
 
 } // namespace
 
-void post_jobs(Ctx &c, int k0, int k1) {
+// late: the augmented rings' offsets may stay on the device (js.late), where
+// label_and_traverse reads them back with its own first values; a group too
+// large for the ordering is then found there, and nothing after the ordering has
+// run.  A read-back costs a small clip 20 us of 400.
+void post_jobs(Ctx &c, int k0, int k1, bool late) {
     SC_REQUIRE(k0 >= 1 && k1 <= c.K && k0 <= k1, SC_EINVAL, "overlay index out of range");
     SC_REQUIRE(int(c.pair_off.size()) == c.K + 1, SC_ESTATE, "candidates not computed");
     hipStream_t s = c.stream;
@@ -655,12 +714,12 @@ void post_jobs(Ctx &c, int k0, int k1) {
         }
         scan_exclusive_u32(ndf, ndf, int64_t(I) + 1, nullptr, s);
         int *slot = c.sp_slot.ensure(Ia), *ndx = c.sp_ndx.ensure(Ia), *edge = c.sp_edge.ensure(Ia);
-        int *sav = c.sp_av.ensure(Ia), *snbr = c.sp_nbr.ensure(Ia), *pos = c.sp_pos.ensure(Ia);
+        int *sav = c.sp_av.ensure(Ia), *snbr = c.sp_nbr.ensure(Ia);
         double *sx = c.sp_x.ensure(Ia), *sy = c.sp_y.ensure(Ia);
         c.sp_lab.ensure(Ia);
         if (I > 0) {
             k_sp_fill<<<grid_for(I), BLK, 0, s>>>(I, c.ordB, c.p_j, c.p_b, ja.p0, ndf, ja.bvoff, c.bpoly, c.p_x,
-                                                  c.p_y, c.p_qa, slot, ndx, edge, sav, snbr, c.sp_lab, sx, sy, pos,
+                                                  c.p_y, c.p_qa, slot, ndx, edge, sav, snbr, c.sp_lab, sx, sy,
                                                   kind, unordered);
             SC_HIP(hipGetLastError());
         }
@@ -675,10 +734,17 @@ void post_jobs(Ctx &c, int k0, int k1) {
         scan_exclusive_u32_2(ub, ub, int64_t(J) + 1, nullptr, uc, uc, int64_t(J) + 1, nullptr, s);
     }
     SC_HIP(hipGetLastError());
-    js.AB.resize(J + 1);
-    js.AC.resize(J + 1);
+    js.late = late && I <= LATE_MAX;
+    js.AB.clear();
+    js.AC.clear();
+    js.cap_b = int64_t(nJB) - J + I;
+    js.cap_c = int64_t(nJC) - J + I;
+    if (!js.late) {
+        js.AB.resize(J + 1);
+        js.AC.resize(J + 1);
+    }
     uint32_t hseg[2 * SEG_CTL] = {};
-    {
+    if (!js.late) {
         ReadBack rb(c);
         rb.add(js.AB.data(), static_cast<const int *>(nba), size_t(J) + 1);
         rb.add(js.AC.data(), static_cast<const int *>(nca), size_t(J) + 1);
@@ -691,9 +757,10 @@ void post_jobs(Ctx &c, int k0, int k1) {
         if (sparse) sparse_slots(nullptr);
     }
     if (hseg[SEG_CTL + 2]) radix_order(false);
-    const int64_t nba_tot = js.AB[J], nca_tot = js.AC[J];
-    c.nbaug = int(nba_tot);
-    c.ncaug = int(nca_tot);
+    const int64_t nba_tot = js.late ? js.cap_b : js.AB[J], nca_tot = js.late ? js.cap_c : js.AC[J];
+    c.nbaug = js.late ? 0 : int(nba_tot);
+    c.ncaug = js.late ? 0 : int(nca_tot);
+    const uint32_t *over = js.late && I > 0 ? segctl : nullptr;
 
     const int64_t nbaA = nba_tot > 0 ? nba_tot : 1, ncaA = nca_tot > 0 ? nca_tot : 1;
     c.aug_cx.ensure(ncaA); c.aug_cy.ensure(ncaA); c.av_c.ensure(ncaA); c.nbr_c.ensure(ncaA); c.lab_c.ensure(ncaA);
@@ -708,30 +775,29 @@ void post_jobs(Ctx &c, int k0, int k1) {
                       c.aug_cy, c.av_c, c.nbr_c, c.lab_c, from_c, c.slot_c};
     // (the sparse base side has slots by the hundred million and none of these arrays)
     const int64_t nsrc = sparse ? nJC : std::max(nJB, nJC);
-    if (std::max<int64_t>(I, nsrc) < SPAN_MIN) {
-        k_augment<true><<<dim3(grid_for(std::max<int64_t>(I, nsrc)), I > 0 ? 4 : 2), BLK, 0, s>>>(
-            J, c.p_j, I, c.p_type, c.p_x, c.p_y, flags, as, 0);
+    if (over || std::max<int64_t>(I, nsrc) < SPAN_MIN) {
+        k_augment<<<dim3(grid_for(std::max<int64_t>(I, nsrc)), I > 0 ? 4 : 2), BLK, 0, s>>>(
+            J, c.p_j, I, c.p_type, c.p_x, c.p_y, flags, as, over);
     } else {
-        k_augment<false><<<dim3(grid_for(nsrc), 2), BLK, 0, s>>>(J, c.p_j, I, c.p_type, c.p_x, c.p_y, flags, as, 0);
-        if (I > 0)
-            k_augment<false><<<dim3(grid_for(I), 2), BLK, 0, s>>>(J, c.p_j, I, c.p_type, c.p_x, c.p_y, flags, as, 2);
+        k_aug_sources<<<dim3(grid_for(nsrc), 2), BLK, 0, s>>>(J, as);
+        if (I > 0) k_aug_segments<<<dim3(grid_for(I), 2), BLK, 0, s>>>(c.p_j, I, c.p_type, c.p_x, c.p_y, flags, as);
     }
     SC_HIP(hipGetLastError());
     if (I > 0) {
         if (sparse) {
-            k_sp_link<<<grid_for(I), BLK, 0, s>>>(I, c.sp_pos, c.p_j, c.sp_slot, c.slot_c, nca, int(nca_tot),
-                                                  c.sp_nbr, c.nbr_c, flags);
-            SC_HIP(hipGetLastError());
-            k_sp_init_labels<<<grid_for(I), BLK, 0, s>>>(I, c.p_j, sparse_view(c), c.sp_nbr, nca, c.aug_cx,
-                                                         c.aug_cy, c.sp_lab, c.lab_c, flags);
-            SC_HIP(hipGetLastError());
-        } else {
+            SpLabelArgs la{I, J, c.p_j, c.ordB, c.slot_c, nca, sparse_view(c), c.aug_cx, c.aug_cy, c.sp_nbr, c.nbr_c,
+                           c.sp_lab, c.lab_c, flags, over};
+            k_sp_link_labels<<<grid_for(I), BLK, 0, s>>>(la);
+        } else if (I > LATE_MAX) {
             k_link<<<grid_for(I), BLK, 0, s>>>(c.slot_b, c.slot_c, c.p_j, I, nba, nca, c.nbr_b, c.nbr_c, flags);
-            SC_HIP(hipGetLastError());
             k_init_labels<<<grid_for(nba_tot), BLK, 0, s>>>(J, nba, nca, c.aug_bx, c.aug_by, c.av_b, c.nbr_b,
                                                             c.aug_cx, c.aug_cy, c.lab_b, c.lab_c, flags);
-            SC_HIP(hipGetLastError());
+        } else {
+            LabelArgs la{J, I, c.p_j, c.ordB, ja.JB, all_b, c.slot_b, c.slot_c, nba, nca, c.aug_bx, c.aug_by, c.aug_cx,
+                         c.aug_cy, c.nbr_b, c.nbr_c, c.lab_b, c.lab_c, flags, over};
+            k_link_labels<<<grid_for(I), BLK, 0, s>>>(la);
         }
+        SC_HIP(hipGetLastError());
     }
     js.flags.assign(size_t(J), 0);
     c.flags_pending = true; // read back later, with the next read-back that needs a wait anyway
