@@ -442,8 +442,6 @@ __global__ __launch_bounds__(HIST_BLK) void k_global_hist(const uint64_t *keys, 
 // until one carries an inclusive prefix, and publishes its own, and each
 // digit's run is written out contiguously at global digit base + prefix.
 // Within a digit keys keep their input order (the sort is stable).
-constexpr int RS_PER_WAVE = RS_TILE / RS_WAVES;
-constexpr int RS_IT = RS_PER_WAVE / WAVE; // = RS_ITEMS
 static_assert(RS_BLOCK == 256, "one thread per 8-bit digit");
 static_assert(RS_TILE <= 65535, "16-bit tile offsets");
 // status word: epoch (8 bits) | flag (2 bits: aggregate, inclusive prefix) | count (54 bits);
@@ -466,7 +464,8 @@ struct SweepArgs {
     unsigned long long epoch;    // 1..255, shifted into place
 };
 
-__device__ inline uint32_t block_excl_sum256(uint32_t x, uint32_t *s_wsum, uint32_t &total) {
+// exclusive scan over the block's first 256 threads (the others pass zero)
+template <int NW> __device__ inline uint32_t block_excl_sum256(uint32_t x, uint32_t *s_wsum, uint32_t &total) {
     const int tid = threadIdx.x, lane = tid & (WAVE - 1), w = tid / WAVE;
     uint32_t inc = x;
 #pragma unroll
@@ -478,7 +477,7 @@ __device__ inline uint32_t block_excl_sum256(uint32_t x, uint32_t *s_wsum, uint3
     __syncthreads();
     uint32_t ex = inc - x;
     total = 0;
-    for (int q = 0; q < RS_WAVES; ++q) {
+    for (int q = 0; q < 256 / WAVE; ++q) {
         if (q < w) ex += s_wsum[q];
         total += s_wsum[q];
     }
@@ -486,39 +485,40 @@ __device__ inline uint32_t block_excl_sum256(uint32_t x, uint32_t *s_wsum, uint3
     return ex;
 }
 
-template <bool VALS> __device__ __forceinline__ void onesweep_tile(const SweepArgs &a) {
+template <bool VALS, int NT> __device__ __forceinline__ void onesweep_tile(const SweepArgs &a) {
+    constexpr int NW = NT / WAVE, PER_WAVE = RS_TILE / NW, IT = PER_WAVE / WAVE;
     __shared__ uint64_t s_k[RS_TILE];
     __shared__ uint32_t s_v[VALS ? RS_TILE : 1];
-    // index digit*RS_WAVES + wave; counts and tile offsets stay below RS_TILE, so
+    // index digit*NW + wave; counts and tile offsets stay below RS_TILE, so
     // 16 bits suffice (the smaller footprint lets three blocks share a CU)
-    __shared__ uint16_t s_cnt[256 * RS_WAVES];
+    __shared__ uint16_t s_cnt[256 * NW];
     __shared__ uint32_t s_gbase[256];          // output offset of the digit minus its tile-local start
-    __shared__ uint32_t s_wsum[RS_WAVES];
+    __shared__ uint32_t s_wsum[NW];
     const int tid = threadIdx.x, lane = tid & (WAVE - 1), w = tid / WAVE;
     const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (WAVE - lane));
-    for (int i = tid; i < 256 * RS_WAVES; i += RS_BLOCK) s_cnt[i] = 0;
+    for (int i = tid; i < 256 * NW; i += NT) s_cnt[i] = 0;
     // a pass in which every key has the same digit keeps the order: copy the tile
-    const bool trivial = __syncthreads_or(uint64_t(a.ghist[tid]) == uint64_t(a.n));
+    const bool trivial = __syncthreads_or(tid < 256 && uint64_t(a.ghist[tid]) == uint64_t(a.n));
     const uint32_t tile = blockIdx.x;
     const int64_t base = int64_t(tile) * RS_TILE;
     if (trivial) {
-        for (int64_t i = base + tid; i < a.n && i < base + RS_TILE; i += RS_BLOCK) {
+        for (int64_t i = base + tid; i < a.n && i < base + RS_TILE; i += NT) {
             a.kout[i] = a.kin[i];
             if (VALS) a.vout[i] = a.vin[i];
         }
         return;
     }
-    uint64_t k[RS_IT];
-    uint32_t v[VALS ? RS_IT : 1], rk[RS_IT];
+    uint64_t k[IT];
+    uint32_t v[VALS ? IT : 1], rk[IT];
 #pragma unroll
-    for (int it = 0; it < RS_IT; ++it) {
-        const int64_t i = base + w * RS_PER_WAVE + it * WAVE + lane;
+    for (int it = 0; it < IT; ++it) {
+        const int64_t i = base + w * PER_WAVE + it * WAVE + lane;
         k[it] = i < a.n ? a.kin[i] : 0ull;
         if (VALS) v[it] = i < a.n ? a.vin[i] : 0u;
     }
 #pragma unroll
-    for (int it = 0; it < RS_IT; ++it) {
-        const int64_t i = base + w * RS_PER_WAVE + it * WAVE + lane;
+    for (int it = 0; it < IT; ++it) {
+        const int64_t i = base + w * PER_WAVE + it * WAVE + lane;
         const bool valid = i < a.n;
         const uint32_t d = uint32_t(k[it] >> a.shift) & a.mask;
         uint64_t m = __ballot(valid);
@@ -530,50 +530,54 @@ template <bool VALS> __device__ __forceinline__ void onesweep_tile(const SweepAr
         }
         const uint32_t r = __popcll(m & lt);
         uint32_t before = 0;
-        if (valid) before = s_cnt[d * RS_WAVES + w];
+        if (valid) before = s_cnt[d * NW + w];
         rk[it] = before + r;
-        if (valid && r == 0) s_cnt[d * RS_WAVES + w] = uint16_t(before + uint32_t(__popcll(m)));
+        if (valid && r == 0) s_cnt[d * NW + w] = uint16_t(before + uint32_t(__popcll(m)));
         __builtin_amdgcn_wave_barrier();
     }
     __syncthreads();
     // thread d: digit d's counts per wave and in the tile
-    uint32_t c[RS_WAVES], cnt = 0;
+    const bool digit = NT == 256 || tid < 256;
+    uint32_t c[NW], cnt = 0;
+    if (digit) {
 #pragma unroll
-    for (int q = 0; q < RS_WAVES; ++q) {
-        c[q] = s_cnt[tid * RS_WAVES + q];
-        cnt += c[q];
+        for (int q = 0; q < NW; ++q) {
+            c[q] = s_cnt[tid * NW + q];
+            cnt += c[q];
+        }
     }
     unsigned long long *my = a.status + size_t(tile) * 256 + tid;
-    __hip_atomic_store(my, a.epoch | (tile == 0 ? ST_PRE : ST_AGG) | cnt, __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
+    if (digit)
+        __hip_atomic_store(my, a.epoch | (tile == 0 ? ST_PRE : ST_AGG) | cnt, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
     uint32_t tot;
-    const uint32_t ex = block_excl_sum256(cnt, s_wsum, tot);
-    {
+    const uint32_t ex = block_excl_sum256<NW>(cnt, s_wsum, tot);
+    if (digit) {
         uint32_t run = ex;
 #pragma unroll
-        for (int q = 0; q < RS_WAVES; ++q) {
-            s_cnt[tid * RS_WAVES + q] = uint16_t(run);
+        for (int q = 0; q < NW; ++q) {
+            s_cnt[tid * NW + q] = uint16_t(run);
             run += c[q];
         }
     }
     // global base of the digit: exclusive scan of the pass histogram
-    const uint32_t gx = block_excl_sum256(a.ghist[tid], s_wsum, tot);
+    const uint32_t gx = block_excl_sum256<NW>(digit ? a.ghist[tid] : 0u, s_wsum, tot);
     // the tile in digit order in LDS (the places inside the tile do not
     // depend on earlier tiles, and the keys' registers are free during the
     // look-back)
 #pragma unroll
-    for (int it = 0; it < RS_IT; ++it) {
-        const int64_t i = base + w * RS_PER_WAVE + it * WAVE + lane;
+    for (int it = 0; it < IT; ++it) {
+        const int64_t i = base + w * PER_WAVE + it * WAVE + lane;
         if (i < a.n) {
             const uint32_t d = uint32_t(k[it] >> a.shift) & a.mask;
-            const uint32_t pos = s_cnt[d * RS_WAVES + w] + rk[it];
+            const uint32_t pos = s_cnt[d * NW + w] + rk[it];
             s_k[pos] = k[it];
             if (VALS) s_v[pos] = v[it];
         }
     }
     // look-back over earlier tiles
     unsigned long long prefix = 0;
-    if (tile > 0) {
+    if (tile > 0 && digit) {
         const unsigned long long EM = 0xffull << ST_EPOCH_SHIFT;
         int64_t t = int64_t(tile) - 1; // next predecessor to account for
         int spins = 0;
@@ -620,10 +624,10 @@ template <bool VALS> __device__ __forceinline__ void onesweep_tile(const SweepAr
         }
         __hip_atomic_store(my, a.epoch | ST_PRE | (prefix + cnt), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    s_gbase[tid] = gx + uint32_t(prefix) - ex;
+    if (digit) s_gbase[tid] = gx + uint32_t(prefix) - ex;
     __syncthreads();
     const int m = int(a.n - base < RS_TILE ? a.n - base : RS_TILE);
-    for (int i = tid; i < m; i += RS_BLOCK) {
+    for (int i = tid; i < m; i += NT) {
         const uint64_t key = s_k[i];
         const uint32_t o = s_gbase[uint32_t(key >> a.shift) & a.mask] + uint32_t(i);
         a.kout[o] = key;
@@ -633,9 +637,26 @@ template <bool VALS> __device__ __forceinline__ void onesweep_tile(const SweepAr
 
 // keys with values; keys only without the values' LDS and registers, which
 // lets four blocks share a CU (three with values)
-__global__ __launch_bounds__(RS_BLOCK) void k_onesweep(SweepArgs a) { onesweep_tile<true>(a); }
+__global__ __launch_bounds__(RS_BLOCK) void k_onesweep(SweepArgs a) { onesweep_tile<true, RS_BLOCK>(a); }
 __global__ __launch_bounds__(RS_BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void k_onesweep_keys(SweepArgs a) {
-    onesweep_tile<false>(a);
+    onesweep_tile<false, RS_BLOCK>(a);
+}
+// The same tiles by four times the threads: a tile alone on its CU is a chain
+// of its waves' steps (260,000 keys are 64 tiles: 15 us a pass, 12.5 so; 24
+// million keys 133 us, 154 so).
+constexpr int RS_WIDE = 1024;
+__global__ __launch_bounds__(RS_WIDE) void k_onesweep_wide(SweepArgs a) { onesweep_tile<true, RS_WIDE>(a); }
+__global__ __launch_bounds__(RS_WIDE) void k_onesweep_keys_wide(SweepArgs a) { onesweep_tile<false, RS_WIDE>(a); }
+constexpr int64_t RS_WIDE_MAX = int64_t(512) * RS_TILE; // two tiles a CU
+void onesweep(const SweepArgs &a, int64_t ntiles, hipStream_t s) {
+    const unsigned g = unsigned(ntiles);
+    if (a.n <= RS_WIDE_MAX) {
+        if (a.vin) k_onesweep_wide<<<g, RS_WIDE, 0, s>>>(a);
+        else k_onesweep_keys_wide<<<g, RS_WIDE, 0, s>>>(a);
+    } else {
+        if (a.vin) k_onesweep<<<g, RS_BLOCK, 0, s>>>(a);
+        else k_onesweep_keys<<<g, RS_BLOCK, 0, s>>>(a);
+    }
 }
 
 // up to SCAN_SET arrays of at most PREF_TILES tiles each in two launches (one
@@ -853,8 +874,7 @@ bool radix_passes(uint64_t *keys, uint32_t *vals, uint64_t *kalt, uint32_t *valt
         a.ghist = gh + size_t(p) * 256;
         a.status = st;
         a.epoch = (unsigned long long)rs.epoch << ST_EPOCH_SHIFT;
-        if (vc) k_onesweep<<<unsigned(ntiles), RS_BLOCK, 0, s>>>(a);
-        else k_onesweep_keys<<<unsigned(ntiles), RS_BLOCK, 0, s>>>(a);
+        onesweep(a, ntiles, s);
         SC_HIP(hipGetLastError());
         std::swap(kc, ko);
         std::swap(vc, vo);
@@ -906,8 +926,7 @@ bool radix_sort_u64_fixed(uint64_t *keys, uint32_t *vals, uint64_t *kalt, uint32
         a.ghist = gh + size_t(p) * 256;
         a.status = st;
         a.epoch = (unsigned long long)(p + 1) << ST_EPOCH_SHIFT;
-        if (vc) k_onesweep<<<unsigned(ntiles), RS_BLOCK, 0, s>>>(a);
-        else k_onesweep_keys<<<unsigned(ntiles), RS_BLOCK, 0, s>>>(a);
+        onesweep(a, ntiles, s);
         SC_HIP(hipGetLastError());
         std::swap(kc, ko);
         std::swap(vc, vo);
