@@ -96,6 +96,37 @@ __global__ __launch_bounds__(BLK) void k_ring_area2(RingSides sides) {
         __syncthreads(); // sh is written again
     }
 }
+// The same for rings of at most RING_WAVE vertices, a wave each: lane l holds the
+// sums of the block's threads l, l + 64, l + 128 and l + 192 and adds them in the
+// block's order (16,384 pairs of 4 to 64 vertices: 28 us with a block per ring,
+// 10 so).
+constexpr int RING_WAVE = BLK;
+__device__ inline double wave_block_sum(double (&s)[BLK / WAVE]) {
+    static_assert(BLK == 4 * WAVE, "the block sum's tree: 128, 64, then 32 to 1");
+    s[0] += s[2];
+    s[1] += s[3];
+    s[0] += s[1];
+    for (int d = WAVE / 2; d > 0; d >>= 1) s[0] += __shfl_down(s[0], d, WAVE);
+    return s[0]; // lane 0
+}
+__global__ __launch_bounds__(BLK) void k_ring_area2_few(RingSides sides) {
+    const RingSide &z = sides.s[blockIdx.y];
+    const int k = int(blockIdx.x) * (BLK / WAVE) + int(threadIdx.x) / WAVE, lane = threadIdx.x & (WAVE - 1);
+    if (k >= z.rings) return;
+    const int r = z.r0 + k;
+    const int64_t a = z.voff[r], n = z.voff[r + 1] - a - 1;
+    double s[BLK / WAVE];
+    for (int q = 0; q < BLK / WAVE; ++q) {
+        const int64_t i = q * WAVE + lane;
+        s[q] = 0.0;
+        if (i < n) {
+            const double *p = z.poly + 2 * (a + i);
+            s[q] += p[0] * p[3] - p[2] * p[1];
+        }
+    }
+    const double t = wave_block_sum(s);
+    if (lane == 0) z.out[k] = t;
+}
 // rings of more than one chunk: its chunks in order
 __global__ void k_ring_parts(RingSides sides) {
     const RingSide &z = sides.s[blockIdx.y];
@@ -118,7 +149,7 @@ __global__ void k_ring_parts(RingSides sides) {
 // large pairs: 0.19 -> 0.06 ms).
 // A longer ring is summed in chunks of AREA_CHUNK vertices, one wave per
 // chunk, and its chunk sums are added in chunk order.
-constexpr int AREA_CHUNK = 64 * WAVE;
+constexpr int AREA_CHUNK = LONG_RING;
 constexpr int AREA_WAVES = 8192; // waves of the short-ring grid (32 per CU)
 constexpr int RING_LANES = 16, RING_SET = WAVE / RING_LANES; // lanes of a short ring, rings a wave takes at once
 
@@ -216,20 +247,45 @@ __global__ void k_ring_chunk_sum(int nrings, const uint32_t *__restrict__ choff,
     out[r] = s;
 }
 
-// twice the unsigned area of each job's output: one block per job, thread t
-// adds |S| of rings t, t + 256, ... of the job, then a fixed tree; with the
-// input rings' sums, the job's areas and IoU
+// The areas and IoU of each job, a block per job: thread t adds |S| of rings t,
+// t + 256, ... (four loaded ahead), then a fixed tree.  Where jobs are many they
+// have a ring or two each and a wave per job adds in the same order (EACH;
+// 16,384 jobs: 14 us with a block per job, 6 so).
+constexpr int JOBS_EACH = 2048;
+template <bool EACH>
 __global__ __launch_bounds__(BLK) void k_job_areas(int J, int paired, const int *__restrict__ jring,
                                                    const double *__restrict__ ring2,
                                                    const double *__restrict__ barea2,
                                                    const double *__restrict__ carea2, double *out4) {
-    __shared__ double sh[BLK];
-    const int j = blockIdx.x;
+    __shared__ double sh[EACH ? 1 : BLK];
+    const int lane = threadIdx.x & (WAVE - 1);
+    const int j = EACH ? int(blockIdx.x) * (BLK / WAVE) + int(threadIdx.x) / WAVE : int(blockIdx.x);
+    if (EACH && j >= J) return; // whole wave
     const int r0 = jring[j], r1 = jring[j + 1];
-    double s = 0.0;
-    for (int r = r0 + int(threadIdx.x); r < r1; r += BLK) s += fabs(ring2[r]);
-    const double t = block_sum(s, sh);
-    if (threadIdx.x != 0) return;
+    double t;
+    if (EACH) {
+        double s[BLK / WAVE] = {};
+        for (int r = r0; r < r1; r += BLK)
+            for (int q = 0; q < BLK / WAVE; ++q) {
+                const int k = r + q * WAVE + lane;
+                if (k < r1) s[q] += fabs(ring2[k]);
+            }
+        t = wave_block_sum(s);
+        if (lane != 0) return;
+    } else {
+        double s = 0.0;
+        int r = r0 + int(threadIdx.x);
+        for (; r + 3 * BLK < r1; r += 4 * BLK) {
+            const double v0 = ring2[r], v1 = ring2[r + BLK], v2 = ring2[r + 2 * BLK], v3 = ring2[r + 3 * BLK];
+            s += fabs(v0);
+            s += fabs(v1);
+            s += fabs(v2);
+            s += fabs(v3);
+        }
+        for (; r < r1; r += BLK) s += fabs(ring2[r]);
+        t = block_sum(s, sh);
+        if (threadIdx.x != 0) return;
+    }
     const double I = 0.5 * t, P = 0.5 * fabs(barea2[paired ? j : 0]), Q = 0.5 * fabs(carea2[j]);
     const double U = P + Q - I;
     out4[j] = I;
@@ -630,17 +686,19 @@ void batch_area(Ctx &c, double *out4) {
         const int64_t wgrid =
             std::min<int64_t>(ceil_div(int64_t(nr), RING_SET * (BLK / WAVE)), AREA_WAVES / (BLK / WAVE));
         k_out_ring_area2<<<unsigned(wgrid), BLK, 0, s>>>(nr, c.d_ring_off, c.d_ring_x, c.d_ring_y, ring2);
-        uint32_t *cnt = a.chunks.ensure(size_t(nr) + 1), *choff = a.choff.ensure(size_t(nr) + 1);
-        uint32_t *tot = a.tot.ensure(1);
-        // a long ring has at most one chunk more than its AREA_CHUNK-vertex
-        // multiples, and there are at most n_out / AREA_CHUNK long rings
-        const int64_t cap = 2 * (c.n_out / AREA_CHUNK) + 1;
-        double *part = a.part.ensure(size_t(cap));
-        k_ring_chunks<<<grid_for(int64_t(nr) + 1), BLK, 0, s>>>(nr, c.d_ring_off, cnt);
-        scan_exclusive_u32(cnt, choff, int64_t(nr) + 1, tot, s);
-        k_out_chunk_area2<<<grid_for(cap, BLK / WAVE), BLK, 0, s>>>(nr, c.d_ring_off, choff, tot, cap, c.d_ring_x,
-                                                                    c.d_ring_y, part);
-        k_ring_chunk_sum<<<grid_for(nr), BLK, 0, s>>>(nr, choff, cap, part, ring2);
+        if (c.long_rings) {
+            uint32_t *cnt = a.chunks.ensure(size_t(nr) + 1), *choff = a.choff.ensure(size_t(nr) + 1);
+            uint32_t *tot = a.tot.ensure(1);
+            // a long ring has at most one chunk more than its AREA_CHUNK-vertex
+            // multiples, and there are at most n_out / AREA_CHUNK long rings
+            const int64_t cap = 2 * (c.n_out / AREA_CHUNK) + 1;
+            double *part = a.part.ensure(size_t(cap));
+            k_ring_chunks<<<grid_for(int64_t(nr) + 1), BLK, 0, s>>>(nr, c.d_ring_off, cnt);
+            scan_exclusive_u32(cnt, choff, int64_t(nr) + 1, tot, s);
+            k_out_chunk_area2<<<grid_for(cap, BLK / WAVE), BLK, 0, s>>>(nr, c.d_ring_off, choff, tot, cap,
+                                                                        c.d_ring_x, c.d_ring_y, part);
+            k_ring_chunk_sum<<<grid_for(nr), BLK, 0, s>>>(nr, choff, cap, part, ring2);
+        }
     }
     RingSides rs;
     const int64_t pb = (c.nb + c.nbr) / RING_CHUNK + c.nbr + 1, pc = (c.nct + c.K) / RING_CHUNK + c.K + 1;
@@ -650,7 +708,9 @@ void batch_area(Ctx &c, double *out4) {
     // blocks for a ring's chunks, where there are not many rings anyway
     const int64_t longest = ceil_div(int64_t(std::max(c.maxbsz, c.maxcsz)), RING_CHUNK);
     const int64_t bx = std::max<int64_t>(1, std::min<int64_t>(longest, 32768 / J));
-    for (int r = 0; r < J; r += 65535) { // grid dimension limit
+    const bool few = std::max(c.maxbsz, c.maxcsz) <= RING_WAVE; // a wave's worth of vertices per ring
+    if (few) k_ring_area2_few<<<dim3(grid_for(J, BLK / WAVE), 2), BLK, 0, s>>>(rs);
+    for (int r = 0; r < J && !few; r += 65535) { // grid dimension limit
         RingSides part_of = rs;
         for (RingSide &z : part_of.s) {
             z.rings = std::max(0, std::min(65535, z.rings - r));
@@ -660,7 +720,10 @@ void batch_area(Ctx &c, double *out4) {
         k_ring_area2<<<dim3(unsigned(bx), unsigned(std::min(65535, J - r)), 2), BLK, 0, s>>>(part_of);
     }
     if (longest > 1) k_ring_parts<<<dim3(grid_for(J), 2), BLK, 0, s>>>(rs);
-    k_job_areas<<<J, BLK, 0, s>>>(J, c.paired ? 1 : 0, js.d_ring, ring2, barea2, carea2, out4);
+    const int paired = c.paired ? 1 : 0;
+    if (J >= JOBS_EACH)
+        k_job_areas<true><<<grid_for(J, BLK / WAVE), BLK, 0, s>>>(J, paired, js.d_ring, ring2, barea2, carea2, out4);
+    else k_job_areas<false><<<J, BLK, 0, s>>>(J, paired, js.d_ring, ring2, barea2, carea2, out4);
     SC_HIP(hipGetLastError());
 }
 

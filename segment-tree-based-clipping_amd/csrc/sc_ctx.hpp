@@ -15,6 +15,8 @@ struct StageTimes {
 // against overlay k0+j.  Host vectors and their device copies; per-edge count
 // arrays hold n+1 slots per job (JB/JC offsets), augmented rings are
 // concatenated job after job (AB/AC offsets, J+1 entries each).
+constexpr int LONG_RING = 4096; // output vertices whose area one wave sums
+
 struct JobSet {
     int k0 = 1, J = 0;
     std::vector<int> p0, bvoff, beoff, nb, nc, cvoff, JB, JC, AB, AC, flags;
@@ -180,6 +182,7 @@ struct Ctx {
     // sequential-route rings walked one per lane (1) or by the single walk
     // (0); results do not depend on it
     int seq_par = 1;
+    bool long_rings = false; // the last output has a ring of more than LONG_RING vertices
     int small_fail = 0; // fallback reasons of the last small-pair batch (0: it ran fused)
     // the small-pair forward captured as a hipGraph (segclip_pairs_area_graph):
     // the buffers it reads and writes belong to it, so a replay never sees a

@@ -1158,10 +1158,12 @@ __global__ void k_ring_heads(int nr, const int *off, uint32_t *head) {
 }
 
 // vertices left of every ring, and whether there are any (nr + 1 threads: the closing entry)
-__global__ void k_ring_counts(int nr, const int *off, const uint32_t *kscan, uint32_t *cnt, uint32_t *nonempty) {
+__global__ void k_ring_counts(int nr, const int *off, const uint32_t *kscan, uint32_t *cnt, uint32_t *nonempty,
+                              uint32_t *longest) {
     const int r = blockIdx.x * blockDim.x + threadIdx.x;
     if (r > nr) return;
     const uint32_t c = r < nr ? kscan[off[r + 1]] - kscan[off[r]] : 0u;
+    if (c > uint32_t(LONG_RING)) *longest = 1u;
     if (r < nr) cnt[r] = c;
     nonempty[r] = c > 0u ? 1u : 0u;
 }
@@ -2498,16 +2500,18 @@ void cleanup_rings(Ctx &c, FosterScratch &f, int nr, int64_t n, int J, const uin
         SC_HIP(hipGetLastError());
         // compaction counts: vertices, surviving rings, the jobs' first rings
         scan_exclusive_u32(keep, kscan, n + 1, jring + J + 1, s);
-        k_ring_counts<<<grid_for(int64_t(nr) + 1), BLK, 0, s>>>(nr, f.off, kscan, rcnt, nonempty);
+        k_ring_counts<<<grid_for(int64_t(nr) + 1), BLK, 0, s>>>(nr, f.off, kscan, rcnt, nonempty, changed + KEEP_ROUNDS);
         SC_HIP(hipGetLastError());
         scan_exclusive_u32(nonempty, nonempty, int64_t(nr) + 1, jring + J + 2, s);
         k_job_rings<<<grid_for(int64_t(J) + 1), BLK, 0, s>>>(J, jr, nonempty, jring, dring);
         SC_HIP(hipGetLastError());
-        uint32_t moved = 0;
+        uint32_t moved = 0, longest = 0;
         ReadBack rb(c);
         rb.add(job_ring.data(), static_cast<const uint32_t *>(jring), size_t(J) + 3);
         if (!rings) rb.add(&moved, static_cast<const uint32_t *>(changed + it - 1), 1);
+        rb.add(&longest, static_cast<const uint32_t *>(changed + KEEP_ROUNDS), 1);
         rb.run();
+        c.long_rings = longest != 0u; // set by a round that was not the last, it costs launches and no more
         if (!moved) break;
     }
     const uint32_t nout = job_ring[size_t(J) + 1];
@@ -3050,7 +3054,7 @@ void label_and_traverse(Ctx &c) {
         fb.add(head, cross ? NV : 0, 0u);
         fb.add(ringid, NV, 0u);
         fb.add(f.keep.ensure(size_t(NV) + 1) + NV, 1, 0u); // closing entry of the clean-up's scan
-        fb.add(f.kctl.ensure(KEEP_ROUNDS), KEEP_ROUNDS, 0u);
+        fb.add(f.kctl.ensure(KEEP_ROUNDS + 1), KEEP_ROUNDS + 1, 0u); // and the long-ring word
         fb.flush();
     }
     int4 *piece = f.piece.ensure(M > 0 ? M : 1);

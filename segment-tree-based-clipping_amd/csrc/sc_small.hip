@@ -800,6 +800,7 @@ bool clip_small_batch(Ctx &c, int k0, int k1) {
     SC_HIP(hipGetLastError());
     c.nrings = NR;
     c.n_out = NV;
+    c.long_rings = false;
     c.undefined = 0;
     c.cur_k = J == 1 ? k0 : 0;
     c.flags_pending = false;
