@@ -4,6 +4,8 @@
 
 #include <algorithm>
 #include <cstring>
+#include <mutex>
+#include <vector>
 
 struct segclip_ctx {
     sc::Ctx c;
@@ -40,18 +42,42 @@ __global__ void k_readback(GatherArgs a) {
         for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < a.words[q]; i += gridDim.x * blockDim.x)
             a.dst[q][i] = a.src[q][i];
 }
-// Two pinned upload buffers per host thread, used in turn: a table is written
-// there and a kernel copies it, which costs a launch instead of a copy command
-// from pageable memory (10 us of host time each).  The event tells when a
-// buffer's last kernel is done.
+// Pinned upload memory of a host thread: a table is written there and a kernel
+// copies it, which costs a launch instead of a copy command from pageable
+// memory (10 us of host time each).  Tables of one call lie one after the
+// other; the memory is free again once the call's stream is drained, which
+// every wait() sees to and settle_uploads() at the end of a call.  No event
+// tells when: it would be asked after its stream may be gone.  A thread that
+// ends hands its memory to the next one that needs some.
 struct UploadStage {
     char *p = nullptr, *dev = nullptr;
-    size_t cap = 0;
-    hipEvent_t ev = nullptr;
-    int device = -1;
+    size_t cap = 0, used = 0;
 };
-thread_local UploadStage tl_up[2];
-thread_local int tl_up_next = 0;
+struct UploadPool {
+    std::mutex m;
+    std::vector<UploadStage> idle; // as many as threads have been alive at once
+};
+UploadPool &upload_pool() {
+    static UploadPool *p = new UploadPool(); // threads may end after static objects are gone
+    return *p;
+}
+struct UploadHold {
+    UploadStage s;
+    UploadHold() {
+        UploadPool &q = upload_pool();
+        std::lock_guard<std::mutex> g(q.m);
+        if (q.idle.empty()) return;
+        s = q.idle.back();
+        q.idle.pop_back();
+    }
+    ~UploadHold() {
+        if (!s.p) return;
+        UploadPool &q = upload_pool();
+        std::lock_guard<std::mutex> g(q.m);
+        q.idle.push_back(s);
+    }
+};
+thread_local UploadHold tl_up;
 constexpr size_t UPLOAD_MAX = size_t(4) << 20; // larger tables are copied
 __global__ void k_upload(const uint32_t *src, uint32_t *dst, uint32_t words) {
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < words; i += gridDim.x * blockDim.x) dst[i] = src[i];
@@ -80,43 +106,40 @@ void Ctx::upload(void *dst, const void *src, size_t bytes) {
         SC_HIP(hipStreamSynchronize(stream)); // the source may be pinned: it is free on return either way
         return;
     }
-    UploadStage &u = tl_up[tl_up_next];
-    tl_up_next ^= 1;
-    if (u.ev && u.device != device) { // events belong to a device
-        SC_HIP(hipEventSynchronize(u.ev));
-        SC_HIP(hipEventDestroy(u.ev));
-        u.ev = nullptr;
+    UploadStage &u = tl_up.s;
+    if (u.used + bytes > u.cap) {
+        if (u.used) wait(); // all of it is this call's, on this stream
+        if (bytes > u.cap) {
+            if (u.p) SC_HIP(hipHostFree(u.p));
+            u = UploadStage{};
+            const size_t want = std::max(size_t(1) << 18, 2 * bytes);
+            void *hp = nullptr, *dp = nullptr;
+            SC_HIP(hipHostMalloc(&hp, want, hipHostMallocDefault));
+            u.p = static_cast<char *>(hp);
+            SC_HIP(hipHostGetDevicePointer(&dp, hp, 0));
+            u.dev = static_cast<char *>(dp);
+            u.cap = want;
+        }
     }
-    if (u.ev) SC_HIP(hipEventSynchronize(u.ev));
-    if (bytes > u.cap) {
-        if (u.p) SC_HIP(hipHostFree(u.p));
-        u.p = u.dev = nullptr;
-        u.cap = 0;
-        const size_t want = std::max(size_t(65536), bytes + bytes / 4);
-        void *hp = nullptr, *dp = nullptr;
-        SC_HIP(hipHostMalloc(&hp, want, hipHostMallocDefault));
-        u.p = static_cast<char *>(hp);
-        SC_HIP(hipHostGetDevicePointer(&dp, hp, 0));
-        u.dev = static_cast<char *>(dp);
-        u.cap = want;
-    }
-    if (!u.ev) {
-        SC_HIP(hipEventCreateWithFlags(&u.ev, hipEventDisableTiming));
-        u.device = device;
-    }
-    std::memcpy(u.p, src, bytes);
+    std::memcpy(u.p + u.used, src, bytes);
     const uint32_t words = uint32_t(bytes / 4);
-    k_upload<<<std::min(1024u, (words + 255u) / 256u), 256, 0, stream>>>(reinterpret_cast<const uint32_t *>(u.dev),
-                                                                       static_cast<uint32_t *>(dst), words);
+    k_upload<<<std::min(1024u, (words + 255u) / 256u), 256, 0, stream>>>(
+        reinterpret_cast<const uint32_t *>(u.dev + u.used), static_cast<uint32_t *>(dst), words);
+    u.used += (bytes + 15) & ~size_t(15); // counts as in use also where the launch failed
     SC_HIP(hipGetLastError());
-    SC_HIP(hipEventRecord(u.ev, stream));
+}
+void Ctx::settle_uploads() {
+    if (!tl_up.s.used) return;
+    if (hipStreamSynchronize(stream) != hipSuccess) (void)hipGetLastError(); // a call that failed
+    tl_up.s.used = 0;
 }
 void Ctx::wait() {
     for (;;) {
         const hipError_t e = hipStreamQuery(stream);
-        if (e == hipSuccess) return;
+        if (e == hipSuccess) break;
         if (e != hipErrorNotReady) SC_HIP(e);
     }
+    tl_up.s.used = 0;
 }
 void ReadBack::run() {
     size_t tot = 0;
@@ -289,18 +312,20 @@ namespace {
 
 template <class F> int guarded(segclip_ctx *h, F &&f) {
     if (!h) return SEGCLIP_EINVAL;
+    int rc = SEGCLIP_OK;
     try {
         SC_HIP(hipSetDevice(h->c.device));
         f(h->c);
         h->c.last_error.clear();
-        return SEGCLIP_OK;
     } catch (const sc::Error &e) {
         h->c.last_error = e.what();
-        return e.code;
+        rc = e.code;
     } catch (const std::exception &e) {
         h->c.last_error = e.what();
-        return SEGCLIP_EHIP;
+        rc = SEGCLIP_EHIP;
     }
+    h->c.settle_uploads();
+    return rc;
 }
 
 int need_space(int64_t n, int64_t cap, int64_t *need) {

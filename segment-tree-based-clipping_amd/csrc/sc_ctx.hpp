@@ -211,6 +211,7 @@ struct Ctx {
     void wait();
     // host words to device memory, in stream order; the host array is free on return
     void upload(void *dst, const void *src, size_t bytes);
+    void settle_uploads(); // the end of a call: its stream drained where uploads may be in flight
     void mark(int i) {
         if (timing) SC_HIP(hipEventRecord(ev[i], stream));
     }
