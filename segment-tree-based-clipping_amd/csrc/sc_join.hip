@@ -33,7 +33,7 @@
 //
 // Measured (tree stages + stab + sort of the duplicates -> join + sort of the
 // pairs): 200,000 x 1,000,000 harmonic rings 2.02 -> 0.37 ms (the join's
-// kernels 0.17 ms), 100,000 x 4,096 star overlays 19.2 -> 2.6 ms, 1,000 x
+// kernels 0.15 ms), 100,000 x 4,096 star overlays 19.2 -> 2.6 ms, 1,000 x
 // 1,000 stars 0.51 -> 0.13 ms, 256 pairs of 10,000 to 200,000 vertices 40 -> 3 ms.
 #include "sc_ctx.hpp"
 #include "sc_fp64.hpp"
@@ -271,10 +271,16 @@ constexpr int QCAP = QNEAR + WAVE;   // queue: a row adds at most 64
 constexpr int HSTG = 10 * WAVE;
 
 // One wave per run of tiles; the grid covers the chip and strides over the
-// tiles.  Bound by VALU issue: about 14 instructions per surviving row and
-// 64 columns, and the classification's FP64 work per near pair.
+// tiles.  A block's waves take its turns from a counter in LDS: tiles differ a
+// lot in the rows that survive, and with a fixed share per wave a third of the
+// launched waves were in flight on average (the join's kernels at 200,000 x
+// 1,000,000 vertices: 192 -> 161 us, at 100,000 x 4,096 overlays: 1.00 -> 0.94
+// ms).  Blocks of five or ten waves share better and run slower (181, 190).
+// Bound by VALU issue: about 14 instructions per surviving row and 64 columns,
+// and the classification's FP64 work per near pair.
 __global__ __launch_bounds__(BLK) void k_join_pairs(PairArgs a) {
     __shared__ uint32_t toff[TILE_SEGS + 1]; // first tile of each segment
+    __shared__ uint32_t next;                // the block's turns taken so far
     __shared__ uint32_t qb[WPB][QCAP], qc[WPB][QCAP], qk[WPB][QCAP];
     __shared__ uint64_t hits_all[WPB][HSTG];
     if (*a.bad == a.call) return; // every block reads the same word
@@ -303,18 +309,22 @@ __global__ __launch_bounds__(BLK) void k_join_pairs(PairArgs a) {
         }
         if (lane == WAVE - 1) toff[TILE_SEGS] = at;
         mx = wave_reduce(mx, [](uint32_t x, uint32_t y) { return max(x, y); });
+        if (lane == 0) next = 0u;
         if (blockIdx.x == 0 && lane == WAVE - 1) {
             a.sum[1] = at;
             a.sum[2] = mx;
         }
     }
     __syncthreads();
-    // Fewer tiles than waves: 2 to 16 waves share a tile, each walking every
-    // 2nd to 16th of its rows or columns (two stars of 1,000 and 1,100 vertices
-    // have 272 tiles, which took 36 us a wave each, 13 shared).
+    // Fewer than eight turns per wave: 2 to 16 waves share a tile, each walking
+    // every 2nd to 16th of its rows or columns (two stars of 1,000 and 1,100
+    // vertices have 272 tiles, which took 36 us a wave each, 13 shared).  At
+    // 200,000 x 1,000,000 vertices, 3 tiles a wave, halves of tiles take the
+    // join from 161 to 153 us; quarters repeat the tiles' set-up too often (with
+    // fixed shares: whole tiles 192 us, halves 176, quarters 205).
     const uint32_t nw = gridDim.x * WPB;
     uint32_t parts = 1;
-    while (parts < 16u && toff[TILE_SEGS] * parts * 2u <= nw) parts *= 2u;
+    while (parts < 16u && uint64_t(toff[TILE_SEGS]) * parts * 2u <= 8u * uint64_t(nw)) parts *= 2u;
     const uint32_t ntile = toff[TILE_SEGS] * parts; // shares of tiles
     const uint64_t share = ~0ull / ((1ull << parts) - 1ull); // every parts-th row
     uint32_t *vb = qb[wv], *vc = qc[wv], *vk = qk[wv];
@@ -369,8 +379,12 @@ __global__ __launch_bounds__(BLK) void k_join_pairs(PairArgs a) {
     };
     const uint32_t per = min(8u, max(1u, ntile / (4u * nw))); // tiles per turn
     int sg = 0;
-    for (uint32_t t0 = (blockIdx.x * WPB + wv) * per; t0 < ntile; t0 += nw * per) {
-        const uint32_t t1 = min(ntile, t0 + per);
+    for (;;) {
+        uint32_t turn = 0;
+        if (lane == 0) turn = atomicAdd(&next, 1u);
+        const uint64_t at0 = (uint64_t(uni(turn)) * gridDim.x + blockIdx.x) * per;
+        if (at0 >= ntile) break;
+        const uint32_t t0 = uint32_t(at0), t1 = min(ntile, t0 + per);
         int hi = TILE_SEGS; // toff[sg] <= t0 < toff[hi]: later turns search on from the last segment
         while (hi - sg > 1) {
             const int mid = (sg + hi) >> 1;
