@@ -5,8 +5,8 @@ Main workload (the value of the JSON line): plain pairwise clip of two
 harmonic star rings, base 200,000 vertices (seed 2001), overlay 1,000,000
 vertices (seed 2002, centre (0.15,-0.1), rotated 17 degrees), FP64.  One step
 = the whole hot path on the device with both rings already resident in HBM:
-edge records, elementary intervals, node intervals, end lists, cover lists,
-stab + candidate dedupe, intersections / augmented rings / initial labels,
+candidate pairs (box join and pair sort; the tree and its stab where a ring
+has key-vertical edges), intersections / augmented rings / initial labels,
 labelling, traversal and clean-up of the output rings.  Value: input edges
 clipped per second (N_b + N_c per step).
 
@@ -21,14 +21,15 @@ GPU loop on a sample of the same pairs):
                 and forward + backward of the area / IoU
   large_pairs   256 pairs of 10k..200k-vertex harmonic stars: forward +
                 backward with the clip recomputed in backward and with the
-                forward's state kept, peak HBM of each, the stab's HBM rate
+                forward's state kept, peak HBM of each, the join's HBM rate
 
-roofline: the stab kernel (the dominant kernel), HBM bound.  Algorithmic
-bytes per launch = 36 (L + E) + 12 K: every cover entry (L) and leaf end entry
-(E; upper-level end lists are ranges of the leaf entries, not stored) read
-once with its 32-byte coordinate record, plus a 12-byte triple per emitted
-candidate (K), divided by the launch time from HIP events on the library's
-stream, against 8 TB/s.  traffic: the kernel's measured bytes per launch
+roofline: the join's kernels (the candidate search).  Algorithmic bytes per
+clip = 16 V + 16 V + 8 P: every vertex (V = N_b + N_c) read once for its leaf's
+box and once for the pair tests, and an 8-byte key per pair found (P), divided by the time of the join's kernels from HIP
+events on the library's stream, against 8 TB/s.  The tree's lists are not
+built by a clip that takes the join; their sizes (L, E, K, W) are counted
+outside the timed region and reported with the stab's 36 (L + E) + 12 K bytes
+that the clip no longer moves.  traffic: the kernels' measured bytes per clip
 from the rocprofv3 FETCH_SIZE / WRITE_SIZE counter runs summarised in
 profiles/clip_harmonic_200k_1m_hbm_traffic.md (default workload only).
 Those counters count L2-to-fabric requests, so Infinity Cache hits are
@@ -51,6 +52,12 @@ sys.path.insert(0, os.path.join(ROOT, "segment-tree-based-clipping_amd", "python
 
 METRIC = "edges clipped/s and pairs/s on 1 GPU, batched vs plain; fwd+bwd area pairs/s"
 HBM_PEAK_GBPS = 8000.0
+
+
+def join_bytes(vertices, pairs):
+    """Algorithmic HBM bytes of the candidate join of one clip: every vertex for
+    its leaf's box and again for the pair tests, an 8-byte key per pair."""
+    return 32 * vertices + 8 * pairs
 
 
 def stab_bytes(cover_entries, end_entries, candidates):
@@ -277,16 +284,16 @@ def bench_large_pairs(steps):
     fwd()
     st = cl.stage_times()
     cnt = cl.counts()
-    sb = stab_bytes(cnt["cover_entries"], cnt["leaf_end_entries"], cnt["candidates"])
     cl.release()
     plain, n = plain_loop_rate(bases, ovs, 8)
     edges = sum(bsz) + sum(csz)
+    jb = join_bytes(edges, cnt["pairs"])
     return {"workload": "256 pairs of harmonic stars, 10k..200k vertices", "pairs": J,
             "fwd_bwd_ms": 1e3 * dt, "fwd_bwd_pairs_per_s": J / dt, "fwd_bwd_edges_per_s": edges / dt,
             "peak_hbm_bytes_fwd_bwd": peak, "fwd_bwd_stored_ms": 1e3 * dts,
             "peak_hbm_bytes_fwd_bwd_stored": peak_stored,
-            "stab_GBps": round(sb / (st["stab_kernel"] * 1e-3) / 1e9, 1) if st["stab_kernel"] > 0 else None,
-            "stab_roofline_frac": round(sb / (st["stab_kernel"] * 1e-3) / 1e9 / HBM_PEAK_GBPS, 4)
+            "join_GBps": round(jb / (st["stab_kernel"] * 1e-3) / 1e9, 1) if st["stab_kernel"] > 0 else None,
+            "join_roofline_frac": round(jb / (st["stab_kernel"] * 1e-3) / 1e9 / HBM_PEAK_GBPS, 4)
             if st["stab_kernel"] > 0 else None,
             "stage_ms": {k: round(v, 3) for k, v in st.items()},
             "fwd_ms": 1e3 * dtf, "fwd_pairs_per_s": J / dtf,
@@ -395,13 +402,13 @@ def main():
     for i in range(args.warmup):
         step()
         log("[bench] warmup %d done" % i)
-    stab_ms, stages = [], []
+    join_ms, stages = [], []
     t0 = time.perf_counter()
     for i in range(args.steps):
         step()
         st = cl.stage_times()
         stages.append(st)
-        stab_ms.append(st["stab_kernel"])
+        join_ms.append(st["stab_kernel"])
     t1 = time.perf_counter()
     ms = 1000.0 * (t1 - t0) / args.steps
     cnt = cl.counts()
@@ -419,18 +426,21 @@ def main():
     cl.release()
     del cl
 
-    stab = sum(stab_ms) / len(stab_ms)
-    algo = stab_bytes(cnt["cover_entries"], cnt["leaf_end_entries"], cnt["candidates"])
-    achieved = algo / (stab * 1e-3) / 1e9 if stab > 0 else 0.0
-    traffic = measured_traffic("stab_stage") if (nb, nc) == (200000, 1000000) else None
+    join = sum(join_ms) / len(join_ms)
+    algo = join_bytes(nb + nc, cnt["pairs"])
+    achieved = algo / (join * 1e-3) / 1e9 if join > 0 else 0.0
+    traffic = measured_traffic("join_stage") if (nb, nc) == (200000, 1000000) else None
     roof = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBPS, "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBPS, 4), "traffic": traffic,
-            "kernel": "stab stage: k_stab + k_stab_rows + k_near_classify", "kernel_ms": round(stab, 4),
-            "algorithmic_bytes": algo, "near_pairs": cnt.get("near_pairs"),
-            "work": "36 (L + E) + 12 K bytes with L=%d cover entries, E=%d leaf end entries, K=%d candidates; "
-                    "W=%d pair tests" % (cnt["cover_entries"], cnt["leaf_end_entries"], cnt["candidates"],
-                                          cnt["tests"]),
-            "traffic_note": "FETCH_SIZE + WRITE_SIZE of the three kernels per stage, scaled by a 1 GiB copy: "
+            "kernel": "join: k_join_leaves + k_join_groups + k_join_tiles + k_join_pairs",
+            "kernel_ms": round(join, 4), "algorithmic_bytes": algo,
+            "work": "32 V + 8 P bytes with V=%d vertices, P=%d pairs" % (nb + nc, cnt["pairs"]),
+            "tree": "not built by the clip: L=%d cover entries, E=%d leaf end entries, K=%d candidates, W=%d pair "
+                    "tests, %d bytes of the stab" % (cnt["cover_entries"], cnt["leaf_end_entries"],
+                                                     cnt["candidates"], cnt["tests"],
+                                                     stab_bytes(cnt["cover_entries"], cnt["leaf_end_entries"],
+                                                                cnt["candidates"])),
+            "traffic_note": "FETCH_SIZE + WRITE_SIZE of the join's kernels per clip, scaled by a 1 GiB copy: "
                             "L2-to-fabric bytes, Infinity Cache hits included"}
     if materialized_end is not None:
         roof["materialized_end_entries"] = materialized_end

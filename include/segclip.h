@@ -102,7 +102,10 @@ int segclip_find_candidates(segclip_ctx *ctx);
 /* Per-overlay bookkeeping (k is 1-based) and labelling / traversal. */
 int segclip_intersections(segclip_ctx *ctx, int k);
 int segclip_label_traverse(segclip_ctx *ctx);
-/* Whole path for overlay k: the tree and candidates are built on first use. */
+/* Whole path for overlay k: the candidates are found on first use, by a join
+ * of bounding boxes or, where a ring has edges vertical in the tree's keys or
+ * values that are not finite, through the tree.  The tree is then built only
+ * when a staged call, a count or a copy-out asks for it. */
 int segclip_clip(segclip_ctx *ctx, int k);
 /* Whole path for overlays (or pairs) k0..k1 as one batch: intersections,
  * labelling, traversal and clean-up of all of them in the same launches.
@@ -155,7 +158,7 @@ int segclip_batch_area_backward_device(segclip_ctx *ctx, const double *g_area, c
 /* Forward areas / IoU (the segclip_batch_area layout, 4*P doubles in out4) of
  * every pair of a paired context whose rings all have at most 64 vertices,
  * replayed as one hipGraph on the context's stream: re-layout of the caller's
- * rings, queue reset and the persistent small-pair kernel with the areas
+ * rings, cleared fallback word and the small-pair kernel with the areas
  * computed in place.  base_xy / ov_xy are device pointers with the layout and
  * sizes of the last segclip_set_pairs* call (rings back to back, no closing
  * vertex); they are read at every replay, so the caller may update them in
@@ -218,6 +221,8 @@ typedef struct {
     int64_t stab_units;       /* work units (waves) of the stab */
     int64_t near_pairs;       /* stab pairs whose single-precision y-extents meet (classified in FP64) */
 } segclip_counts;
+/* Counts of the tree and the stab that a clip did not need are made here, by
+ * building them. */
 int segclip_get_counts(segclip_ctx *ctx, segclip_counts *out);
 
 /* Copy-out (device -> host).  Each returns SEGCLIP_ESPACE and stores the
@@ -286,8 +291,10 @@ int segclip_count_vertical(const double *xy, int n);
 
 /* Per-stage device times in ms of the last segclip_clip with timing enabled,
  * from HIP events on the context's stream: elementary (edges + sort + unique),
- * node intervals, leaf end lists, cover lists, candidates (stab + dedupe),
- * the stab kernel alone, intersections (A11-A15), labelling + traversal. */
+ * node intervals, leaf end lists, cover lists, candidates (join or stab, and
+ * the sort of the pairs), the join's or the stab's kernels alone, intersections
+ * (A11-A15), labelling + traversal.  The first four are 0 where the clip took
+ * the join. */
 int segclip_set_timing(segclip_ctx *ctx, int on);
 int segclip_get_stage_times(segclip_ctx *ctx, float *ms8);
 
@@ -296,19 +303,21 @@ int segclip_get_stage_times(segclip_ctx *ctx, float *ms8);
  * oacc_segment_tree.cpp:6250-6526); they serve
  * the autotuner, which times candidate values on a workload and persists the
  * fastest as JSON (segclip.tune).  Results never depend on a setting.
+ * The two stab settings act where the tree is stabbed: segclip_find_candidates,
+ * and clips that do not take the join.
  *   "stab_tiles"  64-column tiles per stab work unit, 1..16, default 2.
  *   "stab_units_per_wave"  consecutive stab work units one wave runs (near
  *                 pairs staged across them), 1..32, default 2.
  *   "small_fused" 1 (default): a batch of independent pairs whose rings all
  *                 have at most 64 vertices, without provenance, runs as one
- *                 persistent launch, each pair clipped whole in LDS; 0: the
- *                 staged path.  A batch holding a pair the persistent kernel
+ *                 launch, a wave per pair, each pair clipped whole in LDS; 0:
+ *                 the staged path.  A batch holding a pair that this kernel
  *                 does not cover reruns on the staged path.
  *   "seq_parallel_walks"  1 (default): the traversal of a job on the
- *                 sequential route walks its rings one per lane and checks
- *                 that they are the ones the reference's single walk finds
- *                 (taking the single walk when they may not be); 0: the
- *                 single walk always.
+ *                 sequential route runs over the whole device (large jobs) or
+ *                 walks its rings one per lane, and checks that they are the
+ *                 ones the reference's single walk finds (taking the single
+ *                 walk when they may not be); 0: the single walk always.
  * segclip_get_tuning also reads "small_fallback": the fallback reasons of the
  * last small-pair batch (0 when it ran as one launch).
  * An unknown name or a value out of range returns SEGCLIP_EINVAL. */

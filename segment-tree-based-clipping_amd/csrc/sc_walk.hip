@@ -35,7 +35,8 @@
 // fails the check is left to k_sequential (its 'old' word is set).
 //
 // Measured (MI355X, 200,000 x 1,000,000 harmonic rings with 1 to 15 such
-// accidents): labelling 970 to 4,100 ms -> see walk_jobs.
+// accidents): the whole clip 970 to 4,100 ms -> 1.3 to 3.6; 13 to 16 such
+// overlays among 100,000 x 4,096: their labelling 52 -> 12.9 ms.
 #include "sc_fp64.hpp"
 #include "sc_seqroute.hpp"
 

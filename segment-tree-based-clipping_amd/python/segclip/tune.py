@@ -4,8 +4,9 @@ A setting changes how the library splits its work, never its results: the
 stab's "stab_tiles" (64-column tiles per work unit, one wave each) changes the
 number and length of the waves, "stab_units_per_wave" how many consecutive
 units one wave runs, and the candidate list is sorted afterwards,
-so every value yields the same pairs, intersections and rings.  The tuner
-therefore measures speed only; the tests check that results agree across
+so every value yields the same pairs, intersections and rings.  Both act
+where the tree is stabbed: Clipper.find_candidates, and clips of rings that the
+box join does not take.  The tuner therefore measures speed only; the tests check that results agree across
 values.
 
 Usage: time each candidate value on a workload (a function that runs one clip
