@@ -56,3 +56,13 @@ def test_long_output_rings(gpu, n):
     want = abs(np.sum(x * np.roll(y, -1) - np.roll(x, -1) * y)) / 2
     # n terms below 2.1 in size, each product and partial sum rounded to 2^-53
     assert abs(float(got[0, 0] - want)) <= 2.1 * n * 4 * 2.0 ** -53 * max(1.0, np.log2(n))
+
+
+@pytest.mark.parametrize("combs", [13, 14])  # 600 output rings each: 7,800 and 8,400 with 8,192 waves to take them
+def test_output_rings_one_or_four_a_wave(gpu, combs):
+    print("[gpu-area-orders] %d combs of 600 teeth" % combs, flush=True)
+    bases, ovs = [S.star(300, 21), S.star(17, 22), _comb(40)], [S.star(200, 23, 0.1), S.star(9, 24, 0.1), BAND]
+    alone = _areas(bases, ovs)
+    many = _areas(bases + [_comb(600)] * combs, ovs + [BAND] * combs)
+    assert np.array_equal(alone.view(np.uint64), many[:, :3].copy().view(np.uint64))
+    assert len(set(many[0, 3:].tolist())) == 1
