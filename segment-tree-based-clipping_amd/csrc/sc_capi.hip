@@ -282,7 +282,7 @@ void release_derived(Ctx &c) {
     c.sp_x.release();
     c.sp_y.release();
     for (DBuf<int> *b : {&c.etype, &c.eid, &c.after_leaf, &c.before_leaf, &c.p_j, &c.p_b, &c.p_c, &c.p_type,
-                         &c.p_qa, &c.p_qb, &c.ordB, &c.ordC, &c.nd_b, &c.nd_c, &c.all_b, &c.all_c, &c.nbr_b,
+                         &c.p_qa, &c.p_qb, &c.ordB, &c.ordC, &c.dg_b, &c.dg_c, &c.all_b, &c.all_c, &c.nbr_b,
                          &c.nbr_c, &c.av_b, &c.av_c, &c.lab_b, &c.lab_c, &c.slot_b, &c.slot_c, &c.from_b,
                          &c.from_c, &c.arr_b, &c.arr_c})
         b->release();

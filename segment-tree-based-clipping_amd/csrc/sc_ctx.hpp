@@ -134,7 +134,7 @@ struct Ctx {
     DBuf<uint32_t> run_head; // sparse base side: a run of pairs of one edge starts here
     DBuf<int> run_start;     // first pair of every run
     DBuf<uint32_t> seg_wb, seg_wc, seg_bb, seg_bc, seg_ctl; // groups sorted by a wave / a block; list counts
-    DBuf<int> nd_b, nd_c;                // non-degenerate counts -> exclusive scans (n+1 per job)
+    DBuf<int> dg_b, dg_c;                // degenerate counts -> exclusive scans (n+1 per job)
     DBuf<int> all_b, all_c;
     int nbaug = 0, ncaug = 0;
     DBuf<double> aug_bx, aug_by, aug_cx, aug_cy;
