@@ -32,9 +32,9 @@
 // Rings with any of these go to the tree (join_candidates returns false).
 //
 // Measured (tree stages + stab + sort of the duplicates -> join + sort of the
-// pairs): 200,000 x 1,000,000 harmonic rings 2.02 -> 0.37 ms (the join's
-// kernels 0.15 ms), 100,000 x 4,096 star overlays 19.2 -> 2.6 ms, 1,000 x
-// 1,000 stars 0.51 -> 0.13 ms, 256 pairs of 10,000 to 200,000 vertices 40 -> 3 ms.
+// pairs): 200,000 x 1,000,000 harmonic rings 2.02 -> 0.32 ms (the join's
+// kernels 0.15 ms), 100,000 x 4,096 star overlays 19.2 -> 1.94 ms, 1,000 x
+// 1,000 stars 0.51 -> 0.08 ms, 256 pairs of 10,000 to 200,000 vertices 40 -> 1.25 ms.
 #include "sc_ctx.hpp"
 #include "sc_fp64.hpp"
 #include "sc_wave.hpp"
