@@ -470,7 +470,21 @@ __global__ void k_sp_fill(int I, const int *__restrict__ ord, const int *__restr
                           int *av, int *nbr, int *lab, double *x, double *y, const int *kind,
                           const uint32_t *__restrict__ unordered) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= I || (unordered && *unordered)) return;
+    if (i >= I) return;
+    if (unordered && *unordered) {
+        // No slot anywhere until the order is there: the labelling's first kernels
+        // run before the host learns of it, and take an edge from a position that
+        // holds a slot.
+        slot[i] = -1;
+        ndx[i] = 0;
+        edge[i] = 0;
+        av[i] = -100;
+        nbr[i] = -100;
+        lab[i] = 0;
+        x[i] = 0.0;
+        y[i] = 0.0;
+        return;
+    }
     int p = ord[i], j = pj[p], e = pb[p];
     int rel = int(ndg[i] - ndg[p0[j]]);
     int k = kind[i];
