@@ -301,6 +301,7 @@ void release_derived(Ctx &c) {
     c.rs.vals_alt.release();
     release_foster_scratch();
     c.epc = c.nleaves = c.T = 0;
+    c.built = 0;
     c.n_lend = c.n_cov = c.n_cand = c.n_pairs = c.n_mend = 0;
     c.cur_k = 0;
     c.I = 0;
@@ -403,7 +404,7 @@ int segclip_set_pairs_device(segclip_ctx *h, const double *b, const int *bsz, co
 }
 int segclip_build_elementary(segclip_ctx *h) {
     return guarded(h, [&](sc::Ctx &x) {
-        if (x.joined && x.T == 0) {
+        if (x.joined && x.built != sc::TREE_ALL) {
             sc::build_tree(x); // the later stages' results show with it, as after any clip
         } else {
             sc::build_edges(x);
@@ -553,6 +554,7 @@ int segclip_pairs_area_graph(segclip_ctx *h, const double *base_xy, const double
 int segclip_reset(segclip_ctx *h) {
     return guarded(h, [&](sc::Ctx &x) {
         x.epc = x.nleaves = x.T = 0;
+        x.built = 0;
         x.n_lend = x.n_cov = x.n_cand = x.n_pairs = x.n_mend = x.n_near = 0;
         x.cur_k = 0;
         x.pair_off.clear();

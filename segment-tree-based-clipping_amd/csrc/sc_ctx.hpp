@@ -11,6 +11,9 @@ struct StageTimes {
     float elementary = 0, tree = 0, endlist = 0, cover = 0, candidates = 0, stab_kernel = 0, post = 0, label = 0;
 };
 
+// Stages of the tree after the elementary intervals (Ctx::built).
+enum : unsigned { TREE_NODES = 1, TREE_ENDS = 2, TREE_COVERS = 4, TREE_ALL = 7 };
+
 // Jobs of one post-processing batch: job j clips base ring job_base(k0+j)
 // against overlay k0+j.  Host vectors and their device copies; per-edge count
 // arrays hold n+1 slots per job (JB/JC offsets), augmented rings are
@@ -69,6 +72,7 @@ struct Ctx {
     DBuf<double> ea;
     int epc = 0, nleaves = 0, T = 0, depth = 0;
     int ea_count = 0;                    // elementary points before padding
+    unsigned built = 0;                  // the tree's other stages that these rings have (TREE_*)
     DBuf<uint2> ep_lohi;                 // per endpoint: its elementary index range, or NIL (search)
     // ---- A4 ----
     DBuf<double> niv;

@@ -3165,12 +3165,12 @@ void clip_jobs(Ctx &c, int k0, int k1) {
             return;
         }
     }
-    // candidate pairs: from the box join, or from the tree where the join
-    // refuses the rings or the tree is already there with its own pairs
+    // candidate pairs, where no call has found them yet: from the box join, or,
+    // where it refuses the rings, from the tree (built here unless all of it is there)
     const bool cand = int(c.pair_off.size()) != c.K + 1;
     c.mark(10);
     const bool joined = cand && join_candidates(c);
-    const bool tree = cand && !joined && c.T == 0;
+    const bool tree = cand && !joined && c.built != TREE_ALL;
     c.mark(0);
     if (tree) {
         build_edges(c);

@@ -693,7 +693,7 @@ int bits_for(int64_t n) { // bits to hold values in [0, n)
 } // namespace
 
 void find_candidates(Ctx &c) {
-    SC_REQUIRE(c.n_cov >= 0 && c.T > 0 && c.n_lend >= 0, SC_ESTATE, "tree not built");
+    SC_REQUIRE(c.T > 0 && (c.built & TREE_ENDS) && (c.built & TREE_COVERS), SC_ESTATE, "tree not built");
     hipStream_t s = c.stream;
     const int T = c.T;
     c.bits_b = bits_for(c.nb);

@@ -518,6 +518,7 @@ uint64_t read_u64(Ctx &c, const uint64_t *d) {
 namespace {
 void reset_derived(Ctx &c) {
     c.epc = c.nleaves = c.T = c.ea_count = 0;
+    c.built = 0;
     c.n_lend = c.n_cov = c.n_cand = c.n_pairs = c.n_mend = c.n_near = 0;
     c.cur_k = 0;
     c.pair_off.clear();
@@ -710,6 +711,7 @@ void build_node_intervals(Ctx &c) {
     c.niv.ensure(2 * size_t(c.T));
     k_node_intervals<<<grid_for(c.T), BLK, 0, c.stream>>>(c.ea, c.T, c.depth, c.niv);
     SC_HIP(hipGetLastError());
+    c.built |= TREE_NODES;
 }
 
 namespace {
@@ -776,6 +778,7 @@ void build_leaf_end_entries(Ctx &c) {
         k_entry_before<<<grid_for(c.n_lend), BLK, 0, s>>>(vals, c.n_lend, c.before_leaf, c.eyr, bl, bx);
         SC_HIP(hipGetLastError());
     }
+    c.built |= TREE_ENDS;
 }
 
 void build_cover_lists(Ctx &c) {
@@ -824,6 +827,7 @@ void build_cover_lists(Ctx &c) {
     scan_inclusive_max_u32(off + 1, off + 1, T, s);
     k_cover_split<<<grid_for(T), BLK, 0, s>>>(T, off, bend, split);
     SC_HIP(hipGetLastError());
+    c.built |= TREE_COVERS;
 }
 
 void build_tree(Ctx &c) {
@@ -835,7 +839,7 @@ void build_tree(Ctx &c) {
 }
 
 void tree_after_join(Ctx &c) {
-    if (c.joined && c.T == 0) build_tree(c);
+    if (c.joined && c.built != TREE_ALL) build_tree(c); // also where single stages were called
 }
 
 void stab_after_join(Ctx &c) {
