@@ -162,7 +162,9 @@ int segclip_batch_area_backward_device(segclip_ctx *ctx, const double *g_area, c
  * computed in place.  base_xy / ov_xy are device pointers with the layout and
  * sizes of the last segclip_set_pairs* call (rings back to back, no closing
  * vertex); they are read at every replay, so the caller may update them in
- * place between calls.  The graph is captured on the first call, again when
+ * place between calls; the context's rings are then these, and what earlier
+ * calls derived from other ones (pairs, tree) is found again when a call needs
+ * it.  The graph is captured on the first call, again when
  * a pointer changes, and dropped by segclip_set_pairs* / set_polygons*.
  * After the replay one word is read back: when some pair needs the staged
  * path, the batch is clipped on it (areas identical either way) and the next

@@ -270,7 +270,7 @@ void release_derived(Ctx &c) {
     for (DBuf<uint64_t> *b : {&c.join_box, &c.join_leaf, &c.join_tile}) b->release();
     c.join_ctl.release();
     c.out_xy.release();
-    c.joined = false;
+    c.joined = c.moved = false;
     for (DBuf<YRangeF> *b : {&c.eyr, &c.lend_yr, &c.cov_yr}) b->release();
     c.lend_bl.release();
     c.ep_lohi.release();
@@ -336,7 +336,7 @@ int need_space(int64_t n, int64_t cap, int64_t *need) {
 
 // a clip's candidate pairs need no tree: build it for calls that show it
 int need_tree(segclip_ctx *h) {
-    if (!h->c.joined) return SEGCLIP_OK;
+    if (!h->c.joined && !h->c.moved) return SEGCLIP_OK;
     return guarded(h, [](sc::Ctx &x) { sc::tree_after_join(x); });
 }
 
@@ -404,6 +404,7 @@ int segclip_set_pairs_device(segclip_ctx *h, const double *b, const int *bsz, co
 }
 int segclip_build_elementary(segclip_ctx *h) {
     return guarded(h, [&](sc::Ctx &x) {
+        sc::pairs_after_move(x);
         if (x.joined && x.built != sc::TREE_ALL) {
             sc::build_tree(x); // the later stages' results show with it, as after any clip
         } else {
@@ -558,7 +559,7 @@ int segclip_reset(segclip_ctx *h) {
         x.n_lend = x.n_cov = x.n_cand = x.n_pairs = x.n_mend = x.n_near = 0;
         x.cur_k = 0;
         x.pair_off.clear();
-        x.joined = false;
+        x.joined = x.moved = false;
         x.jobs.J = 0;
         x.jobs.AB.clear();
         x.jobs.ring_off.clear();
@@ -687,6 +688,8 @@ int segclip_copy_pairs(segclip_ctx *h, int k, int32_t *b_id, int32_t *c_id, int3
                        int64_t *need) {
     if (!h) return SEGCLIP_EINVAL;
     sc::Ctx &c = h->c;
+    if (c.moved)
+        if (int mrc = guarded(h, [](sc::Ctx &x) { sc::pairs_after_move(x); })) return mrc;
     if (int(c.pair_off.size()) != c.K + 1 || k < 1 || k > c.K) return SEGCLIP_ESTATE;
     int64_t n = c.pair_off[k] - c.pair_off[k - 1];
     int rc = need_space(n, cap, need);

@@ -100,6 +100,7 @@ struct Ctx {
     int64_t n_cov = 0;
     // ---- box join (sc_join.hip): the pairs of a clip without the tree ----
     bool joined = false;                 // pairs come from the join: no tree, no stab counts
+    bool moved = false;                  // the rings moved after pairs or the tree were there: calls that show them find them again
     DBuf<uint64_t> join_box, join_leaf;  // boxes of leaves and base groups; first vertex, size, edge, ring of leaves
     DBuf<uint64_t> join_tile;            // (base leaf, overlay leaf) tiles in segments of join_seg_cap entries
     DBuf<uint32_t> join_ctl;             // totals, flag, segment counters
@@ -244,6 +245,10 @@ void pair_offsets(Ctx &c);             // pair_off of c.n_pairs sorted pairs
 // after a clip whose pairs came from the join: the tree (tree_after_join), and
 // the stab's counts as well (stab_after_join), for calls that show them
 void build_tree(Ctx &c);
+// the rings hold other coordinates of the same sizes: what came from the old
+// ones goes, and pairs_after_move finds the pairs again for calls that need them
+void rings_moved(Ctx &c);
+void pairs_after_move(Ctx &c);
 void tree_after_join(Ctx &c);
 void stab_after_join(Ctx &c);
 void post_jobs(Ctx &c, int k0, int k1, bool late = false); // A11-A15 for overlays k0..k1 in one batch

@@ -3184,6 +3184,7 @@ void clip_jobs(Ctx &c, int k0, int k1) {
     if (tree) build_cover_lists(c);
     c.mark(4);
     if (cand && !joined) find_candidates(c);
+    c.moved = false;
     c.mark(5);
     post_jobs(c, k0, k1, true);
     c.mark(6);

@@ -838,7 +838,10 @@ void fetch_flags(Ctx &c) {
     c.undefined = any;
 }
 
-void post_overlay(Ctx &c, int k) { post_jobs(c, k, k); }
+void post_overlay(Ctx &c, int k) {
+    pairs_after_move(c);
+    post_jobs(c, k, k);
+}
 
 SparseP sparse_view(Ctx &c) {
     SparseP v;

@@ -900,7 +900,7 @@ void pairs_area_graph(Ctx &c, const double *bxy, const double *cxy, double *out4
         g.out4 = out4;
     }
     SC_HIP(hipGraphLaunch(g.exec, s));
-    c.shift_ready = false; // the rings hold other coordinates now
+    rings_moved(c);
     uint32_t anyfail = 0;
     {
         ReadBack rb(c);

@@ -522,7 +522,7 @@ void reset_derived(Ctx &c) {
     c.n_lend = c.n_cov = c.n_cand = c.n_pairs = c.n_mend = c.n_near = 0;
     c.cur_k = 0;
     c.pair_off.clear();
-    c.joined = false;
+    c.joined = c.moved = false;
 }
 
 void load(Ctx &c, const double *bxy, const int *bsz, int nbr, const double *cxy, const int *csz, int K,
@@ -838,11 +838,29 @@ void build_tree(Ctx &c) {
     build_cover_lists(c);
 }
 
+void rings_moved(Ctx &c) {
+    const bool had = c.moved || c.T > 0 || !c.pair_off.empty();
+    reset_derived(c);
+    c.shift_ready = false;
+    c.moved = had;
+}
+
+void pairs_after_move(Ctx &c) {
+    if (!c.moved) return;
+    if (!join_candidates(c)) {
+        if (c.built != TREE_ALL) build_tree(c);
+        find_candidates(c);
+    }
+    c.moved = false;
+}
+
 void tree_after_join(Ctx &c) {
+    pairs_after_move(c);
     if (c.joined && c.built != TREE_ALL) build_tree(c); // also where single stages were called
 }
 
 void stab_after_join(Ctx &c) {
+    pairs_after_move(c);
     if (!c.joined) return;
     tree_after_join(c);
     find_candidates(c); // the same pairs again, with the stab's counts
