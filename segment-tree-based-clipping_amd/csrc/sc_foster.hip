@@ -2463,6 +2463,7 @@ void cleanup_rings(Ctx &c, FosterScratch &f, int nr, int64_t n, int J, const uin
         fb.add(c.d_ring_off.ensure(1), 1, 0u);
         fb.add(dring, int64_t(J) + 1, 0u);
         fb.flush();
+        c.wait(); // the labelling's scratch is the host thread's, for any context and stream
         return;
     }
     int *rstart = f.rstart.ensure(nr);

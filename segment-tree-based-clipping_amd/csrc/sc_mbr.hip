@@ -205,7 +205,10 @@ extern "C" int segclip_mbr_join(const double *a_xy, const int *a_sizes, int na, 
         const int32_t *dp = nullptr;
         const int64_t n = sc::mbr_join(a_xy, a_sizes, na, b_xy, b_sizes, nb, s, &dp);
         if (need) *need = n;
-        if (n > cap) return SEGCLIP_ESPACE;
+        if (n > cap) {
+            SC_HIP(hipStreamSynchronize(s)); // the scratch is the thread's, for any stream
+            return SEGCLIP_ESPACE;
+        }
         if (n > 0) {
             if (!pairs) return SEGCLIP_EINVAL;
             SC_HIP(hipMemcpyAsync(pairs, dp, sizeof(int32_t) * 2 * size_t(n), hipMemcpyDeviceToHost, s));

@@ -798,6 +798,9 @@ bool clip_small_batch(Ctx &c, int k0, int k1) {
     k_small_emit<<<J, 256, 0, s>>>(J, voff, roff, a.job_nr, a.out_x, a.out_y, a.out_len, c.d_ring_x, c.d_ring_y,
                                    c.d_ring_off);
     SC_HIP(hipGetLastError());
+    // the scratch that it reads is the host thread's: another context's batch, on
+    // another stream, may be next to write it
+    c.wait();
     c.nrings = NR;
     c.n_out = NV;
     c.long_rings = false;
@@ -923,6 +926,7 @@ void pairs_area_graph(Ctx &c, const double *bxy, const double *cxy, double *out4
     }
     c.small_fused = keep;
     batch_area(c, out4);
+    c.wait(); // out4 is written on return, and the thread's scratch is free
     c.small_fail = 1;
 }
 
