@@ -204,6 +204,7 @@ constexpr int64_t OUT_CHUNK = int64_t(2) << 20; // vertices per device-side piec
 // pieces of 32 MB and copied.  (Pairing on the host cost a copy to
 // pageable memory and a pass over it: 100 ms for 23.5 M vertices.)
 void rings_to_host(Ctx &c, int32_t *ring_off, double *xy) {
+    SC_REQUIRE(c.d_ring_off.p, SC_ESTATE, "no clip has run"); // a kernel reads the offsets
     const int64_t n = c.n_out;
     const int noff = c.nrings + 1;
     hipStream_t s = c.stream;
