@@ -78,6 +78,14 @@ struct UploadHold {
     }
 };
 thread_local UploadHold tl_up;
+// The stream that may still have work queued on this thread's scratch.  The
+// stream may be gone when another one takes over (its context has drained it
+// then), so it is compared and never waited for: the device is.
+struct ScratchHold {
+    hipStream_t s = nullptr;
+    bool busy = false;
+};
+thread_local ScratchHold tl_hold;
 constexpr size_t UPLOAD_MAX = size_t(4) << 20; // larger tables are copied
 __global__ void k_upload(const uint32_t *src, uint32_t *dst, uint32_t words) {
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < words; i += gridDim.x * blockDim.x) dst[i] = src[i];
@@ -133,13 +141,22 @@ void Ctx::settle_uploads() {
     if (hipStreamSynchronize(stream) != hipSuccess) (void)hipGetLastError(); // a call that failed
     tl_up.s.used = 0;
 }
+void Ctx::hold_scratch() {
+    if (tl_hold.busy && tl_hold.s != stream) SC_HIP(hipDeviceSynchronize());
+    tl_hold.s = stream;
+    tl_hold.busy = true;
+}
+void Ctx::drained() {
+    tl_up.s.used = 0;
+    if (tl_hold.s == stream) tl_hold.busy = false;
+}
 void Ctx::wait() {
     for (;;) {
         const hipError_t e = hipStreamQuery(stream);
         if (e == hipSuccess) break;
         if (e != hipErrorNotReady) SC_HIP(e);
     }
-    tl_up.s.used = 0;
+    drained();
 }
 void ReadBack::run() {
     size_t tot = 0;
@@ -242,6 +259,7 @@ void rings_to_host(Ctx &c, int32_t *ring_off, double *xy) {
         SC_HIP(hipMemcpyAsync(xy + 2 * v, piece, size_t(m) * sizeof(double2), hipMemcpyDeviceToHost, s));
     }
     SC_HIP(hipStreamSynchronize(s));
+    c.drained();
 }
 void Ctx::ensure_side_stream() {
     if (stream2) return;
@@ -487,6 +505,7 @@ int segclip_batch_area(segclip_ctx *h, double *out4, int64_t cap, int64_t *need)
         sc::batch_area(x, d.p);
         d2h(x, out4, d.p, 4 * int64_t(J));
         SC_HIP(hipStreamSynchronize(x.stream));
+        x.drained();
     });
 }
 int segclip_batch_area_device(segclip_ctx *h, double *out4) {
@@ -494,6 +513,7 @@ int segclip_batch_area_device(segclip_ctx *h, double *out4) {
     return guarded(h, [&](sc::Ctx &x) {
         sc::batch_area(x, out4);
         SC_HIP(hipStreamSynchronize(x.stream));
+        x.drained();
     });
 }
 int segclip_batch_area_backward_device(segclip_ctx *h, const double *g_area, const double *g_iou, double *grad_b,

@@ -217,6 +217,10 @@ struct Ctx {
     // host words to device memory, in stream order; the host array is free on return
     void upload(void *dst, const void *src, size_t bytes);
     void settle_uploads(); // the end of a call: its stream drained where uploads may be in flight
+    // Before work on scratch of the host thread that may still be queued when the
+    // call returns: where another stream's may be, it is waited for.
+    void hold_scratch();
+    void drained(); // nothing of this context's stream is queued
     void mark(int i) {
         if (timing) SC_HIP(hipEventRecord(ev[i], stream));
     }
