@@ -2967,6 +2967,7 @@ void label_and_traverse(Ctx &c) {
         SC_HIP(hipGetLastError());
         // scratch per job, sized by its nodes
         int64_t vb = 0, ob = 0, rb = 0;
+        wi.nwalk = 0;
         for (int q = 0; q < nseq; ++q) {
             SeqJob &j = sj[q];
             j.node0 = int(nodeoff[2 * q]);
@@ -2975,6 +2976,7 @@ void label_and_traverse(Ctx &c) {
             j.cap = 2 * (j.nPn + j.nQn) + 64;
             j.out_cap = 2 * (j.nP + j.nQ) + 64;
             j.ring_cap = j.nP + j.nQ + 8;
+            j.walk = j.nPn + j.nQn >= WALK_MIN_NODES ? wi.nwalk++ : -1;
             j.vbase = vb;
             j.obase = ob;
             j.rbase = rb;

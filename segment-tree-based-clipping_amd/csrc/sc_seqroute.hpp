@@ -43,6 +43,7 @@ struct SeqJob {
     int nP, nQ, P0, Q0;        // ring sizes (slots) and first slots in the dense ring arrays
     int node0, nPn, nQn;       // first node, node counts of P and Q
     int cap, out_cap, ring_cap;
+    int walk;                  // its place among the jobs that sc_walk.hip takes, -1: none of them
     int64_t vbase, obase, rbase; // scratch bases: vertices, output vertices, ring offsets
 };
 
@@ -72,6 +73,7 @@ struct SeqBatch {
 struct WalkIn {
     SeqBatch b;
     const std::vector<SeqJob> *jobs; // host copy
+    int nwalk;                       // jobs with a place among them
     const int64_t *nodeoff, *segoff; // 2 * nseq + 1 node / slot offsets (device)
     const uint32_t *nidx;            // node index by slot (exclusive scan of node starts)
     int64_t N;                       // nodes of all jobs
@@ -80,7 +82,7 @@ struct WalkIn {
 // below, one block per job is as fast: on unions of 300 nodes 0.99 ms a clip against
 // 0.98 device-wide, of 1,000 nodes 1.22 against 0.98 (the launches cost 0.15 ms)
 constexpr int WALK_MIN_NODES = 512;
-bool walk_jobs(const WalkIn &in, int *done, hipStream_t s); // false: no job is large enough
+bool walk_jobs(const WalkIn &in, int *done, hipStream_t s); // false: no job is large enough, or no memory for them
 void walk_emit(const WalkIn &in, const int *done, const uint32_t *JV, const uint32_t *JR, double *ox, double *oy,
                int *osrc, int *off, hipStream_t s);
 void release_walk_scratch();

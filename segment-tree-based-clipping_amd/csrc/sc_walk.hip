@@ -102,7 +102,7 @@ struct WalkArgs {
     int64_t N;
     uint32_t cap;            // specials
     WalkJob *gj;
-    uint64_t *lists;         // per job: chain starts, P split list, P crossing list, of LIST entries
+    uint64_t *lists;         // per walking job (SeqJob::walk): chain starts, P split list, P crossing list, of LIST entries
     uint32_t *tab, *tsum;    // state tables by node, per block
     uint32_t *cnt, *ins;     // per node: specials / inserted nodes there, then before it (N + 1)
     // per special
@@ -142,7 +142,7 @@ __global__ void k_walk_init(WalkArgs a) {
     const SeqJob &jb = a.b.jobs[q];
     WalkJob g;
     const int fp = a.firstP[jb.j], fq = a.firstQ[jb.j];
-    g.old = jb.nPn + jb.nQn < WALK_MIN_NODES || jb.nPn + jb.nQn > jb.cap || fp < 0 || fq < 0 ? 1 : 0;
+    g.old = jb.walk < 0 || jb.nPn + jb.nQn > jb.cap || fp < 0 || fq < 0 ? 1 : 0;
     g.V[0] = g.V[1] = 0;
     if (!g.old) { // a first plain slot starts a node
         g.V[0] = int(int64_t(a.nidx[a.segoff[2 * q] + fp]) - a.nodeoff[2 * q]);
@@ -168,7 +168,7 @@ __global__ void k_walk_chain_starts(WalkArgs a) {
     const int lb = a.b.lab[w];
     if (!a.b.inter[w] || (lb != L_LEFT_ON && lb != L_RIGHT_ON)) return;
     const int k = atomicAdd(&a.gj[q].nchain, 1);
-    if (k < LIST) a.lists[int64_t(q) * 3 * LIST + k] = uint64_t(v);
+    if (k < LIST) a.lists[int64_t(a.b.jobs[q].walk) * 3 * LIST + k] = uint64_t(v);
 }
 
 // ascending order of a short list, by one block (every thread calls it)
@@ -196,7 +196,7 @@ __global__ __launch_bounds__(BLK) void k_walk_chains(WalkArgs a) {
         if (threadIdx.x == 0) g.old = 1;
         return;
     }
-    uint64_t *l = a.lists + int64_t(q) * 3 * LIST;
+    uint64_t *l = a.lists + int64_t(a.b.jobs[q].walk) * 3 * LIST;
     sort_list(l, n, s);
     if (threadIdx.x != 0) return;
     const int64_t vb = a.b.jobs[q].vbase;
@@ -380,7 +380,7 @@ __global__ void k_walk_enex(WalkArgs a) {
         a.b.seen[2 * w + (addS ? 0 : 1)] = -1;
     } else if (k < LIST) {
         const int m = int(r1 - r0), p = v > V ? v - V : v - V + m; // place on the walk
-        a.lists[int64_t(q) * 3 * LIST + (addS ? LIST : 2 * LIST) + k] = (uint64_t(uint32_t(p)) << 32) | uint32_t(v);
+        a.lists[int64_t(jb.walk) * 3 * LIST + (addS ? LIST : 2 * LIST) + k] = (uint64_t(uint32_t(p)) << 32) | uint32_t(v);
     }
 }
 
@@ -400,7 +400,7 @@ __global__ __launch_bounds__(BLK) void k_walk_split(WalkArgs a) {
         if (threadIdx.x == 0) wj.old = 1;
         return;
     }
-    uint64_t *lS = a.lists + int64_t(q) * 3 * LIST + LIST, *lC = lS + LIST;
+    uint64_t *lS = a.lists + int64_t(jb.walk) * 3 * LIST + LIST, *lC = lS + LIST;
     sort_list(lS, nS, s);
     sort_list(lC, nC, s);
     if (threadIdx.x != 0) return;
@@ -623,8 +623,9 @@ __global__ void k_walk_cut(WalkArgs a) {
     t.i = i;
     t.cand = NIL;
     t.nst = t.pad = 0;
-    a.terms[int64_t(q) * TERMS + k] = t;
-    a.tpos[i] = uint32_t(int64_t(q) * TERMS + k);
+    const int64_t at = int64_t(a.b.jobs[q].walk) * TERMS + k;
+    a.terms[at] = t;
+    a.tpos[i] = uint32_t(at);
 }
 
 // Doubling over the links.  A record: (smallest value of the window, vertices
@@ -676,7 +677,8 @@ __global__ __launch_bounds__(BLK) void k_walk_walks(WalkArgs a, int again) {
     if (wj.old) return; // uniform: written by earlier launches only
     if (again && wj.wrong == NIL) return;
     const int nt = int(wj.nterm);
-    Term *T = a.terms + int64_t(q) * TERMS;
+    const int walk = a.b.jobs[q].walk;
+    Term *T = a.terms + int64_t(walk) * TERMS;
     const int uni = a.b.uni;
     const int lane = threadIdx.x & (WAVE - 1), wid = threadIdx.x / WAVE;
     int micro = 0; // thread 0: specials stepped over singly so far
@@ -709,7 +711,7 @@ __global__ __launch_bounds__(BLK) void k_walk_walks(WalkArgs a, int again) {
                     const uint32_t w = reached(t.i);
                     if (a.linked[w] == 2 && reached(w) == t.i) {
                         const uint32_t x = a.rec[w].x;
-                        seen = (x & ONCYCLE) || T[a.tpos[x] - uint32_t(int64_t(q) * TERMS)].nst > 0;
+                        seen = (x & ONCYCLE) || a.terms[a.tpos[x]].nst > 0;
                     }
                 }
                 if (!seen) m = min(m, t.i);
@@ -719,7 +721,7 @@ __global__ __launch_bounds__(BLK) void k_walk_walks(WalkArgs a, int again) {
                 bool seen = false;
                 if (a.linked[w] == 2) {
                     const uint32_t x = a.rec[w].x;
-                    seen = (x & ONCYCLE) || T[a.tpos[x] - uint32_t(int64_t(q) * TERMS)].nst > 0;
+                    seen = (x & ONCYCLE) || a.terms[a.tpos[x]].nst > 0;
                 }
                 if (!seen) m = min(m, t.cand);
             }
@@ -732,7 +734,7 @@ __global__ __launch_bounds__(BLK) void k_walk_walks(WalkArgs a, int again) {
                 auto walked = [&](uint32_t i) {
                     const uint4 r = a.rec[i];
                     if (r.x & ONCYCLE) return true;
-                    const Term &t = T[a.tpos[r.x] - uint32_t(int64_t(q) * TERMS)];
+                    const Term &t = a.terms[a.tpos[r.x]];
                     for (uint32_t k = 0; k < t.nst; ++k)
                         if (r.y > t.st[k].lo && r.y <= t.st[k].hi) return true;
                     return false;
@@ -762,7 +764,7 @@ __global__ __launch_bounds__(BLK) void k_walk_walks(WalkArgs a, int again) {
                             wj.old = 1;
                             break;
                         }
-                        Term &t = T[a.tpos[r.x] - uint32_t(int64_t(q) * TERMS)];
+                        Term &t = a.terms[a.tpos[r.x]];
                         uint32_t lo = 0, last = NIL;
                         const uint4 ri = a.rec[I];
                         if (ri.x == r.x && ri.y < r.y) { // jumped to
@@ -853,7 +855,7 @@ __global__ __launch_bounds__(BLK) void k_walk_walks(WalkArgs a, int again) {
                     sg.off = off;
                     sg.ring = I;
                     sg.pad = 0;
-                    a.singles[int64_t(q) * SINGLES + wj.nsingle++] = sg;
+                    a.singles[int64_t(walk) * SINGLES + wj.nsingle++] = sg;
                     off += len;
                     if (closed) break;
                     const uint32_t n = a.snb[c];
@@ -1000,7 +1002,7 @@ __global__ void k_walk_single_heads(WalkArgs a) { // one block per job
     const int q = blockIdx.x;
     if (!a.done[q] || a.gj[q].fail != NIL) return;
     for (uint32_t k = threadIdx.x; k < a.gj[q].nsingle; k += blockDim.x) {
-        const Single t = a.singles[int64_t(q) * SINGLES + k];
+        const Single t = a.singles[int64_t(a.b.jobs[q].walk) * SINGLES + k];
         place(a, q, t.ring, t.off, t.i);
     }
 }
@@ -1084,14 +1086,14 @@ WalkArgs walk_args(const WalkIn &in, int *done) {
     a.firstQ = in.firstQ;
     a.nseq = int(in.jobs->size());
     a.N = in.N;
-    a.cap = uint32_t(in.N) + 2u * uint32_t(LIST) * uint32_t(a.nseq);
+    a.cap = uint32_t(in.N) + 2u * uint32_t(LIST) * uint32_t(in.nwalk);
     a.done = done;
     const SeqJob &lastj = in.jobs->back();
     const int64_t nv = lastj.vbase + lastj.cap, no = lastj.obase + lastj.out_cap;
     a.gj = reinterpret_cast<WalkJob *>(f.gj.ensure(size_t(a.nseq) * ((sizeof(WalkJob) + 7) / 8)));
-    a.lists = f.lists.ensure(size_t(a.nseq) * 3 * LIST);
-    a.terms = reinterpret_cast<Term *>(f.terms.ensure(size_t(a.nseq) * TERMS * sizeof(Term) / 8));
-    a.singles = reinterpret_cast<Single *>(f.singles.ensure(size_t(a.nseq) * SINGLES * sizeof(Single) / 8));
+    a.lists = f.lists.ensure(size_t(in.nwalk) * 3 * LIST);
+    a.terms = reinterpret_cast<Term *>(f.terms.ensure(size_t(in.nwalk) * TERMS * sizeof(Term) / 8));
+    a.singles = reinterpret_cast<Single *>(f.singles.ensure(size_t(in.nwalk) * SINGLES * sizeof(Single) / 8));
     a.rec = reinterpret_cast<uint4 *>(f.rec.ensure(2 * size_t(a.cap)));
     a.rec2 = reinterpret_cast<uint4 *>(f.rec2.ensure(2 * size_t(a.cap)));
     a.tab = f.tab.ensure(size_t(a.N));
@@ -1123,20 +1125,23 @@ static_assert(sizeof(Term) % 8 == 0 && sizeof(Single) % 8 == 0, "allocated in 8-
 } // namespace
 
 bool walk_jobs(const WalkIn &in, int *done, hipStream_t s) {
-    bool any = false;
     uint32_t most = 1;
     for (const SeqJob &j : *in.jobs)
-        if (j.nPn + j.nQn >= WALK_MIN_NODES) {
-            any = true;
-            most = std::max(most, uint32_t(j.nPn + j.nQn) + 2u * uint32_t(LIST));
-        }
+        if (j.walk >= 0) most = std::max(most, uint32_t(j.nPn + j.nQn) + 2u * uint32_t(LIST));
     const int nseq = int(in.jobs->size());
     // specials are counted in 30 bits, output places in 32
     const SeqJob &lastj = in.jobs->back();
-    if (!any || in.N + 2 * int64_t(LIST) * nseq >= (int64_t(1) << 29) ||
+    if (in.nwalk == 0 || in.N + 2 * int64_t(LIST) * in.nwalk >= (int64_t(1) << 29) ||
         lastj.obase + lastj.out_cap >= (int64_t(1) << 32) - 1)
         return false;
-    WalkArgs a = walk_args(in, done);
+    WalkArgs a;
+    try {
+        a = walk_args(in, done);
+    } catch (const Error &e) { // 300 KB a job: k_sequential needs none of it
+        if (e.code != SC_ENOMEM) throw;
+        release_walk_scratch();
+        return false;
+    }
     const int64_t no = lastj.obase + lastj.out_cap;
     const unsigned gn = grid_for(a.N), gs = grid_for(a.cap), gq = grid_for(nseq);
     const unsigned nt = unsigned(ceil_div(a.N, TAB_TILE));
