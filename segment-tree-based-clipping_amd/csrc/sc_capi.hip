@@ -18,8 +18,15 @@ Ctx::~Ctx() {
         for (auto &e : ev) (void)hipEventDestroy(e);
     if (ev_fork) (void)hipEventDestroy(ev_fork);
     if (ev_join) (void)hipEventDestroy(ev_join);
-    if (stream2) (void)hipStreamDestroy(stream2);
-    if (own_stream && stream) (void)hipStreamDestroy(stream);
+    if (stream2) {
+        (void)hipStreamSynchronize(stream2);
+        scan_scratch_back(stream2);
+        (void)hipStreamDestroy(stream2);
+    }
+    if (own_stream && stream) {
+        scan_scratch_back(stream); // drained by segclip_destroy
+        (void)hipStreamDestroy(stream);
+    }
 }
 namespace {
 struct PinnedStage {

@@ -211,6 +211,8 @@ void scan_inclusive_max_u32(const uint32_t *in, uint32_t *out, int64_t n, hipStr
 // two independent arrays in the launches of one scan (same results as two calls)
 void scan_exclusive_u32_2(const uint32_t *in0, uint32_t *out0, int64_t n0, uint32_t *t0, const uint32_t *in1,
                           uint32_t *out1, int64_t n1, uint32_t *t1, hipStream_t s);
+// the end of a stream of the library's own, drained: its scans' scratch goes to other streams
+void scan_scratch_back(hipStream_t s);
 // up to four independent arrays (same results as one call each, no totals)
 void scan_exclusive_u32_4(int count, uint32_t *const *inout, const int64_t *n, hipStream_t s);
 // the last value up to each position that is not zero

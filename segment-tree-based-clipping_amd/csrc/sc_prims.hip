@@ -12,6 +12,10 @@
 #include "sc_common.hpp"
 #include "sc_seg.hpp"
 
+#include <mutex>
+#include <thread>
+#include <vector>
+
 namespace sc {
 
 namespace {
@@ -316,23 +320,48 @@ template <class Op, bool INCL> __global__ __launch_bounds__(SCAN_BLOCK) void k_t
     tile_scan_body<Op, INCL>(q.in, q.out, q.n, q.sums, nullptr, q.d_total, blockIdx.x, s_data, s_wave);
 }
 
-// Per host thread and stream, intentionally never freed: releasing device
-// memory from thread-exit destructors can run after the HIP runtime has shut
-// down.  Keying by stream keeps scans queued on different streams from
-// sharing tile sums.
+// Per host thread and stream: neither scans queued on different streams nor
+// threads that share one may share tile sums.  A context gives back that of its
+// own streams when it goes, and the next new streams take it over; that of a
+// caller's stream stays (releasing device memory from thread-exit destructors
+// can run after the HIP runtime has shut down).
 struct StreamScanScratch {
+    std::thread::id thread;
     hipStream_t stream = nullptr;
+    int device = 0;
     ScanScratch<uint32_t> s32;
     ScanScratch<uint64_t> s64;
 };
 
+constexpr size_t SCAN_IDLE_MAX = 4; // kept for new streams, the rest is freed
+struct ScanPool {
+    std::mutex m;
+    std::vector<StreamScanScratch *> used, idle;
+};
+ScanPool &scan_pool() {
+    static ScanPool *p = new ScanPool();
+    return *p;
+}
+
 StreamScanScratch &stream_scratch(hipStream_t s) {
-    thread_local std::vector<StreamScanScratch *> *v = new std::vector<StreamScanScratch *>();
-    for (StreamScanScratch *p : *v)
-        if (p->stream == s) return *p;
-    StreamScanScratch *p = new StreamScanScratch();
+    ScanPool &q = scan_pool();
+    const std::thread::id me = std::this_thread::get_id();
+    std::lock_guard<std::mutex> g(q.m);
+    for (StreamScanScratch *p : q.used)
+        if (p->stream == s && p->thread == me) return *p;
+    int dev = 0;
+    SC_HIP(hipGetDevice(&dev));
+    StreamScanScratch *p = nullptr;
+    for (size_t i = 0; i < q.idle.size() && !p; ++i)
+        if (q.idle[i]->device == dev) {
+            p = q.idle[i];
+            q.idle.erase(q.idle.begin() + std::ptrdiff_t(i));
+        }
+    if (!p) p = new StreamScanScratch();
+    p->thread = me;
     p->stream = s;
-    v->push_back(p);
+    p->device = dev;
+    q.used.push_back(p);
     return *p;
 }
 
@@ -698,6 +727,23 @@ void scan_u32_set(int count, const uint32_t *const *in, uint32_t *const *out, co
 
 } // namespace
 
+void scan_scratch_back(hipStream_t s) {
+    std::vector<StreamScanScratch *> rest;
+    {
+        ScanPool &q = scan_pool();
+        std::lock_guard<std::mutex> g(q.m);
+        for (size_t i = 0; i < q.used.size();) {
+            StreamScanScratch *p = q.used[i];
+            if (p->stream != s) {
+                ++i;
+                continue;
+            }
+            q.used.erase(q.used.begin() + std::ptrdiff_t(i));
+            (q.idle.size() < SCAN_IDLE_MAX ? q.idle : rest).push_back(p);
+        }
+    }
+    for (StreamScanScratch *p : rest) delete p;
+}
 void scan_exclusive_u32(const uint32_t *in, uint32_t *out, int64_t n, uint32_t *d_total, hipStream_t s) {
     scan_u32_op<OpSum, false>(in, out, n, d_total, s);
 }
