@@ -681,6 +681,7 @@ void batch_area(Ctx &c, double *out4) {
     SC_REQUIRE(!c.uni, SC_ESTATE, "area / IoU are defined for the intersection (a union output may hold holes)");
     JobSet &js = c.jobs;
     SC_REQUIRE(js.J >= 1 && int(js.ring_off.size()) == js.J + 1, SC_ESTATE, "no clipped batch");
+    SC_REQUIRE(js.resident, SC_ESTATE, "the batch was clipped from other rings");
     hipStream_t s = c.stream;
     AreaScratch &a = ascratch(c);
     const int J = js.J;
@@ -734,7 +735,7 @@ void batch_area(Ctx &c, double *out4) {
 
 void batch_area_backward(Ctx &c, const double *g_area, const double *g_iou, double *grad_b, double *grad_c) {
     JobSet &js = c.jobs;
-    SC_REQUIRE(c.prov, SC_ESTATE, "the batch was clipped without provenance (segclip_set_provenance)");
+    SC_REQUIRE(c.prov && js.prov, SC_ESTATE, "the batch was clipped without provenance (segclip_set_provenance)");
     hipStream_t s = c.stream;
     AreaScratch &a = ascratch(c);
     const int J = js.J;

@@ -332,6 +332,8 @@ void release_derived(Ctx &c) {
     c.cur_k = 0;
     c.I = 0;
     c.pair_off.clear();
+    c.jobs.prov = c.jobs.late = false; // what labelling and gradients read is gone
+    c.jobs.AB.clear();
 }
 } // namespace sc
 

@@ -27,6 +27,8 @@ struct JobSet {
     std::vector<int> cin;      // first input vertex (no closing vertices) of each job's overlay
     std::vector<int> route, reason; // labelling route per job (0 crossing, 1 no crossing, 2 sequential), why sequential
     DBuf<int> d_AB, d_AC, d_ring;
+    bool resident = false;     // clipped from the rings that the context holds now
+    bool prov = false;         // the slots' sources are there (from_b, from_c), for the gradients
     bool late = false;         // AB and AC are still on the device (below: the most they end with)
     int64_t cap_b = 0, cap_c = 0;
     // device copies of p0, bvoff, beoff, nb, nc, cvoff, JB, JC, cin: views into

@@ -576,6 +576,8 @@ void post_jobs(Ctx &c, int k0, int k1, bool late) {
     JobSet &js = c.jobs;
     js.k0 = k0;
     js.J = J;
+    js.resident = true;
+    js.prov = c.prov;
     js.p0.assign(J + 1, 0);
     js.bvoff.resize(J);
     js.beoff.resize(J);

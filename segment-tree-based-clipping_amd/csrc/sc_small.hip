@@ -808,6 +808,8 @@ bool clip_small_batch(Ctx &c, int k0, int k1) {
     c.flags_pending = false;
     js.k0 = k0;
     js.J = J;
+    js.resident = true;
+    js.prov = false;
     js.flags.assign(size_t(J), 0);
     js.route = routes;
     js.reason.assign(size_t(J), 0);

@@ -602,6 +602,10 @@ void load(Ctx &c, const double *bxy, const int *bsz, int nbr, const double *cxy,
     c.wait(); // the caller's arrays are free on return
     c.shift_ready = false;
     reset_derived(c);
+    // the last batch's rings and status stay readable; labelling, areas and
+    // gradients would read these rings by the other ones' offsets
+    c.jobs.resident = c.jobs.prov = c.jobs.late = false;
+    c.jobs.AB.clear();
 }
 } // namespace
 
