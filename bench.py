@@ -13,7 +13,7 @@ clipped per second (N_b + N_c per step).
 Batched workloads (reported under "batched", each next to the plain per-pair
 GPU loop on a sample of the same pairs):
   one_to_many   base 100,000-vertex harmonic star against 4,096 star overlays
-                (log-uniform 8..20,000 vertices): one tree, every overlay
+                (log-uniform 8..20,000 vertices): one join, every overlay
                 clipped in one batch
   small_pairs   16,384 pairs of 4..64-vertex rings: clip + area/IoU forward
                 (the small-pair kernel; also replayed as a

@@ -149,7 +149,9 @@ int segclip_init_labels_arrays(segclip_ctx *ctx, int nb_aug, int nc_aug, const d
  * input) and grad_c (2*sum(ov_sizes), the layout of the overlay input) with
  * d/d(vertex) of sum_j g_area[j]*area[j] + g_iou[j]*iou[j], the output
  * combinatorics held fixed; g_area or g_iou may be null (zero).  Device
- * pointers, on the context's device; the call returns after its work is done. */
+ * pointers, on the context's device; the call returns after its work is done.
+ * SEGCLIP_ESTATE where the context holds other rings since, and for gradients of a
+ * batch clipped without provenance or released. */
 int segclip_set_provenance(segclip_ctx *ctx, int on);
 int segclip_batch_area(segclip_ctx *ctx, double *out4, int64_t cap, int64_t *need);
 int segclip_batch_area_device(segclip_ctx *ctx, double *out4);
@@ -167,7 +169,8 @@ int segclip_batch_area_backward_device(segclip_ctx *ctx, const double *g_area, c
  * it.  The graph is captured on the first call, again when
  * a pointer changes, and dropped by segclip_set_pairs* / set_polygons*.
  * After the replay one word is read back: when some pair needs the staged
- * path, the batch is clipped on it (areas identical either way) and the next
+ * path, the batch is clipped on it (areas identical either way, vertical edges
+ * aside: "small_fused" below) and the next
  * call captures again.  Returns when out4 is written.  No counterpart in the
  * reference (its per-pair loop launches every stage, clip:1026-1297). */
 int segclip_pairs_area_graph(segclip_ctx *ctx, const double *base_xy, const double *ov_xy, double *out4);
@@ -304,7 +307,8 @@ int segclip_get_stage_times(segclip_ctx *ctx, float *ms8);
  * (its stab runs one tree node per parallel-loop iteration, countIntersectionsParallel,
  * oacc_segment_tree.cpp:6250-6526); they serve
  * the autotuner, which times candidate values on a workload and persists the
- * fastest as JSON (segclip.tune).  Results never depend on a setting.
+ * fastest as JSON (segclip.tune).  Results do not depend on a setting, but for
+ * edges that are vertical in the tree's keys under "small_fused".
  * The two stab settings act where the tree is stabbed: segclip_find_candidates,
  * and clips that do not take the join.
  *   "stab_tiles"  64-column tiles per stab work unit, 1..16, default 2.
@@ -314,7 +318,10 @@ int segclip_get_stage_times(segclip_ctx *ctx, float *ms8);
  *                 have at most 64 vertices, without provenance, runs as one
  *                 launch, a wave per pair, each pair clipped whole in LDS; 0:
  *                 the staged path.  A batch holding a pair that this kernel
- *                 does not cover reruns on the staged path.
+ *                 does not cover reruns on the staged path.  Same results,
+ *                 but for rings with vertical edges: this kernel tests every
+ *                 pair of edges, the tree's rules can miss one that touches a
+ *                 vertical edge.
  *   "seq_parallel_walks"  1 (default): the traversal of a job on the
  *                 sequential route runs over the whole device (large jobs) or
  *                 walks its rings one per lane, and checks that they are the

@@ -183,9 +183,10 @@ struct Ctx {
     // tuning: consecutive stab work units per wave (1..32); results do not depend on it
     int stab_upw = 2;
     // independent pairs of up to 64 + 64 vertices clipped by the one-launch
-    // small-pair kernel (1) or the staged path (0); results do not depend on it
-    int uni = 0; // operation: 0 intersection, 1 union (UNION of foster/polyclip.h:39)
+    // small-pair kernel (1) or the staged path (0); the same results but for
+    // vertical edges, whose partners the tree can miss
     int small_fused = 1;
+    int uni = 0; // operation: 0 intersection, 1 union (UNION of foster/polyclip.h:39)
     // sequential-route rings walked one per lane (1) or by the single walk
     // (0); results do not depend on it
     int seq_par = 1;

@@ -182,7 +182,12 @@ __global__ void k_copy_order(const uint32_t *__restrict__ vals, int I, int *ord)
 // one launch where sizes, closing entries and their scans took five.  More jobs
 // than one chunk are gathered by as many blocks and scanned in two launches
 // (16,384 jobs: 81 us in four chunks of one block, 14 so).
-constexpr int LATE_MAX = 1 << 16; // pairs up to which launches and read-backs are saved at the price of more loads
+// Pairs up to which launches and read-backs are saved at the price of more loads:
+// a clip with 22,000 pairs takes 368 us instead of 406, with 56,000 448 instead of
+// 496.  Beyond the line it would gain less and less (106,000: 478 for 523, 473,000:
+// 609 for 630), for buffers with a spare slot per pair; with tens of millions of
+// slots the links by slot are the faster ones.
+constexpr int LATE_MAX = 1 << 16;
 constexpr int JOB_BLK = 1024, JOB_PER = 4;
 // Scanned counts of the edges' non-degenerate pairs: of all pairs less the
 // degenerate ones.  Those are few as a rule, so that a pair takes one counting

@@ -676,7 +676,9 @@ __global__ __launch_bounds__(RS_BLOCK) __attribute__((amdgpu_waves_per_eu(4))) v
 constexpr int RS_WIDE = 1024;
 __global__ __launch_bounds__(RS_WIDE) void k_onesweep_wide(SweepArgs a) { onesweep_tile<true, RS_WIDE>(a); }
 __global__ __launch_bounds__(RS_WIDE) void k_onesweep_keys_wide(SweepArgs a) { onesweep_tile<false, RS_WIDE>(a); }
-constexpr int64_t RS_WIDE_MAX = int64_t(512) * RS_TILE; // two tiles a CU
+// Two tiles a CU: a whole sort of keys and values takes 325 us instead of 340 at
+// 512 tiles, 451 instead of 440 at 768.
+constexpr int64_t RS_WIDE_MAX = int64_t(512) * RS_TILE;
 void onesweep(const SweepArgs &a, int64_t ntiles, hipStream_t s) {
     const unsigned g = unsigned(ntiles);
     if (a.n <= RS_WIDE_MAX) {

@@ -24,8 +24,9 @@
 //
 // Bound by VALU issue (FP64 predicates): 2,170 vector instructions per wave
 // for rings of 4 to 64 vertices keep the units about half busy.  16,384 such
-// pairs take 111 us; the version that linked vertices in LDS (28 KB a pair,
-// five pairs a CU) and walked them on one lane took 700.
+// pairs take 112 us where sizes are log-uniform, 160 where they are uniform; the
+// version that linked vertices in LDS (28 KB a pair, five pairs a CU) and walked
+// them on one lane took 700 on the former.
 //
 // Covered here: pairs whose intersection vertices are all labelled CROSSING
 // or BOUNCING, whose rings keep a plain vertex, with no bouncing pair to

@@ -233,7 +233,8 @@ class Clipper:
         self._check(lib().segclip_set_timing(self._h, 1 if on else 0))
 
     def set_tuning(self, name, value):
-        """A tuning setting of this context (see segclip.tune); results do not depend on it."""
+        """A tuning setting of this context (see segclip.tune); results do not depend on it,
+        but for vertical edges under "small_fused" (segclip.h)."""
         self._check(lib().segclip_set_tuning(self._h, name.encode(), int(value)))
         return self
 
